@@ -279,6 +279,46 @@ def test_gemm_partial_sums(ops, act, M, N, K, bias):
     assert err < (1e-5 * scale * math.sqrt(K) if act == "float32" else 4e-3 * scale), (err, scale)
 
 
+@pytest.mark.parametrize("M,N,K,gated", [(65, 100, 36, False), (128, 129, 64, True), (129, 2050, 2048, False), (300, 640, 516, True),
+                                         (1100, 1024, 1412, False), (2100, 2048, 96, True)])
+def test_float_products_on_the_bfloat16_instructions(ops, M, N, K, gated):
+    """Products of more than 64 rows in 32 bits, at the edges of their tiles and runs of k, with rows of very different size
+    and with values that have no split into bfloat16 parts.  Every sum is bounded by its terms: at most k roundings of
+    2^-24 of the terms' sizes added up (and 2^-26 for the products left out), of which a run of them in either direction
+    leaves far less than a quarter; what is infinite or not a number is where the formula has it."""
+    size = 10.0 ** torch.linspace(-25, 25, M)[:, None]
+    a, w, v = rnd((M, K), torch.float32, 31) * size, rnd((N, K), torch.float32, 32, 0.1), rnd((N, K), torch.float32, 33, 0.1)
+    kw = {"w2": v.to(DEV), "activation": "relu2", "out_act": True} if gated else {}
+    if gated:
+        a = a / size
+    got = ops.gemm(a.to(DEV), w.to(DEV), "float32", **kw).cpu().double()
+    x, xs = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    y, ys = (a.double() @ v.double().T, a.double().abs() @ v.double().abs().T) if gated else (None, None)
+    rel = 2.0 ** -24 * (2 + K / 4)
+    if gated:
+        up = x.clamp(min=0)
+        ref, bound = up * up * y, 3 * rel * (xs * xs * ys) + 1e-30
+    else:
+        ref, bound = x, rel * xs + 1e-38
+    assert ((got - ref).abs() <= bound).all(), ((got - ref).abs() / bound).max()
+    # not finite, and beyond the largest bfloat16: the rows that hold such a value, and no others
+    a2 = a.clone()
+    a2[0, 0], a2[M // 2, K - 1], a2[M - 1, 1] = math.inf, math.nan, 3.4e38
+    w2 = w.clone()
+    w2[:, 1] = 0.001
+    odd = ops.gemm(a2.to(DEV), w2.to(DEV), "float32", **kw).cpu()
+    near = [0, M // 2, M - 1]
+    x = a2[near].double() @ w2.double().T
+    if gated:
+        x = x.clamp(min=0) ** 2 * (a2[near].double() @ v.double().T)
+    ref = x.float()
+    assert torch.equal(torch.isnan(odd[near]), torch.isnan(ref)) and torch.equal(torch.isinf(odd[near]), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    assert torch.allclose(odd[near][fine], ref[fine], rtol=1e-4, atol=1e-30)
+    rest = [i for i in range(M) if i not in near]
+    assert torch.isfinite(odd[rest]).all()
+
+
 @pytest.mark.parametrize("act", ACTS)
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "relu2"])
 @pytest.mark.parametrize("M,N,K", [(3, 40, 72), (40, 130, 264), (150, 200, 136), (9, 33, 50)])
