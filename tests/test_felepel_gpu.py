@@ -497,3 +497,69 @@ def test_trace_runner_as_a_program(made, tmp_path):
             check(read(2 + i), wa[81 + i:82 + i], what=f"step {2 + i}")
         else:
             assert not (out / f"{2 + i}.f32").exists()
+
+
+# ------------------------------------------------------------------------------------------------ the delta rule in chunks
+@pytest.mark.parametrize("act", ["float32", "bfloat16"])
+@pytest.mark.parametrize("head_decay", [False, True])
+@pytest.mark.parametrize("lens,H,G,D,V,shift", [([49], 2, 2, 16, 16, -3.0), ([64, 33, 1, 97], 4, 2, 64, 48, -3.0),
+                                                ([31, 32, 129], 2, 1, 128, 128, 8.0), ([96, 0, 50], 3, 3, 144, 32, -3.0),
+                                                ([100], 2, 2, 256, 16, 0.0)])
+def test_the_delta_rule_in_chunks(act, head_decay, lens, H, G, D, V, shift):
+    """Long runs, in chunks of 32 tokens, against the recurrence in 64 bits: ends of chunks and of their halves, a sequence that
+    brings nothing, decays near one and near zero.  A sum is rounded a few hundred times at most on the way (products of 32
+    decays, 32 rows of the triangular system, the state's sums): 2^-24 of its size each, in both directions."""
+    from turboquant_cpp_amd.csrc import ops
+    g = torch.Generator().manual_seed(sum(lens) + D)
+
+    def rnd(*s):
+        return torch.randn(s, generator=g)
+    T, B = sum(lens), len(lens)
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)      # noqa: E731
+    qn, kn = (unit(rnd(T, G, D)) * D ** -0.5).reshape(T, -1), unit(rnd(T, G, D) + 0.3).reshape(T, -1)
+    vc, beta, a_log = rnd(T, H * V), torch.sigmoid(rnd(T, H)), 0.5 * rnd(H)
+    dims = ops.DeltaDims(H, G, D, V, 4, 0, 0, head_decay=True) if head_decay else ops.DeltaDims(H, G, D, V, 4, 8, 8)
+    state = torch.zeros(B + 1, dims.state_floats)
+    state[:, :H * D * V] = 0.1 * rnd(B + 1, H * D * V)
+    slots = torch.arange(B, dtype=torch.int32).flip(0) + 1
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    runs = {"cu_seqlens": cu.to("cuda:0"), "slots": slots.to("cuda:0"), "decode": False}
+    soft = torch.nn.functional.softplus
+    if head_decay:
+        rates = torch.exp(-torch.exp(a_log) * soft(rnd(T, H) + shift))
+        decay = rates.double()[:, :, None].expand(T, H, D)
+    else:
+        ag, dt_bias = rnd(T, H * D + H * V), 0.5 * rnd(H * D) + shift
+        decay = torch.exp(-torch.exp(a_log.double())[:, None] * soft((ag[:, :H * D] + dt_bias).double()).view(T, H, D))
+
+    def run(values, into):
+        lib = ops.library(act)
+        assert lib.tq_delta_chunk_scratch(T, B, H, D, V) > 0
+        if head_decay:
+            return ops.delta_scan_h(qn.to("cuda:0"), kn.to("cuda:0"), values.to("cuda:0"), beta.to("cuda:0"), rates.to("cuda:0"), runs, into, dims, act)
+        return ops.delta_scan(qn.to("cuda:0"), kn.to("cuda:0"), values.to("cuda:0"), beta.to("cuda:0"), ag.to("cuda:0"), a_log.to("cuda:0"), dt_bias.to("cuda:0"), runs,
+                              into, dims, act)
+    into = state.to("cuda:0")
+    o = run(vc, into).cpu().double()
+    k, q = (x.double().view(T, G, D).repeat_interleave(H // G, 1) for x in (kn, qn))
+    want, t = torch.zeros(T, H, V, dtype=torch.float64), 0
+    for b, n in enumerate(lens):
+        S = state[slots[b].item(), :H * D * V].double().view(H, D, V).clone()
+        for _ in range(n):
+            S = S * decay[t][:, :, None]
+            u = beta[t].double()[:, None] * (vc[t].double().view(H, V) - (k[t][:, None] @ S)[:, 0])
+            S = S + k[t][:, :, None] * u[:, None]
+            want[t] = (q[t][:, None] @ S)[:, 0]
+            t += 1
+        got = into[slots[b].item(), :H * D * V].cpu().double().view(H, D, V)
+        assert (got - S).abs().max() <= 4e-6 * max(S.abs().max().item(), 1.0)
+    assert (o.view(T, H, V) - want).abs().max() <= 4e-6 * want.abs().max()
+    assert torch.equal(into[0].cpu(), state[0])
+    # a value that is not a number reaches its own token and those behind it in its sequence, and nothing before it
+    first = next(i for i, n in enumerate(lens) if n > 0)
+    at = lens[first] // 2
+    spoiled = vc.clone()
+    spoiled[at, 0] = float("nan")
+    odd = run(spoiled, state.to("cuda:0")).cpu().view(T, H, V)
+    assert torch.isfinite(odd[:at]).all() and torch.isnan(odd[at, 0, 0])
+    assert torch.isfinite(odd[lens[first]:]).all() and torch.isfinite(odd[:, 1:]).all()

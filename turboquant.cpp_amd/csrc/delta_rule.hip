@@ -13,7 +13,8 @@
 //   delta_decay  (steps of many tokens) the decays of all tokens, in parallel, in place of what they are made from
 //   delta_scan   per (sequence, head, block of value channels): the recurrence over the run's tokens in order, the
 //                state in registers (16 key channels of a value channel per lane), tokens staged through two LDS
-//                buffers in chunks; a short step works out its decays as it stages them
+//                buffers in chunks; a short step works out its decays as it stages them (long runs of sizes that its
+//                tiles take go through delta_chunks.hip instead)
 //   delta_out    per token: norm and gate of every head; and per sequence: the convolution's new state
 //   delta_decode (steps of one token per sequence) the second low-rank products, decays, recurrence, norm, gate and the
 //                convolution's new state in one launch
@@ -24,28 +25,10 @@
 //
 // A sequence's row of state (float): S as [H][D][V], then for every convolution channel (q's, k's, v's) its last
 // taps - 1 inputs, oldest first.  Projections P [T][NP] (float): q (G D) | k (G D) | v (H V) | b (H) | a1 (ra) | g1 (rg).
-#include "common.h"
+#include "delta_rule.h"
 
 #define DR_ROWS 16        // key channels of a value channel that one lane keeps
 #define DR_CHUNK 16       // tokens staged at a time
-
-struct DeltaDims {
-  int H, G, D, V;         // heads, q/k heads, key width, value width
-  int taps;               // of the convolution
-  int ra, rg;             // ranks of the decay's and the gate's first product
-  int mode;               // 0: a decay per head and key channel, behind low-rank products; 1: a decay per head (ra = rg = 0)
-};
-__host__ __device__ __forceinline__ int dd_channels(const DeltaDims& d) { return 2 * d.G * d.D + d.H * d.V; }
-__host__ __device__ __forceinline__ int dd_np(const DeltaDims& d) {
-  return d.mode == 1 ? dd_channels(d) + 2 * d.H + d.H * d.V : dd_channels(d) + d.H + d.ra + d.rg;
-}
-__host__ __device__ __forceinline__ int64_t dd_state(const DeltaDims& d) {
-  return (int64_t)d.H * d.D * d.V + (int64_t)dd_channels(d) * (d.taps - 1);
-}
-
-__device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 // ------------------------------------------------------------------------------------------ per token
 // grid (T, units / 4), block 256: a wave takes one "unit" of its token: one of the G query heads, the G key heads, the H

@@ -99,6 +99,9 @@ _SIGNATURES = {
                       _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "tq_delta_scan": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int,
                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
+    "tq_delta_chunk_scratch": [_c_int, _c_int, _c_int, _c_int, _c_int],
+    "tq_delta_chunks": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int,
+                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
     "tq_delta_decode": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr,
                         _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "tq_delta_out": [_c_ptr, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int,
@@ -240,6 +243,7 @@ def library(dtype) -> ctypes.CDLL:
             f.argtypes, f.restype = sig, _c_int
     lib.tq_sample_topp_scratch.restype = _c_i64
     lib.tq_delta_state_floats.restype = _c_i64
+    lib.tq_delta_chunk_scratch.restype = _c_i64
     for fn in ("tq_attention_decode_scratch", "tq_attention_f32_scratch"):
         if hasattr(lib, fn):
             getattr(lib, fn).restype = _c_i64
@@ -1497,6 +1501,20 @@ def delta_prep(proj: torch.Tensor, slot_of_token: torch.Tensor, state: torch.Ten
     return qn, kn, vc, beta, low
 
 
+def _delta_chunks(k, qn, kn, vc, beta, ag, a_log, dt_bias, runs, state, stride, dims, T, B, o, act) -> bool:
+    """Runs the recurrence in chunks into ``o`` where the library says that this is the better form for the step; ``a_log`` None:
+    ``ag`` holds a decay per head."""
+    lib = library(act)
+    n = lib.tq_delta_chunk_scratch(T, B, dims.heads, dims.dim, dims.vdim)
+    if n == 0 or any(t.data_ptr() % 16 for t in (qn, kn, ag)):
+        return False
+    scratch = torch.empty(n, dtype=torch.float32, device=qn.device)
+    _run(k, lib.tq_delta_chunks(_ptr(qn), _ptr(kn), _ptr(vc), _ptr(beta), _ptr(ag), _ptr(a_log), _ptr(dt_bias), int(a_log is None),
+                                _ptr(runs["cu_seqlens"]), _ptr(runs["slots"]), _ptr(state), stride, *dims.sizes(), T, B,
+                                _ptr(scratch), _ptr(o), _stream()))
+    return True
+
+
 def delta_scan(qn: torch.Tensor, kn: torch.Tensor, vc: torch.Tensor, beta: torch.Tensor, ag: torch.Tensor,
                a_log: torch.Tensor, dt_bias: torch.Tensor, runs: dict, state: torch.Tensor, dims: DeltaDims, act):
     """The recurrence over each sequence's run of tokens, in order, from and into its row of ``state``:
@@ -1515,6 +1533,8 @@ def delta_scan(qn: torch.Tensor, kn: torch.Tensor, vc: torch.Tensor, beta: torch
     _check(runs["cu_seqlens"], k, "cu_seqlens", torch.int32, (B + 1,))
     _check(runs["slots"], k, "slots", torch.int32, (B,))
     o = torch.empty((T, H * V), dtype=torch.float32, device=qn.device)
+    if _delta_chunks(k, qn, kn, vc, beta, ag, a_log, dt_bias, runs, state, stride, dims, T, B, o, act):
+        return o
     _run(k, library(act).tq_delta_scan(_ptr(qn), _ptr(kn), _ptr(vc), _ptr(beta), _ptr(ag), _ptr(a_log), _ptr(dt_bias),
                                        _ptr(runs["cu_seqlens"]), _ptr(runs["slots"]), _ptr(state), stride, *dims.sizes(), T, B,
                                        _ptr(o), _stream()))
@@ -1629,6 +1649,8 @@ def delta_scan_h(qn: torch.Tensor, kn: torch.Tensor, vc: torch.Tensor, beta: tor
     stride = _delta_state(k, state, dims)
     B = _delta_runs(k, runs)
     o = torch.empty((T, H * V), dtype=torch.float32, device=qn.device)
+    if _delta_chunks(k, qn, kn, vc, beta, dec, None, None, runs, state, stride, dims, T, B, o, act):
+        return o
     _run(k, library(act).tq_delta_scan_h(_ptr(qn), _ptr(kn), _ptr(vc), _ptr(beta), _ptr(dec), _ptr(runs["cu_seqlens"]),
                                          _ptr(runs["slots"]), _ptr(state), stride, *dims.sizes(), T, B, _ptr(o), _stream()))
     return o
