@@ -42,12 +42,15 @@ __device__ __forceinline__ int split_place(int row, int q) { return row * SPK + 
 // A tile of 64 MI rows of `a` by 128 rows of w (DUAL: 64 of each matrix) by four waves of 32 MI x 64, 32 of k at a time
 // through one LDS buffer of three planes; three workgroups share a compute unit, so that one splits and stages
 // while the others multiply.  Bound by the matrix instructions at the clock that they leave: 16,385 x 2,048 times
-// 6,144 x 2,048 takes 2.21 ms, 187 TFLOP/s of float products or 1.12 PFLOP/s of bfloat16 ones, where the float
-// instructions took 3.42 ms (121 TFLOP/s; the published peak is 157); without the arithmetic of the split 2.13, so
-// that splitting w once ahead would gain little and cost half as much memory again.  Also measured: tiles of 256 rows
-// (two workgroups to a unit) 2.64 ms, steps of k fetched two ahead (two workgroups) 2.32, 16x16x32 instructions 2.83
+// 6,144 x 2,048 takes 2.25 ms, 183 TFLOP/s of float products or 1.10 PFLOP/s of bfloat16 ones, where the float
+// instructions took 3.42 ms (121 TFLOP/s; the published peak is 157); without the arithmetic of the split 4 % less, so
+// that splitting w once ahead would gain little and cost half as much memory again.  Also measured (beside 2.21):
+// tiles of 256 rows (two workgroups to a unit) 2.64 ms, steps of k fetched two ahead (two workgroups) 2.32, 16x16x32 instructions 2.83
 // (their operands and the next step's rows do not fit the registers of three workgroups).
-// Against 64 bits the sums are closer than the float instructions': 7.0e-7 of the result against 8.1e-7 at k 2,048, since
+// The bfloat16 instructions round a sum down, whatever its sign: left alone, every output ends 1.1e-7 of the result's size
+// (k 2,048) too low, a shift that all outputs share and that layers behind can carry on.  So every 128 of k the sums and
+// the rows of `a` change their sign, and what one block rounds down the next rounds up.
+// Against 64 bits the sums are closer than the float instructions': 6.9e-7 of the result against 8.1e-7 at k 2,048, since
 // k is rounded into the sum in six steps of 16 where those take eight of 2 (and runs of k make them closer still).
 template <int MI, bool DUAL>
 __global__ __launch_bounds__(256, MI == 1 ? 4 : 3) void gemm_f32_split_kernel(F32GemmArgs g, int gm, int gn, int k_per_run, float* part) {
@@ -117,6 +120,16 @@ __global__ __launch_bounds__(256, MI == 1 ? 4 : 3) void gemm_f32_split_kernel(F3
 
   const int k_first = blockIdx.z * k_per_run, k_last = min(g.K, k_first + k_per_run);
   f32x4 next[FETCH];
+  unsigned sign = 0;      // of the sums as they stand
+  auto negate = [&]() {
+    sign ^= 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = -acc[i][j][v];
+  };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   auto fetch = [&](int k0) {
     const bool in = k0 + 4 * chunk < k_last;      // K and the runs are multiples of 4
@@ -128,9 +141,13 @@ __global__ __launch_bounds__(256, MI == 1 ? 4 : 3) void gemm_f32_split_kernel(F3
 #pragma unroll 1
   for (int k0 = k_first; k0 < k_last; k0 += SPK) {
     if (k0 > k_first) __syncthreads();
+    const unsigned now = ((k0 - k_first) / (4 * SPK) & 1) << 31;
 #pragma unroll
     for (int j = 0; j < FETCH; ++j) {
       u32x2 h, m, l;
+      if (j < BM / 32)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) next[j][i] = __uint_as_float(__float_as_uint(next[j][i]) ^ now);
       split3(next[j], h, m, l);
       const int at = split_place(frow + 32 * j, chunk / 2) + 4 * (chunk % 2);
       *reinterpret_cast<u32x2*>(&lds[at]) = h;
@@ -140,6 +157,7 @@ __global__ __launch_bounds__(256, MI == 1 ? 4 : 3) void gemm_f32_split_kernel(F3
     __syncthreads();
     if (k0 + SPK < k_last) fetch(k0 + SPK);
     if (active) {
+      if (now != sign) negate();
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         bf16x8 af[MI][3], wf[2][3];
@@ -165,6 +183,7 @@ __global__ __launch_bounds__(256, MI == 1 ? 4 : 3) void gemm_f32_split_kernel(F3
     }
   }
   if (!active) return;
+  if (sign) negate();
 
   // Whether this lane has outputs in row v of block i, and those outputs from the two sums behind them (the gated pair's,
   // or of columns 32 apart).
