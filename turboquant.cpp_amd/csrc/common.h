@@ -57,15 +57,42 @@ typedef float act_t;
 
 #define TQ_WAVE 64
 
+// v and the value of lane l ^ O put together by f, for the whole wave.  In the vector unit throughout: a step of the shuffle that
+// goes through LDS takes as long as twenty additions, and a short kernel of one token is made of such chains (a sum over a wave: 60
+// clocks instead of 420).
+template <int O, class F>
+__device__ __forceinline__ float with_lane_xor(float v, F f) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "a power of two");
+  if constexpr (O >= 16) {
+    typedef unsigned two __attribute__((ext_vector_type(2)));
+    const unsigned u = __float_as_uint(v);
+    const two s = __builtin_bit_cast(two, O == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                                                  : __builtin_amdgcn_permlane16_swap(u, u, false, false));
+    return f(__uint_as_float(s.x), __uint_as_float(s.y));      // one is the lane's own value, the other its partner's
+  } else {
+    const int i = __float_as_int(v);
+    int o;
+    if constexpr (O == 8) o = __builtin_amdgcn_update_dpp(i, i, 0x128, 0xf, 0xf, false);                 // row_ror:8
+    else if constexpr (O == 4) o = __builtin_amdgcn_update_dpp(i, __builtin_amdgcn_update_dpp(i, i, 0x141, 0xf, 0xf, false), 0x1B, 0xf, 0xf, false);      // half mirror, then [3, 2, 1, 0]
+    else if constexpr (O == 2) o = __builtin_amdgcn_update_dpp(i, i, 0x4E, 0xf, 0xf, false);             // [2, 3, 0, 1]
+    else o = __builtin_amdgcn_update_dpp(i, i, 0xB1, 0xf, 0xf, false);                                   // [1, 0, 3, 2]
+    return f(v, __int_as_float(o));
+  }
+}
+template <class F>
+__device__ __forceinline__ float wave_fold(float v, F f) {
+  v = with_lane_xor<32>(v, f);
+  v = with_lane_xor<16>(v, f);
+  v = with_lane_xor<8>(v, f);
+  v = with_lane_xor<4>(v, f);
+  v = with_lane_xor<2>(v, f);
+  return with_lane_xor<1>(v, f);
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = TQ_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, TQ_WAVE);
-  return v;
+  return wave_fold(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = TQ_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, TQ_WAVE));
-  return v;
+  return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a workgroup in a fixed order: waves reduce by butterfly, wave totals are added
