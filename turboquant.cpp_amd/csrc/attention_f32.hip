@@ -63,12 +63,10 @@ __device__ __forceinline__ void to_own_row(f32x4& t0, f32x4& t1) {
 }
 
 __device__ __forceinline__ float group_max(float v) {       // over the four lanes l, l^16, l^32, l^48
-  v = fmaxf(v, __shfl_xor(v, 16, 64));
-  return fmaxf(v, __shfl_xor(v, 32, 64));
+  return with_lane_xor<32>(with_lane_xor<16>(v, LanesMax()), LanesMax());
 }
 __device__ __forceinline__ float group_sum(float v) {
-  v += __shfl_xor(v, 16, 64);
-  return v + __shfl_xor(v, 32, 64);
+  return with_lane_xor<32>(with_lane_xor<16>(v, LanesSum()), LanesSum());
 }
 
 // One tile of 64 keys for 16 queries: scores from `kf` (reads the key operand of subtile kt, chunk u), softmax

@@ -137,12 +137,10 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {      // round to n
   return __builtin_bit_cast(uint32_t, v);
 }
 __device__ __forceinline__ float group_max(float v) {     // over the four lanes that share l % 16
-  v = fmaxf(v, __shfl_xor(v, 16, 64));
-  return fmaxf(v, __shfl_xor(v, 32, 64));
+  return with_lane_xor<32>(with_lane_xor<16>(v, LanesMax()), LanesMax());
 }
 __device__ __forceinline__ float group_sum(float v) {
-  v += __shfl_xor(v, 16, 64);
-  return v + __shfl_xor(v, 32, 64);
+  return with_lane_xor<32>(with_lane_xor<16>(v, LanesSum()), LanesSum());
 }
 
 

@@ -79,20 +79,26 @@ __device__ __forceinline__ float with_lane_xor(float v, F f) {
     return f(v, __int_as_float(o));
   }
 }
-template <class F>
-__device__ __forceinline__ float wave_fold(float v, F f) {
-  v = with_lane_xor<32>(v, f);
-  v = with_lane_xor<16>(v, f);
-  v = with_lane_xor<8>(v, f);
-  v = with_lane_xor<4>(v, f);
-  v = with_lane_xor<2>(v, f);
-  return with_lane_xor<1>(v, f);
+// Over groups of L neighbouring lanes (L a power of two), from the halves down to the pairs.
+template <int L, class F>
+__device__ __forceinline__ float lanes_fold(float v, F f) {
+  if constexpr (L > 1) {
+    v = with_lane_xor<L / 2>(v, f);
+    return lanes_fold<L / 2>(v, f);
+  }
+  return v;
 }
+struct LanesSum {
+  __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct LanesMax {
+  __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
 __device__ __forceinline__ float wave_sum(float v) {
-  return wave_fold(v, [](float a, float b) { return a + b; });
+  return lanes_fold<TQ_WAVE>(v, LanesSum());
 }
 __device__ __forceinline__ float wave_max(float v) {
-  return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
+  return lanes_fold<TQ_WAVE>(v, LanesMax());
 }
 
 // Sum over a workgroup in a fixed order: waves reduce by butterfly, wave totals are added

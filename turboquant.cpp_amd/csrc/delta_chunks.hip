@@ -148,13 +148,13 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        a[j] += __shfl_xor(a[j], 16, TQ_WAVE);
-        bb[j] += __shfl_xor(bb[j], 16, TQ_WAVE);
+        a[j] = with_lane_xor<16>(a[j], LanesSum());
+        bb[j] = with_lane_xor<16>(bb[j], LanesSum());
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        a[j] += __shfl_xor(a[j], 32, TQ_WAVE);
-        bb[j] += __shfl_xor(bb[j], 32, TQ_WAVE);
+        a[j] = with_lane_xor<32>(a[j], LanesSum());
+        bb[j] = with_lane_xor<32>(bb[j], LanesSum());
       }
       if (lane < 16)
 #pragma unroll

@@ -81,8 +81,7 @@ __global__ __launch_bounds__(256) void lightning_scan_kernel(const float* __rest
         S[r] = fmaf(lam, S[r], kr[r] * val);
         acc = fmaf(S[r], qr[r], acc);
       }
-#pragma unroll
-      for (int off = L / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, TQ_WAVE);
+      acc = lanes_fold<L>(acc, LanesSum());
       if (j == 0 && live) o[(size_t)(t0 + c0 + c) * H * V + (size_t)h * V + v] = acc;
     }
   }

@@ -128,8 +128,7 @@ __global__ __launch_bounds__(256) void mm_scan_kernel(const float* __restrict__ 
         S[r] = fmaf(keep, S[r], kr[r] * val);
         acc = fmaf(S[r], qr[r], acc);
       }
-#pragma unroll
-      for (int off = L / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, TQ_WAVE);
+      acc = lanes_fold<L>(acc, LanesSum());
       if (j == 0 && live) {
         const size_t th = (size_t)(t0 + c0 + c) * H + h;
         if (norm) {
@@ -442,8 +441,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ND > 8 ? 1 
     const float* nb = chunk + (size_t)H * D * V + (size_t)h * D;
     for (int d = part; d < D; d += 4) f = fmaf(qs[t * QLD + d], nb[d], f);
     float nq = fmaf(coef[t], f, s);
-    nq += __shfl_xor(nq, 1, TQ_WAVE);
-    nq += __shfl_xor(nq, 2, TQ_WAVE);
+    nq = with_lane_xor<2>(with_lane_xor<1>(nq, LanesSum()), LanesSum());
     if (part == 0 && t < nc) den[(size_t)(t0 + c * LC_T + t) * H + h] = fmaxf(fabsf(nq), expf(-mt[t])) + MM_EPS;
   }
   if (tid == 0 && (c + 1) * LC_T >= n)

@@ -226,8 +226,7 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(const float* __restrict__
         S[r] = fmaf(keep, S[r], br[r] * val);
         acc = fmaf(S[r], cr[r], acc);
       }
-#pragma unroll
-      for (int off = L / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, TQ_WAVE);
+      acc = lanes_fold<L>(acc, LanesSum());
       if (j == 0 && live) y[((size_t)(t0 + c0 + c) * H + h) * V + v] = fmaf(skip, x, acc);
     }
   }
