@@ -319,6 +319,36 @@ def test_float_products_on_the_bfloat16_instructions(ops, M, N, K, gated):
     assert torch.isfinite(odd[rest]).all()
 
 
+@pytest.mark.parametrize("M,N,K,kind", [(65, 72, 64, "plain"), (128, 6144, 128, "plain"), (129, 4100, 192, "act"), (512, 2050, 576, "plain"),
+                                        (40, 2048, 2048, "runs"), (65, 2048, 5632, "runs"), (511, 100, 1024, "runs"),
+                                        (66, 33, 64, "pair"), (190, 5632, 256, "pair"), (500, 5632, 128, "pair"), (1000, 4099, 192, "pair")])
+def test_some_hundred_rows_of_one_matrix(ops, M, N, K, kind):
+    """Products of up to some hundred rows at the edges of their tiles (rows, columns, a k of fewer tiles than the ring has
+    stages): every rounding of a sum of K terms is at most 2^-23 of the terms' sizes added up; and the bits of the same rows
+    taken through a row index, which go in other tiles.  A last row that is not a number, which stands in for the rows
+    behind the end, reaches no other."""
+    a, w, v = rnd((M, K), torch.bfloat16, 41), rnd((N, K), torch.bfloat16, 42, 0.1), rnd((N, K), torch.bfloat16, 43, 0.1)
+    kw = {"plain": {}, "act": {"out_act": True}, "runs": {"partial_sums": True}, "pair": {"w2": v.to(DEV)}}[kind]
+    y = ops.gemm(a.to(DEV), w.to(DEV), "bfloat16", **kw).cpu()
+    x, xs = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = 2.0 ** -23 * K * xs
+    if kind == "pair":
+        z, zs = a.double() @ v.double().T, a.double().abs() @ v.double().abs().T
+        # |silu'| < 1.1 and |silu(x)| <= |x|; the gate itself is good to 2^-20 of its size
+        bound = 1.1 * bound * z.abs() + x.abs() * 2.0 ** -23 * K * zs + 2.0 ** -20 * (x * z).abs()
+        x = x * torch.sigmoid(x) * z
+    if kind == "act":
+        bound = bound + 2.0 ** -8 * x.abs()
+    got = y.double().sum(0) if kind == "runs" else y.double()
+    assert ((got - x).abs() <= bound).all(), ((got - x).abs() / bound).max()
+    if kind != "runs":
+        rows = torch.arange(M, dtype=torch.int32, device=DEV)
+        assert torch.equal(ops.gemm(a.to(DEV), w.to(DEV), "bfloat16", a_rows=rows, **kw).cpu(), y)
+    a[M - 1] = math.nan
+    odd = ops.gemm(a.to(DEV), w.to(DEV), "bfloat16", **kw).cpu()
+    assert torch.equal(odd[..., : M - 1, :], y[..., : M - 1, :]) and torch.isnan(odd[..., M - 1, :]).all()
+
+
 @pytest.mark.parametrize("act", ACTS)
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "relu2"])
 @pytest.mark.parametrize("M,N,K", [(3, 40, 72), (40, 130, 264), (150, 200, 136), (9, 33, 50)])

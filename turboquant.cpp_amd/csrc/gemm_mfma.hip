@@ -1,7 +1,7 @@
 // Matrix products out[m, n] = sum_k a[m, k] * w[n, k] on the matrix cores, bfloat16 in, float sums.
 //
-// Same contract as the plain product (gemm_generic.hip): optional bias, optional gated pair
-// gate(a w^T) * (a w2^T) (gate: silu or another activation), optional row gather and per-row-tile matrices for experts.  Two kernels:
+// Same contract as the plain product (gemm_generic.hip): optional bias, optional gated pair gate(a w^T) * (a w2^T)
+// (gate: silu or another activation), optional row gather and per-row-tile matrices for experts.  The kernels:
 //
 //  * gemm_stream_kernel, for few rows (decoding): the work is reading w once.  A wave owns 16 rows of w
 //    and streams them straight from memory into the operand registers of v_mfma_f32_16x16x32_bf16 (lane
@@ -15,6 +15,8 @@
 //    through two LDS buffers (16-byte chunks, XOR-swizzled by row so that the operand reads of
 //    v_mfma_f32_32x32x16_bf16 do not collide); while one buffer is multiplied the next tile is written into
 //    the other and the one after that is on its way from memory.
+//  * gemm_few_tiles_kernel and gemm_ring_kernel, for up to some hundred rows of one matrix and for experts with many
+//    rows: smaller or taller tiles through rings of LDS buffers, the same sums.
 //
 // Operand layouts (wave of 64 lanes): 16x16x32: A lane l = row l%16, k 8*(l/16)..+7; B lane l = column l%16,
 // same k; D lane l = column l%16, rows 4*(l/16)+v, v<4.  32x32x16: A lane l = row l%32, k 8*(l/32)..+7;
@@ -308,8 +310,9 @@ __global__ __launch_bounds__(512) void qkv_rope_write_kernel(MfmaGemmArgs g, Rop
 
 // ------------------------------------------------------------------------------------------ many rows
 // grid (row tiles of BM, ceil(N / BN)); block of 8 waves laid WM x WN over the tile of BM x BN outputs (BN = 128
-// unless said): BM = 128 as 4 x 2 (a wave owns 32 x 64 outputs, or 32 x 96 with BN = 192; the experts' gated pair as
-// 2 x 4, 64 x 32 of each of its two products), BM = 256 as 4 x 2 (64 x 64 or 64 x 96), BM = 64 as 2 x 4 (32 x 32).  Eight waves beat four here: twice the waves hide twice the latency.
+// unless said): BM = 128 as 4 x 2 (a wave owns 32 x 64 outputs, or 32 x 96 with BN = 192; the experts' gated pair as 2
+// x 4, 64 x 32 of each of its two products), BM = 256 as 4 x 2 (64 x 64 or 64 x 96), BM = 64 as 2 x 4 (32 x 32).
+// Eight waves beat four here: twice the waves hide twice the latency.
 #define TBN 128
 // Most LDS for the sums of the waves that split k: 128 KB lets the gated pair of 64 rows have 8 waves (22.7 us for the
 // shared expert at 64 rows against 25.1 with 4).
@@ -668,6 +671,105 @@ __global__ __launch_bounds__(1024) void gemm_ring_kernel(MfmaGemmArgs g) {
   }
 }
 
+// ------------------------------------------------------------------------------------------ a few hundred rows, one matrix
+// Tiles of 64 x 32 WN outputs by 2 x WN waves of 32 x 32 each (of either matrix of a gated pair), 64 of k at a time.
+// Such a product has a workgroup or two per compute unit, and its time is the steps of one of them: the tile kernel
+// takes 0.8 us a step here (load, wait, store into LDS, barrier, and every product behind its own reads), for 64 x 128
+// outputs, so that 97 rows by 6,144 x 2,048 kept 96 compute units busy for 26 us.  Here the tiles are smaller where
+// that fills the chip, go from memory straight into a ring of S stages of LDS, S - 1 of them on their way while one is
+// multiplied (as in the ring kernel above), and a wave asks for all the operands of a step at once: 14.5 us, 0.4 us a
+// step.  With the operands read one product at a time, as the compiler puts it by itself: 15.7; two tiles of 64 to a
+// step: 15.9. The sums of an output run over k as in the tile kernel: same bits.
+template <int WN, bool DUAL, bool OUT_ACT, int S>
+__global__ __launch_bounds__(128 * WN) void gemm_few_tiles_kernel(MfmaGemmArgs g) {
+  constexpr int NT = 128 * WN, BM = 64, BN = 32 * WN, ROWS = BM + BN * (DUAL ? 2 : 1), STAGE = ROWS * TBK, L = ROWS * 8 / NT;
+  static_assert(ROWS * 8 % NT == 0 && (S - 2) * L < 16 && S >= 2, "ring");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  bf16_t* ring = (bf16_t*)smem;
+  // a die gets a contiguous run of tiles, a column's row tiles one after the other
+  int tile_m, tile_n;
+  {
+    const int gx = gridDim.x, total = gx * gridDim.y, id = blockIdx.y * gx + blockIdx.x;
+    const int die = id % 8, q = total / 8, rem = total % 8;
+    const int logical = die * q + min(die, rem) + id / 8;
+    tile_m = logical % gx;
+    tile_n = logical / gx;
+  }
+  const int k_lo = blockIdx.z * g.k_per, steps = (min(g.K, k_lo + g.k_per) - k_lo) / TBK;
+  if (blockIdx.z) {
+    g.out = (float*)g.out + blockIdx.z * g.split_stride;
+    g.bias = nullptr;
+  }
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wm = wave / WN, wn = wave % WN;
+  // What this thread asks for of each stage: the chunk that belongs at place tid % 8 of rows tid / 8 + i NT / 8.  Rows past the
+  // end read the last row instead: those outputs are never stored.
+  const bf16_t* src[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int row = tid / 8 + i * (NT / 8), chunk = (tid % 8) ^ ((row >> 1) & 7);
+    const bf16_t* from = row < BM        ? g.a + (size_t)min(m0 + row, g.M - 1) * g.lda
+                         : row < BM + BN ? g.w + (size_t)min(n0 + row - BM, g.N - 1) * g.K
+                                         : g.w2 + (size_t)min(n0 + row - BM - BN, g.N - 1) * g.K;
+    src[i] = from + k_lo + chunk * 8;
+  }
+  auto issue = [&](int stage, int step) {
+#pragma unroll
+    for (int i = 0; i < L; ++i) load_to_lds16(src[i] + step * TBK, ring + stage * STAGE + (i * (NT / 8) + wave * 8) * TBK);
+  };
+  f32x16 acc, acc2;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f, acc2[v] = 0.f;
+  for (int s = 0; s < S - 1 && s < steps; ++s) issue(s, s);
+  const int lr = lane % 32, lc = lane / 32;
+  int cur = 0;
+  for (int t = 0; t < steps; ++t) {
+    // tile t is in LDS once no more loads of this wave are on their way than those of the tiles behind it
+    if (steps - 1 - t >= S - 2)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (S - 2) * L);
+    else
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+    // every wave's share of tile t has landed and every wave is through with tile t - 1, whose stage tile t + S - 1 takes
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + S - 1 < steps) {
+      int nxt = cur + S - 1;
+      if (nxt >= S) nxt -= S;
+      issue(nxt, t + S - 1);
+    }
+    const bf16_t* Ac = ring + cur * STAGE;
+    const bf16_t* Wc = Ac + BM * TBK;
+    const bf16_t* Vc = Wc + BN * TBK;
+    // all reads of the step first: with one or two waves to a SIMD nothing else hides the way through LDS
+    u32x4 af[TBK / 16], wf[TBK / 16], vf[TBK / 16];
+#pragma unroll
+    for (int j = 0; j < TBK / 16; ++j) {
+      af[j] = *reinterpret_cast<const u32x4*>(Ac + swz(wm * 32 + lr, 2 * j + lc));
+      wf[j] = *reinterpret_cast<const u32x4*>(Wc + swz(wn * 32 + lr, 2 * j + lc));
+      if (DUAL) vf[j] = *reinterpret_cast<const u32x4*>(Vc + swz(wn * 32 + lr, 2 * j + lc));
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < TBK / 16; ++j) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[j]), __builtin_bit_cast(bf16x8, wf[j]), acc, 0, 0, 0);
+      if (DUAL)
+        acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[j]), __builtin_bit_cast(bf16x8, vf[j]), acc2, 0, 0, 0);
+    }
+    if (++cur == S) cur = 0;
+  }
+  const int n = n0 + wn * 32 + lr;
+  if (n >= g.N) return;
+  const float b = bias_at(g, n);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int m = m0 + wm * 32 + 8 * (v / 4) + 4 * lc + (v % 4);
+    if (m >= g.M) continue;
+    store_out<OUT_ACT>(g, m, n, DUAL ? gated_pair(acc[v] + b, acc2[v], g.gate, g.limit) : acc[v] + b);
+  }
+}
+
 // ------------------------------------------------------------------------------------------ launch
 // Waves that split k in the streaming kernel: a power of two, enough for about 2048 waves on the chip when one
 // matrix is multiplied and for about 256 per matrix when there is one per expert, each wave keeping at least 256 of
@@ -733,6 +835,34 @@ static int launch_tile(const MfmaGemmArgs& g, bool dual, bool out_act, int split
   return 0;
 }
 
+template <int WN, int S, bool DUAL>
+static int launch_few_tiles(const MfmaGemmArgs& g, bool out_act, int splits, hipStream_t st) {
+  const dim3 grid((g.M + 63) / 64, (g.N + 32 * WN - 1) / (32 * WN), splits);
+  const size_t shmem = (size_t)S * (64 + 32 * WN * (DUAL ? 2 : 1)) * TBK * sizeof(bf16_t);
+  const auto kernel = out_act ? gemm_few_tiles_kernel<WN, DUAL, true, S> : gemm_few_tiles_kernel<WN, DUAL, false, S>;
+  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
+    return TQ_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kernel, grid, dim3(128 * WN), shmem, st, g);
+  return 0;
+}
+
+// Which of its tiles a product of gemm_few_tiles_kernel takes.  Narrow ones, with a deep ring, while there is at most
+// one to a compute unit: then what counts is how soon a tile is done (97 rows by 6,144 x 2,048: 14.5 us against 19.2
+// in wide ones and 26.0 in the tile kernel).  More of them take wide tiles, which read `a` half as often (320 rows:
+// 20.2 against 22.3, tile kernel 26.1).  A gated pair has two matrices' tiles in a stage and so fewer stages (97 rows
+// by twice 5,632 x 2,048: 23.5 us, tile kernel 35.6; 320 rows in wide ones 30.8, 35.7), and where its tiles are many,
+// rings of two stages that leave room for three narrow or two wide tiles on a compute unit: 512 rows 47 in narrow
+// ones, 57 in wide ones of three stages, 61 in the tile kernel; 320 rows by twice 20,480 x 3,584, more than three
+// narrow ones to a unit: 157 in wide ones, 176 in narrow ones, tile kernel 174.
+static int launch_few_tiles(const MfmaGemmArgs& g, bool dual, bool out_act, int splits, hipStream_t st) {
+  const int64_t narrow = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * splits;
+  if (!dual) return narrow <= 256 ? launch_few_tiles<2, 4, false>(g, out_act, splits, st) : launch_few_tiles<4, 3, false>(g, out_act, splits, st);
+  if (narrow <= 256) return launch_few_tiles<2, 3, true>(g, out_act, splits, st);
+  if (narrow <= 512) return launch_few_tiles<4, 3, true>(g, out_act, splits, st);
+  if (narrow <= 768) return launch_few_tiles<2, 2, true>(g, out_act, splits, st);
+  return launch_few_tiles<4, 2, true>(g, out_act, splits, st);
+}
+
 // grid (units of 64 rows: at most so many items, tiles of 256 columns: 128 of a gated pair)
 static int launch_ring(const MfmaGemmArgs& g, bool dual, bool out_act, hipStream_t st) {
   const int cols = dual ? 128 : 256;
@@ -757,6 +887,15 @@ static int launch_ring(const MfmaGemmArgs& g, bool dual, bool out_act, hipStream
 // tiles of 128 columns (a vocabulary).  The tiles read `a` through LDS once per 128 columns, the streaming kernel
 // once per 32 (measured at 151,936 x 2,048 and 64 rows: 159 us against 466 with 16 columns a wave).
 static bool wide_enough_for_tiles(int N) { return (N + TBN - 1) / TBN >= 512 && (N + TBN - 1) / TBN <= 65535; }
+
+// Whether a product in tiles of 64 rows goes to gemm_few_tiles_kernel rather than the tile kernel: rows that follow
+// one another, k in whole tiles, and up to 512 rows (512 by 2,048 x 5,632: 26.6 us against 27.8; 768 rows: 39.7
+// against 38.0), of a very wide matrix up to 128 (128 by 65,536 x 1,024: 49.7 against 53.1; 512 rows: 160 against
+// 151).  A gated pair up to 1,024 (twice 5,632 x 2,048: 86 against 120; 20,480 x 3,584: 422 against 438).
+static bool few_tiles_suit(const MfmaGemmArgs& g, bool dual) {
+  const int most = dual ? 1024 : wide_enough_for_tiles(g.N) ? 128 : 512;
+  return !g.a_rows && g.K % TBK == 0 && g.M <= most;
+}
 
 // Which tile a plain product of many rows takes: 128 x 128, 128 x 192, 256 x 128 or 256 x 192 outputs (0..3).  The
 // larger the tile, the fewer bytes pass through LDS per multiply-add (measured on products that fill the chip
@@ -843,14 +982,13 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
   return s;
 }
 
-// a: bfloat16 [.., K] with row stride lda (a multiple of 8, as K must be); w, w2: bfloat16.
-// tile_rows: with tile_group set, the padding unit of the row order (16, 32, 64, 128 or 256); else a hint that is
-// ignored.  64 + TQ_TILE_PAIRS: units of 64 taken two at a time, by the items that the row order lists behind its
-// row tiles (tile_group[M / 64 ..], n_tiles[1]).
-// splits > 1 (as tq_gemm_mfma_splits says, for a plain product into float): run z of k goes to out + z * M * ldc,
-// the bias to run 0; the sum over the runs is the caller's.
-// gate: the activation of the gated pair; without w2 and with TQ_GEMM_ACT_ALONE added, the activation that the plain
-// product's result (bias included) passes before it is stored (a feed-forward of two matrices needs no launch between them).
+// a: bfloat16 [.., K] with row stride lda (a multiple of 8, as K must be); w, w2: bfloat16. tile_rows: with tile_group
+// set, the padding unit of the row order (16, 32, 64, 128 or 256); else a hint that is ignored.  64 + TQ_TILE_PAIRS:
+// units of 64 taken two at a time, by the items that the row order lists behind its row tiles (tile_group[M / 64 ..],
+// n_tiles[1]). splits > 1 (as tq_gemm_mfma_splits says, for a plain product into float): run z of k goes to out + z *
+// M * ldc, the bias to run 0; the sum over the runs is the caller's. gate: the activation of the gated pair; without
+// w2 and with TQ_GEMM_ACT_ALONE added, the activation that the plain product's result (bias included) passes before it
+// is stored (a feed-forward of two matrices needs no launch between them).
 TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gather, const void* w, const void* w2,
                         int64_t group_stride, const int* tile_group, const int* n_tiles, const void* bias,
                         int bias_type, void* out, int64_t ldc, int out_is_act, int M, int N, int K, int tile_rows,
@@ -907,17 +1045,20 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
     }
   } else if (M <= 16) {
     rc = launch_stream<1>(g, dual, out_act, 1, st);
-  } else if (M <= 64 && wide_enough_for_tiles(N)) {
-    rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);
-  } else if (M <= 64 && splits > 1 && few_rows_in_tiles(M, N, K)) {
-    rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);
+  } else if (M <= 64 && (wide_enough_for_tiles(N) || (splits > 1 && few_rows_in_tiles(M, N, K)))) {
+    if (few_tiles_suit(g, dual))
+      rc = launch_few_tiles(g, dual, out_act, splits, st);
+    else
+      rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);
   } else if (M <= 32) {
     rc = launch_stream<2>(g, dual, out_act, 1, st, splits);
   } else if (M <= 64) {
     rc = launch_stream<4>(g, dual, out_act, 1, st, splits);
   } else {
     if ((N + TBN - 1) / TBN > 65535) return TQ_ERR_UNSUPPORTED;
-    if (M <= 64 * 16 && !dual)
+    if (few_tiles_suit(g, dual))
+      rc = launch_few_tiles(g, dual, out_act, splits, st);
+    else if (M <= 64 * 16 && !dual)
       rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);
     else if (dual && gated_pair_in_tiles_of_64(M, N))
       rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);
@@ -950,12 +1091,12 @@ TQ_API int tq_gemm_mfma_pair_splits(int N1, int K1, int grouped1, int N2, int K2
   return (K2 + k_per - 1) / k_per;
 }
 
-// Two products of few rows in one launch.  d1, d2: 20 numbers each, in the order of tq_gemm_mfma's arguments from
-// `a` to `tile_rows`, then the gate's activation and the bits of the gated pair's limit as a float (0: none).  Both must be products that the streaming kernel takes 16 rows at a time (a matrix per
-// expert with tile_rows 16, or one matrix with M <= 16), both gated or both not, both into the same type.  The
-// waves that split k are those of the first product (the larger one by convention).  splits2 > 1 (as
-// tq_gemm_mfma_pair_splits says, for a plain second product into float): run z of its k goes to
-// out + z * M * ldc, the bias to run 0.
+// Two products of few rows in one launch.  d1, d2: 20 numbers each, in the order of tq_gemm_mfma's arguments from `a`
+// to `tile_rows`, then the gate's activation and the bits of the gated pair's limit as a float (0: none).  Both must
+// be products that the streaming kernel takes 16 rows at a time (a matrix per expert with tile_rows 16, or one matrix
+// with M <= 16), both gated or both not, both into the same type.  The waves that split k are those of the first
+// product (the larger one by convention).  splits2 > 1 (as tq_gemm_mfma_pair_splits says, for a plain second product
+// into float): run z of its k goes to out + z * M * ldc, the bias to run 0.
 TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, hipStream_t st) {
   MfmaGemmArgs g[2];
   int row_tiles[2];
