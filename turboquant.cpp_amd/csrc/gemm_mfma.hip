@@ -940,9 +940,10 @@ static bool gated_pair_in_tiles_of_64(int M, int N) {
 // (64 rows by 2,048 x 2,048: 13.4 us in two runs against 15.2 in one; by 2,048 x 5,632: 17.3 in four against 20.7
 // in two); from 33 rows on the tile kernel with its runs instead, where it may split k.  1 for up to 16 rows.
 // Runs of k for a product that goes in tiles of 64 rows (up to 1,024 rows): a workgroup's time is its steps over k
-// (about 0.6 us each, whatever the memory does), so up to 8 runs, each at least 256 long, while the workgroups stay
+// (about 0.6 us each in the tile kernel, whatever the memory does), so up to 8 runs, each at least 256 long, while the workgroups stay
 // within two to a compute unit and the partial sums within 8 MB, which the kernel behind has to read (128 rows by
-// 2,048 x 2,048: 8.7 us in eight runs against 14.6 in two; by 2,048 x 5,632: 13.7 against 19.3 in four).
+// 2,048 x 2,048: 8.7 us in eight runs against 14.6 in two; by 2,048 x 5,632: 13.7 against 19.3 in four; in the smaller
+// tiles of gemm_few_tiles_kernel the eight runs take 7.9 and 12.3).
 static int tile_runs(int M, int N, int K) {
   const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((N + TBN - 1) / TBN);
   int t = 1;
@@ -954,7 +955,7 @@ static int tile_runs(int M, int N, int K) {
 
 // Whether partial sums of 33 to 64 rows come from the tile kernel rather than the streaming one: where the tile
 // kernel may split k at all.  Its one row tile then has up to eight runs of k to the streaming kernel's two to four
-// (64 rows by 2,048 x 2,048: 7.9 us against 13.1; by 2,048 x 5,632: 12.9 against 17.0; by 3,584 x 20,480: 46 against
+// (64 rows by 2,048 x 2,048: 7.2 us against 13.1; by 2,048 x 5,632: 10.1 against 17.0; by 3,584 x 20,480: 34 against
 // 62).
 // From 17 to 32 rows it is level (2,048 x 2,048: 6.7 to 7.6 us against 7.8 to 8.7; 2,048 x 5,632: 11.9 to 12.7 against
 // 10.6 to 11.8), and the streaming kernel's fewer runs are less for the next kernel to add.
