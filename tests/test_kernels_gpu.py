@@ -281,11 +281,11 @@ def test_gemm_partial_sums(ops, act, M, N, K, bias):
 
 @pytest.mark.parametrize("M,N,K,gated", [(65, 100, 36, False), (128, 129, 64, True), (129, 2050, 2048, False), (300, 640, 516, True),
                                          (1100, 1024, 1412, False), (2100, 2048, 96, True)])
-def test_float_products_on_the_bfloat16_instructions(ops, M, N, K, gated):
-    """Products of more than 64 rows in 32 bits, at the edges of their tiles and runs of k, with rows of very different size
-    and with values that have no split into bfloat16 parts.  Every sum is bounded by its terms: at most k roundings of
-    2^-24 of the terms' sizes added up (and 2^-26 for the products left out), of which a run of them in either direction
-    leaves far less than a quarter; what is infinite or not a number is where the formula has it."""
+def test_float_products_of_many_rows(ops, M, N, K, gated):
+    """Products of more than 64 rows in 32 bits, at the edges of their tiles, with rows of very different size and with values
+    beyond the largest bfloat16.  Every sum is bounded by its terms: at most k roundings of 2^-24 of the terms' sizes added
+    up, of which a run of them in either direction leaves far less than a quarter; what is infinite or not a number is where
+    the formula has it."""
     size = 10.0 ** torch.linspace(-25, 25, M)[:, None]
     a, w, v = rnd((M, K), torch.float32, 31) * size, rnd((N, K), torch.float32, 32, 0.1), rnd((N, K), torch.float32, 33, 0.1)
     kw = {"w2": v.to(DEV), "activation": "relu2", "out_act": True} if gated else {}
@@ -317,6 +317,57 @@ def test_float_products_on_the_bfloat16_instructions(ops, M, N, K, gated):
     assert torch.allclose(odd[near][fine], ref[fine], rtol=1e-4, atol=1e-30)
     rest = [i for i in range(M) if i not in near]
     assert torch.isfinite(odd[rest]).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 72, 36), (128, 640, 2048), (300, 129, 1408), (1100, 1024, 2048)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_float_products_are_summed_in_float(ops, M, N, K, gated):
+    """Products of more than 64 rows in 32 bits keep every bit of their operands.  Of the roundings of a sum of K terms, the one
+    behind k terms is at most 2^-24 of the sum so far, which is about sqrt(k / K) of the result: their root mean square is at
+    most sqrt(K / 2) 2^-24 of the results' (operands of 16 bits instead of 24 leave twice that at k 2,048 and more below),
+    and since they go to the nearest their mean is none: at most a quarter of 2^-24 (sums that are rounded down are 1.8 times
+    2^-24 too low at k 2,048).  Operands of 2^-118, whose lower parts no number of 8 bits holds, lose nothing either."""
+    a, w, v = rnd((M, K), torch.float32, 131), rnd((N, K), torch.float32, 132, 0.1), rnd((N, K), torch.float32, 133, 0.1)
+    for scale in (1.0, 2.0 ** -118):
+        got = ops.gemm((a * scale).to(DEV), w.to(DEV), "float32").cpu().double() / scale
+        ref = a.double() @ w.double().T
+        err, size = got - ref, ref.square().mean().sqrt().item()
+        assert err.square().mean().sqrt().item() <= math.sqrt(K / 2) * 2.0 ** -24 * size
+        assert abs(err.mean().item()) <= 0.25 * 2.0 ** -24 * size + 4 * err.std().item() / math.sqrt(M * N)
+    if gated:
+        # the gated pair's two sums are those of the plain products: four roundings behind them
+        x, y = (ops.gemm(a.to(DEV), m.to(DEV), "float32").cpu().double() for m in (w, v))
+        pair = ops.gemm(a.to(DEV), w.to(DEV), "float32", w2=v.to(DEV), activation="relu2", out_act=True).cpu().double()
+        ref = x.clamp(min=0).square() * y
+        assert ((pair - ref).abs() <= 4 * 2.0 ** -24 * ref.abs() + 1e-37).all()
+
+
+def test_a_rows_float_sums_are_the_same_beside_any_other_rows(ops):
+    """A product of more than 64 rows in 32 bits sums a row over k in one order, the same however many rows there are and in an
+    expert's tiles of 64 rows, taken two at a time or one by one: the same bits."""
+    M, N, K = 1100, 264, 1408
+    a, w = rnd((M, K), torch.float32, 134).to(DEV), rnd((N, K), torch.float32, 135, 0.1).to(DEV)
+    whole = ops.gemm(a, w, "float32")
+    for rows in (65, 128, 129, 577):
+        assert torch.equal(ops.gemm(a[:rows], w, "float32"), whole[:rows])
+    st, slot, te, nt = ops.moe_align(torch.zeros((577, 1), dtype=torch.int32, device=DEV), 1, 64, "float32")
+    for unit in (64, 64 + 1024):
+        y = ops.gemm(a, w[None], "float32", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=unit)
+        assert torch.equal(y[slot.view(-1).long()], whole[:577])
+
+
+def test_float_expert_tiles_without_their_number(ops):
+    """The C entry takes every row tile where no number of live ones is given, and a last tile of fewer than 64 rows."""
+    M, N, K = 100, 40, 72
+    a, w = rnd((M, K), torch.float32, 136).to(DEV), rnd((2, N, K), torch.float32, 137).to(DEV)
+    rows, group = torch.arange(M, dtype=torch.int32, device=DEV), torch.tensor([1, 0], dtype=torch.int32, device=DEV)
+    out = torch.full((M, N), math.nan, device=DEV)
+    lib = ops.library("float32")
+    ops._run("gemm", lib.tq_gemm_f32(a.data_ptr(), K, rows.data_ptr(), 1, w.data_ptr(), None, N * K, group.data_ptr(), None, None, 0,
+                                     out.data_ptr(), N, M, N, K, 64, 0, None, 0, ops._stream()))
+    ref = torch.cat([a[:64].cpu().double() @ w[1].cpu().double().T, a[64:].cpu().double() @ w[0].cpu().double().T])
+    assert (out.cpu().double() - ref).abs().max().item() < 2e-5 * ref.abs().max().item()
+
 
 
 @pytest.mark.parametrize("M,N,K,kind", [(65, 72, 64, "plain"), (128, 6144, 128, "plain"), (129, 4100, 192, "act"), (512, 2050, 576, "plain"),

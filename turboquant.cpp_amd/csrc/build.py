@@ -22,10 +22,10 @@ COMMON_SOURCES = ["elementwise.hip", "gemm_generic.hip", "attention_generic.hip"
                   "lightning.hip", "matrix_memory.hip", "add_layernorm.hip", "token_gate.hip", "attention_prep.hip", "ssd.hip",
                   "host/engine.cpp", "host/vendor.cpp"]
 SOURCES = {
-    "float32": COMMON_SOURCES + ["gemm_f32.hip", "gemm_f32_split.hip", "attention_f32.hip"],
+    "float32": COMMON_SOURCES + ["gemm_f32.hip", "attention_f32.hip"],
     "bfloat16": COMMON_SOURCES + ["gemm_mfma.hip", "attention_mfma.hip", "probe.hip"],
 }
-HEADERS = ["common.h", "value_tiles.h", "linear_chunks.h", "score_mod.h", "gates.def", "no_alloc.h", "gemm_mfma.h", "gemm_f32.h", "delta_rule.h", "turboquant_kernels.h", "host/engine.h", "host/vendor.h",
+HEADERS = ["common.h", "value_tiles.h", "linear_chunks.h", "score_mod.h", "gates.def", "no_alloc.h", "gemm_mfma.h", "delta_rule.h", "turboquant_kernels.h", "host/engine.h", "host/vendor.h",
            "host/host_common.h"]
 DEFINES = {"float32": "-DTQ_ACT_F32", "bfloat16": "-DTQ_ACT_BF16"}
 FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-fno-gpu-rdc",

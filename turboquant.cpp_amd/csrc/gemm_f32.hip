@@ -4,14 +4,13 @@
 // inputs), at twice the rate that the vector unit reaches without packed instructions.  Same contract as the plain
 // product (gemm_generic.hip): optional bias, optional gated pair gate(a w^T) * (a w2^T), optional row gather and
 // per-row-tile matrices for experts; the reference's counterpart is its float matvec
-// (/root/reference/src/engine/tq_ops.c:296-343).  Two kernels here, and gemm_f32_split.hip for more than 64 rows and for
-// experts' units of 64 rows, where multiply-adds bound the product and the bfloat16 instructions make them faster:
+// (/root/reference/src/engine/tq_ops.c:296-343).  Two kernels:
 //
-//  * gemm_f32_tile_kernel, for 17 to 64 rows (a decode step of many sequences): one row of tiles of 64 rows by 128 columns
-//    by four waves, 16 of k at a time through two LDS buffers (rows padded to 20 floats, so that the 16-byte operand
-//    reads of eight neighbouring rows fall on all banks); while one buffer is multiplied the next tile is on its way from
-//    memory.  Multiply-adds and bytes of w are in balance there; a narrow matrix is cut into runs of k so that the chip
-//    has enough workgroups.
+//  * gemm_f32_tile_kernel, for more than 16 rows: tiles of 64 or 128 rows by 128 columns by four waves, 16 of k
+//    at a time through two LDS buffers (rows padded to 20 floats, so that the 16-byte operand reads of eight
+//    neighbouring rows fall on all banks); while one buffer is multiplied the next tile is on its way from memory.
+//    17 to 64 rows (a decode step of many sequences) are one row of tiles, at which multiply-adds and bytes of w
+//    are in balance; a narrow matrix is cut into runs of k so that the chip has enough workgroups.
 //  * gemm_f32_stream_kernel, for few rows (decoding; experts that few tokens chose): the work is reading w once.
 //    A workgroup owns 32 rows of w (every row of `a` that a wave fetches multiplies all of them), its four waves split k
 //    and add their sums in wave order through LDS; the rows of w go from memory straight into the operand
@@ -26,7 +25,34 @@
 // Operand layouts (wave of 64 lanes): 32x32x2: A lane l = row l%32, k l/32; B lane l = column l%32, k l/32; D lane l =
 // column l%32, rows 8*(v/4) + 4*(l/32) + v%4, v<16.  16x16x4: A lane l = row l%16, k l/16; B alike; D lane l = column
 // l%16, rows 4*(l/16) + v, v<4.
-#include "gemm_f32.h"
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+struct F32GemmArgs {
+  const float* a;
+  int64_t lda;
+  const int* a_rows;       // row of `a` that feeds output row m (-1: none), or null for m itself
+  int a_gather;            // 0: a_rows only marks live rows (>= 0) and row m itself is read
+  const float* w;          // [groups][N][K]
+  const float* w2;         // second matrix of the gated pair, or null
+  int64_t group_stride;
+  const int* tile_group;   // group of each row tile, or null (group 0)
+  const int* n_tiles;      // number of live row tiles on the device, or null (all)
+  const void* bias;
+  int bias_type;
+  float* out;
+  int64_t ldc;
+  int M, N, K;
+  int gate;                // activation of the gated pair
+  float limit;             // of the gated pair (gated_pair in common.h); 0: none
+};
+
+__device__ __forceinline__ float f32_bias_at(const F32GemmArgs& g, int n) {
+  if (!g.bias) return 0.f;
+  return g.bias_type == TQ_F32 ? ((const float*)g.bias)[n] : to_f32(((const bf16_t*)g.bias)[n]);
+}
 
 // Row of `a` behind output row m, or null.
 __device__ __forceinline__ const float* f32_row_of(const F32GemmArgs& g, int m) {
@@ -46,15 +72,18 @@ __device__ __forceinline__ const float* f32_row_of(const F32GemmArgs& g, int m) 
 
 // With `part` set the grid's z cuts k into runs of k_per_split and the sums of run z go to part[z] ([run][M][N], the
 // gated pair's second product behind all the first ones) as they are: gemm_f32_reduce_kernel finishes them.
-template <bool DUAL>
+template <int MI, bool DUAL>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k_per_split, float* part) {
-  constexpr int MI = 1, NI = 2, BM = 64 * MI, BN = 64 * NI;
+  constexpr int NI = 2, BM = 64 * MI, BN = 64 * NI;
   __shared__ __align__(16) float As[2][BM * TLD];
   __shared__ __align__(16) float Ws[2][BN * TLD];
   __shared__ __align__(16) float Vs[2][DUAL ? BN * TLD : 4];
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const float* w = g.w;
-  const float* w2 = g.w2;
+  const int tile_m = blockIdx.x, tile_n = blockIdx.y;
+  if (g.n_tiles && tile_m >= g.n_tiles[0]) return;
+  const int group = g.tile_group ? g.tile_group[tile_m] : 0;
+  const float* w = g.w + (size_t)group * g.group_stride;
+  const float* w2 = DUAL ? g.w2 + (size_t)group * g.group_stride : nullptr;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int wave_m = wave / 2, wave_n = wave % 2;
   const int lrow = tid / 4, lchunk = tid % 4;      // what this thread fetches of a tile: rows lrow + 64 j, 4 of k
@@ -394,22 +423,20 @@ static int f32_runs_of_k(int N, int K, int* k_per_split) {
 }
 TQ_API int tq_gemm_f32_runs(int M, int N, int K, int grouped) {
   int per;
-  if (grouped) return 1;
-  return M > 64 ? f32_split_runs(M, N, K, &per) : f32_runs_of_k(N, K, &per);      // (grouped: also a product whose rows are gathered)
+  return (grouped || M > 64) ? 1 : f32_runs_of_k(N, K, &per);      // (grouped: also a product whose rows are gathered)
 }
 
 // tile_rows: 16 or 64 rows of output per row tile; with tile_group set it is the padding unit that the row order
-// was built with, and 64 + TQ_TILE_PAIRS says that units of 64 are taken two at a time, by the items that the row order
-// lists behind its row tiles.  K must be a multiple of 4 and every row of a, w and w2 must start at a multiple of 16 bytes.
-// scratch: for a plain product, tq_gemm_f32_runs(M, N, K, 0) * M * N floats (twice that for a gated pair), unless that
-// number is 1.  keep_runs (plain products into which no second matrix goes): `out` is
+// was built with.  K must be a multiple of 4 and every row of a, w and w2 must start at a multiple of 16 bytes.
+// scratch: for a plain product of up to 64 rows, tq_gemm_f32_runs(M, N, K, 0) * M * N floats (twice that for a gated
+// pair), unless that number is 1.  keep_runs (plain products into which no second matrix goes): `out` is
 // [runs][M][N] and receives the runs apart, the bias in run 0; the caller adds them up in order.
 TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gather, const void* w, const void* w2,
                        int64_t group_stride, const int* tile_group, const int* n_tiles, const void* bias, int bias_type,
                        void* out, int64_t ldc, int M, int N, int K, int tile_rows, int gate, void* scratch, int keep_runs,
                        hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || (tile_rows != 16 && tile_rows != 64 && tile_rows != 64 + TQ_TILE_PAIRS)) return TQ_ERR_BAD_ARG;
+  if (K <= 0 || (tile_rows != 16 && tile_rows != 64)) return TQ_ERR_BAD_ARG;
   if (K % 4 != 0 || lda % 4 != 0 || group_stride % 4 != 0 || ((size_t)a & 15) || ((size_t)w & 15) || ((size_t)w2 & 15))
     return TQ_ERR_UNSUPPORTED;
   if (gate < 0 || gate >= TQ_GATE_COUNT) return TQ_ERR_BAD_ARG;
@@ -419,7 +446,7 @@ TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gath
   const bool grouped = tile_group != nullptr;
   if (keep_runs && (dual || grouped || a_rows || ldc != N)) return TQ_ERR_BAD_ARG;
   int k_per_split = (K + 127) / 128 * 128;
-  const int runs = (grouped || a_rows) ? 1 : M > 64 ? f32_split_runs(M, N, K, &k_per_split) : f32_runs_of_k(N, K, &k_per_split);
+  const int runs = (grouped || a_rows || M > 64) ? 1 : f32_runs_of_k(N, K, &k_per_split);
   float* part = nullptr;
   if (runs > 1) {
     part = keep_runs ? (float*)out : (float*)scratch;
@@ -434,14 +461,18 @@ TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gath
       hipLaunchKernelGGL((gemm_f32_stream_kernel<1, SNT, true>), grid, dim3(256), 0, st, g, k_per_split, k_per_wave, part);
     else
       hipLaunchKernelGGL((gemm_f32_stream_kernel<1, SNT, false>), grid, dim3(256), 0, st, g, k_per_split, k_per_wave, part);
-  } else if (grouped || M > 64) {
-    if (int rc = f32_split_product(g, tile_rows == 64 + TQ_TILE_PAIRS, runs, k_per_split, part, st)) return rc;
   } else {
-    // 17 to 64 rows of one matrix are a single row of tiles, cut into runs of k where the matrix is narrow
-    const dim3 grid(1, (N + 127) / 128, runs);
+    // tiles; 17 to 64 rows of one matrix are a single row of tiles, cut into runs of k where the matrix is narrow
+    const int mi = (grouped || M <= 64) ? 1 : 2;
+    const dim3 grid((M + 64 * mi - 1) / (64 * mi), (N + 127) / 128, runs);
     if (grid.y > 65535) return TQ_ERR_UNSUPPORTED;
-    if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<true>), grid, dim3(256), 0, st, g, k_per_split, part);
-    else hipLaunchKernelGGL((gemm_f32_tile_kernel<false>), grid, dim3(256), 0, st, g, k_per_split, part);
+    if (mi == 1) {
+      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
+      else hipLaunchKernelGGL((gemm_f32_tile_kernel<1, false>), grid, dim3(256), 0, st, g, k_per_split, part);
+    } else {
+      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<2, true>), grid, dim3(256), 0, st, g, k_per_split, part);
+      else hipLaunchKernelGGL((gemm_f32_tile_kernel<2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
+    }
   }
   if (runs > 1) {
     const unsigned blocks = (unsigned)(((int64_t)M * N + 255) / 256);

@@ -142,7 +142,7 @@ int product(Ctx& c, const Product& p, void** out, int* splits, int side = 0) {
   const bool grouped = p.tile_group != nullptr;
   const size_t esz = p.out_act ? TQ_ACT_BYTES : 4;
   const int tile_rows = p.tile_rows ? p.tile_rows : (p.M <= 32 ? 16 : 64);
-  const int unit_rows = tile_rows % TQ_TILE_PAIRS;      // pairs of units are the matrix-core products' alone
+  const int unit_rows = tile_rows % TQ_TILE_PAIRS;      // pairs of units are the matrix-core product's alone
   *splits = 1;
   auto result = [&](size_t bytes) { return p.dest ? p.dest : c.arena.take(bytes); };
   if (!grouped && !p.a_rows && !p.bias.ptr && vendor_product(c, p)) {
@@ -190,7 +190,7 @@ int product(Ctx& c, const Product& p, void** out, int* splits, int side = 0) {
     if (runs > 1 && !p.partial) scratch = c.arena.take((size_t)runs * (p.w2 ? 2 : 1) * p.M * p.N * 4);
     RUN(c, "gemm_f32",
         tq_gemm_f32(p.a, p.lda, p.a_rows, p.gather, p.w.ptr, p.w2, p.gstride, p.tile_group, p.n_tiles, p.bias.ptr,
-                    (int)p.bias.wtype, *out, p.N, p.M, p.N, p.K, tile_rows, p.gate, scratch, p.partial && runs > 1,
+                    (int)p.bias.wtype, *out, p.N, p.M, p.N, p.K, unit_rows, p.gate, scratch, p.partial && runs > 1,
                     c.stream));
     return 0;
   }

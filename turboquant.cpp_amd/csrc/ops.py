@@ -900,8 +900,7 @@ def _gemm_problem(k: str, a, w, act, bias, w2, out_act, a_rows, tile_group, n_ti
               "grouped product needs a_rows, n_tiles and tile_rows of 16, 64, 128 or 256")
         if not _use_mfma(act, a, w, a.shape[1]):
             _need(tile_rows % TILE_PAIRS in (16, 64), k, "tiles of 32, 128 and 256 rows are for the bfloat16 matrix-core product")
-            if not _use_f32(act, a, w, K, w.shape[1] * K):
-                tile_rows %= TILE_PAIRS      # pairs of units are the matrix-core products': the plain one takes unit by unit
+            tile_rows %= TILE_PAIRS      # pairs of units are that product's too: the others take unit by unit
         _check(a_rows, k, "a_rows", torch.int32)
         _check(tile_group, k, "tile_group", torch.int32)
         _check(n_tiles, k, "n_tiles", torch.int32)
@@ -1111,7 +1110,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
     _run(k, lib.tq_gemm_generic(_ptr(a), a.stride(0), _ptr(a_rows), int(gather), _ptr(w), _ptr(w2), _WTYPE[w.dtype], gstride,
                                 _ptr(tile_group), _ptr(n_tiles), _ptr(bias),
                                 _WTYPE[bias.dtype] if bias is not None else 0, _ptr(out), N, int(out_act), M, N, K,
-                                tile_rows % TILE_PAIRS, gate, _stream()), "moe" if grouped else None)
+                                tile_rows, gate, _stream()), "moe" if grouped else None)
     return out
 
 
