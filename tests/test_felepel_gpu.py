@@ -563,3 +563,36 @@ def test_the_delta_rule_in_chunks(act, head_decay, lens, H, G, D, V, shift):
     odd = run(spoiled, state.to("cuda:0")).cpu().view(T, H, V)
     assert torch.isfinite(odd[:at]).all() and torch.isnan(odd[at, 0, 0])
     assert torch.isfinite(odd[lens[first]:]).all() and torch.isfinite(odd[:, 1:]).all()
+
+
+@pytest.mark.parametrize("head_decay", [False, True])
+@pytest.mark.parametrize("told", [False, True])
+def test_a_run_of_the_delta_rule_is_the_same_beside_any_others(head_decay, told):
+    """A run is taken in chunks or token by token for its own length alone: beside others of any lengths, whether the step's
+    longest and shortest run are named or not, it gives the bits that it gives alone."""
+    from turboquant_cpp_amd.csrc import ops
+    H, G, D, V = 4, 2, 64, 48
+    dims = ops.DeltaDims(H, G, D, V, 4, 0, 0, head_decay=True) if head_decay else ops.DeltaDims(H, G, D, V, 4, 8, 8)
+    g = torch.Generator().manual_seed(3)
+    unit = lambda x: (x / x.norm(dim=-1, keepdim=True)).flatten(1)      # noqa: E731
+    rnd = lambda *s: torch.randn(s, generator=g)      # noqa: E731
+    runs_of = {n: (unit(rnd(n, G, D)) * D ** -0.5, unit(rnd(n, G, D) + 0.3), rnd(n, H * V), torch.sigmoid(rnd(n, H)),
+                   torch.sigmoid(rnd(n, H) + 3) if head_decay else rnd(n, H * D + H * V), 0.1 * rnd(1, dims.state_floats))
+               for n in (1, 5, 33, 47, 48, 97, 400)}
+    a_log, dt_bias = (0.5 * rnd(H)).to("cuda:0"), (0.5 * rnd(H * D) - 3).to("cuda:0")
+
+    def step(lens):
+        qn, kn, vc, beta, ag, state = (torch.cat([runs_of[n][i] for n in lens]).to("cuda:0") for i in range(6))
+        cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32).to("cuda:0")
+        runs = {"cu_seqlens": cu, "slots": torch.arange(len(lens), dtype=torch.int32, device="cuda:0"), "decode": False}
+        if told:
+            runs.update(max_new=max(lens), min_new=min(lens))
+        if head_decay:
+            o = ops.delta_scan_h(qn, kn, vc, beta, ag, runs, state, dims, "bfloat16")
+        else:
+            o = ops.delta_scan(qn, kn, vc, beta, ag, a_log, dt_bias, runs, state, dims, "bfloat16")
+        return [(part, state[i]) for i, part in enumerate(o.split(lens))]
+    alone = {n: step([n])[0] for n in runs_of}
+    for lens in ([97] + [1] * 40, [33, 400], [48, 47, 5, 400, 1], [1, 5, 33, 47], [97, 48], [5] * 60):
+        for n, (o, state) in zip(lens, step(lens)):
+            assert torch.equal(o, alone[n][0]) and torch.equal(state, alone[n][1]), (lens, n)

@@ -1,4 +1,5 @@
-// The gated delta rule of delta_rule.hip over long runs, in chunks of 32 tokens.
+// The gated delta rule of delta_rule.hip over long runs, in chunks of 32 tokens.  Which form a run takes is a matter of its own
+// length alone (DC_FROM), so that what a sequence gets does not depend on the others of the step.
 //
 // With S the state before a chunk, G_t the decays of the chunk's tokens multiplied up to and with t (per key channel; one
 // number for all of them in the form with a decay per head) and G_t / G_s the product of those behind s up to t:
@@ -17,18 +18,27 @@
 #include "delta_rule.h"
 
 #define DC_T 32
+// Tokens from which a run goes in chunks: a chunk costs the same whatever it holds, and the two launches 20 us before the first.
+// Chunks and token by token, us, 16 heads of 128 x 128: one sequence of 32 tokens 24 and 23, of 48 25 and 30, of 96 27 and 51, of
+// 1,024 90 and 475; 64 sequences of 32 tokens 195 and 212, of 48 295 and 288, of 64 302 and 364, of 256 970 and 1,291.  Heads of
+// 256 x 256, whose scan spills 196 bytes a lane: 38 and 42 for one of 48 tokens, 1,107 and 1,266 for 64 of them.  Narrow heads in a
+// crowded step, where a chunk's pairs weigh more than the state, are the exception: 64 sequences of 64 tokens and 32 heads of 64 x 64
+// 225 and 215, 16 heads of 128 x 16 135 and 107, while one sequence of 256 tokens of these takes 27 and 127, 38 and 137.
+#define DC_FROM 48
 typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ __forceinline__ int64_t dc_floats(int D, int V) { return (int64_t)DC_T * (3 * D + V) + DC_T * DC_T + D; }
 
-// The sequence and the chunk in it that chunk number `want` of the step is; false behind the last one.  All 64 lanes of a
-// wave call it together.
+__device__ __forceinline__ int dc_chunks(int n) { return n >= DC_FROM ? (n + DC_T - 1) / DC_T : 0; }
+
+// The sequence and the chunk in it that chunk number `want` of the step's long runs is; false behind the last one.  All 64 lanes of
+// a wave call it together.
 __device__ __forceinline__ bool dc_find(const int* __restrict__ cu_seqlens, int B, int want, int& b, int& c) {
   const int lane = threadIdx.x % TQ_WAVE;
   int base = 0;
   for (int b0 = 0; b0 < B; b0 += TQ_WAVE) {
     const int i = b0 + lane;
-    const int own = i < B ? (cu_seqlens[i + 1] - cu_seqlens[i] + DC_T - 1) / DC_T : 0;
+    const int own = i < B ? dc_chunks(cu_seqlens[i + 1] - cu_seqlens[i]) : 0;
     int upto = own;
 #pragma unroll
     for (int o = 1; o < TQ_WAVE; o *= 2) {
@@ -319,9 +329,9 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
   const int h = blockIdx.x % H, vb = blockIdx.x / H, b = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TQ_WAVE), lane = threadIdx.x % TQ_WAVE, r = lane % 16, g4 = lane / 16;
   const int t0 = cu_seqlens[b], n = cu_seqlens[b + 1] - t0;
-  if (n <= 0) return;
+  if (n < DC_FROM) return;
   int base = 0;
-  for (int i = lane; i < b; i += TQ_WAVE) base += (cu_seqlens[i + 1] - cu_seqlens[i] + DC_T - 1) / DC_T;
+  for (int i = lane; i < b; i += TQ_WAVE) base += dc_chunks(cu_seqlens[i + 1] - cu_seqlens[i]);
 #pragma unroll
   for (int o = TQ_WAVE / 2; o > 0; o >>= 1) base += __shfl_xor(base, o, TQ_WAVE);
   base = __builtin_amdgcn_readfirstlane(base);
@@ -480,29 +490,31 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
   }
 }
 
+// The most chunks that the long runs of T tokens of B sequences have: each begins one beyond its whole ones.
+static int64_t dc_bound(int T, int B) { return (int64_t)T / DC_T + (B < T / DC_FROM ? B : T / DC_FROM); }
+
 // Sizes that the tiles take.
 static bool dc_takes(int D, int V) { return D % 16 == 0 && D <= 256 && V % 16 == 0 && V > 0; }
 
-// Floats of scratch that tq_delta_chunks needs for T tokens of B sequences; 0 where the token-by-token form is the better one, or
-// the only one.  In chunks from 48 tokens a sequence on average: a chunk costs the same whatever it holds, and the two launches
-// 20 us before the first (16 heads of 128 x 128, both forms: one sequence of 97 tokens 35 us in chunks and 59 token by token, of
-// 33 tokens 31 and 29, of 8 tokens 30 and 20; 64 sequences of 128 tokens 568 and 680, of 16 tokens 202 and 147).
+// Floats of scratch that tq_delta_chunks needs for T tokens of B sequences; 0 where no run can be long enough for chunks, or the
+// sizes do not fit the tiles.
 TQ_API int64_t tq_delta_chunk_scratch(int T, int B, int H, int D, int V) {
-  if (!dc_takes(D, V) || B < 1 || T < 48 * (int64_t)B) return 0;
-  return ((int64_t)T / DC_T + B) * H * dc_floats(D, V);
+  if (!dc_takes(D, V) || B < 1 || T < DC_FROM) return 0;
+  return dc_bound(T, B) * H * dc_floats(D, V);
 }
 
 // What tq_delta_scan (head_decay 0; ag is only read) and tq_delta_scan_h (head_decay 1; ag [T][H] decays, a_log and dt_bias
-// null) compute, in chunks of 32 tokens of every sequence's run, over `scratch`.
+// null) compute, over `scratch`: runs of DC_FROM tokens and more in chunks, the others token by token in a launch of their own,
+// which all_long (the host knows that there are none) leaves out.
 TQ_API int tq_delta_chunks(const float* qn, const float* kn, const float* vc, const float* beta, const float* ag,
                            const float* a_log, const float* dt_bias, int head_decay, const int* cu_seqlens, const int* slots,
                            float* state, int64_t state_stride, int H, int G, int D, int V, int taps, int T, int B,
-                           float* scratch, float* o_raw, hipStream_t st) {
+                           int all_long, float* scratch, float* o_raw, hipStream_t st) {
   if (B <= 0 || T <= 0) return 0;
   const DeltaDims d{H, G, D, V, taps, head_decay ? 0 : 1, head_decay ? 0 : 1, head_decay ? 1 : 0};
-  if (H < 1 || G < 1 || H % G || taps < 1 || state_stride < dd_state(d) || !scratch || !ag || (!head_decay && (!a_log || !dt_bias)))
+  if (H < 1 || G < 1 || H % G || taps < 1 || taps > 64 || state_stride < dd_state(d) || !scratch || !ag || (!head_decay && (!a_log || !dt_bias)))
     return TQ_ERR_BAD_ARG;
-  const int64_t chunks = (int64_t)T / DC_T + B;
+  const int64_t chunks = dc_bound(T, B);
   if (!dc_takes(D, V) || B > 65535 || chunks > 65535) return TQ_ERR_UNSUPPORTED;
   const int nd = D / 16;
   const int row = DC_T * (D + 4);
@@ -535,5 +547,6 @@ TQ_API int tq_delta_chunks(const float* qn, const float* kn, const float* vc, co
   else TQ_SCAN(4);
 #undef TQ_SCAN
   TQ_LAUNCH_CHECK();
-  return 0;
+  if (all_long) return 0;
+  return delta_short_runs(qn, kn, vc, beta, ag, a_log, dt_bias, cu_seqlens, slots, state, state_stride, d, DC_FROM, T, B, o_raw, st);
 }

@@ -19,3 +19,8 @@ __host__ __device__ __forceinline__ int64_t dd_state(const DeltaDims& d) {
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+
+// The recurrence token by token over the runs of fewer than `below` tokens; ag is only read.
+int delta_short_runs(const float* qn, const float* kn, const float* vc, const float* beta, const float* ag, const float* a_log,
+                     const float* dt_bias, const int* cu_seqlens, const int* slots, float* state, int64_t state_stride,
+                     const DeltaDims& d, int below, int T, int B, float* o_raw, hipStream_t st);

@@ -13,8 +13,8 @@
 //   delta_decay  (steps of many tokens) the decays of all tokens, in parallel, in place of what they are made from
 //   delta_scan   per (sequence, head, block of value channels): the recurrence over the run's tokens in order, the
 //                state in registers (16 key channels of a value channel per lane), tokens staged through two LDS
-//                buffers in chunks; a short step works out its decays as it stages them (long runs of sizes that its
-//                tiles take go through delta_chunks.hip instead)
+//                buffers in chunks; a short step works out its decays as it stages them (runs of 48 tokens and more, of
+//                sizes that its tiles take, go through delta_chunks.hip instead)
 //   delta_out    per token: norm and gate of every head; and per sequence: the convolution's new state
 //   delta_decode (steps of one token per sequence) the second low-rank products, decays, recurrence, norm, gate and the
 //                convolution's new state in one launch
@@ -26,6 +26,7 @@
 // A sequence's row of state (float): S as [H][D][V], then for every convolution channel (q's, k's, v's) its last
 // taps - 1 inputs, oldest first.  Projections P [T][NP] (float): q (G D) | k (G D) | v (H V) | b (H) | a1 (ra) | g1 (rg).
 #include "delta_rule.h"
+#include <limits.h>
 
 #define DR_ROWS 16        // key channels of a value channel that one lane keeps
 #define DR_CHUNK 16       // tokens staged at a time
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
                                                          const float* __restrict__ dt_bias,
                                                          const int* __restrict__ cu_seqlens, const int* __restrict__ slots,
                                                          float* __restrict__ state, int64_t state_stride, DeltaDims dm,
-                                                         int cols, int col_blocks, int head_decay,
+                                                         int cols, int col_blocks, int head_decay, int below,
                                                          float* __restrict__ o_raw) {
   constexpr int DP = DR_ROWS * NSEG, RL = DR_PAD * NSEG;      // rows of a token, and the floats they take in LDS
   constexpr int EV = 16 * CPT / NSEG > 0 ? 16 * CPT / NSEG : 1;      // values of v per thread and chunk, at the most
@@ -153,6 +154,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
   int cloc[CPT];                             // this lane's channels within the block (0 where it has none)
   bool col_ok[CPT];
   const int t0 = cu_seqlens[b], n = cu_seqlens[b + 1] - t0;
+  if (n >= below) return;      // (the whole workgroup: another launch takes this run in chunks)
   float* S = state + (size_t)slots[b] * state_stride + (size_t)h * D * V;
   float s[CPT][DR_ROWS];
 #pragma unroll
@@ -506,10 +508,11 @@ TQ_API int tq_delta_prep_h(const float* P, const int* slot_of_token, const float
                      nullptr, a_log, dt_bias, dec, T, st);
 }
 
-// head_decay: ag is [T][H], the decay of every head, ready to use.
+// head_decay: ag is [T][H], the decay of every head, ready to use.  Runs of `below` tokens and more are left alone; decayed: the
+// decays of the whole step are worked out beforehand, in place.
 static int launch_scan(const float* qn, const float* kn, const float* vc, const float* beta, float* ag, const float* a_log,
                        const float* dt_bias, const int* cu_seqlens, const int* slots, float* state, int64_t state_stride,
-                       const DeltaDims& d, int head_decay, int T, int B, float* o_raw, hipStream_t st) {
+                       const DeltaDims& d, int head_decay, int decayed, int below, int T, int B, float* o_raw, hipStream_t st) {
   if (B <= 0 || T <= 0) return 0;
   if (!dims_ok(d) || state_stride < dd_state(d)) return TQ_ERR_BAD_ARG;
   if (B > 65535) return TQ_ERR_UNSUPPORTED;
@@ -532,8 +535,6 @@ static int launch_scan(const float* qn, const float* kn, const float* vc, const 
   const int dp = DR_ROWS * nseg;
   const int chunk = DR_CHUNK < DR_STAGE * threads / dp ? DR_CHUNK : DR_STAGE * threads / dp;
   const size_t shmem = (size_t)2 * (3 * chunk * DR_PAD * nseg + (chunk * cols + 3) / 4 * 4 + DR_CHUNK) * sizeof(float);
-  // the decays of a long step are worked out beforehand, once for all blocks of value channels
-  const int decayed = head_decay || T > 16 * B || T >= 256;
   if (decayed && !head_decay) {
     const int64_t total = (int64_t)T * H * D;
     hipLaunchKernelGGL(delta_decay_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, ag, a_log, dt_bias,
@@ -546,11 +547,11 @@ static int launch_scan(const float* qn, const float* kn, const float* vc, const 
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);                              \
     hipLaunchKernelGGL((delta_scan_kernel<NS, CP, DEC>), dim3(H * col_blocks, B), dim3(threads), shmem, st, qn, kn,   \
                        vc, beta, ag, a_log, dt_bias, cu_seqlens, slots, state, state_stride, d, cols, col_blocks,     \
-                       head_decay, o_raw);                                                                            \
+                       head_decay, below, o_raw);                                                                     \
   } while (0)
 #define TQ_SCAN_AS(NS, CP)                   \
   do {                                       \
-    if (decayed) TQ_SCAN_WITH(NS, CP, true); \
+    if (decayed || head_decay) TQ_SCAN_WITH(NS, CP, true); \
     else TQ_SCAN_WITH(NS, CP, false);        \
   } while (0)
 #define TQ_SCAN(NS)                  \
@@ -580,8 +581,9 @@ TQ_API int tq_delta_scan(const float* qn, const float* kn, const float* vc, cons
                          const float* a_log, const float* dt_bias, const int* cu_seqlens, const int* slots, float* state,
                          int64_t state_stride, int H, int G, int D, int V, int taps, int T, int B, float* o_raw,
                          hipStream_t st) {
+  // the decays of a long step are worked out beforehand, once for all blocks of value channels
   return launch_scan(qn, kn, vc, beta, ag, a_log, dt_bias, cu_seqlens, slots, state, state_stride,
-                     DeltaDims{H, G, D, V, taps, 1, 1, 0}, 0, T, B, o_raw, st);
+                     DeltaDims{H, G, D, V, taps, 1, 1, 0}, 0, T > 16 * B || T >= 256, INT_MAX, T, B, o_raw, st);
 }
 
 // The same recurrence with one decay per head: dec [T][H] as tq_delta_prep_h wrote it.
@@ -589,7 +591,14 @@ TQ_API int tq_delta_scan_h(const float* qn, const float* kn, const float* vc, co
                            const int* cu_seqlens, const int* slots, float* state, int64_t state_stride, int H, int G, int D,
                            int V, int taps, int T, int B, float* o_raw, hipStream_t st) {
   return launch_scan(qn, kn, vc, beta, const_cast<float*>(dec), nullptr, nullptr, cu_seqlens, slots, state, state_stride,
-                     DeltaDims{H, G, D, V, taps, 0, 0, 1}, 1, T, B, o_raw, st);
+                     DeltaDims{H, G, D, V, taps, 0, 0, 1}, 1, 0, INT_MAX, T, B, o_raw, st);
+}
+
+int delta_short_runs(const float* qn, const float* kn, const float* vc, const float* beta, const float* ag, const float* a_log,
+                     const float* dt_bias, const int* cu_seqlens, const int* slots, float* state, int64_t state_stride,
+                     const DeltaDims& d, int below, int T, int B, float* o_raw, hipStream_t st) {
+  return launch_scan(qn, kn, vc, beta, const_cast<float*>(ag), a_log, dt_bias, cu_seqlens, slots, state, state_stride, d, d.mode, 0,
+                     below, T, B, o_raw, st);
 }
 
 static int launch_out(const float* o_raw, const float* gates, int64_t gate_ld, int gate_kind, const float* norm_w, float eps,

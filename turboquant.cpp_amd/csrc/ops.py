@@ -101,7 +101,7 @@ _SIGNATURES = {
                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "tq_delta_chunk_scratch": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "tq_delta_chunks": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int,
-                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
+                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
     "tq_delta_decode": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr,
                         _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "tq_delta_out": [_c_ptr, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int,
@@ -1500,17 +1500,21 @@ def delta_prep(proj: torch.Tensor, slot_of_token: torch.Tensor, state: torch.Ten
     return qn, kn, vc, beta, low
 
 
+DELTA_CHUNKS_FROM = 48      # tokens from which a run of the delta rule goes in chunks (DC_FROM in delta_chunks.hip)
+
+
 def _delta_chunks(k, qn, kn, vc, beta, ag, a_log, dt_bias, runs, state, stride, dims, T, B, o, act) -> bool:
-    """Runs the recurrence in chunks into ``o`` where the library says that this is the better form for the step; ``a_log`` None:
-    ``ag`` holds a decay per head."""
+    """Runs the recurrence into ``o`` with the long runs in chunks, where there can be some; ``a_log`` None: ``ag`` holds a decay
+    per head.  ``runs`` may name ``max_new`` and ``min_new``, the longest and the shortest run."""
     lib = library(act)
-    n = lib.tq_delta_chunk_scratch(T, B, dims.heads, dims.dim, dims.vdim)
+    longest, shortest = runs.get("max_new", T), runs.get("min_new", T if B == 1 else 0)
+    n = lib.tq_delta_chunk_scratch(T, B, dims.heads, dims.dim, dims.vdim) if longest >= DELTA_CHUNKS_FROM else 0
     if n == 0 or any(t.data_ptr() % 16 for t in (qn, kn, ag)):
         return False
     scratch = torch.empty(n, dtype=torch.float32, device=qn.device)
     _run(k, lib.tq_delta_chunks(_ptr(qn), _ptr(kn), _ptr(vc), _ptr(beta), _ptr(ag), _ptr(a_log), _ptr(dt_bias), int(a_log is None),
                                 _ptr(runs["cu_seqlens"]), _ptr(runs["slots"]), _ptr(state), stride, *dims.sizes(), T, B,
-                                _ptr(scratch), _ptr(o), _stream()))
+                                int(shortest >= DELTA_CHUNKS_FROM), _ptr(scratch), _ptr(o), _stream()))
     return True
 
 
@@ -1518,7 +1522,8 @@ def delta_scan(qn: torch.Tensor, kn: torch.Tensor, vc: torch.Tensor, beta: torch
                a_log: torch.Tensor, dt_bias: torch.Tensor, runs: dict, state: torch.Tensor, dims: DeltaDims, act):
     """The recurrence over each sequence's run of tokens, in order, from and into its row of ``state``:
     S <- diag(g) S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q, with g = exp(-exp(a_log) softplus(a + dt_bias))
-    from the first H*dim columns of ``ag`` [T, H*dim + H*vdim] (which a step of many tokens overwrites with those g).
+    from the first H*dim columns of ``ag`` [T, H*dim + H*vdim] (which a step of many short runs overwrites with those g).  Runs
+    of 48 tokens and more go in chunks of 32, each by its own length whatever else is in the step.
     Returns o, float32 [T, H*vdim]."""
     k = "delta_scan"
     T = qn.shape[0]

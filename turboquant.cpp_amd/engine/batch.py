@@ -72,7 +72,7 @@ class StepBatch:
     def runs(self) -> dict:
         """The step as runs of consecutive positions, one per sequence, for kernels that tile over tokens."""
         return {"cu_seqlens": self.cu_seqlens, "slots": self.slots_dev, "start": self.start_dev,
-                "max_new": self.max_new, "max_end": self.max_end, "decode": self.is_decode}
+                "max_new": self.max_new, "min_new": min(self.n_new), "max_end": self.max_end, "decode": self.is_decode}
 
 
 def pack_step(slots, starts, token_lists, wants, device) -> StepBatch:
