@@ -596,3 +596,40 @@ def test_a_run_of_the_delta_rule_is_the_same_beside_any_others(head_decay, told)
     for lens in ([97] + [1] * 40, [33, 400], [48, 47, 5, 400, 1], [1, 5, 33, 47], [97, 48], [5] * 60):
         for n, (o, state) in zip(lens, step(lens)):
             assert torch.equal(o, alone[n][0]) and torch.equal(state, alone[n][1]), (lens, n)
+
+
+@pytest.mark.parametrize("head_decay", [False, True])
+def test_the_delta_rule_in_more_chunks_than_the_scratch_holds(head_decay):
+    """A step's chunks go through the scratch a window at a time, which ends within runs: the bits of every run by itself in cuts
+    of fifteen chunks, each of which fits a window."""
+    from turboquant_cpp_amd.csrc import ops
+    H, G, D, V = 64, 1, 256, 256
+    lens = [1600, 33, 2080, 1500]
+    dims = ops.DeltaDims(H, G, D, V, 4, 0, 0, head_decay=True) if head_decay else ops.DeltaDims(H, G, D, V, 4, 8, 8)
+    lib = ops.library("bfloat16")
+    chunk = lib.tq_delta_chunk_scratch(48, 1, H, D, V) // 2
+    assert 15 < lib.tq_delta_chunk_scratch(sum(lens), len(lens), H, D, V) // chunk < 50 + 65 + 47
+    g = torch.Generator("cuda:0").manual_seed(4)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda:0")      # noqa: E731
+    unit = lambda x: (x / x.norm(dim=-1, keepdim=True)).flatten(1).contiguous()      # noqa: E731
+    T = sum(lens)
+    tensors = [unit(rnd(T, G, D)) * D ** -0.5, unit(rnd(T, G, D) + 0.3), rnd(T, H * V), torch.sigmoid(rnd(T, H)),
+               torch.sigmoid(rnd(T, H) + 3) if head_decay else rnd(T, H * D + H * V)]
+    a_log, dt_bias, state = 0.5 * rnd(H), 0.5 * rnd(H * D) - 3, 0.1 * rnd(len(lens), dims.state_floats)
+
+    def step(lo, sizes, slots, into):
+        runs = {"cu_seqlens": torch.tensor([0] + torch.tensor(sizes).cumsum(0).tolist(), dtype=torch.int32).to("cuda:0"),
+                "slots": torch.tensor(slots, dtype=torch.int32).to("cuda:0"), "decode": False}
+        qn, kn, vc, beta, ag = (t[lo:lo + sum(sizes)].clone() for t in tensors)
+        if head_decay:
+            return ops.delta_scan_h(qn, kn, vc, beta, ag, runs, into, dims, "bfloat16")
+        return ops.delta_scan(qn, kn, vc, beta, ag, a_log, dt_bias, runs, into, dims, "bfloat16")
+    whole, cut = state.clone(), state.clone()
+    o = step(0, lens, list(range(len(lens))), whole)
+    lo = 0
+    for slot, n in enumerate(lens):
+        for at in range(0, n, 480):
+            size = min(480, n - at)
+            assert torch.equal(step(lo + at, [size], [slot], cut), o[lo + at:lo + at + size]), (slot, at)
+        lo += n
+    assert torch.equal(whole, cut)

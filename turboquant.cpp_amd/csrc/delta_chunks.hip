@@ -12,6 +12,9 @@
 // v_mfma_f32_16x16x4_f32 where it is a product.  No quotient is formed: a ratio G_t / G_s is the product of the factors
 // between, and none is above one, whatever the decays.
 //
+// A step whose chunks do not fit the scratch (DC_SCRATCH) goes through it a window at a time: the same chunks of every run, so that
+// the runs still go side by side, their state through memory from one window to the next; and so many runs at a time.
+//
 // Scratch (float), per chunk and head, in the order in which a wave's lanes of the scan take their operands (four floats a
 // lane, 64 lanes a tile of 16 x 16): W [2 token tiles][D / 16] | G q alike | (G_32 / G) k [D / 16][2] | U0 [V / 16][2] |
 // b [2][2] | G_32 [D].
@@ -25,20 +28,31 @@
 // crowded step, where a chunk's pairs weigh more than the state, are the exception: 64 sequences of 64 tokens and 32 heads of 64 x 64
 // 225 and 215, 16 heads of 128 x 16 135 and 107, while one sequence of 256 tokens of these takes 27 and 127, 38 and 137.
 #define DC_FROM 48
+// Floats of scratch at the most (1 GiB), or those of one chunk: what a step of 30,000 tokens and 16 heads of 128 x 128 fills.  Beyond,
+// a window's launches are a few more (us, in one window and in several of 1 GiB, 512 MiB and 256 MiB: 64 runs of 1,080 tokens 3,791,
+// 3,980, 4,249 and 5,097; four of 32,768 7,007, 7,021, 7,137 and 7,346).
+#define DC_SCRATCH (1 << 28)
 typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ __forceinline__ int64_t dc_floats(int D, int V) { return (int64_t)DC_T * (3 * D + V) + DC_T * DC_T + D; }
 
 __device__ __forceinline__ int dc_chunks(int n) { return n >= DC_FROM ? (n + DC_T - 1) / DC_T : 0; }
 
-// The sequence and the chunk in it that chunk number `want` of the step's long runs is; false behind the last one.  All 64 lanes of
+// The chunks `first` to first + count - 1 of runs b0 to b0 + B - 1.
+struct DeltaWindow {
+  int b0, B, first, count;
+};
+// How many of its chunks a run of n tokens has there.
+__device__ __forceinline__ int dc_inside(const DeltaWindow& w, int n) { return min(max(dc_chunks(n) - w.first, 0), w.count); }
+
+// The run and the chunk of it that chunk number `want` of the window is, run by run; false behind the last one.  All 64 lanes of
 // a wave call it together.
-__device__ __forceinline__ bool dc_find(const int* __restrict__ cu_seqlens, int B, int want, int& b, int& c) {
+__device__ __forceinline__ bool dc_find(const int* __restrict__ cu_seqlens, const DeltaWindow& w, int want, int& b, int& c) {
   const int lane = threadIdx.x % TQ_WAVE;
   int base = 0;
-  for (int b0 = 0; b0 < B; b0 += TQ_WAVE) {
+  for (int b0 = w.b0; b0 < w.b0 + w.B; b0 += TQ_WAVE) {
     const int i = b0 + lane;
-    const int own = i < B ? dc_chunks(cu_seqlens[i + 1] - cu_seqlens[i]) : 0;
+    const int own = i < w.b0 + w.B ? dc_inside(w, cu_seqlens[i + 1] - cu_seqlens[i]) : 0;
     int upto = own;
 #pragma unroll
     for (int o = 1; o < TQ_WAVE; o *= 2) {
@@ -49,7 +63,7 @@ __device__ __forceinline__ bool dc_find(const int* __restrict__ cu_seqlens, int 
     if (reached) {
       const int at = __ffsll((unsigned long long)reached) - 1;
       b = b0 + at;
-      c = want - base - (__shfl(upto, at, TQ_WAVE) - __shfl(own, at, TQ_WAVE));
+      c = w.first + want - base - (__shfl(upto, at, TQ_WAVE) - __shfl(own, at, TQ_WAVE));
       return true;
     }
     base += __shfl(upto, TQ_WAVE - 1, TQ_WAVE);
@@ -57,9 +71,9 @@ __device__ __forceinline__ bool dc_find(const int* __restrict__ cu_seqlens, int 
   return false;
 }
 
-// grid (H, chunks), block 512.  LDS: k, q, decays [32][LD] each, the products of the decays from the start of the token's half of
-// the chunk up to and with it, and (in the decays' place) from behind it to the half's end (halves of 16: what lies between two
-// tokens of different halves is one of each); the partial sums of a and b; a.
+// grid (H, chunks of the window), block 512.  LDS: k, q, decays [32][LD] each, the products of the decays from the start of
+// the token's half of the chunk up to and with it, and (in the decays' place) from behind it to the half's end (halves of 16:
+// what lies between two tokens of different halves is one of each); the partial sums of a and b; a.
 // The pairs of one half are formed channel by channel with the product of the decays between them (a lane keeps k_s times
 // that product for D / 16 channels and walks through t); those of different halves are products of matrices, by waves 0 to 3
 // while the others write the decayed rows out.  The triangular system then takes a column of its right side to a thread.
@@ -70,7 +84,7 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
                                                                const float* __restrict__ vc, const float* __restrict__ beta,
                                                                const float* __restrict__ ag, const float* __restrict__ a_log,
                                                                const float* __restrict__ dt_bias,
-                                                               const int* __restrict__ cu_seqlens, int B, DeltaDims dm,
+                                                               const int* __restrict__ cu_seqlens, DeltaWindow window, DeltaDims dm,
                                                                float* __restrict__ scratch) {
   constexpr int D = 16 * ND, LD = D + 4, SHARES = 8 * 512 > DC_T * LD ? 8 * 512 : DC_T * LD;
   extern __shared__ __align__(16) float dc_lds[];
@@ -86,7 +100,7 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
   const int h = blockIdx.x, tid = threadIdx.x, wave = tid / TQ_WAVE, lane = tid % TQ_WAVE;
   const int H = dm.H, G = dm.G, V = dm.V, gq = h / (H / G);
   int b, c;
-  if (!dc_find(cu_seqlens, B, blockIdx.y, b, c)) return;
+  if (!dc_find(cu_seqlens, window, blockIdx.y, b, c)) return;
   b = __builtin_amdgcn_readfirstlane(b);      // (alike in every lane, and so are the addresses made from them)
   c = __builtin_amdgcn_readfirstlane(c);
   const int t0 = cu_seqlens[b] + c * DC_T, nc = min(DC_T, cu_seqlens[b + 1] - t0);
@@ -311,8 +325,8 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
   }
 }
 
-// grid (H V / 16, B), block 256: a workgroup takes 16 value channels of a head through the sequence's chunks; wave w keeps
-// the rows of the state in key tiles w, w + 4, ... as accumulators, which are the operands of the products with the state as
+// grid (H V / 16, runs of the window), block 256: a workgroup takes 16 value channels of a head through the sequence's chunks in the window;
+// wave w keeps the rows of the state in key tiles w, w + 4, ... as accumulators, which are the operands of the products with the state as
 // they stand (the key channels of a product are taken in the order 0, 4, 8, 12, 1, 5, ...).  Each wave's share of u passes
 // through LDS, one barrier a chunk; its share of o, to which waves 0, 1 and 2 add one of b's three tiles each once u is known,
 // goes along with the next chunk's u.  The next two chunks' operands are on their way meanwhile.  The blocks of a head lie H apart, so
@@ -323,18 +337,22 @@ template <int NB>
 __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __restrict__ scratch,
                                                                const int* __restrict__ cu_seqlens,
                                                                const int* __restrict__ slots, float* __restrict__ state,
-                                                               int64_t state_stride, DeltaDims dm, float* __restrict__ o_raw) {
+                                                               int64_t state_stride, DeltaWindow window, DeltaDims dm,
+                                                               float* __restrict__ o_raw) {
   __shared__ __align__(16) float ex[2][4][4][256];      // [buffer][wave][u, u, the chunk before's o, o][lane][4]
   const int H = dm.H, D = dm.D, V = dm.V, ND = D / 16, VB = V / 16;
-  const int h = blockIdx.x % H, vb = blockIdx.x / H, b = blockIdx.y;
+  const int h = blockIdx.x % H, vb = blockIdx.x / H, b = window.b0 + blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TQ_WAVE), lane = threadIdx.x % TQ_WAVE, r = lane % 16, g4 = lane / 16;
-  const int t0 = cu_seqlens[b], n = cu_seqlens[b + 1] - t0;
-  if (n < DC_FROM) return;
+  int t0 = cu_seqlens[b], n = cu_seqlens[b + 1] - t0;
+  const int chunks = dc_inside(window, n);
+  if (chunks == 0) return;
   int base = 0;
-  for (int i = lane; i < b; i += TQ_WAVE) base += dc_chunks(cu_seqlens[i + 1] - cu_seqlens[i]);
+  for (int i = window.b0 + lane; i < b; i += TQ_WAVE) base += dc_inside(window, cu_seqlens[i + 1] - cu_seqlens[i]);
 #pragma unroll
   for (int o = TQ_WAVE / 2; o > 0; o >>= 1) base += __shfl_xor(base, o, TQ_WAVE);
   base = __builtin_amdgcn_readfirstlane(base);
+  t0 += window.first * DC_T;      // (chunks count from the window's first on)
+  n -= window.first * DC_T;
   const size_t chunk_floats = dc_floats(D, V);
   const float* at = scratch + ((size_t)base * H + h) * chunk_floats;
   float* S = state + (size_t)slots[b] * state_stride + (size_t)h * D * V + vb * 16 + r;
@@ -368,7 +386,6 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
     for (int tb = 0; tb < 2; ++tb) to.u0[tb] = tile(6 * ND + vb * 2 + tb);
     to.bq = tile(6 * ND + 2 * VB + (wave == 0 ? 0 : wave == 1 ? 2 : 3));      // b's tile (0, 0), (1, 0) or (1, 1)
   };
-  const int chunks = (n + DC_T - 1) / DC_T;
   dc_f32x4 po[2] = {zero, zero};      // this wave's share of the o of the chunk that has its u
   // two numbers of the o of chunk c from the waves' shares, in wave order: token tile wave / 2, rows 4 g4 + 2 (wave % 2) on
   auto read_out = [&](const float (*from)[4][256], int c, bool last) {
@@ -496,57 +513,81 @@ static int64_t dc_bound(int T, int B) { return (int64_t)T / DC_T + (B < T / DC_F
 // Sizes that the tiles take.
 static bool dc_takes(int D, int V) { return D % 16 == 0 && D <= 256 && V % 16 == 0 && V > 0; }
 
+// Chunks that the scratch holds.
+static int64_t dc_held(int H, int D, int V) {
+  const int64_t n = DC_SCRATCH / (H * dc_floats(D, V));
+  return n < 1 ? 1 : n < 65535 ? n : 65535;
+}
+
 // Floats of scratch that tq_delta_chunks needs for T tokens of B sequences; 0 where no run can be long enough for chunks, or the
 // sizes do not fit the tiles.
 TQ_API int64_t tq_delta_chunk_scratch(int T, int B, int H, int D, int V) {
-  if (!dc_takes(D, V) || B < 1 || T < DC_FROM) return 0;
-  return dc_bound(T, B) * H * dc_floats(D, V);
+  if (!dc_takes(D, V) || H < 1 || B < 1 || B > 65535 || T < DC_FROM) return 0;
+  const int64_t all = dc_bound(T, B), held = dc_held(H, D, V);
+  return (all < held ? all : held) * H * dc_floats(D, V);
 }
 
 // What tq_delta_scan (head_decay 0; ag is only read) and tq_delta_scan_h (head_decay 1; ag [T][H] decays, a_log and dt_bias
-// null) compute, over `scratch`: runs of DC_FROM tokens and more in chunks, the others token by token in a launch of their own,
-// which all_long (the host knows that there are none) leaves out.
+// null) compute, over `scratch`: runs of DC_FROM tokens and more in chunks, the others token by token in a launch of their own.
+// longest, shortest: bounds that the host knows for the runs' tokens (T and 0 if it knows none).
 TQ_API int tq_delta_chunks(const float* qn, const float* kn, const float* vc, const float* beta, const float* ag,
                            const float* a_log, const float* dt_bias, int head_decay, const int* cu_seqlens, const int* slots,
                            float* state, int64_t state_stride, int H, int G, int D, int V, int taps, int T, int B,
-                           int all_long, float* scratch, float* o_raw, hipStream_t st) {
+                           int longest, int shortest, float* scratch, float* o_raw, hipStream_t st) {
   if (B <= 0 || T <= 0) return 0;
   const DeltaDims d{H, G, D, V, taps, head_decay ? 0 : 1, head_decay ? 0 : 1, head_decay ? 1 : 0};
   if (H < 1 || G < 1 || H % G || taps < 1 || taps > 64 || state_stride < dd_state(d) || !scratch || !ag || (!head_decay && (!a_log || !dt_bias)))
     return TQ_ERR_BAD_ARG;
-  const int64_t chunks = dc_bound(T, B);
-  if (!dc_takes(D, V) || B > 65535 || chunks > 65535) return TQ_ERR_UNSUPPORTED;
+  if (!dc_takes(D, V) || B > 65535 || T < DC_FROM) return TQ_ERR_UNSUPPORTED;
+  if (longest < 0 || longest > T) return TQ_ERR_BAD_ARG;
   const int nd = D / 16;
   const int row = DC_T * (D + 4);
   const size_t shmem = (size_t)(3 * row + (row > 8 * 512 ? row : 8 * 512) + 4 * 512 + DC_T * 36 + DC_T) * sizeof(float);
+  auto launch = [&](const DeltaWindow& w, unsigned chunks) -> int {
 #define TQ_PREP(N, HD)                                                                                                       \
   do {                                                                                                                       \
     if (shmem > 48 * 1024 && hipFuncSetAttribute((const void*)delta_chunk_prep_kernel<N, HD>,                               \
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)      \
       return TQ_ERR_UNSUPPORTED;                                                                                             \
-    hipLaunchKernelGGL((delta_chunk_prep_kernel<N, HD>), dim3(H, (unsigned)chunks), dim3(512), shmem, st, qn, kn, vc, beta,  \
-                       ag, a_log, dt_bias, cu_seqlens, B, d, scratch);                                                       \
+    hipLaunchKernelGGL((delta_chunk_prep_kernel<N, HD>), dim3(H, chunks), dim3(512), shmem, st, qn, kn, vc, beta, ag, a_log, \
+                       dt_bias, cu_seqlens, w, d, scratch);                                                                  \
   } while (0)
 #define TQ_PREP_CASE(N)               \
   case N:                             \
     if (head_decay) TQ_PREP(N, true); \
     else TQ_PREP(N, false);           \
     break;
-  switch (nd) {
-    TQ_PREP_CASE(1) TQ_PREP_CASE(2) TQ_PREP_CASE(3) TQ_PREP_CASE(4) TQ_PREP_CASE(5) TQ_PREP_CASE(6) TQ_PREP_CASE(7)
-    TQ_PREP_CASE(8) TQ_PREP_CASE(9) TQ_PREP_CASE(10) TQ_PREP_CASE(11) TQ_PREP_CASE(12) TQ_PREP_CASE(13) TQ_PREP_CASE(14)
-    TQ_PREP_CASE(15) TQ_PREP_CASE(16)
-  }
+    switch (nd) {
+      TQ_PREP_CASE(1) TQ_PREP_CASE(2) TQ_PREP_CASE(3) TQ_PREP_CASE(4) TQ_PREP_CASE(5) TQ_PREP_CASE(6) TQ_PREP_CASE(7)
+      TQ_PREP_CASE(8) TQ_PREP_CASE(9) TQ_PREP_CASE(10) TQ_PREP_CASE(11) TQ_PREP_CASE(12) TQ_PREP_CASE(13) TQ_PREP_CASE(14)
+      TQ_PREP_CASE(15) TQ_PREP_CASE(16)
+    }
 #undef TQ_PREP_CASE
 #undef TQ_PREP
-  const dim3 grid((unsigned)(H * (V / 16)), B);
+    const dim3 grid((unsigned)(H * (V / 16)), w.B);
 #define TQ_SCAN(NB) \
-  hipLaunchKernelGGL(delta_chunk_scan_kernel<NB>, grid, dim3(256), 0, st, scratch, cu_seqlens, slots, state, state_stride, d, o_raw)
-  if (nd <= 4) TQ_SCAN(1);
-  else if (nd <= 8) TQ_SCAN(2);
-  else TQ_SCAN(4);
+  hipLaunchKernelGGL(delta_chunk_scan_kernel<NB>, grid, dim3(256), 0, st, scratch, cu_seqlens, slots, state, state_stride, w, d, o_raw)
+    if (nd <= 4) TQ_SCAN(1);
+    else if (nd <= 8) TQ_SCAN(2);
+    else TQ_SCAN(4);
 #undef TQ_SCAN
-  TQ_LAUNCH_CHECK();
-  if (all_long) return 0;
+    TQ_LAUNCH_CHECK();
+    return 0;
+  };
+  // windows of as many chunks of every run as the scratch surely holds
+  const int held = (int)dc_held(H, D, V), last = longest / DC_T + (longest % DC_T ? 1 : 0);
+  for (int b0 = 0; b0 < B; b0 += held) {
+    DeltaWindow w{b0, B - b0 < held ? B - b0 : held, 0, 0};
+    const int64_t all = dc_bound(T, w.B);
+    for (; w.first < last; w.first += w.count) {
+      // runs that go on behind the windows before: each has more tokens than those took, and the DC_FROM that make it long
+      const int64_t tokens = (int64_t)w.first * DC_T + 1, most = T / (tokens > DC_FROM ? tokens : DC_FROM), runs = w.B < most ? w.B : most;
+      if (runs == 0) break;
+      const int64_t count = all <= held ? last : held / runs;
+      w.count = (int)(count < last - w.first ? count : last - w.first);
+      if (int rc = launch(w, (unsigned)(all < runs * w.count ? all : runs * w.count))) return rc;
+    }
+  }
+  if (shortest >= DC_FROM) return 0;
   return delta_short_runs(qn, kn, vc, beta, ag, a_log, dt_bias, cu_seqlens, slots, state, state_stride, d, DC_FROM, T, B, o_raw, st);
 }

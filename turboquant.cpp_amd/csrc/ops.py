@@ -101,7 +101,7 @@ _SIGNATURES = {
                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "tq_delta_chunk_scratch": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "tq_delta_chunks": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int,
-                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
+                        _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
     "tq_delta_decode": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr,
                         _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr],
     "tq_delta_out": [_c_ptr, _c_ptr, _c_ptr, _c_f32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int,
@@ -1514,7 +1514,7 @@ def _delta_chunks(k, qn, kn, vc, beta, ag, a_log, dt_bias, runs, state, stride, 
     scratch = torch.empty(n, dtype=torch.float32, device=qn.device)
     _run(k, lib.tq_delta_chunks(_ptr(qn), _ptr(kn), _ptr(vc), _ptr(beta), _ptr(ag), _ptr(a_log), _ptr(dt_bias), int(a_log is None),
                                 _ptr(runs["cu_seqlens"]), _ptr(runs["slots"]), _ptr(state), stride, *dims.sizes(), T, B,
-                                int(shortest >= DELTA_CHUNKS_FROM), _ptr(scratch), _ptr(o), _stream()))
+                                longest, shortest, _ptr(scratch), _ptr(o), _stream()))
     return True
 
 

@@ -145,7 +145,7 @@ int tq_delta_scan_h(const float* qn, const float* kn, const float* vc, const flo
 int64_t tq_delta_chunk_scratch(int T, int B, int H, int D, int V);
 int tq_delta_chunks(const float* qn, const float* kn, const float* vc, const float* beta, const float* ag, const float* a_log,
         const float* dt_bias, int head_decay, const int* cu_seqlens, const int* slots, float* state, int64_t state_stride,
-        int H, int G, int D, int V, int taps, int T, int B, int all_long, float* scratch, float* o_raw, hipStream_t st);
+        int H, int G, int D, int V, int taps, int T, int B, int longest, int shortest, float* scratch, float* o_raw, hipStream_t st);
 int tq_delta_out_h(const float* o_raw, const float* norm_w, float eps, const float* P, int gate_kind,
         const int* cu_seqlens, const int* slots, float* state, int64_t state_stride, int H, int G, int D, int V, int taps,
         int T, int B, void* out, hipStream_t st);
