@@ -400,6 +400,43 @@ def test_some_hundred_rows_of_one_matrix(ops, M, N, K, kind):
     assert torch.equal(odd[..., : M - 1, :], y[..., : M - 1, :]) and torch.isnan(odd[..., M - 1, :]).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 33, 64), (128, 2050, 576), (190, 5632, 256), (500, 5632, 128), (700, 4099, 192)])
+@pytest.mark.parametrize("kind", ["pair", "clamped", "alone", "bias"])
+def test_the_other_forms_of_some_hundred_rows(ops, M, N, K, kind):
+    """The same products as a gated pair into the activation type, as a clamped pair, with an activation of their own behind a
+    bias, and with a bias alone (for the library also of rows that lie further apart than k): what the formula gives (|f'| < 1.13 of either gate; the
+    sums as in the test before; the result rounded to 8 bits, and what the gate is off), and the bits of the same rows taken
+    through a row index, which go in other tiles."""
+    a, w, v = rnd((M, K), torch.bfloat16, 51).to(DEV), rnd((N, K), torch.bfloat16, 52, 0.1), rnd((N, K), torch.bfloat16, 53, 0.1)
+    b, L = rnd((N,), torch.bfloat16, 54), 0.7
+    kw = {"pair": {"w2": v.to(DEV), "out_act": True}, "clamped": {"w2": v.to(DEV), "out_act": True, "pair_limit": L},
+          "alone": {"bias": b.to(DEV), "out_act": True, "activation": "gelu_tanh", "act_alone": True}, "bias": {"bias": b.to(DEV)}}[kind]
+    y = ops.gemm(a, w.to(DEV), "bfloat16", **kw)
+    rows = torch.arange(M, dtype=torch.int32, device=DEV)
+    assert torch.equal(ops.gemm(a, w.to(DEV), "bfloat16", a_rows=rows, **kw), y)
+    if kind == "bias":
+        wide, apart = torch.full((M, K + 24), math.nan, dtype=torch.bfloat16, device=DEV), torch.empty_like(y)
+        wide[:, 8:8 + K] = a
+        wd, bd = w.to(DEV), b.to(DEV)
+        ops._run("gemm", ops.library("bfloat16").tq_gemm_mfma(wide[:, 8:].data_ptr(), K + 24, None, 1, wd.data_ptr(), None, 0, None, None,
+                                                              bd.data_ptr(), ops._WTYPE[bd.dtype], apart.data_ptr(), N, 0, M, N, K, 64, 1,
+                                                              0, ops._stream()))
+        assert torch.equal(apart, y)
+    c = a.cpu().double()
+    x, xe, z, ze = c @ w.double().T, 2.0 ** -23 * K * (c.abs() @ w.double().abs().T), c @ v.double().T, 2.0 ** -23 * K * (c.abs() @ v.double().abs().T)
+    silu, gelu = torch.nn.functional.silu, lambda t: torch.nn.functional.gelu(t, approximate="tanh")
+    if kind == "pair":
+        ref, bound = silu(x) * z, 1.13 * xe * z.abs() + x.abs() * ze
+    elif kind == "clamped":
+        ref, bound = silu(x.clamp(max=L)) * (z.clamp(-L, L) + 1), 1.13 * xe * (L + 1) + x.abs() * ze
+    else:
+        x, xe = x + b.double(), xe + 2.0 ** -23 * (x.abs() + b.double().abs())
+        ref, bound = (gelu(x), 1.13 * xe) if kind == "alone" else (x, xe)
+    if kind != "bias":
+        bound = bound + 2.0 ** -8 * ref.abs() + 2.0 ** -20 * x.abs() * (1 if kind == "alone" else z.abs() + 1)
+    assert ((y.cpu().double() - ref).abs() <= bound).all(), ((y.cpu().double() - ref).abs() / bound).max()
+
+
 @pytest.mark.parametrize("act", ACTS)
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "relu2"])
 @pytest.mark.parametrize("M,N,K", [(3, 40, 72), (40, 130, 264), (150, 200, 136), (9, 33, 50)])

@@ -677,9 +677,10 @@ __global__ __launch_bounds__(1024) void gemm_ring_kernel(MfmaGemmArgs g) {
 // takes 0.8 us a step here (load, wait, store into LDS, barrier, and every product behind its own reads), for 64 x 128
 // outputs, so that 97 rows by 6,144 x 2,048 kept 96 compute units busy for 26 us.  Here the tiles are smaller where
 // that fills the chip, go from memory straight into a ring of S stages of LDS, S - 1 of them on their way while one is
-// multiplied (as in the ring kernel above), and a wave asks for all the operands of a step at once: 14.5 us, 0.4 us a
-// step.  With the operands read one product at a time, as the compiler puts it by itself: 15.7; two tiles of 64 to a
-// step: 15.9. The sums of an output run over k as in the tile kernel: same bits.
+// multiplied (as in the ring kernel above): 15.0 us, 0.4 us a step.  Two tiles of 64 to a step: 15.9.  The compiler puts a
+// step's products between its reads of LDS; all reads before the first product, held there by a scheduling barrier, is
+// level (14.8; a gated pair of 97 rows by twice 5,632 x 2,048 23.6 and 23.6, by twice 20,480 x 3,584 85.9 and 85.2, of
+// 512 rows by that 229 and 240, of 320 161 and 159).  The sums of an output run over k as in the tile kernel: same bits.
 template <int WN, bool DUAL, bool OUT_ACT, int S>
 __global__ __launch_bounds__(128 * WN) void gemm_few_tiles_kernel(MfmaGemmArgs g) {
   constexpr int NT = 128 * WN, BM = 64, BN = 32 * WN, ROWS = BM + BN * (DUAL ? 2 : 1), STAGE = ROWS * TBK, L = ROWS * 8 / NT;
@@ -742,7 +743,6 @@ __global__ __launch_bounds__(128 * WN) void gemm_few_tiles_kernel(MfmaGemmArgs g
     const bf16_t* Ac = ring + cur * STAGE;
     const bf16_t* Wc = Ac + BM * TBK;
     const bf16_t* Vc = Wc + BN * TBK;
-    // all reads of the step first: with one or two waves to a SIMD nothing else hides the way through LDS
     u32x4 af[TBK / 16], wf[TBK / 16], vf[TBK / 16];
 #pragma unroll
     for (int j = 0; j < TBK / 16; ++j) {
@@ -750,7 +750,6 @@ __global__ __launch_bounds__(128 * WN) void gemm_few_tiles_kernel(MfmaGemmArgs g
       wf[j] = *reinterpret_cast<const u32x4*>(Wc + swz(wn * 32 + lr, 2 * j + lc));
       if (DUAL) vf[j] = *reinterpret_cast<const u32x4*>(Vc + swz(wn * 32 + lr, 2 * j + lc));
     }
-    asm volatile("" ::: "memory");
 #pragma unroll
     for (int j = 0; j < TBK / 16; ++j) {
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[j]), __builtin_bit_cast(bf16x8, wf[j]), acc, 0, 0, 0);
@@ -847,7 +846,7 @@ static int launch_few_tiles(const MfmaGemmArgs& g, bool out_act, int splits, hip
 }
 
 // Which of its tiles a product of gemm_few_tiles_kernel takes.  Narrow ones, with a deep ring, while there is at most
-// one to a compute unit: then what counts is how soon a tile is done (97 rows by 6,144 x 2,048: 14.5 us against 19.2
+// one to a compute unit: then what counts is how soon a tile is done (97 rows by 6,144 x 2,048: 15.0 us against 19.2
 // in wide ones and 26.0 in the tile kernel).  More of them take wide tiles, which read `a` half as often (320 rows:
 // 20.2 against 22.3, tile kernel 26.1).  A gated pair has two matrices' tiles in a stage and so fewer stages (97 rows
 // by twice 5,632 x 2,048: 23.5 us, tile kernel 35.6; 320 rows in wide ones 30.8, 35.7), and where its tiles are many,
@@ -983,13 +982,14 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
   return s;
 }
 
-// a: bfloat16 [.., K] with row stride lda (a multiple of 8, as K must be); w, w2: bfloat16. tile_rows: with tile_group
-// set, the padding unit of the row order (16, 32, 64, 128 or 256); else a hint that is ignored.  64 + TQ_TILE_PAIRS:
-// units of 64 taken two at a time, by the items that the row order lists behind its row tiles (tile_group[M / 64 ..],
-// n_tiles[1]). splits > 1 (as tq_gemm_mfma_splits says, for a plain product into float): run z of k goes to out + z *
-// M * ldc, the bias to run 0; the sum over the runs is the caller's. gate: the activation of the gated pair; without
-// w2 and with TQ_GEMM_ACT_ALONE added, the activation that the plain product's result (bias included) passes before it
-// is stored (a feed-forward of two matrices needs no launch between them).
+// a: bfloat16 [.., K] with row stride lda (a multiple of 8, as K must be); w, w2: bfloat16.
+// tile_rows: with tile_group set, the padding unit of the row order (16, 32, 64, 128 or 256); else a hint that is
+// ignored.  64 + TQ_TILE_PAIRS: units of 64 taken two at a time, by the items that the row order lists behind its
+// row tiles (tile_group[M / 64 ..], n_tiles[1]).
+// splits > 1 (as tq_gemm_mfma_splits says, for a plain product into float): run z of k goes to out + z * M * ldc,
+// the bias to run 0; the sum over the runs is the caller's.
+// gate: the activation of the gated pair; without w2 and with TQ_GEMM_ACT_ALONE added, the activation that the plain
+// product's result (bias included) passes before it is stored (a feed-forward of two matrices needs no launch between them).
 TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gather, const void* w, const void* w2,
                         int64_t group_stride, const int* tile_group, const int* n_tiles, const void* bias,
                         int bias_type, void* out, int64_t ldc, int out_is_act, int M, int N, int K, int tile_rows,
