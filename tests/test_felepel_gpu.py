@@ -633,3 +633,47 @@ def test_the_delta_rule_in_more_chunks_than_the_scratch_holds(head_decay):
             assert torch.equal(step(lo + at, [size], [slot], cut), o[lo + at:lo + at + size]), (slot, at)
         lo += n
     assert torch.equal(whole, cut)
+
+
+@pytest.mark.parametrize("head_decay", [False, True])
+def test_the_delta_rule_in_chunks_is_no_further_off(head_decay):
+    """With decays as models have them, a run in chunks is no further from 64 bits than in portions of 47 tokens, which go token by
+    token: its read-outs and its state."""
+    from turboquant_cpp_amd.csrc import ops
+    H, D, V, n = 16, 128, 128, 329
+    dims = ops.DeltaDims(H, H, D, V, 4, 0, 0, head_decay=True) if head_decay else ops.DeltaDims(H, H, D, V, 4, 8, 8)
+    g = torch.Generator().manual_seed(8)
+    rnd = lambda *s: torch.randn(s, generator=g)      # noqa: E731
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)      # noqa: E731
+    qn, kn, vc = (unit(rnd(n, H, D)) * D ** -0.5).flatten(1), unit(rnd(n, H, D)).flatten(1), rnd(n, H * V)
+    beta, a_log, state = torch.sigmoid(rnd(n, H)), 0.5 * rnd(H), 0.1 * rnd(1, dims.state_floats)
+    soft = torch.nn.functional.softplus
+    if head_decay:
+        ag, dt_bias = torch.exp(-torch.exp(a_log) * soft(rnd(n, H) - 3)), None
+        decay = ag.double()[:, :, None].expand(n, H, D)
+    else:
+        ag, dt_bias = rnd(n, H * D + H * V), 0.5 * rnd(H * D) - 3
+        decay = torch.exp(-torch.exp(a_log.double())[:, None] * soft((ag[:, :H * D] + dt_bias).double()).view(n, H, D))
+    S, want = state[0, :H * D * V].double().view(H, D, V), []
+    for t in range(n):
+        S = S * decay[t][:, :, None]
+        k, q = kn[t].double().view(H, 1, D), qn[t].double().view(H, 1, D)
+        u = beta[t].double()[:, None] * (vc[t].double().view(H, V) - (k @ S)[:, 0])
+        S = S + k.transpose(1, 2) * u[:, None]
+        want.append((q @ S)[:, 0].flatten())
+    want = torch.stack(want)
+
+    def off(size):
+        into, parts = state.to("cuda:0"), []
+        for at in range(0, n, size):
+            q, k, v, b, a = (t[at:at + size].to("cuda:0") for t in (qn, kn, vc, beta, ag))
+            runs = {"cu_seqlens": torch.tensor([0, q.shape[0]], dtype=torch.int32, device="cuda:0"),
+                    "slots": torch.zeros(1, dtype=torch.int32, device="cuda:0"), "decode": False}
+            if head_decay:
+                parts.append(ops.delta_scan_h(q, k, v, b, a, runs, into, dims, "float32"))
+            else:
+                parts.append(ops.delta_scan(q, k, v, b, a, a_log.to("cuda:0"), dt_bias.to("cuda:0"), runs, into, dims, "float32"))
+        got = into[0, :H * D * V].cpu().double().view(H, D, V)
+        return (torch.cat(parts).cpu().double() - want).norm().item(), (got - S).norm().item()
+    (o, s), (o1, s1) = off(n), off(47)
+    assert o <= o1 and s <= s1, (o / o1, s / s1)

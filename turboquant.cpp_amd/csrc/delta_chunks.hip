@@ -17,7 +17,8 @@
 //
 // Scratch (float), per chunk and head, in the order in which a wave's lanes of the scan take their operands (four floats a
 // lane, 64 lanes a tile of 16 x 16): W [2 token tiles][D / 16] | G q alike | (G_32 / G) k [D / 16][2] | U0 [V / 16][2] |
-// b [2][2] | G_32 [D].
+// b [2][2] | G_32 [D].  Row 4 g + i of a tile of tokens is token 4 i + g: an instruction then takes four tokens that follow
+// one another, and sums over tokens run in order, the latest and largest term last.
 #include "delta_rule.h"
 
 #define DC_T 32
@@ -42,6 +43,8 @@ __device__ __forceinline__ int dc_chunks(int n) { return n >= DC_FROM ? (n + DC_
 struct DeltaWindow {
   int b0, B, first, count;
 };
+// The token of row r of a tile, and the row of token r.
+__device__ __forceinline__ int dc_turned(int r) { return 4 * (r % 4) + r / 4; }
 // How many of its chunks a run of n tokens has there.
 __device__ __forceinline__ int dc_inside(const DeltaWindow& w, int n) { return min(max(dc_chunks(n) - w.first, 0), w.count); }
 
@@ -76,7 +79,9 @@ __device__ __forceinline__ bool dc_find(const int* __restrict__ cu_seqlens, cons
 // what lies between two tokens of different halves is one of each); the partial sums of a and b; a.
 // The pairs of one half are formed channel by channel with the product of the decays between them (a lane keeps k_s times
 // that product for D / 16 channels and walks through t); those of different halves are products of matrices, by waves 0 to 3
-// while the others write the decayed rows out.  The triangular system then takes a column of its right side to a thread.
+// while the others write the decayed rows out.  The waves' shares of a pair, and the products of decays, are put together in 64
+// bits: a pair's rounding stands alone where token by token the state's rows round each by itself, and would weigh more.
+// The triangular system then takes a column of its right side to a thread.
 // A workgroup is a chain of such steps with a barrier between (19 us alone); two of 80 KB share a compute unit, and 2,048 tokens of
 // 16 heads of 128 x 128, 1,024 workgroups, take 59 us (79 with loads under conditions, each of which is waited for at once).
 template <int ND, bool HEAD>
@@ -190,17 +195,17 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
   }
   __syncthreads();
   const int pt = tid / 16 % 16, ps = tid % 16;              // the pair of a 16 x 16 block that this thread puts together
-  const int b_at = (pt + 16 * (ps / 4)) * 4 + ps % 4;       // and its place in b's tiles: lane pt + 16 (ps / 4), number ps % 4
+  const int b_at = (dc_turned(pt) + 16 * (ps % 4)) * 4 + ps / 4;      // and its place in b's tiles
   {
     const int half = tid / 256, i = tid % 256;
-    float a = 0.f, bb = 0.f;
+    double a = 0., bb = 0.;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       a += part[(half + 2 * w) * 512 + i];
       bb += part[(half + 2 * w) * 512 + 256 + i];
     }
-    am[(16 * half + pt) * 36 + 16 * half + ps] = ps < pt ? bt[16 * half + pt] * a : 0.f;
-    b_out[3 * half * 256 + b_at] = ps <= pt ? bb : 0.f;
+    am[(16 * half + pt) * 36 + 16 * half + ps] = ps < pt ? (float)(bt[16 * half + pt] * a) : 0.f;
+    b_out[3 * half * 256 + b_at] = ps <= pt ? (float)bb : 0.f;
   }
   __syncthreads();
   for (int idx = tid; idx < 2 * D; idx += 512) {
@@ -208,16 +213,16 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
     float g[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) g[i] = gs[(first + i) * LD + d];
-    float p = 1.f;
+    double p = 1.;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       p *= g[i];
-      up[(first + i) * LD + d] = p;
+      up[(first + i) * LD + d] = (float)p;
     }
-    p = 1.f;
+    p = 1.;
 #pragma unroll
     for (int i = 15; i >= 0; --i) {
-      down[(first + i) * LD + d] = p;
+      down[(first + i) * LD + d] = (float)p;
       p *= g[i];
     }
   }
@@ -251,7 +256,7 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
     const int tid2 = tid - 256;
     for (int idx = tid2; idx < 2 * ND * 64; idx += 256) {
       const int l = idx % 64, tile = idx / 64, tb = tile / ND, db = tile % ND;
-      const int t = 16 * tb + l % 16, d = 16 * db + 4 * (l / 16);
+      const int t = 16 * tb + dc_turned(l % 16), d = 16 * db + 4 * (l / 16);
       const dc_f32x4 q = *reinterpret_cast<const dc_f32x4*>(qs + t * LD + d);
       dc_f32x4 p = *reinterpret_cast<const dc_f32x4*>(up + t * LD + d);
       if (tb) p *= *reinterpret_cast<const dc_f32x4*>(up + 15 * LD + d);
@@ -259,25 +264,25 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
     }
     for (int idx = tid2; idx < ND * 2 * 64; idx += 256) {
       const int l = idx % 64, tile = idx / 64, db = tile / 2, tb = tile % 2;
-      const int d = 16 * db + l % 16, t = 16 * tb + 4 * (l / 16);
+      const int d = 16 * db + l % 16, t = 16 * tb + l / 16;
       const float rest = tb ? 1.f : up[31 * LD + d];
       dc_f32x4 k;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) k[i] = ks[(t + i) * LD + d] * down[(t + i) * LD + d] * rest;
+      for (int i = 0; i < 4; ++i) k[i] = ks[(t + 4 * i) * LD + d] * down[(t + 4 * i) * LD + d] * rest;
       *reinterpret_cast<dc_f32x4*>(k_out + (size_t)idx * 4) = k;
     }
     for (int d = tid2; d < D; d += 256) g_out[d] = up[15 * LD + d] * up[31 * LD + d];
   }
   __syncthreads();
   if (tid < 256) {
-    float a = 0.f, bb = 0.f;
+    double a = 0., bb = 0.;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       a += across[w * 512 + tid];
       bb += across[w * 512 + 256 + tid];
     }
-    am[(16 + pt) * 36 + ps] = bt[16 + pt] * a;
-    b_out[2 * 256 + b_at] = bb;
+    am[(16 + pt) * 36 + ps] = (float)(bt[16 + pt] * a);
+    b_out[2 * 256 + b_at] = (float)bb;
   }
   __syncthreads();
   // the triangular system, a column to a thread
@@ -316,11 +321,11 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
 #pragma unroll
       for (int f = 0; f < DC_T / 4; ++f)      // tile (col / 16, f / 4), lane col % 16 + 16 (f % 4)
         *reinterpret_cast<dc_f32x4*>(u_out + ((size_t)(col / 16 * 2 + f / 4) * 64 + col % 16 + 16 * (f % 4)) * 4) =
-            dc_f32x4{x[4 * f], x[4 * f + 1], x[4 * f + 2], x[4 * f + 3]};
+            dc_f32x4{x[f / 4 * 16 + f % 4], x[f / 4 * 16 + f % 4 + 4], x[f / 4 * 16 + f % 4 + 8], x[f / 4 * 16 + f % 4 + 12]};
     } else {
 #pragma unroll
-      for (int t = 0; t < DC_T; ++t)           // tile (t / 16, d / 16), lane t % 16 + 16 (d % 16 / 4), number d % 4 of channel d
-        w_out[((size_t)(t / 16 * ND + (col - V) / 16) * 64 + t % 16 + 16 * ((col - V) % 16 / 4)) * 4 + (col - V) % 4] = -x[t];
+      for (int t = 0; t < DC_T; ++t)           // tile (t / 16, d / 16), lane of t's row + 16 (d % 16 / 4), number d % 4 of channel d
+        w_out[((size_t)(t / 16 * ND + (col - V) / 16) * 64 + dc_turned(t % 16) + 16 * ((col - V) % 16 / 4)) * 4 + (col - V) % 4] = -x[t];
     }
   }
 }
@@ -387,7 +392,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
     to.bq = tile(6 * ND + 2 * VB + (wave == 0 ? 0 : wave == 1 ? 2 : 3));      // b's tile (0, 0), (1, 0) or (1, 1)
   };
   dc_f32x4 po[2] = {zero, zero};      // this wave's share of the o of the chunk that has its u
-  // two numbers of the o of chunk c from the waves' shares, in wave order: token tile wave / 2, rows 4 g4 + 2 (wave % 2) on
+  // two numbers of the o of chunk c from the waves' shares, in wave order: token tile wave / 2, rows 4 g4 + 2 (wave % 2) and the next
   auto read_out = [&](const float (*from)[4][256], int c, bool last) {
     float y0 = 0.f, y1 = 0.f;
 #pragma unroll
@@ -395,10 +400,10 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
       const float2 y = *reinterpret_cast<const float2*>(&from[ww][2 + wave / 2][lane * 4 + 2 * (wave % 2)]);
       y0 += y.x, y1 += y.y;
     }
-    const int t = 16 * (wave / 2) + 4 * g4 + 2 * (wave % 2);
+    const int t = 16 * (wave / 2) + 8 * (wave % 2) + g4;
     float* row = o_raw + ((size_t)(t0 + c * DC_T) * H + h) * V + vb * 16 + ((size_t)t * H * V + r);
     if (!last || c * DC_T + t < n) row[0] = y0;
-    if (!last || c * DC_T + t + 1 < n) row[(size_t)H * V] = y1;
+    if (!last || c * DC_T + t + 4 < n) row[(size_t)4 * H * V] = y1;
   };
   // (neither loads nor stores are under a condition, or the compiler would wait for all loads on their way at each use of some)
   auto one_chunk = [&](int c, Operands& in, bool first) {
@@ -467,13 +472,13 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
         y = before;
 #pragma unroll 1
         for (int t = 0; t < 16; ++t) {
-          const float mine_u = t % 4 == 0 ? us[0] : t % 4 == 1 ? us[1] : t % 4 == 2 ? us[2] : us[3];
-          const float mine_b = t % 4 == 0 ? in.bq[0] : t % 4 == 1 ? in.bq[1] : t % 4 == 2 ? in.bq[2] : in.bq[3];
-          const float ut = __shfl(mine_u, r + 16 * (t / 4), TQ_WAVE);
+          const float mine_u = t / 4 == 0 ? us[0] : t / 4 == 1 ? us[1] : t / 4 == 2 ? us[2] : us[3];
+          const float mine_b = t / 4 == 0 ? in.bq[0] : t / 4 == 1 ? in.bq[1] : t / 4 == 2 ? in.bq[2] : in.bq[3];
+          const float ut = __shfl(mine_u, r + 16 * (t % 4), TQ_WAVE);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float bt = __shfl(mine_b, 4 * g4 + i + 16 * (t / 4), TQ_WAVE);
-            if (t <= 4 * g4 + i) y[i] = fmaf(bt, ut, y[i]);
+            const float bt = __shfl(mine_b, 4 * g4 + i + 16 * (t % 4), TQ_WAVE);
+            if (t <= 4 * i + g4) y[i] = fmaf(bt, ut, y[i]);
           }
         }
       }
