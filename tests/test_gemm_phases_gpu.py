@@ -1,0 +1,76 @@
+"""Products over experts by items of up to four units of 64 rows: the tile of 64 MI rows by 256 columns (128 of a gated pair)
+whose two groups of waves take turns.  Its sums run over k as in the tile kernel, so its bits are the tile kernel's."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from turboquant_cpp_amd.csrc import ops as module
+    return module
+
+
+def drawn(shape, seed, scale=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn(shape, generator=gen) * scale).to(torch.bfloat16).to(DEV)
+
+
+def order(ops, counts, unit=64, item_units=4):
+    """A token per pair, experts in turn with counts[e] tokens each, in a mixed order."""
+    ids = torch.tensor([e for e, n in enumerate(counts) for _ in range(n)], dtype=torch.int32)
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(7))]
+    return ops.moe_align(ids[:, None].contiguous().to(DEV), len(counts), unit, "bfloat16", item_units=item_units)
+
+
+# rows per expert: items of 1, 2, 3 and 4 units, full and with padding, an item of one row behind full ones, an empty expert
+COUNTS = [1, 63, 64, 65, 129, 192, 0, 255, 256, 257, 700]
+
+
+def test_items_of_four_units(ops):
+    """From one workgroup and, from 8,192 pairs on, from several: an expert's row tiles four at a time."""
+    for counts in (COUNTS, [3000, 0, 1, 5000, 191]):
+        st, _slot, te, nt = order(ops, counts)
+        units, items = nt.tolist()
+        of = [-(-n // 64) for n in counts]
+        assert units == sum(of) and te[:units].tolist() == [e for e, n in enumerate(of) for _ in range(n)]
+        first = [sum(of[:e]) for e in range(len(of))]
+        assert te[st.numel() // 64:][:items].tolist() == [first[e] + u for e, n in enumerate(of) for u in range(0, n, 4)]
+
+
+# k: 2, 3, 4, 5 and 9 steps of 64 (the rings hold 2 to 4 tiles); columns: less than a wave's 32, no multiple of 8, one more than a tile
+@pytest.mark.parametrize("K,N", [(128, 24), (192, 100), (256, 129), (320, 256), (576, 263)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_products_by_items_of_four(ops, K, N, gated):
+    T, E = sum(COUNTS), len(COUNTS)
+    st, _slot, te, nt = order(ops, COUNTS)
+    x, w = drawn((T, K), 1), drawn((E, N, K), 2, 0.1)
+    w2 = drawn((E, N, K), 3, 0.1) if gated else None
+    live = st >= 0
+    forms = [dict(w2=w2, out_act=True, activation=a, **more) for a in ("silu", "gelu_tanh") for more in ({}, {"pair_limit": 0.5})] if gated \
+        else [dict(out_act=True), dict(), dict(out_act=True, activation="gelu", act_alone=True)]
+    for form in forms:
+        got, want = (ops.gemm(x, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=rows, **form)
+                     for rows in (64 + ops.TILE_PAIRS, 64))
+        assert torch.equal(got[live], want[live]), form
+    # and the formula: a sum of K products of bfloat16 factors is off by at most K roundings of 32 bits to its largest partial sum
+    if not gated:
+        tokens, expert = st[live].long(), te[torch.nonzero(live)[:, 0] // 64].long()
+        got = ops.gemm(x, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=64 + ops.TILE_PAIRS)[live].double()
+        for e in range(E):
+            rows = expert == e
+            a, b = x[tokens[rows]].double(), w[e].double()
+            assert ((got[rows] - a @ b.T).abs() <= K * 2.0 ** -24 * (a.abs() @ b.abs().T)).all()
+
+
+def test_rows_in_place_and_a_wider_result(ops):
+    """The second product reads row m for row m, and rows of padding are not written."""
+    K, N = 192, 200
+    st, _slot, te, nt = order(ops, COUNTS)
+    h, w = drawn((st.numel(), K), 4), drawn((len(COUNTS), N, K), 5, 0.1)
+    got, want = (ops.gemm(h, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=rows, gather=False)
+                 for rows in (64 + ops.TILE_PAIRS, 64))
+    assert torch.equal(got[st >= 0], want[st >= 0])

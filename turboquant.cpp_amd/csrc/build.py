@@ -23,7 +23,7 @@ COMMON_SOURCES = ["elementwise.hip", "gemm_generic.hip", "attention_generic.hip"
                   "host/engine.cpp", "host/vendor.cpp"]
 SOURCES = {
     "float32": COMMON_SOURCES + ["gemm_f32.hip", "attention_f32.hip"],
-    "bfloat16": COMMON_SOURCES + ["gemm_mfma.hip", "attention_mfma.hip", "probe.hip"],
+    "bfloat16": COMMON_SOURCES + ["gemm_mfma.hip", "gemm_phases.hip", "attention_mfma.hip", "probe.hip"],
 }
 HEADERS = ["common.h", "value_tiles.h", "linear_chunks.h", "score_mod.h", "gates.def", "no_alloc.h", "gemm_mfma.h", "delta_rule.h", "turboquant_kernels.h", "host/engine.h", "host/vendor.h",
            "host/host_common.h"]

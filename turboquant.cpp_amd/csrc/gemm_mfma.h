@@ -67,3 +67,12 @@ __device__ __forceinline__ void store_out(const MfmaGemmArgs& g, int m, int n, f
     ((float*)g.out)[(size_t)m * g.ldc + n] = v;
 }
 
+#define TBK 64      // of k in a tile
+// Straight from memory into LDS, without registers in between: 16 bytes a lane, the wave's 64 chunks one behind the other.
+__device__ __forceinline__ void load_to_lds16(const bf16_t* src, bf16_t* wave_base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)wave_base, 16, 0, 0);
+}
+
+// gemm_phases.hip: products of many rows (K a multiple of TBK), of one matrix or of a matrix per expert by the row order's items
+int launch_gemm_phases(const MfmaGemmArgs& g, bool dual, bool out_act, hipStream_t st);

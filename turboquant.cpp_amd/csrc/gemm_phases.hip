@@ -1,0 +1,388 @@
+// Products of many rows in tiles of up to 256 x 256 outputs by two groups of four waves that take turns: while one group
+// multiplies, the other reads its operands from LDS and asks for what comes later, and a barrier between the two phases
+// lets them change places.  Same contract, operand layouts and order of sums as the tile kernel in gemm_mfma.hip: same bits.
+//
+// What bounds it: a tile of 64 of k is 64 KB on its way through L2 and 8.4 million multiply-adds, 0.85 us of the matrix
+// instructions of a compute unit at their full clock and about as long as its path to L2 takes for the bytes, so each has to go on
+// beside the other:
+//  * a wave owns 32 MI x 64 outputs (MI up to 4), for which its reads from LDS (8 MI + 16 operand reads a tile of 64) take less time
+//    than its products, and the group that multiplies has the matrix instructions to itself;
+//  * loads go straight into LDS and are asked for by the reading group alone, behind its reads.  A wave that asks for more than the
+//    path takes stands still until there is room, and in front of products or reads that time is lost: 13,197 tokens by 8 of 64
+//    experts of 2,560 x 3,584 took 4,215 us with two loads in front of every phase of a wave and 3,739 this way;
+//  * the tiles wait in rings of two (a) and three (w; four where an item has up to 128 rows) tiles, so that a tile of w is asked
+//    for five to seven phases of 0.25 us before it is read: memory's time where an expert's matrices are read once.  Rings of half
+//    tiles of 32 of k are level with two whole ones: rows of 64 bytes halve what L2 gives.
+// One workgroup fills a compute unit's LDS, so what the waves do behind the last tile has nothing to hide behind: outputs go through
+// LDS into stores of 16 bytes a lane, whole lines side by side (a test and a store of a value each took 16 us a tile).
+// Measured, us, against items of two units by 16 waves through a ring of three stages: 64 experts of 2,560 x 3,584 with 1,650 rows
+// each, gated pair 4,760 -> 3,739 (1,036 TFLOP/s), second product 2,590 -> 1,943; 60 experts of 1,408 x 2,048 with 137 rows each
+// 219 -> 173 and 147 -> 103, with 68 rows 149 -> 147 and 96 -> 90.  On operands that are zeros (less power) 8,192 x 8,192 x 8,192
+// takes 638 instead of 880.
+#include "common.h"
+
+#include "gemm_mfma.h"
+
+#define PH_FENCE()                        \
+  do {                                    \
+    asm volatile("" ::: "memory");        \
+    __builtin_amdgcn_sched_barrier(0);    \
+  } while (0)
+#define PH_NEXT()                         \
+  do {                                    \
+    PH_FENCE();                           \
+    __builtin_amdgcn_s_barrier();         \
+    PH_FENCE();                           \
+  } while (0)
+// s_waitcnt: vmcnt in bits 3..0 and 15..14, lgkmcnt in bits 11..8, expcnt in bits 6..4
+#define PH_LDS_DONE() __builtin_amdgcn_s_waitcnt(0xC07F)
+template <int N>
+__device__ __forceinline__ void loads_left() {      // at most N loads of this wave are on their way
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// v[j] = f(v[j]), the switch once for all of them
+template <int N>
+__device__ __forceinline__ void gate_many(float (&v)[N], int kind) {
+  switch (kind) {
+#define TQ_GATE(name, expr)                          \
+  case TQ_GATE_##name:                               \
+    _Pragma("unroll") for (int j = 0; j < N; ++j) {  \
+      const float x = v[j];                          \
+      v[j] = (expr);                                 \
+    }                                                \
+    break;
+#include "gates.def"
+#undef TQ_GATE
+  }
+}
+
+struct No {
+  static constexpr bool value = false;
+};
+struct Yes {
+  static constexpr bool value = true;
+};
+
+struct PhaseTile {
+  int m0, units;               // first row and units of 64 rows (1..4)
+  int n0, n1;                  // first column of either half of 128 columns (the other matrix's same columns for a gated pair)
+  const bf16_t *w, *w2;        // the matrices of the halves
+};
+
+// One tile of 64 MI rows (32 MI of either group of waves).
+template <int MI, bool DUAL, bool OUT_ACT>
+__device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTile& p, bf16_t* lds) {
+  constexpr int A_SLOT = MI * 32 * TBK, W_SLOT = 128 * TBK;      // one group's rows of a, one half of w
+  constexpr int WT = MI > 2 ? 3 : 4;                             // tiles of w in LDS (of a: 2)
+  bf16_t* As = lds;                                              // [2 tiles][2 groups][A_SLOT]
+  bf16_t* Ws = lds + 4 * A_SLOT;                                 // [WT tiles][2 halves][W_SLOT]
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wm = wave / 4, wn = wave % 4;      // group; a wave's 32 columns of either half
+  const int steps = g.K / TBK;
+
+  // What this thread asks for: group 0 the rows of a that group 1 multiplies and the first half of w, group 1 the others; rows
+  // row + 32 i, the chunk of 16 bytes that belongs at place tid % 8 (the swizzle is in what is asked for).  Rows past the end
+  // and rows of padding read some valid row instead: those outputs are never stored.
+  const int row = (tid % 256) / 8, chunk = (tid % 8) ^ ((row >> 1) & 7);
+  const bf16_t *a_src[MI], *w_src[4];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = min(p.m0 + (1 - wm) * 32 * MI + row + 32 * i, g.M - 1);
+    int src = m;
+    if (g.a_rows && g.a_gather) src = max(g.a_rows[m], 0);
+    a_src[i] = g.a + (size_t)src * g.lda + chunk * 8;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w_src[i] = (wm ? p.w2 : p.w) + (size_t)min((wm ? p.n1 : p.n0) + row + 32 * i, g.N - 1) * g.K + chunk * 8;
+  auto ask_a = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) load_to_lds16(a_src[i] + t * TBK, As + ((t & 1) * 2 + 1 - wm) * A_SLOT + (i * 32 + wn * 8) * TBK);
+  };
+  auto ask_w = [&](int t, int slot) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_to_lds16(w_src[i] + t * TBK, Ws + (slot * 2 + wm) * W_SLOT + (i * 32 + wn * 8) * TBK);
+  };
+
+  // which of this wave's rows exist and are no padding (the epilogue's stores; asked for here, where nothing waits behind them)
+  const int mw = p.m0 + wm * 32 * MI;
+  auto alive = [&](int r) { return __ballot(r < 32 * MI && mw + r < g.M && !(g.a_rows && g.a_rows[min(mw + r, g.M - 1)] < 0)); };
+  const unsigned long long live_lo = alive(lane), live_hi = MI > 2 ? alive(64 + lane) : 0;
+
+  f32x16 acc[MI][2];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][b][v] = 0.f;
+  const int lr = lane % 32, lc = lane / 32, x = (lr >> 1) & 7;
+  u32x4 af[2][MI], wf[2][2];
+  // 32 of k: half h of tile t, whose w lies in `slot`
+  auto read = [&](int t, int slot, int h) {
+    const bf16_t* A = As + ((t & 1) * 2 + wm) * A_SLOT + lr * TBK;
+    const bf16_t* W = Ws + slot * 2 * W_SLOT + (wn * 32 + lr) * TBK;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int c = ((2 * (2 * h + j) + lc) ^ x) << 3;
+#pragma unroll
+      for (int b = 0; b < 2; ++b) wf[j][b] = *reinterpret_cast<const u32x4*>(W + b * W_SLOT + c);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) af[j][i] = *reinterpret_cast<const u32x4*>(A + i * 32 * TBK + c);
+    }
+    PH_FENCE();
+  };
+  auto multiply = [&]() {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[j][i]), __builtin_bit_cast(bf16x8, wf[j][b]),
+                                                              acc[i][b], 0, 0, 0);
+    PH_FENCE();
+  };
+
+  // Phases 4 t .. 4 t + 3 of group 0: read the first half of tile t, multiply it, read the second, multiply it; group 1 is one phase
+  // behind.  What a phase asks for goes where every wave has read what lay there (a0, a1: the groups' rows of a; w0, w1: the halves
+  // of w): phase 4 t a1 of t + 1, 4 t + 1 w1 and 4 t + 2 w0 of t + WT - 1 (in the place of tile t - 1's, last read in phase 4 t - 1),
+  // 4 t + 3 a0 of t + 2 (in the place of tile t's, last read in phase 4 t + 2).  A wave waits for its own loads before the barrier
+  // behind which another wave reads them: everything of tile t but a1 is read from phase 4 t on, a1 from 4 t + 1 on.
+  if (wm == 0) {
+    ask_w(0, 0);
+    if (WT == 4 && steps > 1) ask_w(1, 1);
+    ask_a(0);
+    if (WT == 4 ? steps > 2 : steps > 1) ask_w(WT - 2, WT - 2);
+    if (WT == 4) {
+      if (steps > 2) loads_left<MI + 8>();
+      else loads_left<MI>();
+    } else if (steps > 1) loads_left<MI + 4>();
+    else loads_left<MI>();
+  } else {
+    ask_a(0);
+    ask_w(0, 0);
+#pragma unroll
+    for (int t = 1; t < WT - 1; ++t)
+      if (t < steps) ask_w(t, t);
+    if (steps > 1) ask_a(1);
+    if (steps >= WT - 1) loads_left<4 * (WT - 2) + MI>();
+    else loads_left<0>();
+  }
+  PH_NEXT();
+  int slot = 0;      // of tile t's w; the slot of tile t + WT - 1 is the one before it
+  auto before = [](int s) { return s ? s - 1 : WT - 1; };
+  auto behind = [](int s) { return s + 1 < WT ? s + 1 : 0; };
+  // `LAST`: the last tiles, behind which less is asked for
+  auto first_group = [&](int t, auto last) {
+    constexpr bool LAST = decltype(last)::value;
+    read(t, slot, 0);
+    if (!LAST || t + 1 < steps) ask_a(t + 1);
+    // a1 of t has landed: behind it, the w0 asked for in phase 4 t - 2 and the a1 just asked for
+    if (!LAST || t + WT - 2 < steps) loads_left<MI + 4>();
+    else if (t + 1 < steps) loads_left<MI>();
+    else loads_left<0>();
+    PH_LDS_DONE();
+    PH_NEXT();
+    multiply();
+    PH_NEXT();
+    read(t, slot, 1);
+    if (!LAST || t + WT - 1 < steps) ask_w(t + WT - 1, before(slot));
+    PH_LDS_DONE();
+    PH_NEXT();
+    multiply();
+    // w0 of t + 1 has landed
+    if (!LAST || t + WT - 1 < steps) loads_left<(WT == 4 ? 8 : 4) + MI>();
+    else if (WT == 4 && t + 2 < steps) loads_left<4 + MI>();
+    else if (t + 1 < steps) loads_left<MI>();
+    PH_NEXT();
+    slot = behind(slot);
+  };
+  auto second_group = [&](int t, auto last) {
+    constexpr bool LAST = decltype(last)::value;
+    read(t, slot, 0);
+    if (!LAST || t + WT - 1 < steps) ask_w(t + WT - 1, before(slot));
+    PH_LDS_DONE();
+    PH_NEXT();
+    multiply();
+    PH_NEXT();
+    read(t, slot, 1);
+    if (!LAST || t + 2 < steps) ask_a(t + 2);
+    // a0 and w1 of t + 1 have landed: behind them, what this tile's phases asked for
+    if (!LAST || t + WT - 1 < steps) loads_left<4 + MI>();
+    else if (t + 2 < steps) loads_left<MI>();
+    else loads_left<0>();
+    PH_LDS_DONE();
+    PH_NEXT();
+    multiply();
+    PH_NEXT();
+    slot = behind(slot);
+  };
+  int t = 0;
+  if (wm == 0) {
+    for (; t + WT - 1 < steps; ++t) first_group(t, No());
+    for (; t < steps; ++t) first_group(t, Yes());
+    PH_NEXT();      // phase 4 steps, in which group 1 multiplies
+  } else {
+    PH_NEXT();      // phase 0
+    for (; t + WT - 1 < steps; ++t) second_group(t, No());
+    for (; t < steps; ++t) second_group(t, Yes());
+  }
+
+  // The outputs, 32 rows at a time through this wave's own part of LDS, which all waves have read for the last time.
+  constexpr int LD = 72;      // floats of a row: 32 of either half, and lanes 0..31 and 32..63 (four rows apart) on banks of their own
+  float* buf = (float*)lds + wave * 32 * LD;
+  constexpr int V = OUT_ACT ? 8 : 4;                  // outputs of a lane: 16 bytes, a row's lanes side by side
+  constexpr int PER_HALF = 32 / V, PER_ROW = DUAL ? PER_HALF : 2 * PER_HALF;
+  const int part = lane % PER_ROW, in_half = part % PER_HALF * V;
+  const int col = (part / PER_HALF ? p.n1 : p.n0) + wn * 32 + in_half;
+  float bias[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) bias[j] = col + j < g.N ? bias_at(g, col + j) : 0.f;
+  const bool wide = col + V <= g.N && g.ldc % V == 0 && (uintptr_t)g.out % 16 == 0;
+  auto to_lds = [&](const f32x16& first, const f32x16& second) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      float* at = buf + (8 * (v / 4) + 4 * lc + v % 4) * LD + lr;
+      at[0] = first[v];
+      at[32] = second[v];
+    }
+  };
+#pragma unroll 1
+  for (int i = 0; i < MI; ++i) {      // (kept a loop; the sums stay in registers since each case names its own)
+    if (i == 0) to_lds(acc[0][0], acc[0][1]);
+    if constexpr (MI > 1) if (i == 1) to_lds(acc[1][0], acc[1][1]);
+    if constexpr (MI > 2) if (i == 2) to_lds(acc[2][0], acc[2][1]);
+    if constexpr (MI > 3) if (i == 3) to_lds(acc[3][0], acc[3][1]);
+    const int m_first = mw + 32 * i;
+    const unsigned live = (unsigned)((i < 2 ? live_lo : live_hi) >> (i % 2 * 32));
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < PER_ROW / 2; ++q) {
+      const int r = lane / PER_ROW + q * (64 / PER_ROW);
+      float v[V];
+      const float* at = buf + r * LD + (DUAL ? 0 : part / PER_HALF * 32) + in_half;
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[j] = at[j] + bias[j];
+      if (DUAL) {
+        float u[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) u[j] = at[32 + j];
+        if (g.limit > 0.f) {
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            v[j] = fminf(v[j], g.limit);
+            u[j] = fminf(fmaxf(u[j], -g.limit), g.limit) + 1.0f;
+          }
+        }
+        gate_many(v, g.gate);
+#pragma unroll
+        for (int j = 0; j < V; ++j) v[j] *= u[j];
+      } else if (g.act1) {
+        gate_many(v, g.act1 - 1);
+      }
+      if (!((live >> r) & 1)) continue;
+      const size_t off = (size_t)(m_first + r) * g.ldc + col;
+      if constexpr (OUT_ACT) {
+        bf16_t* o = (bf16_t*)g.out + off;
+        if (wide) {
+          u32x4 packed;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) packed[j] = f32_to_bf16(v[2 * j]).bits | (unsigned)f32_to_bf16(v[2 * j + 1]).bits << 16;
+          *reinterpret_cast<u32x4*>(o) = packed;
+        } else {
+#pragma unroll
+          for (int j = 0; j < V; ++j)
+            if (col + j < g.N) o[j] = f32_to_bf16(v[j]);
+        }
+      } else {
+        float* o = (float*)g.out + off;
+        if (wide) {
+          *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int j = 0; j < V; ++j)
+            if (col + j < g.N) o[j] = v[j];
+        }
+      }
+    }
+    asm volatile("" ::: "memory");
+  }
+}
+
+// Which tile this workgroup takes: a die (workgroups are dealt to the 8 of them in turn) gets a contiguous run of tiles.  One
+// matrix: bands of 8 row tiles, down a band's columns.  A matrix per expert: expert by expert, so that an expert's matrices are
+// read by one die, and within an expert column by column with its items side by side.
+template <bool DUAL, bool OUT_ACT>
+__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int gy = gridDim.y, id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int lane = threadIdx.x % 64;
+  PhaseTile p;
+  int tile_n, group = 0;
+  if (g.tile_group) {
+    const int units_all = g.M / 64;
+    const int* items = g.tile_group + units_all;
+    const int n_units = min(g.n_tiles[0], units_all), n_items = min(g.n_tiles[1], units_all);
+    const int total = n_items * gy, die = id % 8, q = total / 8, rem = total % 8;
+    if (id / 8 >= q + (die < rem ? 1 : 0)) return;
+    const int logical = die * q + min(die, rem) + id / 8;
+    const int at = logical / gy;
+    group = g.tile_group[items[at]];
+    // the expert's items lo .. hi - 1, 64 candidates at a time
+    int lo = at, hi = at + 1;
+    for (bool more = true; more;) {
+      const int c = lo - 1 - lane;
+      const unsigned long long same = __ballot(c >= 0 && g.tile_group[items[max(c, 0)]] == group);
+      lo -= ~same ? __builtin_ctzll(~same) : 64;
+      more = !~same;
+    }
+    for (bool more = true; more;) {
+      const int c = hi + lane;
+      const unsigned long long same = __ballot(c < n_items && g.tile_group[items[min(c, n_items - 1)]] == group);
+      hi += ~same ? __builtin_ctzll(~same) : 64;
+      more = !~same;
+    }
+    const int local = logical - lo * gy, n_e = hi - lo;
+    tile_n = local / n_e;
+    const int item = lo + local % n_e, u0 = items[item];
+    p.m0 = u0 * 64;
+    p.units = min((item + 1 < n_items ? items[item + 1] : n_units) - u0, 4);
+  } else {
+    const int gx = gridDim.x, total = gx * gy, die = id % 8, q = total / 8, rem = total % 8;
+    const int logical = die * q + min(die, rem) + id / 8;
+    const int band = logical / (8 * gy), in_band = logical % (8 * gy), bh = min(8, gx - band * 8);
+    tile_n = in_band / bh;
+    p.m0 = (band * 8 + in_band % bh) * 256;
+    p.units = min((g.M - p.m0 + 63) / 64, 4);
+  }
+  p.w = g.w + (size_t)group * g.group_stride;
+  p.w2 = DUAL ? g.w2 + (size_t)group * g.group_stride : p.w;
+  p.n0 = tile_n * (DUAL ? 128 : 256);
+  p.n1 = DUAL ? p.n0 : p.n0 + 128;
+  switch (__builtin_amdgcn_readfirstlane(p.units)) {
+    case 4: phases_tile<4, DUAL, OUT_ACT>(g, p, (bf16_t*)smem); break;
+    case 3: phases_tile<3, DUAL, OUT_ACT>(g, p, (bf16_t*)smem); break;
+    case 2: phases_tile<2, DUAL, OUT_ACT>(g, p, (bf16_t*)smem); break;
+    default: phases_tile<1, DUAL, OUT_ACT>(g, p, (bf16_t*)smem);
+  }
+}
+
+// Grid: (units of 64 rows, at most so many items, or tiles of 256 rows of one matrix; tiles of 256 columns, 128 of a gated pair).
+int launch_gemm_phases(const MfmaGemmArgs& g, bool dual, bool out_act, hipStream_t st) {
+  const int cols = dual ? 128 : 256;
+  const dim3 grid(g.tile_group ? g.M / 64 : (g.M + 255) / 256, (g.N + cols - 1) / cols);
+  const int shmem = 160 * 1024;      // MI = 2 and 4; 144 KB where MI is 1 or 3
+#define TQ_PHASES(D, O)                                                                                                       \
+  do {                                                                                                                        \
+    if (hipFuncSetAttribute((const void*)gemm_phases_kernel<D, O>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem) != hipSuccess) \
+      return TQ_ERR_UNSUPPORTED;                                                                                              \
+    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), grid, dim3(512), shmem, st, g);                                            \
+  } while (0)
+  if (dual && out_act) TQ_PHASES(true, true);
+  else if (dual) TQ_PHASES(true, false);
+  else if (out_act) TQ_PHASES(false, true);
+  else TQ_PHASES(false, false);
+#undef TQ_PHASES
+  return 0;
+}

@@ -372,20 +372,21 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   // outputs of the routing
   int* ids = (int*)c.arena.take((size_t)n_pairs * 4);
   float* weights = (float*)c.arena.take((size_t)n_pairs * 4);
+  // what the products are told: units of 64 up to four at a time where experts have that many rows (ops.expert_product_rows)
+  const int rows = unit == 64 && n_pairs >= s.expert_pairs_from * E ? 64 + TQ_TILE_PAIRS : unit;
+  const int order_unit = rows != unit ? unit + TQ_ITEMS_OF_FOUR : unit;
   float* gate = gated ? (float*)c.arena.take((size_t)T * 4) : nullptr;
   float* logits = (float*)c.arena.take((size_t)T * (E + (gated ? 1 : 0)) * 4);
   int* sorted_token = (int*)c.arena.take((size_t)cap * 4);
   int* pair_slot = (int*)c.arena.take((size_t)n_pairs * 4);
-  int* tile_expert = (int*)c.arena.take((size_t)(cap / unit) * 2 * 4);      // row tiles, then items of two
+  int* tile_expert = (int*)c.arena.take((size_t)(cap / unit) * 2 * 4);      // row tiles, then items
   int* n_tiles = (int*)c.arena.take(2 * 4);
   auto route = [&]() -> int {
     RUN(c, "route",
         tq_route(normed32, f.router.ptr, gated ? f.shared_scale.ptr : nullptr, (int)f.router.wtype, E, k, (int)f.renormalize,
-                 ids, weights, gate, logits, unit, (int)cap, sorted_token, pair_slot, tile_expert, n_tiles, T, H, c.stream));
+                 ids, weights, gate, logits, order_unit, (int)cap, sorted_token, pair_slot, tile_expert, n_tiles, T, H, c.stream));
     return 0;
   };
-  // what the products are told: units of 64 two at a time where experts have that many rows (ops.expert_product_rows)
-  const int rows = unit == 64 && n_pairs >= s.expert_pairs_from * E ? 64 + TQ_TILE_PAIRS : unit;
   Product eg;       // the experts' gated pair over the gathered rows
   eg.a = normed, eg.lda = H, eg.a_rows = sorted_token, eg.w = f.expert_gate, eg.w2 = f.expert_up.ptr, eg.gstride = (int64_t)I * H,
   eg.tile_group = tile_expert, eg.n_tiles = n_tiles, eg.out_act = 1, eg.M = (int)cap, eg.N = I, eg.K = H, eg.tile_rows = rows,

@@ -379,9 +379,10 @@ TQ_API int tq_router_topk(const float* x, const void* wr, const void* shared_w, 
 //   sorted_token[r]  token whose activations feed row r, or -1
 //   pair_slot[i]     row of pair i
 //   tile_expert[j]   expert of row tile j (tiles of `unit` rows), n_tiles[0] tiles in all
-//   tile_expert[cap / unit + p]   first row tile of item p, n_tiles[1] items in all: an expert's row tiles two at a
-//                    time (its last one alone when their number is odd), for the product that takes two tiles of
-//                    one expert per workgroup; item p ends where item p + 1 begins, the last one at n_tiles[0]
+//   tile_expert[cap / unit + p]   first row tile of item p, n_tiles[1] items in all: an expert's row tiles two or, where
+//                    TQ_ITEMS_OF_FOUR is added to `unit`, four at a time (its last item holds what is left), for the product
+//                    that takes several tiles of one expert per workgroup; item p ends where item p + 1 begins, the last one
+//                    at n_tiles[0]
 // One workgroup of 16 waves does all of it.  Wave w owns the w-th sixteenth of the pairs: it goes through
 // them 64 at a time, finds for every lane the lanes that hold the same expert (a ballot per bit of the expert's
 // number), gives it its rank among them in order of lane and adds their number to its count of the expert.
@@ -423,8 +424,8 @@ __device__ __forceinline__ void rank_segment(const int* ids, int seg_beg, int se
 
 // Wave 0 of a workgroup turns the experts' padded sizes starts[e] into their first rows (an exclusive scan, each lane
 // a contiguous run of experts) and writes the row tiles' experts, the items and their numbers.
-__device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int cap, int* __restrict__ tile_expert,
-                                            int* __restrict__ n_tiles) {
+__device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int per_item, int cap,
+                                            int* __restrict__ tile_expert, int* __restrict__ n_tiles) {
   const int lane = threadIdx.x % TQ_WAVE;
   {
     const int chunk = (E + TQ_WAVE - 1) / TQ_WAVE;
@@ -432,7 +433,7 @@ __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int ca
     int sum = 0, isum = 0;
     for (int e = e0; e < e1; ++e) {
       sum += starts[e];
-      isum += (starts[e] / unit + 1) / 2;
+      isum += (starts[e] / unit + per_item - 1) / per_item;
     }
     int incl = sum, iincl = isum;
 #pragma unroll
@@ -451,7 +452,7 @@ __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int ca
       starts[e] = row;
       for (int j = 0; j < padded / unit; ++j) {
         tile_expert[row / unit + j] = e;
-        if (j % 2 == 0) items[item++] = row / unit + j;
+        if (j % per_item == 0) items[item++] = row / unit + j;
       }
       row += padded;
     }
@@ -465,7 +466,7 @@ __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int ca
 // ids may lie in LDS or in memory; cnt: (NW + 1) * E ints of LDS ([NW][E] counts, then E starts).  All NW waves
 // of the workgroup call it together.
 template <int NW>
-__device__ __forceinline__ void align_pairs(const int* ids, int n_pairs, int E, int topk, int unit, int cap,
+__device__ __forceinline__ void align_pairs(const int* ids, int n_pairs, int E, int topk, int unit, int per_item, int cap,
                                             int* __restrict__ sorted_token, int* __restrict__ pair_slot,
                                             int* __restrict__ tile_expert, int* __restrict__ n_tiles, int* cnt,
                                             int n_real = 1 << 30) {
@@ -495,7 +496,7 @@ __device__ __forceinline__ void align_pairs(const int* ids, int n_pairs, int E, 
     starts[e] = e < n_real ? (total + unit - 1) / unit * unit : 0;
   }
   __syncthreads();
-  if (wave == 0) scan_starts(starts, E, unit, cap, tile_expert, n_tiles);
+  if (wave == 0) scan_starts(starts, E, unit, per_item, cap, tile_expert, n_tiles);
   __syncthreads();
   if (one_batch) {
     if (my_e >= n_real) {
@@ -521,13 +522,13 @@ __device__ __forceinline__ void align_pairs(const int* ids, int n_pairs, int E, 
 }
 
 __global__ __launch_bounds__(64 * AW) void moe_align_kernel(const int* __restrict__ ids, int n_pairs, int E,
-                                                            int topk, int unit, int cap,
+                                                            int topk, int unit, int per_item, int cap,
                                                             int* __restrict__ sorted_token,
                                                             int* __restrict__ pair_slot,
                                                             int* __restrict__ tile_expert,
                                                             int* __restrict__ n_tiles, int n_real) {
   extern __shared__ int cnt[];
-  align_pairs<AW>(ids, n_pairs, E, topk, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles, cnt, n_real);
+  align_pairs<AW>(ids, n_pairs, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, cnt, n_real);
 }
 
 // The same order by several workgroups, for steps of many tokens (one workgroup's waves go through 32,768 pairs in
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(64 * AW) void align_count_kernel(const int* __restr
   for (int e = lane; e < E; e += TQ_WAVE) table[(size_t)v * E + e] = cnt[wave * E + e];
 }
 
-__global__ __launch_bounds__(64 * AW) void align_scan_kernel(int* __restrict__ table, int V, int E, int unit, int cap,
+__global__ __launch_bounds__(64 * AW) void align_scan_kernel(int* __restrict__ table, int V, int E, int unit, int per_item, int cap,
                                                              int* __restrict__ tile_expert, int* __restrict__ n_tiles,
                                                              int n_real) {
   extern __shared__ int sm_a[];        // [chunks][E] sums of AC waves' counts, then E starts
@@ -593,7 +594,7 @@ __global__ __launch_bounds__(64 * AW) void align_scan_kernel(int* __restrict__ t
         total += cv[u];
       }
   }
-  if (threadIdx.x / TQ_WAVE == 0) scan_starts(starts, E, unit, cap, tile_expert, n_tiles);
+  if (threadIdx.x / TQ_WAVE == 0) scan_starts(starts, E, unit, per_item, cap, tile_expert, n_tiles);
   __syncthreads();
   for (int e = threadIdx.x; e < E; e += blockDim.x) table[(size_t)V * E + e] = starts[e];
 }
@@ -648,7 +649,7 @@ static int align_workgroups(int n_pairs, int E, size_t table_ints) {
   return g;
 }
 
-static int launch_align_multi(const int* ids, int n_pairs, int E, int topk, int unit, int cap, int* sorted_token,
+static int launch_align_multi(const int* ids, int n_pairs, int E, int topk, int unit, int per_item, int cap, int* sorted_token,
                               int* pair_slot, int* tile_expert, int* n_tiles, int* table, int g, hipStream_t st,
                               int n_real = 1 << 30) {
   const int V = g * AW, chunks = (V + AC - 1) / AC;
@@ -662,7 +663,7 @@ static int launch_align_multi(const int* ids, int n_pairs, int E, int topk, int 
   }
   hipLaunchKernelGGL(align_count_kernel, dim3(g), dim3(64 * AW), lds_count, st, ids, n_pairs, E, cap, sorted_token,
                      pair_slot, table);
-  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(64 * AW), lds_scan, st, table, V, E, unit, cap, tile_expert,
+  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(64 * AW), lds_scan, st, table, V, E, unit, per_item, cap, tile_expert,
                      n_tiles, n_real);
   hipLaunchKernelGGL(align_place_kernel, dim3(g), dim3(64 * AW), lds_place, st, ids, n_pairs, E, topk, table, pair_slot,
                      sorted_token, n_real);
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(64 * NW) void select_align_kernel(const float* __re
                                                                int topk, int renorm, int groups, int keep,
                                                                int* __restrict__ ids, float* __restrict__ weights,
                                                                float* __restrict__ shared_gate, int T, int unit,
-                                                               int cap, int* __restrict__ sorted_token,
+                                                               int per_item, int cap, int* __restrict__ sorted_token,
                                                                int* __restrict__ pair_slot,
                                                                int* __restrict__ tile_expert,
                                                                int* __restrict__ n_tiles,
@@ -692,12 +693,19 @@ __global__ __launch_bounds__(64 * NW) void select_align_kernel(const float* __re
     select_token(logits + (size_t)wave * rows, rows, E, topk, renorm, groups, keep, lg + wave * E, ids + (size_t)wave * topk,
                  ids_l + wave * topk, weights + (size_t)wave * topk, shared_gate + wave, correction, n_real, wscale);
   __syncthreads();
-  align_pairs<NW>(ids_l, T * topk, E, topk, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles, cnt, n_real);
+  align_pairs<NW>(ids_l, T * topk, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, cnt, n_real);
+}
+
+// Row tiles that an item holds at most; takes TQ_ITEMS_OF_FOUR off `unit`.
+static int units_per_item(int& unit) {
+  if (unit < TQ_ITEMS_OF_FOUR) return 2;
+  unit -= TQ_ITEMS_OF_FOUR;
+  return 4;
 }
 
 // cap: rows that sorted_token holds, a multiple of unit and at least n_pairs + min(E, n_pairs) * (unit - 1);
 // tile_expert holds 2 * cap / unit entries (row tiles, then items), n_tiles two.
-static int moe_align_impl(const int* ids, int n_pairs, int E, int topk, int unit, int cap, int* sorted_token,
+static int moe_align_impl(const int* ids, int n_pairs, int E, int topk, int unit, int per_item, int cap, int* sorted_token,
                           int* pair_slot, int* tile_expert, int* n_tiles, hipStream_t st, int n_real) {
   if (n_pairs <= 0) return 0;
   if (unit < 1 || cap % unit != 0 || cap < n_pairs + (E < n_pairs ? E : n_pairs) * (unit - 1)) return TQ_ERR_BAD_ARG;
@@ -705,7 +713,7 @@ static int moe_align_impl(const int* ids, int n_pairs, int E, int topk, int unit
   if (shmem > 160 * 1024) return TQ_ERR_UNSUPPORTED;
   if (shmem > 48 * 1024)
     (void)hipFuncSetAttribute((const void*)moe_align_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * AW), shmem, st, ids, n_pairs, E, topk, unit, cap,
+  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * AW), shmem, st, ids, n_pairs, E, topk, unit, per_item, cap,
                      sorted_token, pair_slot, tile_expert, n_tiles, n_real);
   TQ_LAUNCH_CHECK();
   return 0;
@@ -713,7 +721,8 @@ static int moe_align_impl(const int* ids, int n_pairs, int E, int topk, int unit
 
 TQ_API int tq_moe_align(const int* ids, int n_pairs, int E, int topk, int unit, int cap, int* sorted_token,
                         int* pair_slot, int* tile_expert, int* n_tiles, hipStream_t st) {
-  return moe_align_impl(ids, n_pairs, E, topk, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles, st, E);
+  const int per_item = units_per_item(unit);
+  return moe_align_impl(ids, n_pairs, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, st, E);
 }
 
 // tq_router_topk followed by tq_moe_align; up to 16 tokens take two kernels instead of three, and from 8,192 pairs on
@@ -725,6 +734,7 @@ static int route_impl(const float* x, const void* wr, const void* shared_w, cons
                       float* logits, int unit, int cap, int* sorted_token, int* pair_slot, int* tile_expert,
                       int* n_tiles, int T, int H, hipStream_t st, const float* correction, int n_real, float wscale = 1.0f) {
   if (T <= 0) return 0;
+  const int per_item = units_per_item(unit);
   if (!groups_ok(E, topk, groups, keep)) return TQ_ERR_BAD_ARG;
   const size_t shmem = ((size_t)(AW + 1) * E + (size_t)AW * topk + (size_t)AW * E) * 4;
   if (T > AW || shmem > 64 * 1024) {
@@ -734,9 +744,9 @@ static int route_impl(const float* x, const void* wr, const void* shared_w, cons
     // once the experts are chosen the logits are done with: the order by several workgroups keeps its table there
     const int n = T * topk;
     const int g = align_workgroups(n, E, (size_t)T * (E + (shared_w ? 1 : 0)));
-    if (g == 0) return moe_align_impl(ids, n, E, topk, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles, st, n_real);
+    if (g == 0) return moe_align_impl(ids, n, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, st, n_real);
     if (unit < 1 || cap % unit != 0 || cap < n + (E < n ? E : n) * (unit - 1)) return TQ_ERR_BAD_ARG;
-    return launch_align_multi(ids, n, E, topk, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles, (int*)logits, g,
+    return launch_align_multi(ids, n, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, (int*)logits, g,
                               st, n_real);
   }
   if (topk < 1 || topk > 64 || topk > E || E > 8192) return TQ_ERR_UNSUPPORTED;
@@ -747,7 +757,7 @@ static int route_impl(const float* x, const void* wr, const void* shared_w, cons
   if (T == 1) {      // one wave: its barriers cost nothing
     const size_t shmem1 = ((size_t)2 * E + topk + E) * 4;
     hipLaunchKernelGGL(select_align_kernel<1>, dim3(1), dim3(64), shmem1, st, logits, E + (shared_w ? 1 : 0), E, topk,
-                       renorm, groups, keep, ids, weights, shared_gate, T, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles,
+                       renorm, groups, keep, ids, weights, shared_gate, T, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles,
                        correction, n_real, wscale);
     TQ_LAUNCH_CHECK();
     return 0;
@@ -755,7 +765,7 @@ static int route_impl(const float* x, const void* wr, const void* shared_w, cons
   if (shmem > 48 * 1024)
     (void)hipFuncSetAttribute((const void*)select_align_kernel<AW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   hipLaunchKernelGGL(select_align_kernel<AW>, dim3(1), dim3(64 * AW), shmem, st, logits, E + (shared_w ? 1 : 0), E, topk,
-                     renorm, groups, keep, ids, weights, shared_gate, T, unit, cap, sorted_token, pair_slot, tile_expert, n_tiles,
+                     renorm, groups, keep, ids, weights, shared_gate, T, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles,
                        correction, n_real, wscale);
   TQ_LAUNCH_CHECK();
   return 0;

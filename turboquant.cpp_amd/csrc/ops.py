@@ -837,11 +837,11 @@ def _use_mfma(act, a: torch.Tensor, w: torch.Tensor, K: int) -> bool:
 
 
 EXPERT_16_UPTO, EXPERT_32_UPTO = 5, 10
-# Rows per expert on average from which the row order's unit is 128 and 256: never, since units of 64 taken two at a
+# Rows per expert on average from which the row order's unit is 128 and 256: never, since units of 64 taken several at a
 # time do better wherever the taller units did (see expert_tile_rows); tests lower them to run those kernels.
 EXPERT_128_FROM = EXPERT_256_FROM = 1 << 30
-TILE_PAIRS = 1024            # added to tile_rows 64: two units of one expert per workgroup (TQ_TILE_PAIRS)
-EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken two at a time
+TILE_PAIRS = 1024            # added to tile_rows 64: the units of an item, two or four of one expert, per workgroup (TQ_TILE_PAIRS)
+EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken several at a time
 
 
 def expert_tile_rows(n_pairs: int, num_experts: int, act, a: torch.Tensor, w: torch.Tensor,
@@ -858,9 +858,8 @@ def expert_tile_rows(n_pairs: int, num_experts: int, act, a: torch.Tensor, w: to
     faster with units of 16 than of 32).
     Without the matrix-core product 16 up to 12.  Units of 128 and 256 rows (EXPERT_128_FROM, EXPERT_256_FROM) are
     not chosen: they were 8 to 17 % faster than single tiles of 64 rows from 256 rows per expert on, but units of 64
-    taken two at a time (expert_product_rows) are faster than either (60 experts of 1,408 x 2,048, both products:
-    396 us against 448 at 205 rows per expert, 492 against 565 at 273, 841 against 949 at 546; 64 experts of
-    2,560 x 3,584 at 1,650 rows each: a prompt step of 425 ms against 436 with units of 256)."""
+    taken several at a time (expert_product_rows) are faster than either (60 experts of 1,408 x 2,048, both products, already two at
+    a time: 396 us against 448 at 205 rows per expert, 492 against 565 at 273, 841 against 949 at 546; now 715 at 546)."""
     # (``w_behind``: the matrices of the product that follows on the same row order, over another k: the units that only
     # the matrix-core product takes are chosen where both products run there)
     mfma = _use_mfma(act, a, w, a.shape[1]) and (w_behind is None or _use_mfma(act, a, w_behind, w_behind.shape[-1]))
@@ -875,12 +874,11 @@ def expert_tile_rows(n_pairs: int, num_experts: int, act, a: torch.Tensor, w: to
 
 def expert_product_rows(unit: int, n_pairs: int, num_experts: int) -> int:
     """The ``tile_rows`` that a product over experts is called with when the row order has units of ``unit`` rows: from
-    48 rows per expert on average, units of 64 two at a time (measured on 60 experts of 1,408 x 2,048, four per
-    token, both products together: 251 us against 286 at 68 rows per expert, 260 against 307 at 102, 346 against 360
-    at 137; level below; a prompt step of 24 layers: 10.3 ms against 10.9 at 1,024 tokens, 15.8 against 17.0 at
-    2,048, 22.3 against 23.7 at 3,072; where the border lies, by such steps: 9.42 ms against 9.73 at 55 rows per
-    expert and 9.75 against 10.22 at 60, which already gives many experts a second unit, level at 43 and 47, 7.97
-    against 7.81 at 34)."""
+    48 rows per expert on average, units of 64 up to four at a time by the order's items (csrc/gemm_phases.hip).  Measured on
+    60 experts of 1,408 x 2,048, four per token, evenly dealt, both products together against items of two through a ring of LDS
+    stages, which unit by unit trailed by 13 % and more: 237 us against 247 at 68 rows per expert, 275 against 367 at 137, 480 against
+    541 at 273, 715 against 918 at 546; 64 experts of 2,560 x 3,584 at 1,650 rows each 5.7 ms against 7.5.  Below 48
+    rows nearly every expert has one unit, and unit by unit is level."""
     if unit == 64 and n_pairs >= EXPERT_PAIRS_FROM * num_experts:
         return 64 + TILE_PAIRS
     return unit
@@ -1363,7 +1361,7 @@ def _align_outputs(T: int, topk: int, num_experts: int, unit: int, dev):
     cap = (cap + unit - 1) // unit * unit
     sorted_token = torch.empty((cap,), dtype=torch.int32, device=dev)
     pair_slot = torch.empty((T, topk), dtype=torch.int32, device=dev)
-    tile_expert = torch.empty((2 * (cap // unit),), dtype=torch.int32, device=dev)      # row tiles, then items of two
+    tile_expert = torch.empty((2 * (cap // unit),), dtype=torch.int32, device=dev)      # row tiles, then items
     n_tiles = torch.empty((2,), dtype=torch.int32, device=dev)
     return cap, sorted_token, pair_slot, tile_expert, n_tiles
 
@@ -1371,7 +1369,7 @@ def _align_outputs(T: int, topk: int, num_experts: int, unit: int, dev):
 def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | None, top_k: int, renormalize: bool,
           unit: int, act, groups: tuple[int, int] | None = None, bias: torch.Tensor | None = None,
           correction: torch.Tensor | None = None, identity: int = 0, sigmoid: bool = False, weight_scale: float = 1.0,
-          pair_groups: bool = False):
+          pair_groups: bool = False, item_units: int = 2):
     """``router_topk`` followed by ``moe_align`` in one call: (ids, weights, gate, sorted_token, pair_slot,
     tile_expert, n_tiles), with the same results; a handful of tokens takes one kernel less.
 
@@ -1379,8 +1377,9 @@ def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | 
     all E rows of the router, the choice is by score + correction and the weights are the scores themselves.  ``identity`` n
     (with ``correction``): the router's last n rows are experts without matrices whose output is their input; their pairs
     get ``pair_slot`` -1 and no rows in the order, and ``gate`` [T] is the sum of each token's weights for them.
-    ``sigmoid``, ``weight_scale``, ``pair_groups``: as for ``router_topk``."""
+    ``sigmoid``, ``weight_scale``, ``pair_groups``: as for ``router_topk``; ``item_units``: as for ``moe_align``."""
     k = "route"
+    listed = _order_unit(k, unit, item_units)
     T, H, E, ids, weights, gate, logits = _router_outputs(k, x32, router, shared_scale, top_k)
     _need(unit in (16, 32, 64, 128, 256), k, "unit must be 16, 32, 64, 128 or 256")
     if correction is not None:
@@ -1391,7 +1390,7 @@ def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | 
             gate = torch.empty((T,), dtype=torch.float32, device=x32.device)
         cap, sorted_token, pair_slot, tile_expert, n_tiles = _align_outputs(T, top_k, E, unit, x32.device)
         _run(k, library(act).tq_route_scored(_ptr(x32), _ptr(router), _ptr(correction), _WTYPE[router.dtype], E, E - identity,
-                                             top_k, _ptr(ids), _ptr(weights), _ptr(gate), _ptr(logits), unit, cap,
+                                             top_k, _ptr(ids), _ptr(weights), _ptr(gate), _ptr(logits), listed, cap,
                                              _ptr(sorted_token), _ptr(pair_slot), _ptr(tile_expert), _ptr(n_tiles), T, H,
                                              _stream()))
         return ids, weights, gate, sorted_token, pair_slot, tile_expert, n_tiles
@@ -1405,31 +1404,38 @@ def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | 
     if sigmoid:
         _run(k, library(act).tq_route_sigmoid(_ptr(x32), _ptr(router), _ptr(shared_scale), _ptr(bias), _WTYPE[router.dtype], E,
                                               top_k, count, keep, int(pair_groups), float(weight_scale), _ptr(ids), _ptr(weights),
-                                              _ptr(gate), _ptr(logits), unit, cap, _ptr(sorted_token), _ptr(pair_slot),
+                                              _ptr(gate), _ptr(logits), listed, cap, _ptr(sorted_token), _ptr(pair_slot),
                                               _ptr(tile_expert), _ptr(n_tiles), T, H, _stream()))
         return ids, weights, gate, sorted_token, pair_slot, tile_expert, n_tiles
     if weight_scale != 1.0:
         _run(k, library(act).tq_route_weighted(_ptr(x32), _ptr(router), _ptr(shared_scale), _ptr(bias), _WTYPE[router.dtype], E,
                                                top_k, count, keep, float(weight_scale), _ptr(ids), _ptr(weights), _ptr(gate),
-                                               _ptr(logits), unit, cap, _ptr(sorted_token), _ptr(pair_slot), _ptr(tile_expert),
+                                               _ptr(logits), listed, cap, _ptr(sorted_token), _ptr(pair_slot), _ptr(tile_expert),
                                                _ptr(n_tiles), T, H, _stream()))
         return ids, weights, gate, sorted_token, pair_slot, tile_expert, n_tiles
     _run(k, library(act).tq_route_biased(_ptr(x32), _ptr(router), _ptr(shared_scale), _ptr(bias), _WTYPE[router.dtype], E, top_k,
                                          int(bool(renormalize)), count, keep, _ptr(ids), _ptr(weights), _ptr(gate),
-                                         _ptr(logits), unit, cap, _ptr(sorted_token), _ptr(pair_slot), _ptr(tile_expert),
+                                         _ptr(logits), listed, cap, _ptr(sorted_token), _ptr(pair_slot), _ptr(tile_expert),
                                          _ptr(n_tiles), T, H, _stream()))
     return ids, weights, gate, sorted_token, pair_slot, tile_expert, n_tiles
 
 
-def moe_align(ids: torch.Tensor, num_experts: int, unit: int, act):
+def _order_unit(k: str, unit: int, item_units: int) -> int:
+    """The ``unit`` that the library is told, with how many row tiles an item holds at most (TQ_ITEMS_OF_FOUR)."""
+    _need(item_units in (2, 4), k, "an item holds up to 2 or 4 row tiles")
+    return unit + 2048 if item_units == 4 else unit
+
+
+def moe_align(ids: torch.Tensor, num_experts: int, unit: int, act, item_units: int = 2):
     """Orders the (token, expert) pairs by expert.  Returns sorted_token [cap], pair_slot [T, k],
-    tile_expert [cap/unit], n_tiles [1]; each expert's rows start at a multiple of ``unit``."""
+    tile_expert [2 cap/unit], n_tiles [2]; each expert's rows start at a multiple of ``unit``.  Behind the row tiles'
+    experts stand the items, runs of up to ``item_units`` (2 or 4) row tiles of one expert."""
     k = "moe_align"
     _check(ids, k, "ids", torch.int32)
     T, topk = ids.shape
     n_pairs = T * topk
     cap, sorted_token, pair_slot, tile_expert, n_tiles = _align_outputs(T, topk, num_experts, unit, ids.device)
-    _run(k, library(act).tq_moe_align(_ptr(ids), n_pairs, num_experts, topk, unit, cap, _ptr(sorted_token),
+    _run(k, library(act).tq_moe_align(_ptr(ids), n_pairs, num_experts, topk, _order_unit(k, unit, item_units), cap, _ptr(sorted_token),
                                       _ptr(pair_slot), _ptr(tile_expert), _ptr(n_tiles), _stream()))
     return sorted_token, pair_slot, tile_expert, n_tiles
 
