@@ -6,9 +6,15 @@
 // per-row-tile matrices for experts; the reference's counterpart is its float matvec
 // (/root/reference/src/engine/tq_ops.c:296-343).  Two kernels:
 //
-//  * gemm_f32_tile_kernel, for more than 16 rows: tiles of 64 or 128 rows by 128 columns by four waves, 16 of k
-//    at a time through two LDS buffers (rows padded to 20 floats, so that the 16-byte operand reads of eight
-//    neighbouring rows fall on all banks); while one buffer is multiplied the next tile is on its way from memory.
+//  * gemm_f32_tile_kernel, for more than 16 rows: tiles of 64 or 128 rows by 128 columns (64 of a gated pair of 128 rows) by four
+//    waves, 16 of k at a time.  What bounds it is the matrix instructions (64 clocks each), so what counts is that a SIMD always
+//    has a wave with products to do: 64 sums a wave and no more, so that three workgroups share a compute unit, and tiles that go
+//    straight from memory into a ring of three LDS stages, two on their way, with one bare barrier a tile and no branch around a
+//    load (with tiles through registers and loads behind predicates a gated pair of 128 x 128 had one wave to a SIMD).
+//    16,385 rows, ms, before and now: by 6,144 x 2,048 3.46 and 3.20 (129 TFLOP/s; the instructions alone give 153), by 2,048 x 5,632 3.48
+//    and 3.22, gated pair of twice 5,632 x 2,048 7.55 and 5.78; 60 experts of 1,408 x 2,048, four per token, 6.85 and
+//    6.12, their second product 3.80 and 3.22; 1,000 rows by twice 5,632 x 2,048 655 and 402 us.  Rings of two stages 1 to 3 % slower,
+//    of four level; four waves to a SIMD (128 registers) level.
 //    17 to 64 rows (a decode step of many sequences) are one row of tiles, at which multiply-adds and bytes of w
 //    are in balance; a narrow matrix is cut into runs of k so that the chip has enough workgroups.
 //  * gemm_f32_stream_kernel, for few rows (decoding; experts that few tokens chose): the work is reading w once.
@@ -68,37 +74,86 @@ __device__ __forceinline__ const float* f32_row_of(const F32GemmArgs& g, int m) 
 
 // ------------------------------------------------------------------------------------------ many rows
 #define TBK 16
-#define TLD (TBK + 4)
+#define TSTAGES 3
+// Where chunk c (4 of k) of a tile's row lies in the row: eight neighbouring rows' reads of one chunk, and sixteen neighbouring rows'
+// where the 64 banks serve them together, fall on banks of their own.
+__device__ __forceinline__ int f32_place(int row, int c) { return c ^ (((((row >> 1) ^ (row >> 3)) & 1) << 1) | ((row >> 2) & 1)); }
+__device__ __forceinline__ void f32_to_lds16(const float* src, float* wave_base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)wave_base, 16, 0, 0);
+}
 
 // With `part` set the grid's z cuts k into runs of k_per_split and the sums of run z go to part[z] ([run][M][N], the
 // gated pair's second product behind all the first ones) as they are: gemm_f32_reduce_kernel finishes them.
-template <int MI, bool DUAL>
+template <int MI, int NI, bool DUAL>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k_per_split, float* part) {
-  constexpr int NI = 2, BM = 64 * MI, BN = 64 * NI;
-  __shared__ __align__(16) float As[2][BM * TLD];
-  __shared__ __align__(16) float Ws[2][BN * TLD];
-  __shared__ __align__(16) float Vs[2][DUAL ? BN * TLD : 4];
-  const int tile_m = blockIdx.x, tile_n = blockIdx.y;
-  if (g.n_tiles && tile_m >= g.n_tiles[0]) return;
+  constexpr int BM = 64 * MI, BN = 64 * NI, ROWS = BM + BN * (DUAL ? 2 : 1), STAGE = ROWS * TBK, L = ROWS / 64;
+  __shared__ __align__(16) float ring[TSTAGES * STAGE];
+  // Which tile: a die (workgroups are dealt to the 8 of them in turn) gets a contiguous run.  One matrix: bands of 8 row tiles, down
+  // a band's columns.  A matrix per expert: expert by expert, within one column by column with its row tiles side by side.
+  int tile_m, tile_n;
+  {
+    const int gx = g.n_tiles ? min(g.n_tiles[0], (int)gridDim.x) : (int)gridDim.x, gy = gridDim.y, total = gx * gy;
+    const int id = blockIdx.y * gridDim.x + blockIdx.x, die = id % 8, q = total / 8, rem = total % 8;
+    if (id / 8 >= q + (die < rem ? 1 : 0)) return;
+    const int logical = die * q + min(die, rem) + id / 8;
+    if (g.tile_group) {
+      const int at = logical / gy, e = g.tile_group[at], l = threadIdx.x % 64;
+      int lo = at, hi = at + 1;
+      for (bool more = true; more;) {
+        const int c = lo - 1 - l;
+        const unsigned long long same = __ballot(c >= 0 && g.tile_group[max(c, 0)] == e);
+        lo -= ~same ? __builtin_ctzll(~same) : 64;
+        more = !~same;
+      }
+      for (bool more = true; more;) {
+        const int c = hi + l;
+        const unsigned long long same = __ballot(c < gx && g.tile_group[min(c, gx - 1)] == e);
+        hi += ~same ? __builtin_ctzll(~same) : 64;
+        more = !~same;
+      }
+      const int local = logical - lo * gy;
+      tile_n = local / (hi - lo);
+      tile_m = lo + local % (hi - lo);
+    } else {
+      const int band = logical / (8 * gy), in_band = logical % (8 * gy), bh = min(8, gx - band * 8);
+      tile_m = band * 8 + in_band % bh;
+      tile_n = in_band / bh;
+    }
+  }
   const int group = g.tile_group ? g.tile_group[tile_m] : 0;
   const float* w = g.w + (size_t)group * g.group_stride;
   const float* w2 = DUAL ? g.w2 + (size_t)group * g.group_stride : nullptr;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wave_m = wave / 2, wave_n = wave % 2;
-  const int lrow = tid / 4, lchunk = tid % 4;      // what this thread fetches of a tile: rows lrow + 64 j, 4 of k
 
-  const float* arow[MI];
-  const float* wrow[NI];
-  const float* vrow[DUAL ? NI : 1];
+  // What this thread asks for of each stage: place tid % 4 of rows tid / 4 + 64 i (a's rows, then w's, then w2's).  Rows that do not
+  // exist read some valid row instead: those outputs are never stored.
+  const float* src[L];
 #pragma unroll
-  for (int j = 0; j < MI; ++j) arow[j] = f32_row_of(g, m0 + lrow + 64 * j);
-#pragma unroll
-  for (int j = 0; j < NI; ++j) {
-    const int n = n0 + lrow + 64 * j;
-    wrow[j] = n < g.N ? w + (size_t)n * g.K : nullptr;
-    if (DUAL) vrow[j] = n < g.N ? w2 + (size_t)n * g.K : nullptr;
+  for (int i = 0; i < L; ++i) {
+    const int r = tid / 4 + 64 * i;      // (a load's 64 rows lie in one of the three: all heights are multiples of 64)
+    if (64 * i < BM) {
+      const float* from = f32_row_of(g, min(m0 + r, g.M - 1));
+      src[i] = from ? from : g.a;
+    } else if (64 * i < BM + BN) {
+      src[i] = w + (size_t)min(n0 + r - BM, g.N - 1) * g.K;
+    } else {
+      src[i] = w2 + (size_t)min(n0 + r - BM - BN, g.N - 1) * g.K;
+    }
   }
+  const int k_first = blockIdx.z * k_per_split, k_last = min(g.K, k_first + k_per_split);
+  const int chunk = 4 * f32_place(tid / 4, tid % 4);      // (64 rows on the place is the same)
+  auto ask = [&](int step) {
+    float* base = ring + step % TSTAGES * STAGE + wave * 16 * TBK;
+#pragma unroll
+    for (int i = 0; i < L; ++i) f32_to_lds16(src[i] + k_first + step * TBK + chunk, base + 64 * i * TBK);
+  };
+  // which of this wave's rows exist and are no padding
+  const int mw = m0 + wave_m * 32 * MI;
+  const unsigned long long live =
+      __ballot(lane < 32 * MI && mw + lane < g.M && !(g.a_rows && g.a_rows[min(mw + lane, g.M - 1)] < 0));
 
   f32x16 acc[MI][NI], acc2[DUAL ? MI : 1][DUAL ? NI : 1];
 #pragma unroll
@@ -111,49 +166,20 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k
         if (DUAL) acc2[i][j][v] = 0.f;
       }
     }
-
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 ra[MI], rw[NI], rv[DUAL ? NI : 1];
-  const int k_first = blockIdx.z * k_per_split, k_last = min(g.K, k_first + k_per_split);
-  auto fetch = [&](int k0) {
-    const int k = k0 + 4 * lchunk;
-    const bool in = k < k_last;       // K and the runs are multiples of 4: a chunk lies inside or outside as a whole
-#pragma unroll
-    for (int j = 0; j < MI; ++j) ra[j] = in && arow[j] ? *reinterpret_cast<const f32x4*>(arow[j] + k) : zero;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      rw[j] = in && wrow[j] ? *reinterpret_cast<const f32x4*>(wrow[j] + k) : zero;
-      if (DUAL) rv[j] = in && vrow[j] ? *reinterpret_cast<const f32x4*>(vrow[j] + k) : zero;
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < MI; ++j) *reinterpret_cast<f32x4*>(&As[buf][(lrow + 64 * j) * TLD + 4 * lchunk]) = ra[j];
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      *reinterpret_cast<f32x4*>(&Ws[buf][(lrow + 64 * j) * TLD + 4 * lchunk]) = rw[j];
-      if (DUAL) *reinterpret_cast<f32x4*>(&Vs[buf][(lrow + 64 * j) * TLD + 4 * lchunk]) = rv[j];
-    }
-  };
-
-  const int nk = (k_last - k_first + TBK - 1) / TBK;
-  fetch(k_first);
-  stage(0);
-  __syncthreads();
   const int r32 = lane % 32, kk = lane / 32;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) fetch(k_first + (kt + 1) * TBK);
+  auto multiply = [&](const float* at) {
+    const float* A = at + (wave_m * 32 * MI + r32) * TBK;
+    const float* W = at + (BM + wave_n * 32 * NI + r32) * TBK;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      const int c = 4 * f32_place(r32, 2 * h + kk);
       f32x4 af[MI], wf[NI], vf[DUAL ? NI : 1];
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
-        af[i] = *reinterpret_cast<const f32x4*>(&As[buf][(wave_m * 32 * MI + i * 32 + r32) * TLD + 8 * h + 4 * kk]);
+      for (int i = 0; i < MI; ++i) af[i] = *reinterpret_cast<const f32x4*>(A + i * 32 * TBK + c);
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
-        wf[j] = *reinterpret_cast<const f32x4*>(&Ws[buf][(wave_n * 32 * NI + j * 32 + r32) * TLD + 8 * h + 4 * kk]);
-        if (DUAL) vf[j] = *reinterpret_cast<const f32x4*>(&Vs[buf][(wave_n * 32 * NI + j * 32 + r32) * TLD + 8 * h + 4 * kk]);
+        wf[j] = *reinterpret_cast<const f32x4*>(W + j * 32 * TBK + c);
+        if (DUAL) vf[j] = *reinterpret_cast<const f32x4*>(W + (BN + j * 32) * TBK + c);
       }
 #pragma unroll
       for (int s = 0; s < 4; ++s)
@@ -165,31 +191,53 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k
             if (DUAL) acc2[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][s], vf[j][s], acc2[i][j], 0, 0, 0);
           }
     }
-    if (kt + 1 < nk) stage(buf ^ 1);
+  };
+
+  const int steps = (k_last - k_first) / TBK, left = (k_last - k_first) % TBK;
+  for (int s = 0; s < TSTAGES - 1 && s < steps; ++s) ask(s);
+  for (int t = 0; t < steps; ++t) {
+    // tile t has landed once no more of this wave's loads are on their way than those of the tile behind it
+    if (t + 1 < steps) __builtin_amdgcn_s_waitcnt(0x0F70 | L);
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();      // and every wave is through with tile t - 1, whose stage tile t + 2 takes
+    asm volatile("" ::: "memory");
+    if (t + TSTAGES - 1 < steps) ask(t + TSTAGES - 1);
+    multiply(ring + t % TSTAGES * STAGE);
+  }
+  if (left) {      // the last 4, 8 or 12 of k, through registers, zeros behind them
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4*>(&ring[(tid / 4 + 64 * i) * TBK + tid % 4 * 4]) =
+          chunk < left ? *reinterpret_cast<const f32x4*>(src[i] + k_first + steps * TBK + chunk) : zero;
+    }
+    __syncthreads();
+    multiply(ring);
   }
 
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int j = 0; j < NI; ++j) {
+    const int n = n0 + wave_n * 32 * NI + j * 32 + r32;
+    if (n >= g.N) continue;
+    const float bias = part ? 0.f : f32_bias_at(g, n);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = m0 + wave_m * 32 * MI + i * 32 + 8 * (v / 4) + 4 * kk + v % 4;
-      if (m >= g.M) continue;
-      if (g.a_rows && g.a_rows[m] < 0) continue;
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j) {
-        const int n = n0 + wave_n * 32 * NI + j * 32 + r32;
-        if (n >= g.N) continue;
+      for (int v = 0; v < 16; ++v) {
+        const int r = i * 32 + 8 * (v / 4) + 4 * kk + v % 4, m = mw + r;
+        if (!((live >> r) & 1)) continue;
         if (part) {
           part[((size_t)blockIdx.z * g.M + m) * g.N + n] = acc[i][j][v];
           if (DUAL) part[((size_t)(gridDim.z + blockIdx.z) * g.M + m) * g.N + n] = acc2[i][j][v];
           continue;
         }
-        float x = acc[i][j][v] + f32_bias_at(g, n);
+        float x = acc[i][j][v] + bias;
         if (DUAL) x = gated_pair(x, acc2[i][j][v], g.gate, g.limit);
         g.out[(size_t)m * g.ldc + n] = x;
       }
-    }
+  }
 }
 
 // ------------------------------------------------------------------------------------------ few rows
@@ -463,15 +511,15 @@ TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gath
       hipLaunchKernelGGL((gemm_f32_stream_kernel<1, SNT, false>), grid, dim3(256), 0, st, g, k_per_split, k_per_wave, part);
   } else {
     // tiles; 17 to 64 rows of one matrix are a single row of tiles, cut into runs of k where the matrix is narrow
-    const int mi = (grouped || M <= 64) ? 1 : 2;
-    const dim3 grid((M + 64 * mi - 1) / (64 * mi), (N + 127) / 128, runs);
+    const int mi = (grouped || M <= 64) ? 1 : 2, columns = mi == 2 && dual ? 64 : 128;
+    const dim3 grid((M + 64 * mi - 1) / (64 * mi), (N + columns - 1) / columns, runs);
     if (grid.y > 65535) return TQ_ERR_UNSUPPORTED;
     if (mi == 1) {
-      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
-      else hipLaunchKernelGGL((gemm_f32_tile_kernel<1, false>), grid, dim3(256), 0, st, g, k_per_split, part);
+      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, true>), grid, dim3(256), 0, st, g, k_per_split, part);
+      else hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
     } else {
-      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<2, true>), grid, dim3(256), 0, st, g, k_per_split, part);
-      else hipLaunchKernelGGL((gemm_f32_tile_kernel<2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
+      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<2, 1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
+      else hipLaunchKernelGGL((gemm_f32_tile_kernel<2, 2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
     }
   }
   if (runs > 1) {
