@@ -94,6 +94,180 @@ TQ_API int tq_move_rows(const void* src, const int* idx, void* dst, int n, int64
 // A thread takes four consecutive elements at a time when H is a multiple of four (every load is 16 bytes and
 // all of a thread's loads can be on their way at once), else one element at a time; what is computed per
 // element is the same.
+//
+// Rows of whole runs of four numbers, up to 8,192 of them, wait in registers instead (the row kernels below; the kernels that
+// go through LDS serve what is left): a thread asks for its runs of everything that does not hang on another load at
+// once, the norms' weights too, the experts' rows are looked up by the workgroup as a whole, and a sum over the workgroup takes
+// one barrier.  What is computed per element, and the order of every sum, is the same.  For one token that is a chain of waits (a launch,
+// the slots, the rows, a barrier a norm, the store): the sum of a normed part and its norm 3.7 us instead of 5.0, of eight tokens' parts
+// side by side 4.8 (5.0), one norm level; for a prompt's rows it is memory: 2,048 rows of 2,048 behind four experts with two
+// norms 17.8 us instead of 27.1, with one 18.7 (21.3), 13,197 rows of 3,584 behind eight 222 (237; 5.5 TB/s).
+__device__ __forceinline__ void lds_barrier() {      // what the waves wrote to LDS is seen; loads from memory stay on their way
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+// block_sum for THREADS threads with a place in LDS that nothing else uses
+template <int THREADS>
+__device__ __forceinline__ float sum_over_threads(float v, float* red) {
+  v = wave_sum(v);
+  if (threadIdx.x % TQ_WAVE == 0) red[threadIdx.x / TQ_WAVE] = v;
+  lds_barrier();
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < THREADS / TQ_WAVE; ++i) t += red[i];
+  return t;
+}
+// A thread's runs of a row, run u at 4 (threadIdx.x + u THREADS), as they are stored: what is beyond the row is read from its last
+// run, so that no load waits behind a branch, and becomes zeros in `row_of`.
+template <class T>
+struct RawRun {
+  typedef f32x4 type;
+};
+template <>
+struct RawRun<bf16_t> {
+  typedef uint2 type;
+};
+template <int THREADS, int NV, class T>
+__device__ __forceinline__ void load_raw(typename RawRun<T>::type (&v)[NV], const T* __restrict__ p, int H) {
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+    v[u] = *reinterpret_cast<const typename RawRun<T>::type*>(p + min(4 * ((int)threadIdx.x + u * THREADS), H - 4));
+}
+__device__ __forceinline__ f32x4 widened(const f32x4& v) { return v; }
+__device__ __forceinline__ f32x4 widened(const uint2& v) {
+  return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
+}
+template <int THREADS, int NV, class R>
+__device__ __forceinline__ void row_of(f32x4 (&v)[NV], const R (&raw)[NV], int H) {
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+    v[u] = 4 * ((int)threadIdx.x + u * THREADS) < H ? widened(raw[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+template <int THREADS, int NV, class T>
+__device__ __forceinline__ void store_row(T* __restrict__ p, const f32x4 (&v)[NV], int H) {
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const int i = 4 * ((int)threadIdx.x + u * THREADS);
+    if (i < H) store4(p + i, v[u]);
+  }
+}
+// v += coef * part[s] for the S partial sums, one after the other, fetched four at a time (coef 1 without the product: ONE)
+template <int THREADS, int NV, bool ONE>
+__device__ __forceinline__ void add_parts(f32x4 (&v)[NV], const float* __restrict__ part, int S, size_t stride, float coef, int H) {
+  for (int s = 0; s < S; s += 4) {
+    f32x4 t[4][NV];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) load_raw<THREADS, NV>(t[k], part + min(s + k, S - 1) * stride, H);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (s + k < S)
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+          if (ONE) v[u] += t[k][u];
+          else v[u] += coef * t[k][u];
+        }
+  }
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+    if (4 * ((int)threadIdx.x + u * THREADS) >= H) v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// v += sum_j wgt[j] * y[slot[j]], j ascending; slot and wgt are the same for the whole workgroup.  A slot of -1 is a pair without a
+// row: a row of zeros, or (SKIP) nothing.
+template <int THREADS, int NV, bool SKIP>
+__device__ __forceinline__ void add_experts(f32x4 (&v)[NV], const float* __restrict__ y, const int* __restrict__ slot,
+                                            const float* __restrict__ wgt, int topk, int H) {
+  for (int j = 0; j < topk; j += 4) {
+    f32x4 t[4][NV];
+    int at[4];
+    float wt[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      at[k] = slot[min(j + k, topk - 1)];
+      wt[k] = wgt[min(j + k, topk - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) load_raw<THREADS, NV>(t[k], y + (size_t)max(at[k], 0) * H, H);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (j + k < topk && (!SKIP || at[k] >= 0))
+#pragma unroll
+        for (int u = 0; u < NV; ++u) v[u] += wt[k] * (SKIP || at[k] >= 0 ? t[k][u] : f32x4{0.f, 0.f, 0.f, 0.f});
+  }
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+    if (4 * ((int)threadIdx.x + u * THREADS) >= H) v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+template <int NV>
+__device__ __forceinline__ float sum_of_squares(const f32x4 (&v)[NV]) {
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    ss += v[u].x * v[u].x;
+    ss += v[u].y * v[u].y;
+    ss += v[u].z * v[u].z;
+    ss += v[u].w * v[u].w;
+  }
+  return ss;
+}
+// The threads of a row and runs of a thread that the row kernels take for rows of H numbers (a function of H alone: a row's sums do
+// not depend on what else the step holds), as body(THREADS, NV); rows that they do not take go on behind it.
+#define TQ_ROW_KERNELS(H, BODY)             \
+  do {                                      \
+    if ((H) % 4 == 0 && (H) <= 8192) {      \
+      if ((H) <= 1024) BODY(256, 1);        \
+      else if ((H) < 2048) BODY(256, 2);    \
+      else if ((H) <= 2048) BODY(512, 1);   \
+      else if ((H) <= 4096) BODY(512, 2);   \
+      else BODY(512, 4);                    \
+      TQ_LAUNCH_CHECK();                    \
+      return 0;                             \
+    }                                       \
+  } while (0)
+
+template <class W, int THREADS, int NV>
+__global__ __launch_bounds__(THREADS) void add_rmsnorm_row_kernel(
+    float* __restrict__ x, const float* __restrict__ delta, int S, size_t delta_stride, const float* __restrict__ y,
+    const int* __restrict__ pair_slot, const float* __restrict__ weights, int topk, const float* __restrict__ gate,
+    const W* __restrict__ w, float eps, const int* __restrict__ rows, act_t* __restrict__ out, float* __restrict__ out32, int H) {
+  __shared__ float red[THREADS / TQ_WAVE];
+  const int r = blockIdx.x, row = rows ? rows[r] : r;
+  float* xr = x + (size_t)row * H;
+  const float* dr = delta + (size_t)row * H;
+  f32x4 a[NV], xv[NV];
+  typename RawRun<W>::type wv[NV];
+  load_raw<THREADS, NV>(xv, xr, H);
+  load_raw<THREADS, NV>(wv, w, H);
+  row_of<THREADS, NV>(a, xv, H);
+  if (y) {
+    const float g = gate ? gate[row] : 1.0f;
+    f32x4 acc[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    add_experts<THREADS, NV, false>(acc, y, pair_slot + (size_t)row * topk, weights + (size_t)row * topk, topk, H);
+    if (S > 0) {
+      f32x4 sh[NV];
+#pragma unroll
+      for (int u = 0; u < NV; ++u) sh[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      add_parts<THREADS, NV, true>(sh, dr, S, delta_stride, 1.f, H);
+#pragma unroll
+      for (int u = 0; u < NV; ++u) acc[u] += g * sh[u];
+    }
+#pragma unroll
+    for (int u = 0; u < NV; ++u) a[u] += acc[u];
+  } else {
+    add_parts<THREADS, NV, true>(a, dr, S, delta_stride, 1.f, H);
+  }
+  if (!rows) store_row<THREADS, NV>(xr, a, H);
+  const float ss = sum_over_threads<THREADS>(sum_of_squares(a), red) / (float)H + eps;
+  const float rs = 1.0f / sqrtf(ss);
+#pragma unroll
+  for (int u = 0; u < NV; ++u) a[u] = a[u] * rs * widened(wv[u]);
+  if (out) store_row<THREADS, NV>(out + (size_t)r * H, a, H);
+  if (out32) store_row<THREADS, NV>(out32 + (size_t)r * H, a, H);
+}
+
 template <class W>
 __global__ void add_rmsnorm_kernel(float* __restrict__ x, const float* __restrict__ delta, int S,
                                    size_t delta_stride, const float* __restrict__ y,
@@ -215,8 +389,13 @@ TQ_API int tq_add_rmsnorm(float* x, const float* delta, int S, int64_t delta_str
                           hipStream_t st) {
   if (R <= 0) return 0;
   if (y && (topk < 1 || topk > 64 || !pair_slot || !weights)) return TQ_ERR_BAD_ARG;
-  // a row of 2,048 and more by 512 threads, so that each takes its four elements in one go and all of a row's loads
-  // are on their way at once (a function of H alone: a row's sums do not depend on what else the step holds)
+#define TQ_BODY(THREADS, NV)                                                                                                        \
+  TQ_DISPATCH_W(wtype, {                                                                                                            \
+    hipLaunchKernelGGL((add_rmsnorm_row_kernel<W, THREADS, NV>), dim3(R), dim3(THREADS), 0, st, x, delta, S, (size_t)delta_stride,  \
+                       y, pair_slot, weights, topk, gate, (const W*)w, eps, rows, (act_t*)out, out32, H);                           \
+  })
+  TQ_ROW_KERNELS(H, TQ_BODY);
+#undef TQ_BODY
   const int threads = (H % 4 == 0 && H >= 2048) ? 512 : 256;
   const size_t shmem = (size_t)((H + 3) / 4 * 4 + threads / TQ_WAVE) * sizeof(float);
   if (shmem > 150 * 1024) return TQ_ERR_UNSUPPORTED;
@@ -346,6 +525,46 @@ __global__ void add_terms_rmsnorm_kernel(float* __restrict__ x, TermArgs terms, 
   }
 }
 
+template <class W, int THREADS, int NV>
+__global__ __launch_bounds__(THREADS) void add_terms_rmsnorm_row_kernel(
+    float* __restrict__ x, TermArgs terms, size_t delta_stride, const float* __restrict__ vec, const float* __restrict__ y,
+    const int* __restrict__ pair_slot, const float* __restrict__ weights, int topk, const W* __restrict__ w, float eps,
+    const int* __restrict__ rows, act_t* __restrict__ out, float* __restrict__ out32, int H) {
+  __shared__ float red[THREADS / TQ_WAVE];
+  const int r = blockIdx.x, row = rows ? rows[r] : r;
+  float* xr = x + (size_t)row * H;
+  f32x4 a[NV], xv[NV], t[NV];
+  typename RawRun<W>::type wv[NV];
+  load_raw<THREADS, NV>(xv, xr, H);
+  if (w) load_raw<THREADS, NV>(wv, w, H);
+  if (vec) load_raw<THREADS, NV>(t, vec, H);
+  row_of<THREADS, NV>(a, xv, H);
+  if (vec) {
+    row_of<THREADS, NV>(t, t, H);
+#pragma unroll
+    for (int u = 0; u < NV; ++u) a[u] += t[u];
+  }
+  if (y) {
+    f32x4 acc[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    add_experts<THREADS, NV, false>(acc, y, pair_slot + (size_t)row * topk, weights + (size_t)row * topk, topk, H);
+#pragma unroll
+    for (int u = 0; u < NV; ++u) a[u] += acc[u];
+  }
+#pragma unroll
+  for (int g = 0; g < TERMS; ++g)
+    if (g < terms.n) add_parts<THREADS, NV, false>(a, terms.delta[g] + (size_t)row * H, terms.S[g], delta_stride, terms.coef[g], H);
+  if (!rows) store_row<THREADS, NV>(xr, a, H);
+  if (!w) return;
+  const float ss = sum_over_threads<THREADS>(sum_of_squares(a), red);
+  const float rs = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int u = 0; u < NV; ++u) a[u] = a[u] * rs * widened(wv[u]);
+  if (out) store_row<THREADS, NV>(out + (size_t)r * H, a, H);
+  if (out32) store_row<THREADS, NV>(out32 + (size_t)r * H, a, H);
+}
+
 // deltas, S, coef: n parts (host arrays; n may be 0), all with partial sums delta_stride floats apart.
 TQ_API int tq_add_terms_rmsnorm(float* x, const int64_t* deltas, const int* S, const float* coef, int n, int64_t delta_stride,
                                 const float* vec, const float* y, const int* pair_slot, const float* weights, int topk,
@@ -366,6 +585,13 @@ TQ_API int tq_add_terms_rmsnorm(float* x, const int64_t* deltas, const int* S, c
   }
   t.n = n;
   if (slices > TERM_SLICES) return TQ_ERR_UNSUPPORTED;
+#define TQ_BODY(THREADS, NV)                                                                                                            \
+  TQ_DISPATCH_W(wtype, {                                                                                                                \
+    hipLaunchKernelGGL((add_terms_rmsnorm_row_kernel<W, THREADS, NV>), dim3(R), dim3(THREADS), 0, st, x, t, (size_t)delta_stride, vec,  \
+                       y, pair_slot, weights, topk, (const W*)w, eps, rows, (act_t*)out, out32, H);                                     \
+  })
+  TQ_ROW_KERNELS(H, TQ_BODY);
+#undef TQ_BODY
   const int threads = (H % 4 == 0 && H >= 2048) ? 512 : 256;
   const size_t shmem = (size_t)((H + 3) / 4 * 4 + threads / TQ_WAVE) * sizeof(float);
   if (shmem > 150 * 1024) return TQ_ERR_UNSUPPORTED;
@@ -1057,6 +1283,67 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ x, const float* __
   }
 }
 
+template <class W, int THREADS, int NV>
+__global__ __launch_bounds__(THREADS) void add_normed_rmsnorm_row_kernel(
+    float* __restrict__ x, const float* __restrict__ delta, int S, size_t delta_stride, const float* __restrict__ y,
+    const int* __restrict__ pair_slot, const float* __restrict__ weights, int topk, const float* __restrict__ gate,
+    const W* __restrict__ wd, float eps_d, const W* __restrict__ w, float eps, const int* __restrict__ rows, act_t* __restrict__ out,
+    float* __restrict__ out32, int H, const float* __restrict__ shift_w, float* __restrict__ shift_state,
+    const int* __restrict__ shift_slots) {
+  __shared__ float red[2][THREADS / TQ_WAVE];
+  const int r = blockIdx.x, row = rows ? rows[r] : r;
+  float* xr = x + (size_t)row * H;
+  const float* dr = delta + (size_t)row * H;
+  f32x4 a[NV], d[NV], was[NV], sw[NV];
+  typename RawRun<W>::type wdv[NV], wv[NV];
+  load_raw<THREADS, NV>(a, xr, H);
+  load_raw<THREADS, NV>(wdv, wd, H);
+  if (w) load_raw<THREADS, NV>(wv, w, H);
+  float* kept = shift_state ? shift_state + (size_t)shift_slots[row] * H : nullptr;
+  if (kept) {
+    load_raw<THREADS, NV>(was, kept, H);
+    load_raw<THREADS, NV>(sw, shift_w, H);
+  }
+#pragma unroll
+  for (int u = 0; u < NV; ++u) d[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (y) {
+    const float g = gate ? gate[row] : 1.0f;
+    add_experts<THREADS, NV, true>(d, y, pair_slot + (size_t)row * topk, weights + (size_t)row * topk, topk, H);
+    if (S > 0) {
+      f32x4 sh[NV];
+#pragma unroll
+      for (int u = 0; u < NV; ++u) sh[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      add_parts<THREADS, NV, true>(sh, dr, S, delta_stride, 1.f, H);
+#pragma unroll
+      for (int u = 0; u < NV; ++u) d[u] += g * sh[u];
+    }
+  } else {
+    add_parts<THREADS, NV, true>(d, dr, S, delta_stride, 1.f, H);
+  }
+  const float ss = sum_over_threads<THREADS>(sum_of_squares(d), red[0]);
+  const float rd = 1.0f / sqrtf(ss / (float)H + eps_d);
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+    a[u] = 4 * ((int)threadIdx.x + u * THREADS) < H ? a[u] + (d[u] * rd) * widened(wdv[u]) : f32x4{0.f, 0.f, 0.f, 0.f};
+  if (!rows) store_row<THREADS, NV>(xr, a, H);
+  if (!w) {      // the summed stream itself, for a part that reads it un-normed
+    if (!out) return;
+    if (kept) {
+      store_row<THREADS, NV>(kept, a, H);
+#pragma unroll
+      for (int u = 0; u < NV; ++u) a[u] = a[u] + (was[u] - a[u]) * sw[u];
+    }
+    store_row<THREADS, NV>(out + (size_t)r * H, a, H);
+    return;
+  }
+  const float s2 = sum_over_threads<THREADS>(sum_of_squares(a), red[1]);
+  const float rs = 1.0f / sqrtf(s2 / (float)H + eps);
+#pragma unroll
+  for (int u = 0; u < NV; ++u) a[u] = a[u] * rs * widened(wv[u]);
+  if (out) store_row<THREADS, NV>(out + (size_t)r * H, a, H);
+  if (out32) store_row<THREADS, NV>(out32 + (size_t)r * H, a, H);
+}
+
 TQ_API int tq_add_normed_rmsnorm_shift(float* x, const float* delta, int S, int64_t delta_stride, const float* y,
                                        const int* pair_slot, const float* weights, int topk, const float* gate,
                                        const void* wd, float eps_d, const void* w, int wtype, float eps, const int* rows,
@@ -1084,6 +1371,16 @@ TQ_API int tq_add_normed_rmsnorm_shift(float* x, const float* delta, int S, int6
   if (shift_state && (w || rows || !out || !shift_w || !shift_slots)) return TQ_ERR_BAD_ARG;
   if (!wd || (y && (topk < 1 || topk > 64 || !pair_slot || !weights))) return TQ_ERR_BAD_ARG;
   if (!y && (S < 1 || !delta)) return TQ_ERR_BAD_ARG;
+#define TQ_BODY(THREADS, NV)                                                                                                       \
+  TQ_DISPATCH_W(wtype, {                                                                                                           \
+    hipLaunchKernelGGL((add_normed_rmsnorm_row_kernel<W, THREADS, NV>), dim3(R), dim3(THREADS), 0, st, x, delta, S,                \
+                       (size_t)delta_stride, y, pair_slot, weights, topk, gate, (const W*)wd, eps_d, (const W*)w, eps, rows,       \
+                       (act_t*)out, out32, H, shift_w, shift_state, shift_slots);                                                  \
+  })
+  // (the kernel through LDS reads all but the terms number by number: rows that do not start at whole runs are its own)
+  const uintptr_t starts = (uintptr_t)x | (uintptr_t)wd | (uintptr_t)w | (uintptr_t)out | (uintptr_t)out32 | (uintptr_t)shift_w | (uintptr_t)shift_state;
+  if (starts % 16 == 0 && delta_stride % 4 == 0) TQ_ROW_KERNELS(H, TQ_BODY);
+#undef TQ_BODY
   const int threads = (H % 4 == 0 && H >= 2048) ? 512 : 256;
   const size_t shmem = (size_t)((H + 3) / 4 * 4 + threads / TQ_WAVE) * sizeof(float);
   if (shmem > 150 * 1024) return TQ_ERR_UNSUPPORTED;
