@@ -104,6 +104,18 @@ __device__ __forceinline__ float wave_max(float v) {
   return lanes_fold<TQ_WAVE>(v, LanesMax());
 }
 
+// Inclusive sum over the lanes up to one's own, in the vector unit as well: within rows of 16 by shifts, then the rows' last lanes
+// into the rows behind them.
+__device__ __forceinline__ int wave_scan_add(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);      // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);     // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);     // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 // Sum over a workgroup in a fixed order: waves reduce by butterfly, wave totals are added
 // in wave order.  `red` holds one float per wave.  Every thread gets the total.
 __device__ __forceinline__ float block_sum(float v, float* red) {
