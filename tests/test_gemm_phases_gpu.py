@@ -74,3 +74,34 @@ def test_rows_in_place_and_a_wider_result(ops):
     got, want = (ops.gemm(h, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=rows, gather=False)
                  for rows in (64 + ops.TILE_PAIRS, 64))
     assert torch.equal(got[st >= 0], want[st >= 0])
+
+
+# the second product: fewer rows than a tile, more than one row of tiles; k in one run and (5,632 beside 192) in several, the last shorter
+@pytest.mark.parametrize("T,K,N,K2,N2", [(65, 192, 100, 128, 130), (300, 256, 263, 640, 72), (777, 192, 64, 5632, 200), (515, 128, 40, 2112, 256)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_a_product_beside_the_experts(ops, T, K, N, K2, N2, gated):
+    """Both products of gemm_pair in one launch: the experts' rows bit for bit as alone, the other's as unit by unit in one run of k, and
+    its partial sums in as many runs as it says, each within the rounding of its sum."""
+    st, _slot, te, nt = order(ops, COUNTS)
+    x, w = drawn((sum(COUNTS), K), 1), drawn((len(COUNTS), N, K), 2, 0.1)
+    a, b = drawn((T, K2), 6), drawn((N2, K2), 7, 0.1)
+    first = dict(a=x, w=w, a_rows=st, tile_group=te, n_tiles=nt, tile_rows=64 + ops.TILE_PAIRS)
+    second = dict(a=a, w=b)
+    if gated:
+        first.update(w2=drawn(w.shape, 3, 0.1), out_act=True, activation="silu", pair_limit=0.7)
+        second.update(w2=drawn(b.shape, 8, 0.1), out_act=True, activation="gelu_tanh")
+    else:
+        second.update(partial_sums=True)
+    y1, y2 = ops.gemm_pair(dict(first), dict(second), "bfloat16")
+    want = ops.gemm(first.pop("a"), first.pop("w"), "bfloat16", **first)
+    assert torch.equal(y1[st >= 0], want[st >= 0])
+    if gated:
+        alone = ops.gemm(a, b, "bfloat16", w2=second["w2"], out_act=True, activation="gelu_tanh")
+        assert torch.equal(y2, alone)
+    else:
+        runs = y2.shape[0]
+        assert (runs > 1) == (K2 >= 2048)
+        per = -(-(K2 // 64) // runs) * 64
+        for z in range(runs):
+            az, bz = a[:, z * per:(z + 1) * per].double(), b[:, z * per:(z + 1) * per].double()
+            assert ((y2[z].double() - az @ bz.T).abs() <= K2 * 2.0 ** -24 * (az.abs() @ bz.abs().T)).all()

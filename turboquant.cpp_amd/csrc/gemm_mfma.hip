@@ -855,7 +855,7 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
     } else if (tile_rows == 64 || tile_rows == 64 + TQ_TILE_PAIRS) {
       if ((N + TBN - 1) / TBN > 65535 || M % 64) return TQ_ERR_UNSUPPORTED;
       if (tile_rows != 64 && K % TBK == 0 && K >= 2 * TBK)
-        rc = launch_gemm_phases(g, dual, out_act, st);
+        rc = launch_gemm_phases(g, nullptr, dual, out_act, st);
       else
         rc = launch_tile<64, 2, 4>(g, dual, out_act, 1, st);
     } else if (tile_rows == 128) {     // experts with hundreds of rows each: the taller tile's rate for little padding
@@ -934,11 +934,14 @@ TQ_API int tq_gemm_mfma_pair_splits(int N1, int K1, int grouped1, int N2, int K2
 // with M <= 16), both gated or both not, both into the same type.  The waves that split k are those of the first
 // product (the larger one by convention).  splits2 > 1 (as tq_gemm_mfma_pair_splits says, for a plain second product
 // into float): run z of its k goes to out + z * M * ldc, the bias to run 0.
+TQ_API int tq_gemm_phases_pair_splits(int M1, int N1, int K1, int M2, int N2, int K2);
+
 TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, hipStream_t st) {
   MfmaGemmArgs g[2];
   int row_tiles[2];
   bool dual[2], out_act[2];
   const int64_t* d[2] = {d1, d2};
+  const bool many = d1[17] == 64 + TQ_TILE_PAIRS;
   for (int i = 0; i < 2; ++i) {
     const int64_t* p = d[i];
     const int M = (int)p[14], N = (int)p[15], K = (int)p[16], tile_rows = (int)p[17];
@@ -953,6 +956,10 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
     if (g[i].gate < 0 || g[i].gate >= TQ_GATE_COUNT) return TQ_ERR_BAD_ARG;
     dual[i] = p[5] != 0;
     out_act[i] = p[13] != 0;
+    if (many) {
+      if (K % TBK || K < 2 * TBK || (i == 0 ? M % 64 || !g[i].tile_group : g[i].tile_group || g[i].a_rows)) return TQ_ERR_BAD_ARG;
+      continue;
+    }
     if (g[i].tile_group) {
       if (tile_rows != 16 || M % 16) return TQ_ERR_BAD_ARG;
       row_tiles[i] = M / 16;
@@ -963,6 +970,16 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
   }
   if (dual[0] != dual[1] || out_act[0] != out_act[1]) return TQ_ERR_BAD_ARG;
   if (splits2 < 1) return TQ_ERR_BAD_ARG;
+  if (many) {
+    if (splits2 > 1) {
+      if (dual[1] || out_act[1] || splits2 != tq_gemm_phases_pair_splits(g[0].M, g[0].N, g[0].K, g[1].M, g[1].N, g[1].K)) return TQ_ERR_BAD_ARG;
+      g[1].k_per = (g[1].K / TBK + splits2 - 1) / splits2 * TBK;
+      g[1].split_stride = (int64_t)g[1].M * g[1].ldc;
+    }
+    if (const int rc = launch_gemm_phases(g[0], &g[1], dual[0], out_act[0], st)) return rc;
+    TQ_LAUNCH_CHECK();
+    return 0;
+  }
   if (splits2 > 1) {
     if (dual[1] || out_act[1] || g[1].a_rows || g[1].tile_group) return TQ_ERR_BAD_ARG;
     g[1].k_per = pair_run_of_k(g[0].N, g[0].K, g[0].tile_group != nullptr, g[1].N, g[1].K, false);

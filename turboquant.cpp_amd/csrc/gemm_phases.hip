@@ -79,7 +79,7 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
   bf16_t* Ws = lds + 4 * A_SLOT;                                 // [WT tiles][2 halves][W_SLOT]
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wm = wave / 4, wn = wave % 4;      // group; a wave's 32 columns of either half
-  const int steps = g.K / TBK;
+  const int steps = g.k_per / TBK;
 
   // What this thread asks for: group 0 the rows of a that group 1 multiplies and the first half of w, group 1 the others; rows
   // row + 32 i, the chunk of 16 bytes that belongs at place tid % 8 (the swizzle is in what is asked for).  Rows past the end
@@ -310,23 +310,17 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
   }
 }
 
-// Which tile this workgroup takes: a die (workgroups are dealt to the 8 of them in turn) gets a contiguous run of tiles.  One
-// matrix: bands of 8 row tiles, down a band's columns.  A matrix per expert: expert by expert, so that an expert's matrices are
-// read by one die, and within an expert column by column with its items side by side.
-template <bool DUAL, bool OUT_ACT>
-__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int gy = gridDim.y, id = blockIdx.y * gridDim.x + blockIdx.x;
+// Tile `logical` of a product in the order in which a die goes through its run of them.  One matrix: bands of 8 row tiles, down a
+// band's columns (a run of k behind the other).  A matrix per expert: expert by expert, so that an expert's matrices are read by one
+// die, and within an expert column by column with its items side by side.
+template <bool DUAL>
+__device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int gx, int gy, int height, PhaseTile& p) {
   const int lane = threadIdx.x % 64;
-  PhaseTile p;
   int tile_n, group = 0;
   if (g.tile_group) {
     const int units_all = g.M / 64;
     const int* items = g.tile_group + units_all;
-    const int n_units = min(g.n_tiles[0], units_all), n_items = min(g.n_tiles[1], units_all);
-    const int total = n_items * gy, die = id % 8, q = total / 8, rem = total % 8;
-    if (id / 8 >= q + (die < rem ? 1 : 0)) return;
-    const int logical = die * q + min(die, rem) + id / 8;
+    const int n_units = min(g.n_tiles[0], units_all), n_items = gx;
     const int at = logical / gy;
     group = g.tile_group[items[at]];
     // the expert's items lo .. hi - 1, 64 candidates at a time
@@ -349,35 +343,90 @@ __global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g) {
     p.m0 = u0 * 64;
     p.units = min((item + 1 < n_items ? items[item + 1] : n_units) - u0, 4);
   } else {
-    const int gx = gridDim.x, total = gx * gy, die = id % 8, q = total / 8, rem = total % 8;
-    const int logical = die * q + min(die, rem) + id / 8;
+    const int run = logical / (gx * gy);
+    logical %= gx * gy;
+    if (g.k_per < g.K) {      // partial sums: run z of k, its sums to out + z * split_stride, the bias with run 0
+      const int k_lo = run * g.k_per;
+      g.a += k_lo;
+      g.w += k_lo;
+      g.out = (float*)g.out + run * g.split_stride;
+      if (run) g.bias = nullptr;
+      g.k_per = min(g.k_per, g.K - k_lo);
+    }
     const int band = logical / (8 * gy), in_band = logical % (8 * gy), bh = min(8, gx - band * 8);
     tile_n = in_band / bh;
-    p.m0 = (band * 8 + in_band % bh) * 256;
-    p.units = min((g.M - p.m0 + 63) / 64, 4);
+    p.m0 = (band * 8 + in_band % bh) * 64 * height;
+    p.units = min((g.M - p.m0 + 63) / 64, height);
   }
   p.w = g.w + (size_t)group * g.group_stride;
   p.w2 = DUAL ? g.w2 + (size_t)group * g.group_stride : p.w;
   p.n0 = tile_n * (DUAL ? 128 : 256);
   p.n1 = DUAL ? p.n0 : p.n0 + 128;
+}
+template <bool DUAL, bool OUT_ACT>
+__device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int gy, int height, bf16_t* lds) {
+  PhaseTile p;
+  phase_tile_of<DUAL>(g, logical, gx, gy, height, p);
   switch (__builtin_amdgcn_readfirstlane(p.units)) {
-    case 4: phases_tile<4, DUAL, OUT_ACT>(g, p, (bf16_t*)smem); break;
-    case 3: phases_tile<3, DUAL, OUT_ACT>(g, p, (bf16_t*)smem); break;
-    case 2: phases_tile<2, DUAL, OUT_ACT>(g, p, (bf16_t*)smem); break;
-    default: phases_tile<1, DUAL, OUT_ACT>(g, p, (bf16_t*)smem);
+    case 4: phases_tile<4, DUAL, OUT_ACT>(g, p, lds); break;
+    case 3: phases_tile<3, DUAL, OUT_ACT>(g, p, lds); break;
+    case 2: phases_tile<2, DUAL, OUT_ACT>(g, p, lds); break;
+    default: phases_tile<1, DUAL, OUT_ACT>(g, p, lds);
   }
 }
 
-// Grid: (units of 64 rows, at most so many items, or tiles of 256 rows of one matrix; tiles of 256 columns, 128 of a gated pair).
-int launch_gemm_phases(const MfmaGemmArgs& g, bool dual, bool out_act, hipStream_t st) {
+// A die (workgroups are dealt to the 8 of them in turn) gets a contiguous run of the tiles of the first product and one of the
+// second, if there is one (n2 tiles, gx2 x gy2 a run of k): `first2`: the second's before the first's, else spread among them.
+template <bool DUAL, bool OUT_ACT>
+__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gx, int gy, int height, int runs, MfmaGemmArgs g2, int gx2,
+                                                          int gy2, int n2, int first2) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if (g.tile_group) gx = min(g.n_tiles[1], g.M / 64);
+  const int id = blockIdx.x, die = id % 8, i = id / 8;
+  const int n1 = gx * gy * runs;
+  const int q1 = n1 / 8, rem1 = n1 % 8, mine1 = q1 + (die < rem1 ? 1 : 0);
+  const int q2 = n2 / 8, rem2 = n2 % 8, mine2 = q2 + (die < rem2 ? 1 : 0);
+  if (i >= mine1 + mine2) return;
+  int in2;      // how many of the second's tiles stand before this place
+  bool second;
+  if (first2) {
+    in2 = min(i, mine2);
+    second = i < mine2;
+  } else {
+    in2 = (int)((int64_t)i * mine2 / (mine1 + mine2));
+    second = (int)((int64_t)(i + 1) * mine2 / (mine1 + mine2)) > in2;
+  }
+  const int logical = second ? die * q2 + min(die, rem2) + in2 : die * q1 + min(die, rem1) + i - in2;
+  if (second) {
+    g = g2;
+    gx = gx2;
+    gy = gy2;
+    height = 4;
+  }
+  phases<DUAL, OUT_ACT>(g, logical, gx, gy, height, (bf16_t*)smem);
+}
+
+// g2 (null: none): a second product, of one matrix and of the same kind, whose tiles fill the chip beside the first's; its k may be
+// in runs (k_per, split_stride).
+int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual, bool out_act, hipStream_t st, int height) {
   const int cols = dual ? 128 : 256;
-  const dim3 grid(g.tile_group ? g.M / 64 : (g.M + 255) / 256, (g.N + cols - 1) / cols);
+  // (units of 64 rows, at most so many items, or tiles of `height` units of one matrix)
+  const int gx = g.tile_group ? g.M / 64 : (g.M + 64 * height - 1) / (64 * height), gy = (g.N + cols - 1) / cols;
+  const int runs = g.tile_group ? 1 : (g.K + g.k_per - 1) / g.k_per;
+  int gx2 = 1, gy2 = 1, n2 = 0, first2 = 0;
+  if (g2) {
+    gx2 = (g2->M + 255) / 256, gy2 = (g2->N + cols - 1) / cols;
+    n2 = gx2 * gy2 * ((g2->K + g2->k_per - 1) / g2->k_per);
+    first2 = g2->k_per >= 3 * g.K / 2;      // tiles that take longer start first
+  }
+  const int64_t per_die = ((int64_t)gx * gy * runs + 7) / 8 + (n2 + 7) / 8;
+  if (per_die * 8 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
   const int shmem = 160 * 1024;      // MI = 2 and 4; 144 KB where MI is 1 or 3
 #define TQ_PHASES(D, O)                                                                                                       \
   do {                                                                                                                        \
     if (hipFuncSetAttribute((const void*)gemm_phases_kernel<D, O>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem) != hipSuccess) \
       return TQ_ERR_UNSUPPORTED;                                                                                              \
-    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), grid, dim3(512), shmem, st, g);                                            \
+    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), dim3((unsigned)(per_die * 8)), dim3(512), shmem, st, g, gx, gy, height, runs, g2 ? *g2 : g, gx2, gy2, n2, first2); \
   } while (0)
   if (dual && out_act) TQ_PHASES(true, true);
   else if (dual) TQ_PHASES(true, false);
@@ -385,4 +434,15 @@ int launch_gemm_phases(const MfmaGemmArgs& g, bool dual, bool out_act, hipStream
   else TQ_PHASES(false, false);
 #undef TQ_PHASES
   return 0;
+}
+
+// Into how many runs the second product's k goes beside a first of M1 rows (at most): so many that none of its tiles takes longer than
+// the chip has to do for both, while a run keeps 1,024 of k and the partial sums, which the kernel behind reads, stay within 256 MB.
+TQ_API int tq_gemm_phases_pair_splits(int M1, int N1, int K1, int M2, int N2, int K2) {
+  const int64_t tiles1 = (int64_t)(M1 + 255) / 256 * ((N1 + 255) / 256), tiles2 = (int64_t)(M2 + 255) / 256 * ((N2 + 255) / 256);
+  const int64_t all = (tiles1 * K1 + tiles2 * K2) / 256;
+  int s = 1;
+  while (s < 8 && K2 / s > all && K2 / (2 * s) >= 1024 && (int64_t)2 * s * M2 * N2 * 4 <= (256 << 20)) s *= 2;
+  while (s > 1 && (int64_t)(s - 1) * (((K2 + TBK - 1) / TBK + s - 1) / s * TBK) >= K2) s /= 2;      // every run begins before the end of k
+  return s;
 }

@@ -213,21 +213,29 @@ void pair_desc(const Product& p, void* out, int tile_rows, int64_t* d) {
 #endif
 
 // Two products that do not depend on each other; mirrors ops.gemm_pair (only the second may leave partial sums).
+// Whether a product over experts by items of several units and one of one matrix go out together (mirrors ops.gemm_pair).
+bool tiles_together(const Product& p1, const Product& p2) {
+  auto suits = [](const Product& p) { return use_mfma(p.w, p.K) && p.K % 64 == 0 && p.K >= 128; };
+  return p1.tile_group && p1.tile_rows == 64 + TQ_TILE_PAIRS && !p2.tile_group && !p2.a_rows && p2.M >= 64 && suits(p1) && suits(p2);
+}
+
 int product_pair(Ctx& c, const Product& p1, const Product& p2, void** out1, void** out2, int* splits2) {
   *splits2 = 1;
 #if defined(TQ_ACT_BF16)
   const Product* ps[2] = {&p1, &p2};
   bool fused = true;
   int tile_rows[2];
+  const bool many = tiles_together(p1, p2);
   for (int i = 0; i < 2; ++i) {
     const Product& p = *ps[i];
     tile_rows[i] = p.tile_rows ? p.tile_rows : (p.M <= 32 ? 16 : 64);
     const bool few = p.tile_group ? tile_rows[i] == 16 : p.M <= 16;
-    fused = fused && few && use_mfma(p.w, p.K);
+    fused = fused && (few || many) && use_mfma(p.w, p.K);
   }
   fused = fused && (p1.w2 == nullptr) == (p2.w2 == nullptr) && p1.out_act == p2.out_act;
   if (fused) {
-    if (p2.partial) *splits2 = tq_gemm_mfma_pair_splits(p1.N, p1.K, p1.tile_group != nullptr, p2.N, p2.K, 0);
+    if (p2.partial && many) *splits2 = tq_gemm_phases_pair_splits(p1.M, p1.N, p1.K, p2.M, p2.N, p2.K);
+    else if (p2.partial) *splits2 = tq_gemm_mfma_pair_splits(p1.N, p1.K, p1.tile_group != nullptr, p2.N, p2.K, 0);
     *out1 = c.arena.take((size_t)p1.M * p1.N * (p1.out_act ? TQ_ACT_BYTES : 4));
     *out2 = c.arena.take((size_t)*splits2 * p2.M * p2.N * (p2.out_act ? TQ_ACT_BYTES : 4));
     int64_t d1[20], d2[20];
@@ -401,8 +409,9 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   sd.lda = Is, sd.w = f.shared_down, sd.M = T, sd.N = H, sd.K = Is, sd.partial = true;
   *pending = Pending();
   pending->pair_slot = pair_slot, pending->weights = weights, pending->topk = k, pending->gate = gate;
-  if (Is > 0 && T <= 16 && unit == 16) {
-    // a handful of tokens: the shared expert's two products ride in the launches of the routed experts'
+  if (Is > 0 && ((T <= 16 && unit == 16) || (tiles_together(eg, sg) && tiles_together(ed, sd)))) {
+    // a handful of tokens: the shared expert's two products ride in the launches of the routed experts'; a long prompt: their
+    // tiles fill the chip together (parts/ffn.py)
     if (int rc = route()) return rc;
     void *h, *hs, *y, *shared;
     int one, splits;

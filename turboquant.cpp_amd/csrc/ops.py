@@ -175,6 +175,7 @@ _OPTIONAL = {
     "tq_gemm_mfma": [_c_ptr, _c_i64, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int,
                      _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "tq_gemm_mfma_splits": [_c_int, _c_int, _c_int],
+    "tq_gemm_phases_pair_splits": [_c_int] * 6,
     "tq_gemm_mfma_pair_splits": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "tq_gemm_mfma_pair": [_c_ptr, _c_ptr, _c_int, _c_ptr],
     "tq_qkv_rope_write": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr,
@@ -1114,9 +1115,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
 
 def gemm_pair(first: dict, second: dict, act) -> tuple[torch.Tensor, torch.Tensor]:
     """Two products that do not depend on each other; ``first`` and ``second`` hold the arguments of ``gemm``
-    (``partial_sums`` only in the second).  Products of few rows of the same kind (both gated or both plain, into
-    the same type) go out in one launch, so that the smaller one costs no launch of its own; anything else is two
-    calls."""
+    (``partial_sums`` only in the second).  Products of the same kind (both gated or both plain, into the same type) go out
+    in one launch where both have few rows, so that the smaller one costs no launch of its own, or where the first is over
+    experts by items of several units of rows (``expert_product_rows``) and the second of one matrix and 64 rows and more,
+    so that the tiles of both fill the chip; anything else is two calls."""
     k = "gemm_pair"
     keys = ("bias", "w2", "out_act", "a_rows", "tile_group", "n_tiles", "tile_rows", "gather", "partial_sums", "activation",
             "pair_limit")
@@ -1133,12 +1135,16 @@ def gemm_pair(first: dict, second: dict, act) -> tuple[torch.Tensor, torch.Tenso
     lib = library(act) if dtype_name(act) == "bfloat16" else None
     fused = lib is not None and hasattr(lib, "tq_gemm_mfma_pair")
     dims = []
+    many = probs[0]["tile_group"] is not None and probs[0]["tile_rows"] == 64 + TILE_PAIRS
     for p in probs:
         M, N, K, tile_rows, gstride = _gemm_problem(k, p["a"], p["w"], act, p["bias"], p["w2"], p["out_act"], p["a_rows"],
                                                     p["tile_group"], p["n_tiles"], p["tile_rows"], p["gather"])
         dims.append((M, N, K, tile_rows, gstride))
-        few = (p["tile_group"] is not None and tile_rows == 16) or (p["tile_group"] is None and M <= 16)
-        fused = fused and few and _use_mfma(act, p["a"], p["w"], K) and (p["bias"] is None or p["bias"].dtype in _WTYPE)
+        if many:
+            suits = K % 64 == 0 and K >= 128 and (p is probs[0] or (p["tile_group"] is None and p["a_rows"] is None and M >= 64))
+        else:
+            suits = (p["tile_group"] is not None and tile_rows == 16) or (p["tile_group"] is None and M <= 16)
+        fused = fused and suits and _use_mfma(act, p["a"], p["w"], K) and (p["bias"] is None or p["bias"].dtype in _WTYPE)
     fused = fused and (probs[0]["w2"] is None) == (probs[1]["w2"] is None) and probs[0]["out_act"] == probs[1]["out_act"]
     if not fused:
         return tuple(gemm(p["a"], p["w"], act, **{n: p[n] for n in keys}) for p in probs)
@@ -1149,8 +1155,8 @@ def gemm_pair(first: dict, second: dict, act) -> tuple[torch.Tensor, torch.Tenso
         p2 = probs[1]
         _need(p2["w2"] is None and not p2["out_act"] and p2["tile_group"] is None and p2["a_rows"] is None, k,
               "partial sums are for plain products into float32")
-        splits = lib.tq_gemm_mfma_pair_splits(dims[0][1], dims[0][2], int(probs[0]["tile_group"] is not None),
-                                              dims[1][1], dims[1][2], 0)
+        splits = lib.tq_gemm_phases_pair_splits(*dims[0][:3], *dims[1][:3]) if many else \
+            lib.tq_gemm_mfma_pair_splits(dims[0][1], dims[0][2], int(probs[0]["tile_group"] is not None), dims[1][1], dims[1][2], 0)
     for p, (M, N, K, tile_rows, gstride) in zip(probs, dims):
         shape = (splits, M, N) if p["partial_sums"] else (M, N)
         out = torch.empty(shape, dtype=adt if p["out_act"] else torch.float32, device=p["a"].device)

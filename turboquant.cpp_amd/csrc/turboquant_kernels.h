@@ -74,6 +74,7 @@ int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gather, co
         void* out, int64_t ldc, int out_is_act, int M, int N, int K, int tile_rows, int splits, int gate,
         hipStream_t st);
 int tq_gemm_mfma_pair_splits(int N1, int K1, int grouped1, int N2, int K2, int grouped2);
+int tq_gemm_phases_pair_splits(int M1, int N1, int K1, int M2, int N2, int K2);
 int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, hipStream_t st);
 int tq_qkv_rope_write(const void* a, int64_t lda, const void* w, const void* bias, int bias_type, int T, int K,
         const int* positions, const int* seq_of_token, const int* block_table, int bt_stride,

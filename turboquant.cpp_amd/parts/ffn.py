@@ -194,10 +194,12 @@ class SparseMoE(Part):
                                   **({} if self.weight_scale == 1.0 else {"weight_scale": self.weight_scale}),
                                   **({} if not self.sigmoid_scores else {"sigmoid": True, "pair_groups": self.pair_groups}), **items)
         limit = {} if self.pair_limit is None else {"pair_limit": self.pair_limit}
-        if self.shared_size > 0 and T <= 16 and unit == 16:
-            # a handful of tokens: the shared expert's two products ride in the launches of the routed experts'
+        if self.shared_size > 0 and ((T <= 16 and unit == 16) or self._tiles_together(normed, ctx, rows)):
+            # a handful of tokens: the shared expert's two products ride in the launches of the routed experts'; a long prompt: the
+            # tiles of both fill the chip together, those that wait for memory beside those that do not (2,048 tokens, 60 experts
+            # of 1,408 x 2,048 and a shared one of 5,632: 302 + 170 us a layer; on a second stream 343 + 146 behind 340 of its own)
             _, weights, gate, sorted_token, pair_slot, tile_expert, n_tiles = route()
-            experts = dict(a_rows=sorted_token, tile_group=tile_expert, n_tiles=n_tiles, tile_rows=unit)
+            experts = dict(a_rows=sorted_token, tile_group=tile_expert, n_tiles=n_tiles, tile_rows=rows)
             h, hs = ops.gemm_pair(dict(a=normed, w=self.expert_gate, w2=self.expert_up, out_act=True,
                                        activation=self.activation, **experts, **limit),
                                   dict(a=normed, w=self.shared_gate, w2=self.shared_up, out_act=True,
@@ -251,6 +253,13 @@ class SparseMoE(Part):
         # a token's weights for the experts that are the identity multiply its own float32 row, which rides where a shared
         # expert's output would
         return ops.GatheredSum(y, pair_slot, weights, normed32[None] if self.identity else None, own if self.identity else None)
+
+    def _tiles_together(self, normed, ctx, rows) -> bool:
+        """Whether the shared expert's products go out with the routed experts' in tiles of many rows (what ops.gemm_pair joins)."""
+        return rows == 64 + ops.TILE_PAIRS and normed.is_cuda and all(
+            K % 64 == 0 and K >= 128 and w.dtype == torch.bfloat16 and ops.dtype_name(ctx.act) == "bfloat16"
+            for K, w in ((self.hidden_size, self.expert_gate), (self.expert_size, self.expert_down),
+                         (self.hidden_size, self.shared_gate), (self.shared_size, self.shared_down)))
 
     def _shared_limit(self) -> dict:
         return {} if self.shared_limit is None else {"pair_limit": self.shared_limit}
