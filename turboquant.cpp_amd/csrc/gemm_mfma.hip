@@ -11,6 +11,7 @@
 //    are read the same way, without the hint, and stay in cache.  The waves of a workgroup split k among them and
 //    add their partial sums in wave order through LDS, so that even a narrow matrix gives the chip enough
 //    waves and bytes in flight.  How k is split depends on N and K only, never on the number of rows.
+//    gemm_lean_kernel is the same for whole lines of k and whole tiles of columns, which nearly all products are.
 //  * gemm_tile_kernel, for many rows (prompts): tiles of BM x 128 outputs by eight waves, 64 of k at a time staged
 //    through two LDS buffers (16-byte chunks, XOR-swizzled by row so that the operand reads of
 //    v_mfma_f32_32x32x16_bf16 do not collide); while one buffer is multiplied the next tile is written into
@@ -219,6 +220,166 @@ __global__ __launch_bounds__(1024) void gemm_stream_pair_kernel(MfmaGemmArgs g1,
     stream_body<1, DUAL, OUT_ACT>(g2, id % nx2, id / nx2 % rows2, id / nx2 / rows2, red);
   else
     stream_body<1, DUAL, OUT_ACT>(g1, (id - n2) % nx1, (id - n2) / nx1, 0, red);
+}
+
+// ------------------------------------------------------------------------------------------ few rows, whole lines
+// The streaming kernel for what nearly every product of a decode step is: k in whole lines of 64, columns in whole tiles of 16, up to
+// 16 rows a tile.  Same sums in the same order as stream_body, so the same bits, but no lane asks whether its chunk or its row is
+// there: a row that is none reads the tile's first row instead (what it gives is never stored: a row of the product depends on its
+// own row of `a` alone), and a last round with fewer lines is a branch of the whole wave.
+//
+// What bounds it: the matrices' way from memory, and for the small ones what a launch and a wave's chain of first load, products, LDS
+// and store take.  Every load a branch of its own, as stream_body has them, kept the last of a round from being asked for until the
+// first had come, and cost a microsecond of 5 to 9.
+// Measured, us a launch in a captured graph, one row: 2,048 x 2,048 5.4 -> 4.4 (a plain read of its bytes: 3.6), 2,048 x 5,632 9.1 ->
+// 6.8, a gated pair of 5,632 x 2,048 12.6 -> 10.4 (read: 8.8), four of 60 experts' pairs of 1,408 x 2,048 12.3 -> 10.6 and second
+// products 8.3 -> 6.7, 32,000 x 2,048 24.2 -> 22.5.  Asking for more lines at once (R) made large products slower: 4 KB of every stream
+// and wave fill the path.
+//
+// NT streams of COLS columns (1, or a gated pair's two matrices), wb[t] their first line of this wave's share, `lines` lines of 64 of
+// k.  A lane's loads are whole lines as above.  COLS 8: the operands of columns 8..15 are other columns' and nothing is stored of
+// them.  A8: the tile has no row behind its eighth, so `a` is read as such a w is (ap: row r % 8, chunk q); else in the operands' own
+// layout (ap: row r, chunk c).
+// v of lane l ^ 8
+__device__ __forceinline__ u32x4 from_other_half(const u32x4& v) {
+  u32x4 s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = __builtin_amdgcn_update_dpp(0, v[i], 0x128, 0xf, 0xf, false);      // row_ror:8
+  return s;
+}
+// row of lane l % 8 of its 16
+__device__ __forceinline__ int row_of_eight(int row) { return __builtin_amdgcn_update_dpp(row, row, 0x128, 0xf, 0xc, false); }
+typedef const __attribute__((address_space(1))) char* global_bytes;
+typedef const __attribute__((address_space(1))) u32x4* global_u32x4;
+template <int COLS, int NT, int R, bool A8, bool FULL>
+__device__ __forceinline__ void lean_round(const global_bytes (&wb)[NT], unsigned off, unsigned off8, global_bytes ap, int lines,
+                                           f32x4 (&acc)[NT]) {
+  u32x4 wf[NT][R][COLS / 8], af[R][2];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    if (!FULL && j && j >= lines) break;
+    af[j][0] = *(global_u32x4)(ap + 128 * j);
+    if (!A8) af[j][1] = *(global_u32x4)(ap + 128 * j + 64);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      wf[t][j][0] = __builtin_nontemporal_load((global_u32x4)(wb[t] + off + 128 * j));
+      if (COLS > 8) wf[t][j][COLS / 8 - 1] = __builtin_nontemporal_load((global_u32x4)(wb[t] + off8 + 128 * j));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    if (!FULL && j && j >= lines) break;
+    if (A8) af[j][1] = from_other_half(af[j][0]);
+    u32x4 second[NT];      // the operand of the line's second half
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (COLS > 8) {
+        to_own_row(wf[t][j][0], wf[t][j][COLS / 8 - 1]);
+        second[t] = wf[t][j][COLS / 8 - 1];
+      } else {
+        second[t] = from_other_half(wf[t][j][0]);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[j][h]),
+                                                         __builtin_bit_cast(bf16x8, h ? second[t] : wf[t][j][0]), acc[t], 0, 0, 0);
+  }
+}
+template <int COLS, int NT, int R, bool A8>
+__device__ __forceinline__ void lean_accumulate(global_bytes (&wb)[NT], unsigned off, unsigned off8, global_bytes ap, int lines,
+                                                f32x4 (&acc)[NT]) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (; lines >= R; lines -= R) {
+    lean_round<COLS, NT, R, A8, true>(wb, off, off8, ap, R, acc);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wb[t] += 128 * R;
+    ap += 128 * R;
+  }
+  if (lines > 0) lean_round<COLS, NT, R, A8, false>(wb, off, off8, ap, lines, acc);
+}
+
+// One workgroup's COLS columns of tile `tile_m` (run z of k); GROUP: a matrix per row tile, by the row order's lists.
+template <bool DUAL, bool OUT_ACT, bool GROUP, int COLS>
+__device__ __forceinline__ void lean_body(const MfmaGemmArgs& g, int tile_n, int tile_m, int z, float* red) {
+  constexpr int NT = DUAL ? 2 : 1, R = 4 / NT;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), nw = blockDim.x / 64;
+  const int r = lane % 16, c = lane / 16, q = c + 4 * (r / 8);
+  const int m0 = GROUP ? tile_m * 16 : 0, n0 = tile_n * COLS;
+  // which matrix and which rows, asked for together
+  const int live_tiles = GROUP ? g.n_tiles[0] : 1, group = GROUP ? g.tile_group[tile_m] : 0;
+  const int src = GROUP ? g.a_rows[m0 + r] : r < g.M ? r : -1;
+  if (GROUP) asm volatile("" ::"s"(group), "v"(src));
+  if (GROUP && tile_m >= live_tiles) return;
+  const unsigned live = (unsigned)__ballot(src >= 0) & 0xffff;
+  const int own = !GROUP || g.a_gather ? src : m0 + r;
+  const int first = __builtin_amdgcn_readfirstlane(own);      // (by all lanes: lane 0 has the tile's first row, which is never padding)
+  const int row = max(src >= 0 ? own : first, 0);
+  const int k_lo = z * g.k_per, k_hi = min(g.K, k_lo + g.k_per);
+  const int steps = (k_hi - k_lo + 31) / 32, per = ((steps + nw - 1) / nw + 1) & ~1;
+  const int k_beg = k_lo + wave * per * 32, lines = (min(k_hi, k_beg + per * 32) - k_beg) / 64;
+  global_bytes wb[NT];
+  wb[0] = (global_bytes)(g.w + (size_t)group * g.group_stride + (size_t)n0 * g.K + k_beg);
+  if (DUAL) wb[NT - 1] = (global_bytes)(g.w2 + (size_t)group * g.group_stride + (size_t)n0 * g.K + k_beg);
+  const unsigned off = ((unsigned)(r % 8) * g.K + q * 8) * 2;
+  f32x4 acc[NT];
+  if (live >> 8)
+    lean_accumulate<COLS, NT, R, false>(wb, off, off + 16 * g.K, (global_bytes)(g.a + (size_t)row * g.lda + k_beg + 8 * c), lines, acc);
+  else
+    lean_accumulate<COLS, NT, R, true>(wb, off, off + 16 * g.K, (global_bytes)(g.a + (size_t)row_of_eight(row) * g.lda + k_beg + 8 * q), lines, acc);
+  float* out = (float*)g.out + z * g.split_stride;      // (runs of k go out as floats)
+  auto store = [&](int i, float s, float s2) {
+    const int on = n0 + i % 16, om = 4 * (i % 64 / 16) + i / 64;
+    if ((COLS < 16 && i % 16 >= COLS) || !((live >> om) & 1)) return;
+    float o = s + (z ? 0.f : bias_at(g, on));
+    if (DUAL) o = gated_pair(o, s2, g.gate, g.limit);
+    if (g.act1) o = gate_fn(o, g.act1 - 1);
+    const size_t at = (size_t)(m0 + om) * g.ldc + on;
+    if (OUT_ACT) ((bf16_t*)g.out)[at] = f32_to_bf16(o);
+    else out[at] = o;
+  };
+  if (nw > 1) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[((wave * NT + t) * 4 + v) * 64 + lane] = acc[t][v];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) {
+      float s = 0.f, s2 = 0.f;
+      for (int w = 0; w < nw; w += 2) {      // (an even number of waves)
+        const float* at = red + w * NT * 256 + i;
+        const float a0 = at[0], a1 = at[NT * 256], b0 = DUAL ? at[256] : 0.f, b1 = DUAL ? at[NT * 256 + 256] : 0.f;
+        s += a0;
+        s += a1;
+        if (DUAL) {
+          s2 += b0;
+          s2 += b1;
+        }
+      }
+      store(i, s, s2);
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) store(v * 64 + lane, acc[0][v], acc[NT - 1][v]);
+  }
+}
+
+template <bool DUAL, bool OUT_ACT, bool GROUP, int COLS>
+__global__ __launch_bounds__(1024) void gemm_lean_kernel(MfmaGemmArgs g) {
+  extern __shared__ float red[];
+  lean_body<DUAL, OUT_ACT, GROUP, COLS>(g, blockIdx.x, blockIdx.y, blockIdx.z, red);
+}
+// (as gemm_stream_pair_kernel; the first over experts, the second of one matrix)
+template <bool DUAL, bool OUT_ACT>
+__global__ __launch_bounds__(1024) void gemm_lean_pair_kernel(MfmaGemmArgs g1, int nx1, MfmaGemmArgs g2, int nx2, int n2) {
+  extern __shared__ float red[];
+  const int id = blockIdx.x;
+  if (id < n2) lean_body<DUAL, OUT_ACT, false, 8>(g2, id % nx2, 0, id / nx2, red);
+  else lean_body<DUAL, OUT_ACT, true, 8>(g1, (id - n2) % nx1, (id - n2) / nx1, 0, red);
 }
 
 // ------------------------------------------------------------------------------------------ q, k, v of a few tokens
@@ -638,6 +799,22 @@ static int split_k_waves(int N, int K, bool grouped) {
 }
 
 // MT row tiles of 16; more than one (17 to 64 rows of one matrix) go with two column tiles per wave.
+// Whether lean_body takes a product of at most 16 rows a tile.
+static bool lean_suits(const MfmaGemmArgs& g) {
+  return g.K % 64 == 0 && g.N % 16 == 0 && g.K < (1 << 26) && g.k_per % 64 == 0 &&
+         (g.tile_group ? g.a_rows && g.n_tiles : !g.a_rows && !g.n_tiles && g.M <= 16);
+}
+// A workgroup's columns there.  Tiles of 8 leave fewer compute units without work (one row by 2,048 x 5,632: 6.9 us against 8.5 in
+// tiles of 16, 2,048 x 8,448 8.7 against 11.7, a gated pair of 5,632 x 2,048 10.4 against 12.4; experts' pairs 10.6 against 11.8,
+// 151,936 x 2,048 106 against 110) but read `a` twice as often: tiles of 16 where they give every compute unit a full workgroup
+// (8 rows by 4,096 x 4,096: 9.3 against 10.3) and for more than 8 rows of many columns (32,000 x 2,048: 24.2 against 26.2).
+static int lean_columns(const MfmaGemmArgs& g, int nw, bool dual) {
+  const int tiles = g.N / 16;
+  if (tiles < 192) return 8;
+  if (tiles <= 256 && nw == 8 && !g.tile_group) return 16;
+  return dual || g.tile_group || g.M <= 8 ? 8 : 16;
+}
+
 template <int MT>
 static int launch_stream(MfmaGemmArgs g, bool dual, bool out_act, int row_tiles, hipStream_t st, int splits = 1) {
   constexpr int NTL = MT > 1 ? 2 : 1;
@@ -651,6 +828,26 @@ static int launch_stream(MfmaGemmArgs g, bool dual, bool out_act, int row_tiles,
   const dim3 grid((g.N + 16 * NTL - 1) / (16 * NTL), row_tiles, splits);
   const size_t shmem = nw > 1 ? nw * per_wave : 0;
   if (shmem > TQ_STREAM_LDS) return TQ_ERR_UNSUPPORTED;
+  if constexpr (MT == 1) {
+    if (lean_suits(g)) {
+      const int cols = lean_columns(g, nw, dual);
+      const dim3 lean_grid(g.N / cols, row_tiles, splits);
+#define TQ_LEAN(D, O, G, C) hipLaunchKernelGGL((gemm_lean_kernel<D, O, G, C>), lean_grid, dim3(64 * nw), shmem, st, g)
+#define TQ_LEAN_OF(D, O)                        \
+  do {                                          \
+    if (g.tile_group) TQ_LEAN(D, O, true, 8);   \
+    else if (cols == 8) TQ_LEAN(D, O, false, 8); \
+    else TQ_LEAN(D, O, false, 16);              \
+  } while (0)
+      if (dual && out_act) TQ_LEAN_OF(true, true);
+      else if (dual) TQ_LEAN_OF(true, false);
+      else if (out_act) TQ_LEAN_OF(false, true);
+      else TQ_LEAN_OF(false, false);
+#undef TQ_LEAN_OF
+#undef TQ_LEAN
+      return 0;
+    }
+  }
 #define TQ_STREAM(D, O)                                                                                       \
   do {                                                                                                        \
     if (shmem > 48 * 1024)                                                                                    \
@@ -992,6 +1189,18 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
   const int64_t n1 = (int64_t)nx1 * row_tiles[0], n2 = (int64_t)nx2 * row_tiles[1] * splits2;
   if (n1 + n2 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)(n1 + n2));
+  if (g[0].tile_group && !g[1].tile_group && lean_suits(g[0]) && lean_suits(g[1])) {
+    const int lx1 = g[0].N / 8, lx2 = g[1].N / 8, l2 = lx2 * splits2;
+    if ((int64_t)lx1 * row_tiles[0] + l2 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
+#define TQ_PAIR(D, O) hipLaunchKernelGGL((gemm_lean_pair_kernel<D, O>), dim3(lx1 * row_tiles[0] + l2), dim3(64 * nw), shmem, st, g[0], lx1, g[1], lx2, l2)
+    if (dual[0] && out_act[0]) TQ_PAIR(true, true);
+    else if (dual[0]) TQ_PAIR(true, false);
+    else if (out_act[0]) TQ_PAIR(false, true);
+    else TQ_PAIR(false, false);
+#undef TQ_PAIR
+    TQ_LAUNCH_CHECK();
+    return 0;
+  }
 #define TQ_PAIR(D, O) \
   hipLaunchKernelGGL((gemm_stream_pair_kernel<D, O>), grid, dim3(64 * nw), shmem, st, g[0], nx1, g[1], nx2, row_tiles[1], (int)n2)
   if (dual[0] && out_act[0]) TQ_PAIR(true, true);
