@@ -8,7 +8,7 @@
 // sigmoid gate.  Everything here is float arithmetic on both libraries; the products around it are the library's.
 //
 // The kernels, for prompts and for decoding alike (a decoded token is a run of one):
-//   delta_prep   per token: convolution (its first inputs from the sequence's state), silu, unit vectors, beta, and
+//   delta_prep   per token (many tokens: per run of eight): convolution (its first inputs from the sequence's state), silu, unit vectors, beta, and
 //                the low-rank activations of the decay and the gate in the activation type, for the product behind
 //   delta_decay  (steps of many tokens) the decays of all tokens, in parallel, in place of what they are made from
 //   delta_scan   per (sequence, head, block of value channels): the recurrence over the run's tokens in order, the
@@ -89,6 +89,110 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(const float* __restrict
     const float f = (1.0f / sqrtf(ss + 1e-6f)) * (u < G ? 1.0f / sqrtf((float)D) : 1.0f);
     for (int i = lane; i < width; i += TQ_WAVE) dst[i] *= f;
   }
+}
+
+// The same for steps of many tokens, four taps and heads of 64, 128 or 256 channels, same bits: a wave takes its unit of DP_RUN tokens,
+// a lane NU channels of it, whose taps wait in registers and whose inputs are read once, all of them asked for before the first is
+// used.  INSIDE: all of them and the three in front of them are one sequence's, so that no token asks where it begins.  What bounds
+// it: memory, and the chain of a token's sum over the wave.  A token to a wave, as above, reads every input four times, a value at
+// a time behind the search for the run's start: 16 heads of 128, 2,048 tokens (100 MB in and out) 75 us, this way 32; 3,258 tokens
+// of the form with a decay per head 137 and 53.
+#define DP_RUN 8
+template <int NU, bool INSIDE>
+__device__ __forceinline__ void prep_run(const float* __restrict__ P, int NP, int T, int t0, int c0, const int (&slot)[DP_RUN + 3],
+                                         const float* __restrict__ state, int64_t state_stride, int64_t hist_at,
+                                         const float* __restrict__ conv_w, float* __restrict__ dst, int64_t dst_stride, bool unit, float scale) {
+  const int lane = threadIdx.x % TQ_WAVE;
+  float x[DP_RUN + 3][NU], w[4][NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j][u] = conv_w[(size_t)(c0 + lane + u * TQ_WAVE) * 4 + j];
+#pragma unroll
+  for (int i = 0; i < DP_RUN + 3; ++i)
+#pragma unroll
+    for (int u = 0; u < NU; ++u) x[i][u] = P[(size_t)min(max(t0 + i - 3, 0), T - 1) * NP + c0 + lane + u * TQ_WAVE];
+#pragma unroll
+  for (int i = 0; i < DP_RUN; ++i) {
+    if (!INSIDE && t0 + i >= T) return;
+    const int own = slot[i + 3];      // (tokens before the step have a slot that is none)
+    const int before = slot[i + 2] != own ? 0 : slot[i + 1] != own ? 1 : slot[i] != own ? 2 : 3;
+    float y[NU], ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      float in[4] = {x[i][u], x[i + 1][u], x[i + 2][u], x[i + 3][u]};
+      if (!INSIDE && before < 3) {
+        const float* hist = state + (size_t)own * state_stride + hist_at + (size_t)(c0 + lane + u * TQ_WAVE) * 3;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (3 - j > before) in[j] = hist[j + before];
+      }
+      float v = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v = fmaf(w[j][u], in[j], v);
+      y[u] = silu_f(v);
+      ss = fmaf(y[u], y[u], ss);
+    }
+    const float f = unit ? (1.0f / sqrtf(wave_sum(ss) + 1e-6f)) * scale : 1.0f;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) dst[(size_t)(t0 + i) * dst_stride + lane + u * TQ_WAVE] = unit ? y[u] * f : y[u];
+  }
+}
+__global__ __launch_bounds__(256) void delta_prep_runs_kernel(const float* __restrict__ P, const int* __restrict__ slot_of_token,
+                                                              const float* __restrict__ state, int64_t state_stride,
+                                                              const float* __restrict__ conv_w, DeltaDims dm, int T,
+                                                              float* __restrict__ qn, float* __restrict__ kn,
+                                                              float* __restrict__ vc, float* __restrict__ beta,
+                                                              act_t* __restrict__ low, const float* __restrict__ a_log,
+                                                              const float* __restrict__ dt_bias, float* __restrict__ dec) {
+  const int t0 = blockIdx.x * DP_RUN, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TQ_WAVE), lane = threadIdx.x % TQ_WAVE;
+  const int G = dm.G, D = dm.D, H = dm.H, V = dm.V, NP = dd_np(dm), C = dd_channels(dm);
+  const int units = 2 * G + H + 1;
+  int slot[DP_RUN + 3];
+#pragma unroll
+  for (int i = 0; i < DP_RUN + 3; ++i) slot[i] = t0 + i >= 3 ? slot_of_token[min(t0 + i - 3, T - 1)] : -1;
+  bool inside = t0 + DP_RUN <= T;
+#pragma unroll
+  for (int i = 0; i < DP_RUN + 2; ++i) inside = inside && slot[i] == slot[DP_RUN + 2];
+  for (int u = blockIdx.y * 4 + wave; u < units; u += 4 * gridDim.y) {
+    if (u == units - 1) {
+      for (int t = t0; t < min(t0 + DP_RUN, T); ++t) {
+        const float* row = P + (size_t)t * NP;
+        for (int h = lane; h < H; h += TQ_WAVE) beta[(size_t)t * H + h] = sigmoid_f(row[C + h]);
+        if (dm.mode == 1) {
+          for (int h = lane; h < H; h += TQ_WAVE)
+            dec[(size_t)t * H + h] = expf(-expf(a_log[h]) * softplus_f(row[C + H + h] + dt_bias[h]));
+          continue;
+        }
+        for (int i = lane; i < dm.ra + dm.rg; i += TQ_WAVE)
+          low[(size_t)t * (dm.ra + dm.rg) + i] = from_f32<act_t>(row[C + H + i]);
+      }
+      continue;
+    }
+    const bool is_v = u >= 2 * G;
+    const int width = is_v ? V : D, c0 = is_v ? 2 * G * D + (u - 2 * G) * V : u * D;
+    float* dst = is_v ? vc + (size_t)(u - 2 * G) * V : (u < G ? qn + (size_t)u * D : kn + (size_t)(u - G) * D);
+    const int64_t dst_stride = is_v ? (int64_t)H * V : (int64_t)G * D;
+    const float scale = u < G ? 1.0f / sqrtf((float)D) : 1.0f;
+#define TQ_PREP_AT(NU, INSIDE) \
+  prep_run<NU, INSIDE>(P, NP, T, t0, c0, slot, state, state_stride, (int64_t)H * D * V, conv_w, dst, dst_stride, !is_v, scale)
+#define TQ_PREP(NU)                    \
+  do {                                 \
+    if (inside) TQ_PREP_AT(NU, true);  \
+    else TQ_PREP_AT(NU, false);        \
+  } while (0)
+    if (width == 64) TQ_PREP(1);
+    else if (width == 128) TQ_PREP(2);
+    else TQ_PREP(4);
+#undef TQ_PREP
+#undef TQ_PREP_AT
+  }
+}
+// From so many tokens on: below, a wave's eight tokens in turn take longer than a wave to each (16 heads of 128, us by a token to a wave
+// and by runs: 64 tokens 5.0 and 7.5, 128 6.9 and 7.8, 192 9.6 and 9.2, 256 12.8 and 9.4, 512 22.9 and 15.5).
+static bool prep_in_runs(const DeltaDims& d, int T) {
+  auto width = [](int n) { return n == 64 || n == 128 || n == 256; };
+  return T >= 192 && d.taps == 4 && width(d.D) && width(d.V);
 }
 
 // ------------------------------------------------------------------------------------------ decays of a long step
@@ -482,6 +586,12 @@ static int launch_prep(const float* P, const int* slot_of_token, const float* st
   if (T <= 0) return 0;
   if (!dims_ok(d) || state_stride < dd_state(d)) return TQ_ERR_BAD_ARG;
   const int units = 2 * d.G + d.H + 1;
+  if (prep_in_runs(d, T)) {
+    hipLaunchKernelGGL(delta_prep_runs_kernel, dim3((T + DP_RUN - 1) / DP_RUN, (units + 3) / 4 < 65535 ? (units + 3) / 4 : 65535), dim3(256),
+                       0, st, P, slot_of_token, state, state_stride, conv_w, d, T, qn, kn, vc, beta, (act_t*)low, a_log, dt_bias, dec);
+    TQ_LAUNCH_CHECK();
+    return 0;
+  }
   hipLaunchKernelGGL(delta_prep_kernel, dim3(T, (units + 3) / 4 < 65535 ? (units + 3) / 4 : 65535), dim3(256), 0, st, P,
                      slot_of_token, state, state_stride, conv_w, d, qn, kn, vc, beta, (act_t*)low, a_log, dt_bias, dec);
   TQ_LAUNCH_CHECK();
