@@ -1375,7 +1375,7 @@ def _align_outputs(T: int, topk: int, num_experts: int, unit: int, dev):
 def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | None, top_k: int, renormalize: bool,
           unit: int, act, groups: tuple[int, int] | None = None, bias: torch.Tensor | None = None,
           correction: torch.Tensor | None = None, identity: int = 0, sigmoid: bool = False, weight_scale: float = 1.0,
-          pair_groups: bool = False, item_units: int = 2):
+          pair_groups: bool = False):
     """``router_topk`` followed by ``moe_align`` in one call: (ids, weights, gate, sorted_token, pair_slot,
     tile_expert, n_tiles), with the same results; a handful of tokens takes one kernel less.
 
@@ -1383,9 +1383,9 @@ def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | 
     all E rows of the router, the choice is by score + correction and the weights are the scores themselves.  ``identity`` n
     (with ``correction``): the router's last n rows are experts without matrices whose output is their input; their pairs
     get ``pair_slot`` -1 and no rows in the order, and ``gate`` [T] is the sum of each token's weights for them.
-    ``sigmoid``, ``weight_scale``, ``pair_groups``: as for ``router_topk``; ``item_units``: as for ``moe_align``."""
+    ``sigmoid``, ``weight_scale``, ``pair_groups``: as for ``router_topk``.  ``unit`` may be a ``RowUnit``, whose items are as for ``moe_align``."""
     k = "route"
-    listed = _order_unit(k, unit, item_units)
+    listed = _order_unit(k, int(unit), getattr(unit, "item_units", 2))
     T, H, E, ids, weights, gate, logits = _router_outputs(k, x32, router, shared_scale, top_k)
     _need(unit in (16, 32, 64, 128, 256), k, "unit must be 16, 32, 64, 128 or 256")
     if correction is not None:
@@ -1424,6 +1424,17 @@ def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | 
                                          _ptr(logits), listed, cap, _ptr(sorted_token), _ptr(pair_slot), _ptr(tile_expert),
                                          _ptr(n_tiles), T, H, _stream()))
     return ids, weights, gate, sorted_token, pair_slot, tile_expert, n_tiles
+
+
+class RowUnit(int):
+    """The unit of a row order (rows of a tile) together with how many of its tiles an item holds at most: 2, as for a plain
+    int, or 4."""
+    item_units: int
+
+    def __new__(cls, rows: int, item_units: int):
+        unit = super().__new__(cls, rows)
+        unit.item_units = item_units
+        return unit
 
 
 def _order_unit(k: str, unit: int, item_units: int) -> int:

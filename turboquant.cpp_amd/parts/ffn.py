@@ -184,15 +184,15 @@ class SparseMoE(Part):
                                     **({} if self.expert_size % 8 == 0 else {"w_behind": self.expert_down}))
         # what the experts' products are called with, and the items of the row order that they go by
         rows = ops.expert_product_rows(unit, T * self.top_k, self.num_experts)
-        items = {} if rows == unit else {"item_units": 4}
+        unit = unit if rows == unit else ops.RowUnit(unit, 4)
         if self.score_correction or not self.gated:
-            return self._forward_scored(normed, normed32, ctx, unit, rows, items)
+            return self._forward_scored(normed, normed32, ctx, unit, rows)
         route = lambda: ops.route(normed32, self.router, self.shared_scale if self.shared_gated else None,
                                   self.top_k, self.renormalize, unit, ctx.act,
                                   **({} if self.groups is None else {"groups": self.groups}),
                                   **({} if self.router_bias is None else {"bias": self.router_bias}),
                                   **({} if self.weight_scale == 1.0 else {"weight_scale": self.weight_scale}),
-                                  **({} if not self.sigmoid_scores else {"sigmoid": True, "pair_groups": self.pair_groups}), **items)
+                                  **({} if not self.sigmoid_scores else {"sigmoid": True, "pair_groups": self.pair_groups}))
         limit = {} if self.pair_limit is None else {"pair_limit": self.pair_limit}
         if self.shared_size > 0 and ((T <= 16 and unit == 16) or self._tiles_together(normed, ctx, rows)):
             # a handful of tokens: the shared expert's two products ride in the launches of the routed experts'; a long prompt: the
@@ -236,13 +236,13 @@ class SparseMoE(Part):
         # the weighted sum over the chosen experts and the shared expert is left to the next norm
         return ops.GatheredSum(y, pair_slot, weights, shared, gate)
 
-    def _forward_scored(self, normed, normed32, ctx, unit, rows, items):
+    def _forward_scored(self, normed, normed32, ctx, unit, rows):
         """Experts of two matrices, and routers that choose by corrected scores with experts that are the identity."""
         T = normed.shape[0]
         extra = {"correction": self.correction, "identity": self.identity} if self.score_correction else \
             ({} if self.groups is None else {"groups": self.groups}) | ({} if self.router_bias is None else {"bias": self.router_bias})
         _, weights, own, sorted_token, pair_slot, tile_expert, n_tiles = ops.route(
-            normed32, self.router, None, self.top_k, self.renormalize, unit, ctx.act, **extra, **items)
+            normed32, self.router, None, self.top_k, self.renormalize, unit, ctx.act, **extra)
         order = dict(a_rows=sorted_token, tile_group=tile_expert, n_tiles=n_tiles, tile_rows=rows)
         if self.gated:
             h = ops.gemm(normed, self.expert_gate, ctx.act, w2=self.expert_up, out_act=True, activation=self.activation,
