@@ -96,3 +96,27 @@ def test_sum_of_several_parts(ops, H):
     out, out32 = ops.add_rmsnorm(x, ops.Terms([(0.5, a), (2.0, b)], gathered, vec), w, eps, "float32", want_f32=True)
     v = x0.double() + vec.double() + total + 0.5 * a.double().sum(0) + 2.0 * b.double().sum(0)
     assert close(x, v, 64) and close(out, rms(v, w, eps), 256) and torch.equal(out, out32)
+
+
+@pytest.mark.parametrize("act", ["float32", "bfloat16"])
+def test_rows_of_no_numbers(ops, act):
+    """Empty rows come back empty; the library's entries read and write nothing for them."""
+    import ctypes
+    dt = torch.float32 if act == "float32" else torch.bfloat16
+    x, w = drawn((5, 0), 1), drawn((0,), 2, dtype=dt)
+    rows = torch.tensor([4, 0, 4], dtype=torch.int32, device=DEV)
+    for delta in (None, drawn((2, 5, 0), 3), experts(ops, 5, 0, 3, 2, 4)[0]):
+        for picked in (None, rows):
+            out, out32 = ops.add_rmsnorm(x, delta, w, 1e-5, act, rows=picked, want_f32=True)
+            assert out.shape == out32.shape == (5 if picked is None else 3, 0)
+    lib, st = ops.library(act), torch.cuda.current_stream().cuda_stream
+    buf = [drawn((64,), seed) for seed in range(5)]
+    was = [b.clone() for b in buf]
+    x, delta, w, out, out32 = (b.data_ptr() for b in buf)
+    assert lib.tq_add_rmsnorm(x, delta, 2, 8, None, None, None, 0, None, w, 0, 1e-5, None, 5, out, out32, 0, st) == 0
+    assert lib.tq_add_terms_rmsnorm(x, (ctypes.c_int64 * 1)(delta), (ctypes.c_int * 1)(2), (ctypes.c_float * 1)(0.5), 1, 8, None, None,
+                                    None, None, 0, w, 0, 1e-5, None, 5, out, out32, 0, st) == 0
+    assert lib.tq_add_normed_rmsnorm_shift(x, delta, 2, 8, None, None, None, 0, None, w, 1e-5, w, 0, 1e-5, None, 5, out, out32, 0,
+                                           None, None, None, st) == 0
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(buf, was))

@@ -212,18 +212,19 @@ __device__ __forceinline__ float sum_of_squares(const f32x4 (&v)[NV]) {
   return ss;
 }
 // The threads of a row and runs of a thread that the row kernels take for rows of H numbers (a function of H alone: a row's sums do
-// not depend on what else the step holds), as body(THREADS, NV); rows that they do not take go on behind it.
-#define TQ_ROW_KERNELS(H, BODY)             \
-  do {                                      \
-    if ((H) % 4 == 0 && (H) <= 8192) {      \
-      if ((H) <= 1024) BODY(256, 1);        \
-      else if ((H) < 2048) BODY(256, 2);    \
-      else if ((H) <= 2048) BODY(512, 1);   \
-      else if ((H) <= 4096) BODY(512, 2);   \
-      else BODY(512, 4);                    \
-      TQ_LAUNCH_CHECK();                    \
-      return 0;                             \
-    }                                       \
+// not depend on what else the step holds), as body(THREADS, NV); rows that they do not take go on behind it: rows of no
+// numbers too, which have no last run for a load to stay within.
+#define TQ_ROW_KERNELS(H, BODY)                       \
+  do {                                                \
+    if ((H) > 0 && (H) % 4 == 0 && (H) <= 8192) {     \
+      if ((H) <= 1024) BODY(256, 1);                  \
+      else if ((H) < 2048) BODY(256, 2);              \
+      else if ((H) <= 2048) BODY(512, 1);             \
+      else if ((H) <= 4096) BODY(512, 2);             \
+      else BODY(512, 4);                              \
+      TQ_LAUNCH_CHECK();                              \
+      return 0;                                       \
+    }                                                 \
   } while (0)
 
 template <class W, int THREADS, int NV>
