@@ -84,6 +84,18 @@ def test_sum_and_norm(ops, act, H):
             x2 = x0.clone()
             ops.add_rmsnorm(x2, ops.NormedDelta(delta, off, eps), w, eps, act)
             assert close(x2, v, 256)
+            # the sums' order does not hang on where anything starts: the same bits, also where a shared part starts so
+            x1 = x0.clone()
+            want = ops.add_rmsnorm(x1, normed, w, eps, act, want_f32=True)
+            cases = [(delta, off)]
+            if kind == "experts" and parts:
+                dense = torch.cat([delta.dense.flatten()[:1], delta.dense.flatten()])[1:].view_as(delta.dense)
+                assert dense.data_ptr() % 16
+                cases += [(ops.GatheredSum(delta.y, delta.pair_slot, delta.weights, dense, delta.gate), n) for n in (wd, off)]
+            for moved, norm in cases:
+                x2 = x0.clone()
+                got = ops.add_rmsnorm(x2, ops.NormedDelta(moved, norm, eps), w, eps, act, want_f32=True)
+                assert torch.equal(x1, x2) and torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
 
 
 @pytest.mark.parametrize("H", LENGTHS)

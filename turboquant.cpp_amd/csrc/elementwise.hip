@@ -1378,8 +1378,10 @@ TQ_API int tq_add_normed_rmsnorm_shift(float* x, const float* delta, int S, int6
                        (size_t)delta_stride, y, pair_slot, weights, topk, gate, (const W*)wd, eps_d, (const W*)w, eps, rows,       \
                        (act_t*)out, out32, H, shift_w, shift_state, shift_slots);                                                  \
   })
-  // (the kernel through LDS reads all but the terms number by number: rows that do not start at whole runs are its own)
-  const uintptr_t starts = (uintptr_t)x | (uintptr_t)wd | (uintptr_t)w | (uintptr_t)out | (uintptr_t)out32 | (uintptr_t)shift_w | (uintptr_t)shift_state;
+  // (the row kernel reads and writes everything by whole runs, the kernel through LDS the experts' rows and what is normed alone:
+  // whatever does not start at a whole run is the latter's)
+  const uintptr_t starts = (uintptr_t)x | (uintptr_t)delta | (uintptr_t)y | (uintptr_t)wd | (uintptr_t)w | (uintptr_t)out | (uintptr_t)out32 |
+                           (uintptr_t)shift_w | (uintptr_t)shift_state;
   if (starts % 16 == 0 && delta_stride % 4 == 0) TQ_ROW_KERNELS(H, TQ_BODY);
 #undef TQ_BODY
   const int threads = (H % 4 == 0 && H >= 2048) ? 512 : 256;
