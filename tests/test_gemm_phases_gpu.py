@@ -41,6 +41,20 @@ def test_items_of_four_units(ops):
         assert te[st.numel() // 64:][:items].tolist() == [first[e] + u for e, n in enumerate(of) for u in range(0, n, 4)]
 
 
+@pytest.mark.parametrize("item_units", [2, 4])
+@pytest.mark.parametrize("unit", [1, 2047, 2048, 2112, 4096])
+def test_items_of_any_unit(ops, unit, item_units):
+    """A unit is a number of rows, small or large, whatever its items hold."""
+    counts = [1, 2049, 0, 9000, 4096]
+    st, slot, te, nt = order(ops, counts, unit, item_units)
+    of = [-(-n // unit) for n in counts]
+    first = [sum(of[:e]) for e in range(len(of))]
+    units, items = nt.tolist()
+    assert st.numel() % unit == 0 and units == sum(of) and te[:units].tolist() == [e for e, n in enumerate(of) for _ in range(n)]
+    assert te[st.numel() // unit:][:items].tolist() == [first[e] + u for e, n in enumerate(of) for u in range(0, n, item_units)]
+    assert sorted(slot.flatten().tolist()) == [first[e] * unit + i for e, n in enumerate(counts) for i in range(n)]
+
+
 # k: 2, 3, 4, 5 and 9 steps of 64 (the rings hold 2 to 4 tiles); columns: less than a wave's 32, no multiple of 8, one more than a tile
 @pytest.mark.parametrize("K,N", [(128, 24), (192, 100), (256, 129), (320, 256), (576, 263)])
 @pytest.mark.parametrize("gated", [True, False])

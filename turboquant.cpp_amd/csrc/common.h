@@ -17,8 +17,9 @@
 // added to a tile_rows of 64 of a product over experts: the units that the row order's items hold, two or four of one
 // expert, per workgroup (see tq_gemm_mfma)
 #define TQ_TILE_PAIRS 1024
-// added to the unit of the order of pairs by expert: its items hold four row tiles instead of two (see moe.hip)
-#define TQ_ITEMS_OF_FOUR 2048
+// added to the unit of the order of pairs by expert: its items hold four row tiles instead of two (see moe.hip).  Above every unit:
+// a unit of rows may be any number whose rows fit the order.
+#define TQ_ITEMS_OF_FOUR (1 << 30)
 #define TQ_GEMM_ACT_ALONE 256      // added to tq_gemm_mfma's gate: the activation of a plain product's result
 
 struct bf16_t {

@@ -842,6 +842,7 @@ EXPERT_16_UPTO, EXPERT_32_UPTO = 5, 10
 # time do better wherever the taller units did (see expert_tile_rows); tests lower them to run those kernels.
 EXPERT_128_FROM = EXPERT_256_FROM = 1 << 30
 TILE_PAIRS = 1024            # added to tile_rows 64: the units of an item, two or four of one expert, per workgroup (TQ_TILE_PAIRS)
+ITEMS_OF_FOUR = 1 << 30      # added to the row order's unit: its items hold four row tiles instead of two (TQ_ITEMS_OF_FOUR)
 EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken several at a time
 
 
@@ -1438,9 +1439,9 @@ class RowUnit(int):
 
 
 def _order_unit(k: str, unit: int, item_units: int) -> int:
-    """The ``unit`` that the library is told, with how many row tiles an item holds at most (TQ_ITEMS_OF_FOUR)."""
+    """The ``unit`` that the library is told, with how many row tiles an item holds at most (ITEMS_OF_FOUR)."""
     _need(item_units in (2, 4), k, "an item holds up to 2 or 4 row tiles")
-    return unit + 2048 if item_units == 4 else unit
+    return unit + ITEMS_OF_FOUR if item_units == 4 else unit
 
 
 def moe_align(ids: torch.Tensor, num_experts: int, unit: int, act, item_units: int = 2):
