@@ -40,6 +40,20 @@ def test_products_in_tiles(ops, M, N, K):
     assert ((got - exact).abs() <= (2 * u.abs() * bound + bound ** 2) * (v.abs() + bound2) + u ** 2 * bound2 + 4 * 2.0 ** -24 * exact.abs() + 1e-30).all()
 
 
+@pytest.mark.parametrize("N", [4194240, 4194241, 8388480])
+def test_gated_pairs_of_as_many_columns_as_the_grid_has_room_for(ops, N):
+    """The last width in tiles of 64 columns, the first in tiles of 128 and the last of those: the same bits, column by column."""
+    M, K = 65, 4
+    a, w, w2 = drawn((M, K), 1), drawn((4096, K), 2, 0.2), drawn((4096, K), 3, 0.2)
+    many = [m.repeat(-(-N // 4096), 1)[:N].contiguous() for m in (w, w2)]
+    want = ops.gemm(a, w, "float32", w2=w2)
+    got = ops.gemm(a, many[0], "float32", w2=many[1])
+    whole = N // 4096 * 4096
+    assert (got[:, :whole].view(M, -1, 4096) == want[:, None]).all() and torch.equal(got[:, whole:], want[:, :N - whole])
+    with pytest.raises(Exception, match="not supported"):
+        ops.gemm(a, w.repeat(2049, 1)[:8388481].contiguous(), "float32", w2=w2.repeat(2049, 1)[:8388481].contiguous())
+
+
 @pytest.mark.parametrize("K,N", [(12, 40), (52, 129), (64, 128)])
 @pytest.mark.parametrize("gated", [True, False])
 def test_experts_in_row_tiles(ops, K, N, gated):

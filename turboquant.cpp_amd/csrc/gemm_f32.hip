@@ -510,8 +510,11 @@ TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gath
     else
       hipLaunchKernelGGL((gemm_f32_stream_kernel<1, SNT, false>), grid, dim3(256), 0, st, g, k_per_split, k_per_wave, part);
   } else {
-    // tiles; 17 to 64 rows of one matrix are a single row of tiles, cut into runs of k where the matrix is narrow
-    const int mi = (grouped || M <= 64) ? 1 : 2, columns = mi == 2 && dual ? 64 : 128;
+    // tiles; 17 to 64 rows of one matrix are a single row of tiles, cut into runs of k where the matrix is narrow.  A gated pair of
+    // more rows goes in tiles of 128 rows by 64 columns, as long as the grid's y has room for as many columns of tiles (4,194,240
+    // columns of either matrix), beyond that in tiles of 64 by 128, whose sums run over k alike.
+    const bool tall = !grouped && M > 64 && !(dual && (N + 63) / 64 > 65535);
+    const int mi = tall ? 2 : 1, columns = tall && dual ? 64 : 128;
     const dim3 grid((M + 64 * mi - 1) / (64 * mi), (N + columns - 1) / columns, runs);
     if (grid.y > 65535) return TQ_ERR_UNSUPPORTED;
     if (mi == 1) {
