@@ -196,11 +196,12 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k
   const int steps = (k_last - k_first) / TBK, left = (k_last - k_first) % TBK;
   for (int s = 0; s < TSTAGES - 1 && s < steps; ++s) ask(s);
   for (int t = 0; t < steps; ++t) {
-    // tile t has landed once no more of this wave's loads are on their way than those of the tile behind it
-    if (t + 1 < steps) __builtin_amdgcn_s_waitcnt(0x0F70 | L);
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    // Tile t has landed once no more of this wave's loads are on their way than those of the tile behind it.  And every wave is
+    // through with tile t - 1, whose stage tile t + 2 takes: its reads of it have come back, wherever their products stand.
+    if (t + 1 < steps) __builtin_amdgcn_s_waitcnt(0x0070 | L);
+    else __builtin_amdgcn_s_waitcnt(0x0070);
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();      // and every wave is through with tile t - 1, whose stage tile t + 2 takes
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (t + TSTAGES - 1 < steps) ask(t + TSTAGES - 1);
     multiply(ring + t % TSTAGES * STAGE);

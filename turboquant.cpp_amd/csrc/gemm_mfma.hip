@@ -743,11 +743,12 @@ __global__ __launch_bounds__(128 * WN) void gemm_few_tiles_kernel(MfmaGemmArgs g
   const int lr = lane % 32, lc = lane / 32;
   int cur = 0;
   for (int t = 0; t < steps; ++t) {
-    // tile t is in LDS once no more loads of this wave are on their way than those of the tiles behind it
+    // tile t is in LDS once no more loads of this wave are on their way than those of the tiles behind it, and its reads of tile
+    // t - 1 have come back, wherever their products stand
     if (steps - 1 - t >= S - 2)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (S - 2) * L);
+      __builtin_amdgcn_s_waitcnt(0x0070 | (S - 2) * L);
     else
-      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __builtin_amdgcn_s_waitcnt(0x0070);
     // every wave's share of tile t has landed and every wave is through with tile t - 1, whose stage tile t + S - 1 takes
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
