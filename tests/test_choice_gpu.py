@@ -96,3 +96,22 @@ def test_logits_that_are_no_numbers(ops, E):
             one = ops.route(x[t:t + 1].contiguous(), router, None, topk, renorm, 16, "float32")
             assert torch.equal(one[0], ids[t:t + 1]) and torch.equal(one[1].isnan(), weights[t:t + 1].isnan())
             assert ((one[4] >= 0) & (one[4] < one[3].numel())).all()
+
+
+@pytest.mark.parametrize("E", [8, 60, 64, 80, 128, 132])
+def test_corrections_that_are_no_numbers(ops, E):
+    """Experts whose correction is NaN are not chosen; where all are, it is the first one, with its own score as its weight."""
+    H, topk = 64, 3
+    x, router = drawn((20, H), 1), drawn((E, H), 2, 0.3)
+    score = torch.softmax(x.double() @ router.double().T, -1)
+    for real in ([], [1], [0, E - 2, E - 1, 2]):
+        correction = torch.full((E,), torch.nan, device=DEV)
+        correction[real] = 0.0
+        ids, weights, *_ = ops.route(x, router, None, topk, False, 16, "float32", correction=correction)
+        if not real:
+            assert (ids == 0).all()
+        assert torch.isin(ids[:, :len(real)], torch.tensor(real or [0], dtype=torch.int32, device=DEV)).all()
+        assert (weights.double() - score.gather(1, ids.long()))[:, :max(len(real), 1)].abs().max() < 1e-6
+        for t in (0, 7):
+            one = ops.route(x[t:t + 1].contiguous(), router, None, topk, False, 16, "float32", correction=correction)
+            assert torch.equal(one[0], ids[t:t + 1]) and torch.equal(one[1], weights[t:t + 1])

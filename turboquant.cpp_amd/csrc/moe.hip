@@ -218,8 +218,8 @@ __device__ __forceinline__ int select_small(const float (&logit)[NL], int E, int
   int sel_id = -1;
   for (int k = 0; k < topk; ++k) {
     const float best = largest();
-    int bi = 0;
-    float raw = 0.f;
+    int bi = 0;      // (none: only if every score is NaN, through its correction)
+    float raw = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(logit[0])));
 #pragma unroll
     for (int u = 0; u < NL; ++u) {      // (the later, the higher the index)
       const unsigned long long at = __ballot(mine[u] && v[u] == best);
