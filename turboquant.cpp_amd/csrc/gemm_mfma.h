@@ -74,7 +74,6 @@ __device__ __forceinline__ void load_to_lds16(const bf16_t* src, bf16_t* wave_ba
                                    (__attribute__((address_space(3))) void*)wave_base, 16, 0, 0);
 }
 
-// gemm_phases.hip: products of many rows (K a multiple of TBK), of one matrix or of a matrix per expert by the row order's items;
-// g2 (or null): another of one matrix, in the same launch; k of one matrix may be in runs of k_per.  height: units of 64 rows of a tile
-// of one matrix (1 .. 4)
-int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual, bool out_act, hipStream_t st, int height = 4);
+// gemm_phases.hip: products of many rows (K a multiple of TBK, 2 TBK and more) with a matrix per expert, by the row order's items; g2 (or
+// null): another of one matrix in the same launch, whose k may be in runs of k_per
+int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual, bool out_act, hipStream_t st);

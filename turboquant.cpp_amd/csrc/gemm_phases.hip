@@ -2,10 +2,10 @@
 // multiplies, the other reads its operands from LDS and asks for what comes later, and a barrier between the two phases
 // lets them change places.  Same contract, operand layouts and order of sums as the tile kernel in gemm_mfma.hip: same bits.
 //
-// What bounds it: a tile of 64 of k is 64 KB on its way through L2 and 8.4 million multiply-adds, 0.85 us of the matrix
+// What bounds it: a tile of 64 of k is 64 KB on its way through L2 and 4.2 million multiply-adds, 0.85 us of the matrix
 // instructions of a compute unit at their full clock and about as long as its path to L2 takes for the bytes, so each has to go on
 // beside the other:
-//  * a wave owns 32 MI x 64 outputs (MI up to 4), for which its reads from LDS (8 MI + 16 operand reads a tile of 64) take less time
+//  * a wave owns 32 MI x 64 outputs (MI up to 4), for which its reads from LDS (4 MI + 8 operand reads a tile of 64) take less time
 //    than its products, and the group that multiplies has the matrix instructions to itself;
 //  * loads go straight into LDS and are asked for by the reading group alone, behind its reads.  A wave that asks for more than the
 //    path takes stands still until there is room, and in front of products or reads that time is lost: 13,197 tokens by 8 of 64
@@ -17,8 +17,7 @@
 // LDS into stores of 16 bytes a lane, whole lines side by side (a test and a store of a value each took 16 us a tile).
 // Measured, us, against items of two units by 16 waves through a ring of three stages: 64 experts of 2,560 x 3,584 with 1,650 rows
 // each, gated pair 4,760 -> 3,739 (1,036 TFLOP/s), second product 2,590 -> 1,943; 60 experts of 1,408 x 2,048 with 137 rows each
-// 219 -> 173 and 147 -> 103, with 68 rows 149 -> 147 and 96 -> 90.  On operands that are zeros (less power) 8,192 x 8,192 x 8,192
-// takes 638 instead of 880.
+// 219 -> 173 and 147 -> 103, with 68 rows 149 -> 147 and 96 -> 90.
 #include "common.h"
 
 #include "gemm_mfma.h"
@@ -310,11 +309,11 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
   }
 }
 
-// Tile `logical` of a product in the order in which a die goes through its run of them.  One matrix: bands of 8 row tiles, down a
-// band's columns (a run of k behind the other).  A matrix per expert: expert by expert, so that an expert's matrices are read by one
-// die, and within an expert column by column with its items side by side.
+// Tile `logical` of a product in the order in which a die goes through its run of them.  A matrix per expert (the first product): expert
+// by expert, so that an expert's matrices are read by one die, and within an expert column by column with its items side by side.
+// One matrix (the second): tiles of 256 rows in bands of 8, down a band's columns, a run of k behind the other.
 template <bool DUAL>
-__device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int gx, int gy, int height, PhaseTile& p) {
+__device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int gx, int gy, PhaseTile& p) {
   const int lane = threadIdx.x % 64;
   int tile_n, group = 0;
   if (g.tile_group) {
@@ -355,8 +354,8 @@ __device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int 
     }
     const int band = logical / (8 * gy), in_band = logical % (8 * gy), bh = min(8, gx - band * 8);
     tile_n = in_band / bh;
-    p.m0 = (band * 8 + in_band % bh) * 64 * height;
-    p.units = min((g.M - p.m0 + 63) / 64, height);
+    p.m0 = (band * 8 + in_band % bh) * 256;
+    p.units = min((g.M - p.m0 + 63) / 64, 4);
   }
   p.w = g.w + (size_t)group * g.group_stride;
   p.w2 = DUAL ? g.w2 + (size_t)group * g.group_stride : p.w;
@@ -364,9 +363,9 @@ __device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int 
   p.n1 = DUAL ? p.n0 : p.n0 + 128;
 }
 template <bool DUAL, bool OUT_ACT>
-__device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int gy, int height, bf16_t* lds) {
+__device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int gy, bf16_t* lds) {
   PhaseTile p;
-  phase_tile_of<DUAL>(g, logical, gx, gy, height, p);
+  phase_tile_of<DUAL>(g, logical, gx, gy, p);
   switch (__builtin_amdgcn_readfirstlane(p.units)) {
     case 4: phases_tile<4, DUAL, OUT_ACT>(g, p, lds); break;
     case 3: phases_tile<3, DUAL, OUT_ACT>(g, p, lds); break;
@@ -378,12 +377,11 @@ __device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int
 // A die (workgroups are dealt to the 8 of them in turn) gets a contiguous run of the tiles of the first product and one of the
 // second, if there is one (n2 tiles, gx2 x gy2 a run of k): `first2`: the second's before the first's, else spread among them.
 template <bool DUAL, bool OUT_ACT>
-__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gx, int gy, int height, int runs, MfmaGemmArgs g2, int gx2,
-                                                          int gy2, int n2, int first2) {
+__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gy, MfmaGemmArgs g2, int gx2, int gy2, int n2, int first2) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  if (g.tile_group) gx = min(g.n_tiles[1], g.M / 64);
+  int gx = min(g.n_tiles[1], g.M / 64);
   const int id = blockIdx.x, die = id % 8, i = id / 8;
-  const int n1 = gx * gy * runs;
+  const int n1 = gx * gy;
   const int q1 = n1 / 8, rem1 = n1 % 8, mine1 = q1 + (die < rem1 ? 1 : 0);
   const int q2 = n2 / 8, rem2 = n2 % 8, mine2 = q2 + (die < rem2 ? 1 : 0);
   if (i >= mine1 + mine2) return;
@@ -401,32 +399,30 @@ __global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gx
     g = g2;
     gx = gx2;
     gy = gy2;
-    height = 4;
   }
-  phases<DUAL, OUT_ACT>(g, logical, gx, gy, height, (bf16_t*)smem);
+  phases<DUAL, OUT_ACT>(g, logical, gx, gy, (bf16_t*)smem);
 }
 
 // g2 (null: none): a second product, of one matrix and of the same kind, whose tiles fill the chip beside the first's; its k may be
 // in runs (k_per, split_stride).
-int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual, bool out_act, hipStream_t st, int height) {
+int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual, bool out_act, hipStream_t st) {
+  if (!g.tile_group || !g.n_tiles) return TQ_ERR_BAD_ARG;
   const int cols = dual ? 128 : 256;
-  // (units of 64 rows, at most so many items, or tiles of `height` units of one matrix)
-  const int gx = g.tile_group ? g.M / 64 : (g.M + 64 * height - 1) / (64 * height), gy = (g.N + cols - 1) / cols;
-  const int runs = g.tile_group ? 1 : (g.K + g.k_per - 1) / g.k_per;
+  const int gx = g.M / 64, gy = (g.N + cols - 1) / cols;      // (units of 64 rows: at most so many items)
   int gx2 = 1, gy2 = 1, n2 = 0, first2 = 0;
   if (g2) {
     gx2 = (g2->M + 255) / 256, gy2 = (g2->N + cols - 1) / cols;
     n2 = gx2 * gy2 * ((g2->K + g2->k_per - 1) / g2->k_per);
     first2 = g2->k_per >= 3 * g.K / 2;      // tiles that take longer start first
   }
-  const int64_t per_die = ((int64_t)gx * gy * runs + 7) / 8 + (n2 + 7) / 8;
+  const int64_t per_die = ((int64_t)gx * gy + 7) / 8 + (n2 + 7) / 8;
   if (per_die * 8 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
   const int shmem = 160 * 1024;      // MI = 2 and 4; 144 KB where MI is 1 or 3
 #define TQ_PHASES(D, O)                                                                                                       \
   do {                                                                                                                        \
     if (hipFuncSetAttribute((const void*)gemm_phases_kernel<D, O>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem) != hipSuccess) \
       return TQ_ERR_UNSUPPORTED;                                                                                              \
-    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), dim3((unsigned)(per_die * 8)), dim3(512), shmem, st, g, gx, gy, height, runs, g2 ? *g2 : g, gx2, gy2, n2, first2); \
+    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), dim3((unsigned)(per_die * 8)), dim3(512), shmem, st, g, gy, g2 ? *g2 : g, gx2, gy2, n2, first2); \
   } while (0)
   if (dual && out_act) TQ_PHASES(true, true);
   else if (dual) TQ_PHASES(true, false);
