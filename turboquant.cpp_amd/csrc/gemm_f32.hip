@@ -8,7 +8,8 @@
 //
 //  * gemm_f32_tile_kernel, for more than 16 rows: tiles of 64 or 128 rows by 128 columns (64 of a gated pair of 128 rows) by four
 //    waves, 16 of k at a time.  What bounds it is the matrix instructions (64 clocks each), so what counts is that a SIMD always
-//    has a wave with products to do: 64 sums a wave and no more, so that three workgroups share a compute unit, and tiles that go
+//    has a wave with products to do: 64 sums a wave and no more, so that three workgroups share a compute unit (two of an
+//    expert's gated pair, and of one of up to 64 rows, whose stages hold 64 rows and 128 of either matrix: 60 KB a ring), and tiles that go
 //    straight from memory into a ring of three LDS stages, two on their way, with one bare barrier a tile and no branch around a
 //    load (with tiles through registers and loads behind predicates a gated pair of 128 x 128 had one wave to a SIMD).
 //    16,385 rows, ms, before and now: by 6,144 x 2,048 3.46 and 3.20 (129 TFLOP/s; the instructions alone give 153), by 2,048 x 5,632 3.48

@@ -694,7 +694,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(MfmaGemmArgs g)
 // takes 0.8 us a step here (load, wait, store into LDS, barrier, and every product behind its own reads), for 64 x 128
 // outputs, so that 97 rows by 6,144 x 2,048 kept 96 compute units busy for 26 us.  Here the tiles are smaller where
 // that fills the chip, go from memory straight into a ring of S stages of LDS, S - 1 of them on their way while one is
-// multiplied (as in the ring kernel above): 15.0 us, 0.4 us a step.  Two tiles of 64 to a step: 15.9.  The compiler puts a
+// multiplied (global_load_lds_dwordx4: no registers in between; a load instruction of a wave fills eight rows of 128 bytes, lane l
+// the l-th chunk of 16, so the swizzle is in what a lane asks for): 15.0 us, 0.4 us a step.  Two tiles of 64 to a step: 15.9.  The compiler puts a
 // step's products between its reads of LDS; all reads before the first product, held there by a scheduling barrier, is
 // level (14.8; a gated pair of 97 rows by twice 5,632 x 2,048 23.6 and 23.6, by twice 20,480 x 3,584 85.9 and 85.2, of
 // 512 rows by that 229 and 240, of 320 161 and 159).  The sums of an output run over k as in the tile kernel: same bits.
@@ -799,7 +800,6 @@ static int split_k_waves(int N, int K, bool grouped) {
   return s;
 }
 
-// MT row tiles of 16; more than one (17 to 64 rows of one matrix) go with two column tiles per wave.
 // Whether lean_body takes a product of at most 16 rows a tile.
 static bool lean_suits(const MfmaGemmArgs& g) {
   return g.K % 64 == 0 && g.N % 16 == 0 && g.K < (1 << 26) && g.k_per % 64 == 0 &&
@@ -807,8 +807,9 @@ static bool lean_suits(const MfmaGemmArgs& g) {
 }
 // A workgroup's columns there.  Tiles of 8 leave fewer compute units without work (one row by 2,048 x 5,632: 6.9 us against 8.5 in
 // tiles of 16, 2,048 x 8,448 8.7 against 11.7, a gated pair of 5,632 x 2,048 10.4 against 12.4; experts' pairs 10.6 against 11.8,
-// 151,936 x 2,048 106 against 110) but read `a` twice as often: tiles of 16 where they give every compute unit a full workgroup
-// (8 rows by 4,096 x 4,096: 9.3 against 10.3) and for more than 8 rows of many columns (32,000 x 2,048: 24.2 against 26.2).
+// 151,936 x 2,048 106 against 110) but read `a` twice as often: tiles of 16 where there are 192 to 256 of them with eight waves each,
+// one to nearly every compute unit (8 rows by 4,096 x 4,096: 9.3 against 10.3), and for more than 8 rows of plain products with more
+// columns than that (32,000 x 2,048: 24.2 against 26.2).
 static int lean_columns(const MfmaGemmArgs& g, int nw, bool dual) {
   const int tiles = g.N / 16;
   if (tiles < 192) return 8;
@@ -816,6 +817,7 @@ static int lean_columns(const MfmaGemmArgs& g, int nw, bool dual) {
   return dual || g.tile_group || g.M <= 8 ? 8 : 16;
 }
 
+// MT row tiles of 16; more than one (17 to 64 rows of one matrix) go with two column tiles per wave.
 template <int MT>
 static int launch_stream(MfmaGemmArgs g, bool dual, bool out_act, int row_tiles, hipStream_t st, int splits = 1) {
   constexpr int NTL = MT > 1 ? 2 : 1;
@@ -1126,14 +1128,17 @@ TQ_API int tq_gemm_mfma_pair_splits(int N1, int K1, int grouped1, int N2, int K2
   return (K2 + k_per - 1) / k_per;
 }
 
-// Two products of few rows in one launch.  d1, d2: 20 numbers each, in the order of tq_gemm_mfma's arguments from `a`
-// to `tile_rows`, then the gate's activation and the bits of the gated pair's limit as a float (0: none).  Both must
-// be products that the streaming kernel takes 16 rows at a time (a matrix per expert with tile_rows 16, or one matrix
-// with M <= 16), both gated or both not, both into the same type.  The waves that split k are those of the first
-// product (the larger one by convention).  splits2 > 1 (as tq_gemm_mfma_pair_splits says, for a plain second product
-// into float): run z of its k goes to out + z * M * ldc, the bias to run 0.
 TQ_API int tq_gemm_phases_pair_splits(int M1, int N1, int K1, int M2, int N2, int K2);
 
+// Two products in one launch.  d1, d2: 20 numbers each, in the order of tq_gemm_mfma's arguments from `a`
+// to `tile_rows`, then the gate's activation and the bits of the gated pair's limit as a float (0: none); both gated or
+// both not, both into the same type.  Either
+//  * few rows: both products that the streaming kernel takes 16 rows at a time (a matrix per expert with tile_rows 16, or
+//    one matrix with M <= 16).  The waves that split k are those of the first product (the larger one by convention);
+//  * or many, where tile_rows of the first is 64 + TQ_TILE_PAIRS: the first over experts by the row order's items, the second
+//    of one matrix whose rows follow one another, k of either a multiple of 64 and 128 and more (gemm_phases.hip).
+// splits2 > 1 (as tq_gemm_mfma_pair_splits says of few rows and tq_gemm_phases_pair_splits of many, for a plain second
+// product into float): run z of its k goes to out + z * M * ldc, the bias to run 0.
 TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, hipStream_t st) {
   MfmaGemmArgs g[2];
   int row_tiles[2];

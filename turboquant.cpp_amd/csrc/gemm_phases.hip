@@ -413,7 +413,12 @@ int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual,
   if (g2) {
     gx2 = (g2->M + 255) / 256, gy2 = (g2->N + cols - 1) / cols;
     n2 = gx2 * gy2 * ((g2->K + g2->k_per - 1) / g2->k_per);
-    first2 = g2->k_per >= 3 * g.K / 2;      // tiles that take longer start first
+    // Tiles that take longer start first.  60 experts of 2,048 x 1,408, us with the second's tiles first and spread among the first's:
+    // 2,048 rows beside runs of 2,816 of k 143 and 164, beside 1,024 x 2,048 of 2,048 107 and 126, 13,197 rows of 5,632 613 and 706.
+    // Tiles of about the same time gain less: 2,048 rows of k 1,920 131 and 144, of 1,408 136 and 139, of 704 130 and 130; 1,100 rows
+    // in runs of 1,408 120 and 131; 6,000 rows of 1,408 to 2,112 level (and vary by 4 %); gated pairs beside 1,408 columns 195 and 204,
+    // beside 5,632 261 and 266.  No side where spreading wins was found: the line is no border between two, only where the gain is sure.
+    first2 = g2->k_per >= 3 * g.K / 2;
   }
   const int64_t per_die = ((int64_t)gx * gy + 7) / 8 + (n2 + 7) / 8;
   if (per_die * 8 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;

@@ -142,7 +142,7 @@ int product(Ctx& c, const Product& p, void** out, int* splits, int side = 0) {
   const bool grouped = p.tile_group != nullptr;
   const size_t esz = p.out_act ? TQ_ACT_BYTES : 4;
   const int tile_rows = p.tile_rows ? p.tile_rows : (p.M <= 32 ? 16 : 64);
-  const int unit_rows = tile_rows % TQ_TILE_PAIRS;      // pairs of units are the matrix-core product's alone
+  const int unit_rows = tile_rows % TQ_TILE_PAIRS;      // items of several units are the matrix-core product's alone
   *splits = 1;
   auto result = [&](size_t bytes) { return p.dest ? p.dest : c.arena.take(bytes); };
   if (!grouped && !p.a_rows && !p.bias.ptr && vendor_product(c, p)) {
@@ -212,13 +212,13 @@ void pair_desc(const Product& p, void* out, int tile_rows, int64_t* d) {
 }
 #endif
 
-// Two products that do not depend on each other; mirrors ops.gemm_pair (only the second may leave partial sums).
 // Whether a product over experts by items of several units and one of one matrix go out together (mirrors ops.gemm_pair).
 bool tiles_together(const Product& p1, const Product& p2) {
   auto suits = [](const Product& p) { return use_mfma(p.w, p.K) && p.K % 64 == 0 && p.K >= 128; };
   return p1.tile_group && p1.tile_rows == 64 + TQ_TILE_PAIRS && !p2.tile_group && !p2.a_rows && p2.M >= 64 && suits(p1) && suits(p2);
 }
 
+// Two products that do not depend on each other; mirrors ops.gemm_pair (only the second may leave partial sums).
 int product_pair(Ctx& c, const Product& p1, const Product& p2, void** out1, void** out2, int* splits2) {
   *splits2 = 1;
 #if defined(TQ_ACT_BF16)

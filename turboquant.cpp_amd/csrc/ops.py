@@ -900,7 +900,7 @@ def _gemm_problem(k: str, a, w, act, bias, w2, out_act, a_rows, tile_group, n_ti
               "grouped product needs a_rows, n_tiles and tile_rows of 16, 64, 128 or 256")
         if not _use_mfma(act, a, w, a.shape[1]):
             _need(tile_rows % TILE_PAIRS in (16, 64), k, "tiles of 32, 128 and 256 rows are for the bfloat16 matrix-core product")
-            tile_rows %= TILE_PAIRS      # pairs of units are that product's too: the others take unit by unit
+            tile_rows %= TILE_PAIRS      # items of several units are that product's too: the others take unit by unit
         _check(a_rows, k, "a_rows", torch.int32)
         _check(tile_group, k, "tile_group", torch.int32)
         _check(n_tiles, k, "n_tiles", torch.int32)

@@ -14,7 +14,8 @@
 
 #define TQ_ERR_BAD_ARG (-1)
 #define TQ_ERR_UNSUPPORTED (-2)
-// added to a tile_rows of 64 of a product over experts: two units of one expert per workgroup (see tq_gemm_mfma)
+// added to a tile_rows of 64 of a product over experts: the units that the row order's items hold, two or four of one
+// expert, per workgroup (see tq_gemm_mfma)
 #define TQ_TILE_PAIRS 1024
 #define TQ_ITEMS_OF_FOUR (1 << 30)      /* added to the unit of the order of pairs by expert: its items hold four row tiles, not two */
 #define TQ_GEMM_ACT_ALONE 256      // added to tq_gemm_mfma's gate: the activation of a plain product's result
