@@ -98,6 +98,27 @@ def test_logits_that_are_no_numbers(ops, E):
             assert ((one[4] >= 0) & (one[4] < one[3].numel())).all()
 
 
+@pytest.mark.parametrize("E", [8, 60, 80, 132])
+@pytest.mark.parametrize("renorm", [False, True])
+def test_logits_that_are_infinite(ops, E, renorm):
+    """Infinities without a NaN among them: the search by the rule, the highest index first among equals, a chosen expert then the least."""
+    H, topk = 64, 3
+    x, router = drawn((20, H), 1), drawn((E, H), 2, 0.3)
+    router[:, 0], router[1, 0] = -router[:, 0].abs(), 0.5      # one expert at +infinity and the others at -infinity, or the other way about
+    x[3, 0], x[7, 0], x[11, 5] = torch.inf, -torch.inf, torch.inf
+    ids, weights, *_ = ops.route(x, router, None, topk, renorm, 16, "float32")
+    z = (x.double() @ router.double().T).cpu()
+    for t in (3, 7, 11):
+        v, want = z[t].clone(), []
+        assert v.isinf().all()
+        for _ in range(topk):
+            want.append(max(range(E), key=lambda e: (v[e].item(), e)))
+            v[want[-1]] = -torch.inf
+        one = ops.route(x[t:t + 1].contiguous(), router, None, topk, renorm, 16, "float32")
+        assert ids[t].tolist() == want and one[0][0].tolist() == want and torch.equal(one[1].isnan(), weights[t:t + 1].isnan())
+        assert ((one[4] >= 0) & (one[4] < one[3].numel())).all()
+
+
 @pytest.mark.parametrize("E", [8, 60, 64, 80, 128, 132])
 def test_corrections_that_are_no_numbers(ops, E):
     """Experts whose correction is NaN are not chosen; where all are, it is the first one, with its own score as its weight."""

@@ -89,7 +89,7 @@ def test_the_executor_at_the_layer_sizes_of_a_real_checkpoint(act, monkeypatch):
     eager and replayed.  A step of 900 tokens hands its plain bfloat16 products to the vendor's library; the executor
     calls that library itself where the parts go through torch, and the two may be served by different kernels of it:
     there both are compared with each other at the bound of a bfloat16 product, and with every product in this
-    library's kernels the bits agree again, also between the experts' units taken two at a time and one by one."""
+    library's kernels the bits agree again, also between the experts' units taken up to four at a time and one by one."""
     from turboquant_cpp_amd.csrc import ops
     from turboquant_cpp_amd.engine.model import random_model
     from turboquant_cpp_amd.engine.step import Engine
@@ -143,7 +143,7 @@ def test_the_executor_at_the_layer_sizes_of_a_real_checkpoint(act, monkeypatch):
             assert torch.equal(own[0], own[1])
             scale = own[0].abs().max().item()
             assert (own[0] - a[n]).abs().max().item() < 0.04 * scale
-        # 1,100 tokens are 73 rows per expert: units of 64 two at a time; one by one they give the same bits
+        # 1,100 tokens are 73 rows per expert: units of 64 up to four at a time; one by one they give the same bits
         monkeypatch.setattr(ops, "EXPERT_PAIRS_FROM", 1 << 30)
         for eng in engines:
             slot = eng.open(1)

@@ -55,6 +55,29 @@ def test_items_of_any_unit(ops, unit, item_units):
     assert sorted(slot.flatten().tolist()) == [first[e] * unit + i for e, n in enumerate(counts) for i in range(n)]
 
 
+@pytest.mark.parametrize("form", [{}, {"shared_size": 128}, {"sigmoid_scores": True, "renormalize": True}, {"score_correction": True, "identity": 2},
+                                  {"gated": False}, {"expert_size": 72}])
+def test_the_feed_forward_asks_for_items_of_four(ops, monkeypatch, form):
+    """Every kind of routed experts with 48 rows each and more has its row order list items of up to four units (an order with items of two
+    gives the same results more slowly), and with fewer of two."""
+    from types import SimpleNamespace
+    from turboquant_cpp_amd.parts.ffn import SparseMoE
+    form = dict({"expert_size": 128}, **form)
+    part = SparseMoE(128, 5, 2, **form)
+    for i, (name, spec) in enumerate(part.param_specs().items()):
+        setattr(part, name, drawn(spec.shape, i, 0.1))
+    part.prepare(DEV, "bfloat16")
+    seen, route = [], ops.route
+    monkeypatch.setattr(ops, "route", lambda *a, **k: seen.append(route(*a, **k)) or seen[-1])
+    for T, per in ((601, 4), (100, 2)):
+        x = drawn((T, 128), 50)
+        part.forward(x, x.float(), SimpleNamespace(act="bfloat16"))
+        ids, _w, _g, st, _slot, _te, nt = seen.pop()
+        of = [-(-int((ids == e).sum()) // 64) for e in range(5)]
+        assert nt.tolist() == [sum(of), sum(-(-n // per) for n in of)]
+        assert per == 2 or max(of) > 2
+
+
 # k: 2, 3, 4, 5 and 9 steps of 64 (the rings hold 2 to 4 tiles); columns: less than a wave's 32, no multiple of 8, one more than a tile
 @pytest.mark.parametrize("K,N", [(128, 24), (192, 100), (256, 129), (320, 256), (576, 263)])
 @pytest.mark.parametrize("gated", [True, False])
@@ -64,8 +87,9 @@ def test_products_by_items_of_four(ops, K, N, gated):
     x, w = drawn((T, K), 1), drawn((E, N, K), 2, 0.1)
     w2 = drawn((E, N, K), 3, 0.1) if gated else None
     live = st >= 0
-    forms = [dict(w2=w2, out_act=True, activation=a, **more) for a in ("silu", "gelu_tanh") for more in ({}, {"pair_limit": 0.5})] if gated \
-        else [dict(out_act=True), dict(), dict(out_act=True, activation="gelu", act_alone=True)]
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(4)).to(DEV)
+    forms = [dict(w2=w2, out_act=True, activation=a, **more) for a in ("silu", "gelu_tanh") for more in ({}, {"pair_limit": 0.5}, {"bias": bias})] if gated \
+        else [dict(out_act=True), dict(), dict(out_act=True, activation="gelu", act_alone=True), dict(bias=bias), dict(out_act=True, bias=bias.bfloat16())]
     for form in forms:
         got, want = (ops.gemm(x, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=rows, **form)
                      for rows in (64 + ops.TILE_PAIRS, 64))
@@ -80,14 +104,26 @@ def test_products_by_items_of_four(ops, K, N, gated):
             assert ((got[rows] - a @ b.T).abs() <= K * 2.0 ** -24 * (a.abs() @ b.abs().T)).all()
 
 
-def test_rows_in_place_and_a_wider_result(ops):
-    """The second product reads row m for row m, and rows of padding are not written."""
-    K, N = 192, 200
+# a result whose rows stand further apart than it is wide: by whole runs of 16 bytes, and not
+@pytest.mark.parametrize("N,ldc", [(200, 208), (200, 203), (263, 264), (256, 512)])
+@pytest.mark.parametrize("out_act", [True, False])
+def test_rows_in_place_and_a_wider_result(ops, N, ldc, out_act):
+    """The second product reads row m for row m.  What padding holds does not matter, and neither its rows nor what lies beside a row
+    of the result are written."""
+    K, act = 192, "bfloat16"
     st, _slot, te, nt = order(ops, COUNTS)
+    live = st >= 0
     h, w = drawn((st.numel(), K), 4), drawn((len(COUNTS), N, K), 5, 0.1)
-    got, want = (ops.gemm(h, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=rows, gather=False)
-                 for rows in (64 + ops.TILE_PAIRS, 64))
-    assert torch.equal(got[st >= 0], want[st >= 0])
+    h[~live] = float("nan")
+    lib, outs = ops.library(act), []
+    for rows in (64 + ops.TILE_PAIRS, 64):
+        out = torch.full((st.numel(), ldc), 7.5, dtype=torch.bfloat16 if out_act else torch.float32, device=DEV)
+        assert lib.tq_gemm_mfma(h.data_ptr(), K, st.data_ptr(), 0, w.data_ptr(), None, N * K, te.data_ptr(), nt.data_ptr(), None, 0,
+                                out.data_ptr(), ldc, int(out_act), st.numel(), N, K, rows, 1, 0, torch.cuda.current_stream().cuda_stream) == 0
+        outs.append(out)
+    got, want = outs
+    assert torch.equal(got, want) and got[live].isfinite().all()
+    assert (got[~live] == 7.5).all() and (got[:, N:] == 7.5).all()
 
 
 # the second product: fewer rows than a tile, more than one row of tiles; k in one run and (5,632 beside 192) in several, the last shorter
@@ -95,7 +131,7 @@ def test_rows_in_place_and_a_wider_result(ops):
 @pytest.mark.parametrize("gated", [True, False])
 def test_a_product_beside_the_experts(ops, T, K, N, K2, N2, gated):
     """Both products of gemm_pair in one launch: the experts' rows bit for bit as alone, the other's as unit by unit in one run of k, and
-    its partial sums in as many runs as it says, each within the rounding of its sum."""
+    its partial sums in as many runs as it says, each within the rounding of its sum and of the bias added to the first."""
     st, _slot, te, nt = order(ops, COUNTS)
     x, w = drawn((sum(COUNTS), K), 1), drawn((len(COUNTS), N, K), 2, 0.1)
     a, b = drawn((T, K2), 6), drawn((N2, K2), 7, 0.1)
@@ -105,7 +141,8 @@ def test_a_product_beside_the_experts(ops, T, K, N, K2, N2, gated):
         first.update(w2=drawn(w.shape, 3, 0.1), out_act=True, activation="silu", pair_limit=0.7)
         second.update(w2=drawn(b.shape, 8, 0.1), out_act=True, activation="gelu_tanh")
     else:
-        second.update(partial_sums=True)
+        bias = torch.randn(N2, generator=torch.Generator().manual_seed(9)).to(DEV)
+        second.update(partial_sums=True, bias=bias)
     y1, y2 = ops.gemm_pair(dict(first), dict(second), "bfloat16")
     want = ops.gemm(first.pop("a"), first.pop("w"), "bfloat16", **first)
     assert torch.equal(y1[st >= 0], want[st >= 0])
@@ -118,4 +155,5 @@ def test_a_product_beside_the_experts(ops, T, K, N, K2, N2, gated):
         per = -(-(K2 // 64) // runs) * 64
         for z in range(runs):
             az, bz = a[:, z * per:(z + 1) * per].double(), b[:, z * per:(z + 1) * per].double()
-            assert ((y2[z].double() - az @ bz.T).abs() <= K2 * 2.0 ** -24 * (az.abs() @ bz.abs().T)).all()
+            exact = az @ bz.T + (bias.double() if z == 0 else 0.0)      # the bias goes with the first run alone
+            assert ((y2[z].double() - exact).abs() <= K2 * 2.0 ** -24 * (az.abs() @ bz.abs().T) + 2.0 ** -23 * exact.abs()).all()

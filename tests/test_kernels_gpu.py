@@ -478,7 +478,7 @@ def test_gemm_rows_do_not_depend_on_the_batch(ops, act):
 
 def test_the_height_of_expert_tiles(ops, monkeypatch):
     """16 up to 5 pairs per expert and 32 up to 10 where the bfloat16 matrix-core product runs (else 16 up to 12), 64
-    beyond, which the products take two at a time from 48 rows per expert on; 128 and 256 only where their borders
+    beyond, which the products take up to four at a time from 48 rows per expert on; 128 and 256 only where their borders
     are lowered, and only for the bfloat16 matrix-core product."""
     a16, w16 = torch.zeros((1, 64), dtype=torch.bfloat16), torch.zeros((1, 8, 64), dtype=torch.bfloat16)
     a32, w32 = a16.float(), w16.float()

@@ -327,7 +327,7 @@ def test_the_configurations_whose_bfloat16_logits_lay_furthest_off(run, case, tm
 
 # ------------------------------------------------------------------------------------------------ a long prompt's experts
 def test_a_long_prompt_takes_the_taller_expert_tiles(sharp, monkeypatch):
-    """Where the borders of the taller units are lowered (by default units of 64 stay, taken two at a time), the bfloat16
+    """Where the borders of the taller units are lowered (by default units of 64 stay, taken up to four at a time), the bfloat16
     products over experts take tiles of 128 rows from 256 rows per expert on: a prompt of 1,400 tokens
     with one expert of five per token goes that way through the engine (and one of 700 does not), and every
     position agrees with the plain model.  With the second border at 256 rows too the row order's unit is 256."""
