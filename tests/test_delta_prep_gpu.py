@@ -6,8 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-# sequences of the step: shorter than the taps, one token to each side of a run of eight and of a step of 128
-LENGTHS = [1, 2, 3, 4, 7, 8, 9, 1, 1, 127, 16, 100]
+# sequences of the step: shorter than the taps, one token to each side of a run of eight and of a step of 128; in all tokens enough for
+# runs with the fewest heads, and none of them alone
+LENGTHS = [1, 2, 3, 4, 7, 8, 9, 1, 1, 127, 16, 100] * 8
 
 
 @pytest.mark.parametrize("act", ["float32", "bfloat16"])

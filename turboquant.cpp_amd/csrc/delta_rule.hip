@@ -188,11 +188,14 @@ __global__ __launch_bounds__(256) void delta_prep_runs_kernel(const float* __res
 #undef TQ_PREP_AT
   }
 }
-// From so many tokens on: below, a wave's eight tokens in turn take longer than a wave to each (16 heads of 128, us by a token to a wave
-// and by runs: 64 tokens 5.0 and 7.5, 128 6.9 and 7.8, 192 9.6 and 9.2, 256 12.8 and 9.4, 512 22.9 and 15.5).
+// From so many waves' worth of work on (a token of a unit each): with less, the chip is not full and a wave's eight tokens in turn take
+// longer than a wave to each.  By a token to a wave and by runs, us, tokens of one sequence and of sequences of one token (whose inputs
+// come from the states): 2 heads of 128 (7 units) 256 tokens 4.7 4.6 and 8.8 9.0, 1,500 tokens (10,500) 11.3 11.6 and 10.8 12.0, 4,000
+// 25.2 25.1 and 14.2 17.3; 8 heads of 64 x 256 (13 units) 700 tokens (9,100) 13.1 13.9 and 11.6 14.0; 16 heads of 128 (49 units) 192
+// tokens (9,408) 10.0 11.0 and 10.8 11.4, 256 (12,544) 13.0 13.6 and 11.1 12.4, 700 30.7 30.8 and 18.0 24.7.
 static bool prep_in_runs(const DeltaDims& d, int T) {
   auto width = [](int n) { return n == 64 || n == 128 || n == 256; };
-  return T >= 192 && d.taps == 4 && width(d.D) && width(d.V);
+  return (int64_t)T * (2 * d.G + d.H + 1) >= 12000 && d.taps == 4 && width(d.D) && width(d.V);
 }
 
 // ------------------------------------------------------------------------------------------ decays of a long step
