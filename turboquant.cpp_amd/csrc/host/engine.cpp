@@ -382,7 +382,9 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   float* weights = (float*)c.arena.take((size_t)n_pairs * 4);
   // what the products are told: units of 64 up to four at a time where experts have that many rows (ops.expert_product_rows)
   const int rows = unit == 64 && n_pairs >= s.expert_pairs_from * E ? 64 + TQ_TILE_PAIRS : unit;
-  const int order_unit = rows != unit ? unit + TQ_ITEMS_OF_FOUR : unit;
+  // how many of them (ops.expert_item_units)
+  const bool four = n_pairs >= 112 * (int64_t)E && n_pairs * ((I + 127) / 128) / 256 >= 256;
+  const int order_unit = rows != unit && four ? unit + TQ_ITEMS_OF_FOUR : unit;
   float* gate = gated ? (float*)c.arena.take((size_t)T * 4) : nullptr;
   float* logits = (float*)c.arena.take((size_t)T * (E + (gated ? 1 : 0)) * 4);
   int* sorted_token = (int*)c.arena.take((size_t)cap * 4);

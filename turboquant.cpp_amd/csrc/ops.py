@@ -843,6 +843,7 @@ EXPERT_16_UPTO, EXPERT_32_UPTO = 5, 10
 EXPERT_128_FROM = EXPERT_256_FROM = 1 << 30
 TILE_PAIRS = 1024            # added to tile_rows 64: the units of an item, two or four of one expert, per workgroup (TQ_TILE_PAIRS)
 ITEMS_OF_FOUR = 1 << 30      # added to the row order's unit: its items hold four row tiles instead of two (TQ_ITEMS_OF_FOUR)
+ITEMS_OF_FOUR_FROM = 112     # rows per expert on average from which items may hold four units (expert_item_units)
 EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken several at a time
 
 
@@ -884,6 +885,21 @@ def expert_product_rows(unit: int, n_pairs: int, num_experts: int) -> int:
     if unit == 64 and n_pairs >= EXPERT_PAIRS_FROM * num_experts:
         return 64 + TILE_PAIRS
     return unit
+
+
+def expert_item_units(n_pairs: int, num_experts: int, inner: int, gated: bool = True) -> int:
+    """How many units of 64 rows an item of the row order holds at most: 4 from 112 rows per expert on average and as many
+    tiles of four units (by 128 columns of a gated pair's two matrices of ``inner`` rows, or by 256 of one) as the chip has
+    compute units, else 2.  Tall tiles have the higher rate, but where they are few each of them is all that a compute
+    unit does, and it lasts twice as long; and where experts have fewer rows than two units, only those that a skewed
+    router favours have tall items, which the others then wait for.  Both products, us, by items of two and of four:
+    8 experts of 1,024 x 512 with 200 rows each (50 tiles of four units) 37 and 56; 32 of 768 x 1,024 with 260 rows
+    (195) 89 and 110, with 350 (262) 113 and 113, with 500 154 and 138; 60 of 1,408 x 2,048 with 130 rows 321 and 285, behind
+    a router whose experts' shares fall as 1 / n 326 and 371, with 500 rows 737 and 646, 737 and 665; 64 of that size
+    with 100 rows 269 and 266, 296 and 351; 32 of 4,096 x 4,096 with 70 rows 603 and 601, 660 and 857, with 130 rows 812 and
+    679, 808 and 861."""
+    tiles = n_pairs * -(-inner // (128 if gated else 256)) // 256
+    return 4 if n_pairs >= ITEMS_OF_FOUR_FROM * num_experts and tiles >= 256 else 2
 
 
 def _gemm_problem(k: str, a, w, act, bias, w2, out_act, a_rows, tile_group, n_tiles, tile_rows, gather):

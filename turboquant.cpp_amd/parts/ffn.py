@@ -184,7 +184,8 @@ class SparseMoE(Part):
                                     **({} if self.expert_size % 8 == 0 else {"w_behind": self.expert_down}))
         # what the experts' products are called with, and the items of the row order that they go by
         rows = ops.expert_product_rows(unit, T * self.top_k, self.num_experts)
-        unit = unit if rows == unit else ops.RowUnit(unit, 4)
+        if rows != unit:
+            unit = ops.RowUnit(unit, ops.expert_item_units(T * self.top_k, self.num_experts, self.expert_size, self.gated))
         if self.score_correction or not self.gated:
             return self._forward_scored(normed, normed32, ctx, unit, rows)
         route = lambda: ops.route(normed32, self.router, self.shared_scale if self.shared_gated else None,
