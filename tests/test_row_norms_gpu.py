@@ -110,6 +110,23 @@ def test_sum_of_several_parts(ops, H):
     assert close(x, v, 64) and close(out, rms(v, w, eps), 256) and torch.equal(out, out32)
 
 
+@pytest.mark.parametrize("H", [64, 512, 1020, 1024, 4096, 4100, 8192])
+def test_parts_of_many_rows(ops, H):
+    """Many rows of short or long runs take another kernel than few: a row's bits are the same."""
+    T, eps = 257, 1e-5
+    w, vec, x0 = drawn((H,), 1, 0.1) + 1, drawn((H,), 2), drawn((T, H), 3)
+    a, b = drawn((1, T, H), 4), drawn((5, T, H), 5)
+    gathered, _ = experts(ops, T, H, 3, 0, 6)
+
+    def run(n):
+        x = x0[:n].clone()
+        part = ops.GatheredSum(gathered.y, gathered.pair_slot[:n].contiguous(), gathered.weights[:n].contiguous(), None, None)
+        return x, *ops.add_rmsnorm(x, ops.Terms([(0.5, a[:, :n].contiguous()), (2.0, b[:, :n].contiguous())], part, vec), w, eps, "bfloat16", want_f32=True)
+
+    for many, few in zip(run(T), run(T - 1)):
+        assert torch.equal(many[:T - 1], few)
+
+
 @pytest.mark.parametrize("act", ["float32", "bfloat16"])
 def test_rows_of_no_numbers(ops, act):
     """Empty rows come back empty; the library's entries read and write nothing for them."""

@@ -591,7 +591,12 @@ TQ_API int tq_add_terms_rmsnorm(float* x, const int64_t* deltas, const int* S, c
     hipLaunchKernelGGL((add_terms_rmsnorm_row_kernel<W, THREADS, NV>), dim3(R), dim3(THREADS), 0, st, x, t, (size_t)delta_stride, vec,  \
                        y, pair_slot, weights, topk, (const W*)w, eps, rows, (act_t*)out, out32, H);                                     \
   })
-  TQ_ROW_KERNELS(H, TQ_BODY);
+  // Both kernels give the same bits.  Many rows: up to 4,096 numbers in registers, where the terms' sums one behind the other do not leave
+  // a row's loads too few (4,000 rows of three terms and four experts, us in registers and through LDS: 5,120 numbers 118 and 107, 8,192
+  // 189 and 170, 4,096 81 and 81, 2,048 41 and 42, 1,024 23 and 23), and from 1,024 on, where every thread has a run (512 15.4 and 15.4,
+  // 256 11.8 and 9.8, 64 10.6 and 8.3; 700 rows of 512 5.0 and 4.8).  Few rows wait for latency: always (8 rows of 64 3.8 and 4.2,
+  // of 4,096 5.4 and 5.9, of 8,192 7.8 and 8.8).
+  if (R <= 256 || (H >= 1024 && H <= 4096)) TQ_ROW_KERNELS(H, TQ_BODY);
 #undef TQ_BODY
   const int threads = (H % 4 == 0 && H >= 2048) ? 512 : 256;
   const size_t shmem = (size_t)((H + 3) / 4 * 4 + threads / TQ_WAVE) * sizeof(float);
