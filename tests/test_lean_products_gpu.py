@@ -26,8 +26,8 @@ def forms(w2, pair_limit=None):
 
 
 # k: one line; fewer lines than a round; a round and a remainder over two waves; shares of sixteen waves of which one has none;
-# columns: one tile, a few, every compute unit a workgroup of 16 columns (4,096 with eight waves), many
-@pytest.mark.parametrize("K,N", [(64, 16), (192, 48), (1408, 208), (5632, 512), (2048, 4096), (320, 17408)])
+# columns: one tile, a few, every compute unit a workgroup of 16 columns, one and a half, many
+@pytest.mark.parametrize("K,N", [(64, 16), (192, 48), (1408, 208), (5632, 512), (2048, 4096), (128, 6144), (320, 17408)])
 @pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
 @pytest.mark.parametrize("gated", [True, False])
 def test_one_matrix(ops, K, N, M, gated):
@@ -52,8 +52,8 @@ def rows_of(ops, counts, T):
     return dict(a_rows=st, tile_group=te, n_tiles=nt, tile_rows=16)
 
 
-# experts with one row, eight, nine, sixteen, seventeen (a second tile of one), none
-@pytest.mark.parametrize("counts,T", [([0, 1, 0, 0], 1), ([1, 8, 0, 9, 16, 17, 1], 52)])
+# experts with one row, eight, nine, sixteen, seventeen (a second tile of one), none; more row tiles than the narrow columns are for
+@pytest.mark.parametrize("counts,T", [([0, 1, 0, 0], 1), ([1, 8, 0, 9, 16, 17, 1], 52), ([1] * 20 + [12], 16)])
 @pytest.mark.parametrize("K,N", [(64, 16), (1408, 240), (2048, 1408)])
 def test_experts_and_a_second_product_beside_them(ops, counts, T, K, N):
     E = len(counts)

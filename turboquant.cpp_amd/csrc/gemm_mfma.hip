@@ -374,12 +374,12 @@ __global__ __launch_bounds__(1024) void gemm_lean_kernel(MfmaGemmArgs g) {
   lean_body<DUAL, OUT_ACT, GROUP, COLS>(g, blockIdx.x, blockIdx.y, blockIdx.z, red);
 }
 // (as gemm_stream_pair_kernel; the first over experts, the second of one matrix)
-template <bool DUAL, bool OUT_ACT>
+template <bool DUAL, bool OUT_ACT, int COLS>
 __global__ __launch_bounds__(1024) void gemm_lean_pair_kernel(MfmaGemmArgs g1, int nx1, MfmaGemmArgs g2, int nx2, int n2) {
   extern __shared__ float red[];
   const int id = blockIdx.x;
-  if (id < n2) lean_body<DUAL, OUT_ACT, false, 8>(g2, id % nx2, 0, id / nx2, red);
-  else lean_body<DUAL, OUT_ACT, true, 8>(g1, (id - n2) % nx1, (id - n2) / nx1, 0, red);
+  if (id < n2) lean_body<DUAL, OUT_ACT, false, COLS>(g2, id % nx2, 0, id / nx2, red);
+  else lean_body<DUAL, OUT_ACT, true, COLS>(g1, (id - n2) % nx1, (id - n2) / nx1, 0, red);
 }
 
 // ------------------------------------------------------------------------------------------ q, k, v of a few tokens
@@ -805,16 +805,22 @@ static bool lean_suits(const MfmaGemmArgs& g) {
   return g.K % 64 == 0 && g.N % 16 == 0 && g.K < (1 << 26) && g.k_per % 64 == 0 &&
          (g.tile_group ? g.a_rows && g.n_tiles : !g.a_rows && !g.n_tiles && g.M <= 16);
 }
-// A workgroup's columns there.  Tiles of 8 leave fewer compute units without work (one row by 2,048 x 5,632: 6.9 us against 8.5 in
-// tiles of 16, 2,048 x 8,448 8.7 against 11.7, a gated pair of 5,632 x 2,048 10.4 against 12.4; experts' pairs 10.6 against 11.8,
-// 151,936 x 2,048 106 against 110) but read `a` twice as often: tiles of 16 where there are 192 to 256 of them with eight waves each,
-// one to nearly every compute unit (8 rows by 4,096 x 4,096: 9.3 against 10.3), and for more than 8 rows of plain products with more
-// columns than that (32,000 x 2,048: 24.2 against 26.2).
-static int lean_columns(const MfmaGemmArgs& g, int nw, bool dual) {
-  const int tiles = g.N / 16;
-  if (tiles < 192) return 8;
-  if (tiles <= 256 && nw == 8 && !g.tile_group) return 16;
-  return dual || g.tile_group || g.M <= 8 ? 8 : 16;
+// A workgroup's columns there.  Tiles of 8 leave fewer compute units without work but read `a` twice as often, which costs the more
+// the more rows there are and the less `w` has of them (a gated pair reads two lines of w for one of a).
+// One matrix: 8 where tiles of 16 do not give three quarters of the compute units one (one row by 2,048 x 5,632: 6.9 us against 8.7 in
+// tiles of 16; sixteen 10.8 and 13.3; from five eighths on for up to 8 rows: sixteen by 2,816 x 1,024 5.5 and 4.7), and where they
+// come out unevenly for up to 8 rows, 12 of a gated pair (384 tiles, one row by 6,144 x 2,048 7.3 and 8.0; eight of a pair 12.9 and
+// 13.8); else few rows of wide matrices alone (one row by 20,480 x 3,584 24.6 and 26.0, four of a pair 48.5 and 50.4; of a pair by
+// 8,192 x 4,096 25.6 and 23.8; eight rows by 151,936 x 2,048 144 and 116, sixteen of a pair by 11,008 x 4,096 47.7 and 37.1).
+// A matrix per expert: while row tiles are few (60 experts of 1,408 x 2,048, four a token, us of the pair and of the second product: one
+// token 9.7 7.2 and 11.2 7.1, four 27.8 17.0 and 27.6 14.7, sixteen 69.8 36.9 and 66.4 34.5, 64 109 65 and 108 54; with a second
+// product beside them sixteen 70.3 39.8 and 70.3 37.5).
+static int lean_columns(const MfmaGemmArgs& g, int row_tiles, bool dual) {
+  if (g.tile_group) return row_tiles <= (dual ? 16 : 6) ? 8 : 16;
+  const int tiles = g.N / 16, rounds = (tiles + 255) / 256;
+  if (tiles <= 256) return tiles < (g.M > 8 ? 160 : 192) ? 8 : 16;
+  const bool uneven = rounds * 256 > tiles + tiles / 4;
+  return g.M <= (dual ? (uneven ? 12 : tiles > 512 ? 4 : 0) : (uneven ? 8 : 1)) ? 8 : 16;
 }
 
 // MT row tiles of 16; more than one (17 to 64 rows of one matrix) go with two column tiles per wave.
@@ -833,14 +839,15 @@ static int launch_stream(MfmaGemmArgs g, bool dual, bool out_act, int row_tiles,
   if (shmem > TQ_STREAM_LDS) return TQ_ERR_UNSUPPORTED;
   if constexpr (MT == 1) {
     if (lean_suits(g)) {
-      const int cols = lean_columns(g, nw, dual);
+      const int cols = lean_columns(g, row_tiles, dual);
       const dim3 lean_grid(g.N / cols, row_tiles, splits);
 #define TQ_LEAN(D, O, G, C) hipLaunchKernelGGL((gemm_lean_kernel<D, O, G, C>), lean_grid, dim3(64 * nw), shmem, st, g)
-#define TQ_LEAN_OF(D, O)                        \
-  do {                                          \
-    if (g.tile_group) TQ_LEAN(D, O, true, 8);   \
-    else if (cols == 8) TQ_LEAN(D, O, false, 8); \
-    else TQ_LEAN(D, O, false, 16);              \
+#define TQ_LEAN_OF(D, O)                                            \
+  do {                                                              \
+    if (g.tile_group && cols == 8) TQ_LEAN(D, O, true, 8);          \
+    else if (g.tile_group) TQ_LEAN(D, O, true, 16);                 \
+    else if (cols == 8) TQ_LEAN(D, O, false, 8);                    \
+    else TQ_LEAN(D, O, false, 16);                                  \
   } while (0)
       if (dual && out_act) TQ_LEAN_OF(true, true);
       else if (dual) TQ_LEAN_OF(true, false);
@@ -1196,14 +1203,21 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
   if (n1 + n2 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)(n1 + n2));
   if (g[0].tile_group && !g[1].tile_group && lean_suits(g[0]) && lean_suits(g[1])) {
-    const int lx1 = g[0].N / 8, lx2 = g[1].N / 8, l2 = lx2 * splits2;
+    const int cols = lean_columns(g[0], row_tiles[0], dual[0]), lx1 = g[0].N / cols, lx2 = g[1].N / cols, l2 = lx2 * splits2;
     if ((int64_t)lx1 * row_tiles[0] + l2 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
-#define TQ_PAIR(D, O) hipLaunchKernelGGL((gemm_lean_pair_kernel<D, O>), dim3(lx1 * row_tiles[0] + l2), dim3(64 * nw), shmem, st, g[0], lx1, g[1], lx2, l2)
+#define TQ_PAIR_OF(D, O, C) \
+  hipLaunchKernelGGL((gemm_lean_pair_kernel<D, O, C>), dim3(lx1 * row_tiles[0] + l2), dim3(64 * nw), shmem, st, g[0], lx1, g[1], lx2, l2)
+#define TQ_PAIR(D, O)                     \
+  do {                                    \
+    if (cols == 8) TQ_PAIR_OF(D, O, 8);   \
+    else TQ_PAIR_OF(D, O, 16);            \
+  } while (0)
     if (dual[0] && out_act[0]) TQ_PAIR(true, true);
     else if (dual[0]) TQ_PAIR(true, false);
     else if (out_act[0]) TQ_PAIR(false, true);
     else TQ_PAIR(false, false);
 #undef TQ_PAIR
+#undef TQ_PAIR_OF
     TQ_LAUNCH_CHECK();
     return 0;
   }
