@@ -54,6 +54,20 @@ def test_gated_pairs_of_as_many_columns_as_the_grid_has_room_for(ops, N):
         ops.gemm(a, w.repeat(2049, 1)[:8388481].contiguous(), "float32", w2=w2.repeat(2049, 1)[:8388481].contiguous())
 
 
+def test_an_experts_pair_in_either_width(ops):
+    """Experts' gated pairs go in tiles of 64 columns and, where those are many, of 128: a column's bits are the same."""
+    K, N, E = 36, 8192, 3
+    ids = torch.tensor([0] * 700 + [1] * 65 + [2], dtype=torch.int32)[torch.randperm(766, generator=torch.Generator().manual_seed(7))].to(DEV)
+    st, _slot, te, nt = ops.moe_align(ids[:, None].contiguous(), E, 64, "float32")
+    assert st.numel() // 64 * (N // 128) <= 5 * 512 < st.numel() // 64 * (4 * N // 128)
+    x, w, w2 = drawn((766, K), 1), drawn((E, N, K), 2, 0.2), drawn((E, N, K), 3, 0.2)
+    order = dict(a_rows=st, tile_group=te, n_tiles=nt, tile_rows=64)
+    want = ops.gemm(x, w, "float32", w2=w2, **order)
+    got = ops.gemm(x, w.repeat(1, 4, 1), "float32", w2=w2.repeat(1, 4, 1), **order)
+    live = st >= 0
+    assert (got[live].view(-1, 4, N) == want[live][:, None]).all()
+
+
 @pytest.mark.parametrize("K,N", [(12, 40), (52, 129), (64, 128)])
 @pytest.mark.parametrize("gated", [True, False])
 def test_experts_in_row_tiles(ops, K, N, gated):

@@ -6,10 +6,10 @@
 // per-row-tile matrices for experts; the reference's counterpart is its float matvec
 // (/root/reference/src/engine/tq_ops.c:296-343).  Two kernels:
 //
-//  * gemm_f32_tile_kernel, for more than 16 rows: tiles of 64 or 128 rows by 128 columns (64 of a gated pair of 128 rows) by four
+//  * gemm_f32_tile_kernel, for more than 16 rows: tiles of 64 or 128 rows by 128 columns (64 of most gated pairs) by four
 //    waves, 16 of k at a time.  What bounds it is the matrix instructions (64 clocks each), so what counts is that a SIMD always
-//    has a wave with products to do: 64 sums a wave and no more, so that three workgroups share a compute unit (two of an
-//    expert's gated pair, and of one of up to 64 rows, whose stages hold 64 rows and 128 of either matrix: 60 KB a ring), and tiles that go
+//    has a wave with products to do: 64 sums a wave and no more, so that three workgroups share a compute unit (two of a
+//    gated pair of 64 rows by 128 columns, whose ring is 60 KB, four by 64), and tiles that go
 //    straight from memory into a ring of three LDS stages, two on their way, with one bare barrier a tile and no branch around a
 //    load (with tiles through registers and loads behind predicates a gated pair of 128 x 128 had one wave to a SIMD).
 //    16,385 rows, ms, before and now: by 6,144 x 2,048 3.46 and 3.20 (129 TFLOP/s; the instructions alone give 153), by 2,048 x 5,632 3.48
@@ -513,14 +513,22 @@ TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gath
       hipLaunchKernelGGL((gemm_f32_stream_kernel<1, SNT, false>), grid, dim3(256), 0, st, g, k_per_split, k_per_wave, part);
   } else {
     // tiles; 17 to 64 rows of one matrix are a single row of tiles, cut into runs of k where the matrix is narrow.  A gated pair of
-    // more rows goes in tiles of 128 rows by 64 columns, as long as the grid's y has room for as many columns of tiles (4,194,240
-    // columns of either matrix), beyond that in tiles of 64 by 128, whose sums run over k alike.
-    const bool tall = !grouped && M > 64 && !(dual && (N + 63) / 64 > 65535);
-    const int mi = tall ? 2 : 1, columns = tall && dual ? 64 : 128;
+    // more rows goes in tiles of 128 rows by 64 columns, as long as the grid's y has room for as many (4,194,240 columns of either
+    // matrix), beyond that in tiles of 64 rows, whose sums run over k alike.
+    // A gated pair in tiles of 64 rows: by 128 columns two workgroups share a compute unit, by 64 columns four, but `a` passes twice as
+    // often.  64 columns while the tiles of 128 are within five rounds of those two (us by 128 and by 64 columns: 24 rows by twice 6,144
+    // x 2,048 58 and 48, 64 by 20,480 x 3,584 250 and 203; 60 experts of 1,408 x 2,048, four per token, 250 tokens 523 and 429, 2,000
+    // (2,035 tiles) 1,035 and 979, 3,000 (2,717) 1,338 and 1,381, 18,000 6,550 and 6,901; 32 of 4,096 x 2,048, two per token, 2,000
+    // tokens (3,008) 1,359 and 1,406; 8 of 4,096 x 1,024 3,000 tokens (3,264) 898 and 863).
+    const bool fits = (N + 63) / 64 <= 65535;
+    const int mi = (grouped || M <= 64 || (dual && !fits)) ? 1 : 2;
+    const bool narrow = dual && fits && (mi == 2 || (int64_t)((M + 63) / 64) * ((N + 127) / 128) <= 5 * 512);
+    const int columns = narrow ? 64 : 128;
     const dim3 grid((M + 64 * mi - 1) / (64 * mi), (N + columns - 1) / columns, runs);
     if (grid.y > 65535) return TQ_ERR_UNSUPPORTED;
     if (mi == 1) {
-      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, true>), grid, dim3(256), 0, st, g, k_per_split, part);
+      if (narrow) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
+      else if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, true>), grid, dim3(256), 0, st, g, k_per_split, part);
       else hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
     } else {
       if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<2, 1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
