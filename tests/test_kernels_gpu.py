@@ -492,7 +492,10 @@ def test_the_height_of_expert_tiles(ops, monkeypatch):
     assert ops.expert_product_rows(64, 60 * 48 - 1, 60) == 64
     assert ops.expert_product_rows(64, 60 * 48, 60) == 64 + ops.TILE_PAIRS
     assert ops.expert_product_rows(16, 60 * 64, 60) == 16 and ops.expert_product_rows(256, 60 * 2000, 60) == 256
-    # items of four units: 112 rows per expert and 256 tiles of four units by 128 columns of either matrix (256 of one)
+    # items of four units: 112 rows per expert and 256 tiles of four units by 128 columns of either matrix (256 of one), or 88 and 450
+    assert ops.expert_item_units(88, 1, 64, beside=True) == 4 and ops.expert_item_units(87, 1, 1 << 20, beside=True) == 2
+    assert ops.expert_item_units(64 * 90, 64, 2560) == 4 and ops.expert_item_units(64 * 89, 64, 2560) == 2
+    assert ops.expert_item_units(64 * 88, 64, 4096) == 4 and ops.expert_item_units(64 * 88 - 1, 64, 4096) == 2
     assert ops.expert_item_units(112 * 60, 60, 1408) == 4 and ops.expert_item_units(112 * 60 - 1, 60, 1408) == 2
     assert ops.expert_item_units(8192, 32, 1024) == 4 and ops.expert_item_units(8191, 32, 1024) == 2
     assert ops.expert_item_units(16384, 32, 1024, gated=False) == 4 and ops.expert_item_units(16383, 32, 1024, gated=False) == 2

@@ -382,9 +382,7 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   float* weights = (float*)c.arena.take((size_t)n_pairs * 4);
   // what the products are told: units of 64 up to four at a time where experts have that many rows (ops.expert_product_rows)
   const int rows = unit == 64 && n_pairs >= s.expert_pairs_from * E ? 64 + TQ_TILE_PAIRS : unit;
-  // how many of them (ops.expert_item_units)
-  const bool four = n_pairs >= 112 * (int64_t)E && n_pairs * ((I + 127) / 128) / 256 >= 256;
-  const int order_unit = rows != unit && four ? unit + TQ_ITEMS_OF_FOUR : unit;
+  int order_unit = unit;
   float* gate = gated ? (float*)c.arena.take((size_t)T * 4) : nullptr;
   float* logits = (float*)c.arena.take((size_t)T * (E + (gated ? 1 : 0)) * 4);
   int* sorted_token = (int*)c.arena.take((size_t)cap * 4);
@@ -411,7 +409,12 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   sd.lda = Is, sd.w = f.shared_down, sd.M = T, sd.N = H, sd.K = Is, sd.partial = true;
   *pending = Pending();
   pending->pair_slot = pair_slot, pending->weights = weights, pending->topk = k, pending->gate = gate;
-  if (Is > 0 && ((T <= 16 && unit == 16) || (tiles_together(eg, sg) && tiles_together(ed, sd)))) {
+  const bool beside = Is > 0 && tiles_together(eg, sg) && tiles_together(ed, sd);
+  if (rows != unit) {      // how many units an item holds (ops.expert_item_units)
+    const int64_t tiles = n_pairs * ((I + 127) / 128) / 256;
+    if ((beside || tiles >= 256) && n_pairs >= (beside || tiles >= 450 ? 88 : 112) * (int64_t)E) order_unit += TQ_ITEMS_OF_FOUR;
+  }
+  if (beside || (Is > 0 && T <= 16 && unit == 16)) {
     // a handful of tokens: the shared expert's two products ride in the launches of the routed experts'; a long prompt: their
     // tiles fill the chip together (parts/ffn.py)
     if (int rc = route()) return rc;

@@ -843,7 +843,7 @@ EXPERT_16_UPTO, EXPERT_32_UPTO = 5, 10
 EXPERT_128_FROM = EXPERT_256_FROM = 1 << 30
 TILE_PAIRS = 1024            # added to tile_rows 64: the units of an item, two or four of one expert, per workgroup (TQ_TILE_PAIRS)
 ITEMS_OF_FOUR = 1 << 30      # added to the row order's unit: its items hold four row tiles instead of two (TQ_ITEMS_OF_FOUR)
-ITEMS_OF_FOUR_FROM = 112     # rows per expert on average from which items may hold four units (expert_item_units)
+ITEMS_OF_FOUR_FROM = 112, 88 # rows per expert on average from which items may hold four units, by expert_item_units
 EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken several at a time
 
 
@@ -887,19 +887,26 @@ def expert_product_rows(unit: int, n_pairs: int, num_experts: int) -> int:
     return unit
 
 
-def expert_item_units(n_pairs: int, num_experts: int, inner: int, gated: bool = True) -> int:
+def expert_item_units(n_pairs: int, num_experts: int, inner: int, gated: bool = True, beside: bool = False) -> int:
     """How many units of 64 rows an item of the row order holds at most: 4 from 112 rows per expert on average and as many
     tiles of four units (by 128 columns of a gated pair's two matrices of ``inner`` rows, or by 256 of one) as the chip has
-    compute units, else 2.  Tall tiles have the higher rate, but where they are few each of them is all that a compute
-    unit does, and it lasts twice as long; and where experts have fewer rows than two units, only those that a skewed
-    router favours have tall items, which the others then wait for.  Both products, us, by items of two and of four:
-    8 experts of 1,024 x 512 with 200 rows each (50 tiles of four units) 37 and 56; 32 of 768 x 1,024 with 260 rows
-    (195) 89 and 110, with 350 (262) 113 and 113, with 500 154 and 138; 60 of 1,408 x 2,048 with 130 rows 321 and 285, behind
-    a router whose experts' shares fall as 1 / n 326 and 371, with 500 rows 737 and 646, 737 and 665; 64 of that size
-    with 100 rows 269 and 266, 296 and 351; 32 of 4,096 x 4,096 with 70 rows 603 and 601, 660 and 857, with 130 rows 812 and
-    679, 808 and 861."""
+    compute units, from 88 rows on where there are 450 of them, among which a crowded expert's last the less, or where the
+    shared expert's tiles go out in the same launches (``beside``), which are as tall anyway; else 2.  Tall tiles have the
+    higher rate, but where they are few each of them is all that a compute unit does, and it lasts twice as long; and
+    where experts have fewer rows than two units, only those that a skewed router favours have tall items, which the others
+    then wait for.
+    Both products, us, by items of two and of four: 8 experts of 1,024 x 512 with 200 rows each (50 tiles of four units) 37 and
+    56; 32 of 768 x 1,024 with 260 rows (195) 89 and 110, with 350 (262) 113 and 113, with 500 154 and 138; 60 of 1,408 x
+    2,048 with 130 rows 321 and 285, behind a router whose experts' shares fall as 1 / n 326 and 371, with 500 rows 737 and
+    646, 737 and 665; 64 of that size with 100 rows 269 and 266, 296 and 351; 32 of 4,096 x 4,096 with 70 rows 603 and 601,
+    660 and 857, with 130 rows 812 and 679, 808 and 861; 64 of 2,560 x 3,584 with 70 rows (350) 727 and 700, 811 and 848, with
+    100 rows (500) 764 and 727, 833 and 841.  With a shared expert's beside them: 32 of 768 x 1,024 with 80 rows 67 and 69, with
+    115 rows 71 and 71, 89 and 73, with 256 rows 126 and 111; 60 of 1,408 x 2,048 with 64 rows 335 and 338, 343 and 356, with 100
+    rows 373 and 370, 406 and 395; 64 of 2,560 x 3,584 with 64 rows 888 and 883, 956 and 1,012, with 100 rows 1,097 and 1,100, 1,201
+    and 1,214, with 128 rows 1,389 and 1,216."""
     tiles = n_pairs * -(-inner // (128 if gated else 256)) // 256
-    return 4 if n_pairs >= ITEMS_OF_FOUR_FROM * num_experts and tiles >= 256 else 2
+    most = beside or tiles >= 450
+    return 4 if (beside or tiles >= 256) and n_pairs >= ITEMS_OF_FOUR_FROM[most] * num_experts else 2
 
 
 def _gemm_problem(k: str, a, w, act, bias, w2, out_act, a_rows, tile_group, n_tiles, tile_rows, gather):

@@ -184,8 +184,9 @@ class SparseMoE(Part):
                                     **({} if self.expert_size % 8 == 0 else {"w_behind": self.expert_down}))
         # what the experts' products are called with, and the items of the row order that they go by
         rows = ops.expert_product_rows(unit, T * self.top_k, self.num_experts)
+        beside = self.gated and self.shared_size > 0 and self._tiles_together(normed, ctx, rows)
         if rows != unit:
-            unit = ops.RowUnit(unit, ops.expert_item_units(T * self.top_k, self.num_experts, self.expert_size, self.gated))
+            unit = ops.RowUnit(unit, ops.expert_item_units(T * self.top_k, self.num_experts, self.expert_size, self.gated, beside))
         if self.score_correction or not self.gated:
             return self._forward_scored(normed, normed32, ctx, unit, rows)
         route = lambda: ops.route(normed32, self.router, self.shared_scale if self.shared_gated else None,
@@ -195,7 +196,7 @@ class SparseMoE(Part):
                                   **({} if self.weight_scale == 1.0 else {"weight_scale": self.weight_scale}),
                                   **({} if not self.sigmoid_scores else {"sigmoid": True, "pair_groups": self.pair_groups}))
         limit = {} if self.pair_limit is None else {"pair_limit": self.pair_limit}
-        if self.shared_size > 0 and ((T <= 16 and unit == 16) or self._tiles_together(normed, ctx, rows)):
+        if beside or (self.shared_size > 0 and T <= 16 and unit == 16):
             # a handful of tokens: the shared expert's two products ride in the launches of the routed experts'; a long prompt: the
             # tiles of both fill the chip together, those that wait for memory beside those that do not (2,048 tokens, 60 experts
             # of 1,408 x 2,048 and a shared one of 5,632: 302 + 170 us a layer; on a second stream 343 + 146 behind 340 of its own)
