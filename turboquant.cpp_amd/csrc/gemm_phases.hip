@@ -13,11 +13,15 @@
 //  * the tiles wait in rings of two (a) and three (w; four where an item has up to 128 rows) tiles, so that a tile of w is asked
 //    for five to seven phases of 0.25 us before it is read: memory's time where an expert's matrices are read once.  Rings of half
 //    tiles of 32 of k are level with two whole ones: rows of 64 bytes halve what L2 gives.
-// One workgroup fills a compute unit's LDS, so what the waves do behind the last tile has nothing to hide behind: outputs go through
-// LDS into stores of 16 bytes a lane, whole lines side by side (a test and a store of a value each took 16 us a tile).
-// Measured, us, against items of two units by 16 waves through a ring of three stages: 64 experts of 2,560 x 3,584 with 1,650 rows
-// each, gated pair 4,760 -> 3,739 (1,036 TFLOP/s), second product 2,590 -> 1,943; 60 experts of 1,408 x 2,048 with 137 rows each
-// 219 -> 173 and 147 -> 103, with 68 rows 149 -> 147 and 96 -> 90.
+// One workgroup fills a compute unit's LDS, so what the waves do behind the last tile has nothing to hide behind: with w as the products'
+// first operand a lane ends with columns side by side, and the outputs go from the registers into stores of 16 bytes a lane.
+// What the matrix instructions cost is power: on random values the chip runs 32x32x16 products alone at 1,858 TFLOP/s and 16x16x32
+// products at 2,183 (1.7 GHz in this kernel either way, where 2.4 is the peak), so these are the small ones.  They add k in groups of
+// eight, one behind the other, as the large ones do: same bits.
+// Measured, us, with items of two units by 16 waves through a ring of three stages, then these tiles by 32x32x16 products and outputs
+// through LDS, then as it is: 13,197 tokens by 8 of 64 experts of 2,560 x 3,584 beside a shared expert of 20,480, gated pairs 7,551 ->
+// 6,334 (1,223 TFLOP/s), second products 3,496 -> 3,051 (the experts alone 4,760 -> 3,739 and 2,590 -> 1,943 before); 2,048 tokens by 4
+// of 60 experts of 1,408 x 2,048 beside one of 5,632 293 -> 260 and 165 -> 154 (the experts alone 219 -> 173 and 147 -> 103 before).
 #include "common.h"
 
 #include "gemm_mfma.h"
@@ -69,6 +73,11 @@ struct PhaseTile {
   const bf16_t *w, *w2;        // the matrices of the halves
 };
 
+// What the place of a chunk of 16 bytes in row r of w's tile is turned by: sixteen lanes that read one chunk of the rows of a product's
+// operand (16 neighbours, or four of every eight) find it in 16 places of 16 bytes of the 256 that the banks serve together.
+template <bool OUT_ACT>
+__device__ __forceinline__ int w_place(int r) { return OUT_ACT ? ((r >> 1) & 1) | ((r >> 3) & 3) << 1 : (r >> 1) & 7; }
+
 // One tile of 64 MI rows (32 MI of either group of waves).
 template <int MI, bool DUAL, bool OUT_ACT>
 __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTile& p, bf16_t* lds) {
@@ -83,7 +92,7 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
   // What this thread asks for: group 0 the rows of a that group 1 multiplies and the first half of w, group 1 the others; rows
   // row + 32 i, the chunk of 16 bytes that belongs at place tid % 8 (the swizzle is in what is asked for).  Rows past the end
   // and rows of padding read some valid row instead: those outputs are never stored.
-  const int row = (tid % 256) / 8, chunk = (tid % 8) ^ ((row >> 1) & 7);
+  const int row = (tid % 256) / 8, chunk = (tid % 8) ^ ((row >> 1) & 7), w_chunk = (tid % 8) ^ w_place<OUT_ACT>(row);
   const bf16_t *a_src[MI], *w_src[4];
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
@@ -93,7 +102,7 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
     a_src[i] = g.a + (size_t)src * g.lda + chunk * 8;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w_src[i] = (wm ? p.w2 : p.w) + (size_t)min((wm ? p.n1 : p.n0) + row + 32 * i, g.N - 1) * g.K + chunk * 8;
+  for (int i = 0; i < 4; ++i) w_src[i] = (wm ? p.w2 : p.w) + (size_t)min((wm ? p.n1 : p.n0) + row + 32 * i, g.N - 1) * g.K + w_chunk * 8;
   auto ask_a = [&](int t) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) load_to_lds16(a_src[i] + t * TBK, As + ((t & 1) * 2 + 1 - wm) * A_SLOT + (i * 32 + wn * 8) * TBK);
@@ -108,38 +117,43 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
   auto alive = [&](int r) { return __ballot(r < 32 * MI && mw + r < g.M && !(g.a_rows && g.a_rows[min(mw + r, g.M - 1)] < 0)); };
   const unsigned long long live_lo = alive(lane), live_hi = MI > 2 ? alive(64 + lane) : 0;
 
-  f32x16 acc[MI][2];
+  // The products are v_mfma_f32_16x16x32_bf16 with w as the first operand: a lane's four sums are four columns of one row, D lane l =
+  // row l % 16 of a, columns 4 (l / 16) + v of w.  Which of the wave's 32 columns of a half a tile's column i is, is free: where the
+  // result is of 16 bits, 8 (i / 4) + 4 j + i % 4 for the half's tiles j = 0 and 1, so that a lane ends with eight columns side by side.
+  f32x4 acc[2 * MI][2][2];      // [rows 16 i ..][half][tile of its columns]
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int i = 0; i < 2 * MI; ++i)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][b][v] = 0.f;
-  const int lr = lane % 32, lc = lane / 32, x = (lr >> 1) & 7;
-  u32x4 af[2][MI], wf[2][2];
+      for (int j = 0; j < 2; ++j) acc[i][b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int lr = lane % 16, lq = lane / 16, a_x = (lr >> 1) & 7;
+  u32x4 af[2 * MI], wf[2][2];
   // 32 of k: half h of tile t, whose w lies in `slot`
   auto read = [&](int t, int slot, int h) {
     const bf16_t* A = As + ((t & 1) * 2 + wm) * A_SLOT + lr * TBK;
-    const bf16_t* W = Ws + slot * 2 * W_SLOT + (wn * 32 + lr) * TBK;
+    const bf16_t* W = Ws + slot * 2 * W_SLOT + wn * 32 * TBK;
+    const int c = 4 * h + lq;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int c = ((2 * (2 * h + j) + lc) ^ x) << 3;
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) wf[j][b] = *reinterpret_cast<const u32x4*>(W + b * W_SLOT + c);
+      for (int j = 0; j < 2; ++j) {
+        const int r = OUT_ACT ? 8 * (lr / 4) + 4 * j + lr % 4 : 16 * j + lr;
+        wf[b][j] = *reinterpret_cast<const u32x4*>(W + b * W_SLOT + r * TBK + ((c ^ w_place<OUT_ACT>(r)) << 3));
+      }
 #pragma unroll
-      for (int i = 0; i < MI; ++i) af[j][i] = *reinterpret_cast<const u32x4*>(A + i * 32 * TBK + c);
-    }
+    for (int i = 0; i < 2 * MI; ++i) af[i] = *reinterpret_cast<const u32x4*>(A + i * 16 * TBK + ((c ^ a_x) << 3));
     PH_FENCE();
   };
   auto multiply = [&]() {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < 2 * MI; ++i)
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[j][i]), __builtin_bit_cast(bf16x8, wf[j][b]),
-                                                              acc[i][b], 0, 0, 0);
+        for (int j = 0; j < 2; ++j)
+          acc[i][b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[b][j]), __builtin_bit_cast(bf16x8, af[i]),
+                                                                 acc[i][b][j], 0, 0, 0);
     PH_FENCE();
   };
 
@@ -228,84 +242,82 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
     for (; t < steps; ++t) second_group(t, Yes());
   }
 
-  // The outputs, 32 rows at a time through this wave's own part of LDS, which all waves have read for the last time.
-  constexpr int LD = 72;      // floats of a row: 32 of either half, and lanes 0..31 and 32..63 (four rows apart) on banks of their own
-  float* buf = (float*)lds + wave * 32 * LD;
-  constexpr int V = OUT_ACT ? 8 : 4;                  // outputs of a lane: 16 bytes, a row's lanes side by side
-  constexpr int PER_HALF = 32 / V, PER_ROW = DUAL ? PER_HALF : 2 * PER_HALF;
-  const int part = lane % PER_ROW, in_half = part % PER_HALF * V;
-  const int col = (part / PER_HALF ? p.n1 : p.n0) + wn * 32 + in_half;
-  float bias[V];
+  // The outputs, 16 rows at a time, from the registers: a lane's pieces of 16 bytes, the four lanes of a row side by side.
+  constexpr int V = OUT_ACT ? 8 : 4, HALVES = DUAL ? 1 : 2, J = OUT_ACT ? 1 : 2;      // columns of a piece; pieces of a lane's row
+  const int col0 = wn * 32 + (OUT_ACT ? 8 : 4) * lq;
+  float bias[HALVES][J][V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) bias[j] = col + j < g.N ? bias_at(g, col + j) : 0.f;
-  const bool wide = col + V <= g.N && g.ldc % V == 0 && (uintptr_t)g.out % 16 == 0;
-  auto to_lds = [&](const f32x16& first, const f32x16& second) {
+  for (int b = 0; b < HALVES; ++b)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      float* at = buf + (8 * (v / 4) + 4 * lc + v % 4) * LD + lr;
-      at[0] = first[v];
-      at[32] = second[v];
-    }
-  };
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const int n = (b ? p.n1 : p.n0) + col0 + 16 * j + v;
+        bias[b][j][v] = n < g.N ? bias_at(g, n) : 0.f;
+      }
+  const bool aligned = g.ldc % V == 0 && (uintptr_t)g.out % 16 == 0;
 #pragma unroll 1
-  for (int i = 0; i < MI; ++i) {      // (kept a loop; the sums stay in registers since each case names its own)
-    if (i == 0) to_lds(acc[0][0], acc[0][1]);
-    if constexpr (MI > 1) if (i == 1) to_lds(acc[1][0], acc[1][1]);
-    if constexpr (MI > 2) if (i == 2) to_lds(acc[2][0], acc[2][1]);
-    if constexpr (MI > 3) if (i == 3) to_lds(acc[3][0], acc[3][1]);
-    const int m_first = mw + 32 * i;
-    const unsigned live = (unsigned)((i < 2 ? live_lo : live_hi) >> (i % 2 * 32));
-    asm volatile("" ::: "memory");
+  for (int i = 0; i < 2 * MI; ++i) {      // (kept a loop; the sums stay in registers since each case names its own)
+    f32x4 sums[2][2];
+#define PH_TAKE(n)                                                        \
+  if constexpr (2 * MI > n)                                               \
+    if (i == n) {                                                         \
+      _Pragma("unroll") for (int b = 0; b < 2; ++b)                       \
+          _Pragma("unroll") for (int j = 0; j < 2; ++j) sums[b][j] = acc[n][b][j]; \
+    }
+    PH_TAKE(0) PH_TAKE(1) PH_TAKE(2) PH_TAKE(3) PH_TAKE(4) PH_TAKE(5) PH_TAKE(6) PH_TAKE(7)
+#undef PH_TAKE
+    if (!(((i < 4 ? live_lo : live_hi) >> (i % 4 * 16 + lr)) & 1)) continue;
+    const size_t row = (size_t)(mw + 16 * i + lr) * g.ldc;
 #pragma unroll
-    for (int q = 0; q < PER_ROW / 2; ++q) {
-      const int r = lane / PER_ROW + q * (64 / PER_ROW);
-      float v[V];
-      const float* at = buf + r * LD + (DUAL ? 0 : part / PER_HALF * 32) + in_half;
+    for (int b = 0; b < HALVES; ++b)
 #pragma unroll
-      for (int j = 0; j < V; ++j) v[j] = at[j] + bias[j];
-      if (DUAL) {
-        float u[V];
+      for (int j = 0; j < J; ++j) {
+        const int col = (b ? p.n1 : p.n0) + col0 + 16 * j;
+        float v[V];
 #pragma unroll
-        for (int j = 0; j < V; ++j) u[j] = at[32 + j];
-        if (g.limit > 0.f) {
+        for (int k = 0; k < V; ++k) v[k] = sums[b][OUT_ACT ? k / 4 : j][k % 4] + bias[b][j][k];
+        if (DUAL) {
+          float u[V];
 #pragma unroll
-          for (int j = 0; j < V; ++j) {
-            v[j] = fminf(v[j], g.limit);
-            u[j] = fminf(fmaxf(u[j], -g.limit), g.limit) + 1.0f;
+          for (int k = 0; k < V; ++k) u[k] = sums[1][OUT_ACT ? k / 4 : j][k % 4];
+          if (g.limit > 0.f) {
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+              v[k] = fminf(v[k], g.limit);
+              u[k] = fminf(fmaxf(u[k], -g.limit), g.limit) + 1.0f;
+            }
+          }
+          gate_many(v, g.gate);
+#pragma unroll
+          for (int k = 0; k < V; ++k) v[k] *= u[k];
+        } else if (g.act1) {
+          gate_many(v, g.act1 - 1);
+        }
+        const bool wide = aligned && col + V <= g.N;
+        if constexpr (OUT_ACT) {
+          bf16_t* o = (bf16_t*)g.out + row + col;
+          if (wide) {
+            u32x4 packed;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) packed[k] = f32_to_bf16(v[2 * k]).bits | (unsigned)f32_to_bf16(v[2 * k + 1]).bits << 16;
+            *reinterpret_cast<u32x4*>(o) = packed;
+          } else {
+#pragma unroll
+            for (int k = 0; k < V; ++k)
+              if (col + k < g.N) o[k] = f32_to_bf16(v[k]);
+          }
+        } else {
+          float* o = (float*)g.out + row + col;
+          if (wide) {
+            *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
+          } else {
+#pragma unroll
+            for (int k = 0; k < V; ++k)
+              if (col + k < g.N) o[k] = v[k];
           }
         }
-        gate_many(v, g.gate);
-#pragma unroll
-        for (int j = 0; j < V; ++j) v[j] *= u[j];
-      } else if (g.act1) {
-        gate_many(v, g.act1 - 1);
       }
-      if (!((live >> r) & 1)) continue;
-      const size_t off = (size_t)(m_first + r) * g.ldc + col;
-      if constexpr (OUT_ACT) {
-        bf16_t* o = (bf16_t*)g.out + off;
-        if (wide) {
-          u32x4 packed;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) packed[j] = f32_to_bf16(v[2 * j]).bits | (unsigned)f32_to_bf16(v[2 * j + 1]).bits << 16;
-          *reinterpret_cast<u32x4*>(o) = packed;
-        } else {
-#pragma unroll
-          for (int j = 0; j < V; ++j)
-            if (col + j < g.N) o[j] = f32_to_bf16(v[j]);
-        }
-      } else {
-        float* o = (float*)g.out + off;
-        if (wide) {
-          *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int j = 0; j < V; ++j)
-            if (col + j < g.N) o[j] = v[j];
-        }
-      }
-    }
-    asm volatile("" ::: "memory");
   }
 }
 
