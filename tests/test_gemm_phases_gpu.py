@@ -158,3 +158,46 @@ def test_a_product_beside_the_experts(ops, T, K, N, K2, N2, gated):
             az, bz = a[:, z * per:(z + 1) * per].double(), b[:, z * per:(z + 1) * per].double()
             exact = az @ bz.T + (bias.double() if z == 0 else 0.0)      # the bias goes with the first run alone
             assert ((y2[z].double() - exact).abs() <= K2 * 2.0 ** -24 * (az.abs() @ bz.abs().T) + 2.0 ** -23 * exact.abs()).all()
+
+
+# rows, columns, k and the height of the tiles that suits: each height; the fewest rows of each rule (65 and 129, 513 to 1,024, 1,025);
+# a few columns past a tile, less than a wave's 32; two and three steps of k; a last tile of one row; and columns it leaves to the tile kernel
+@pytest.mark.parametrize("M,N,K", [(1025, 24, 128), (1100, 4200, 128), (700, 3104, 512), (65, 66048, 512), (1030, 4104, 192), (515, 16600, 512), (130, 33000, 576),
+                                   (2049, 6400, 192), (3001, 5000, 128), (2999, 8000, 320), (1025, 4100, 128)])
+def test_products_of_one_matrix(ops, M, N, K):
+    """Plain products in these tiles are the tile kernel's bits (which gathered rows keep to), with a bias, into either type, through an
+    activation and in runs of k; and the formula's values."""
+    a, w = drawn((M, K), 1), drawn((N, K), 2, 0.1)
+    every = torch.arange(M, dtype=torch.int32, device=DEV)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(4)).to(DEV)
+    for form in (dict(), dict(bias=bias), dict(out_act=True, bias=bias.bfloat16()), dict(out_act=True, activation="gelu", act_alone=True, bias=bias)):
+        assert torch.equal(ops.gemm(a, w, "bfloat16", **form), ops.gemm(a, w, "bfloat16", a_rows=every, **form)), form
+    runs = ops.gemm(a, w, "bfloat16", bias=bias, partial_sums=True)
+    x, y = a.double(), w.double()
+    assert ((runs.double().sum(0) - (x @ y.T + bias.double())).abs() <= (K + 4) * 2.0 ** -24 * (x.abs() @ y.abs().T + bias.double().abs())).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 16500, 128), (1500, 2100, 192), (129, 20000, 128), (200, 16500, 192), (2049, 5000, 192), (1025, 8, 128)])
+def test_gated_pairs_of_one_matrix(ops, M, N, K):
+    """As above, of two matrices behind each other and apart, with and without a limit."""
+    a, both = drawn((M, K), 1), drawn((2 * N, K), 2, 0.1)
+    w, w2, every = both[:N], both[N:], torch.arange(M, dtype=torch.int32, device=DEV)
+    for form in (dict(out_act=True), dict(), dict(out_act=True, pair_limit=0.6), dict(out_act=True, activation="gelu_tanh")):
+        want = ops.gemm(a, w, "bfloat16", w2=w2, a_rows=every, **form)
+        assert torch.equal(ops.gemm(a, w, "bfloat16", w2=w2.clone(), **form), want), form
+        assert torch.equal(ops.gemm(a, w, "bfloat16", w2=w2, **form), want) or M >= ops.VENDOR_MIN_ROWS, form
+
+
+def test_runs_of_k_of_one_matrix(ops):
+    """Many rows of a long k in two runs and more, each within the rounding of its sum, the bias in the first alone."""
+    for M, N, K in ((1025, 2048, 8448), (2100, 1024, 4160), (1100, 1504, 6400)):
+        a, w = drawn((M, K), 1), drawn((N, K), 2, 0.1)
+        bias = torch.randn(N, generator=torch.Generator().manual_seed(4)).to(DEV)
+        got = ops.gemm(a, w, "bfloat16", bias=bias, partial_sums=True)
+        runs = got.shape[0]
+        assert runs > 1 and runs == ops.library("bfloat16").tq_gemm_mfma_splits(M, N, K)
+        per = -(-(K // 64) // runs) * 64
+        for z in range(runs):
+            x, y = a[:, z * per:(z + 1) * per].double(), w[:, z * per:(z + 1) * per].double()
+            want = x @ y.T + (bias.double() if z == 0 else 0.0)
+            assert ((got[z].double() - want).abs() <= (per + 4) * 2.0 ** -24 * (x.abs() @ y.abs().T + bias.double().abs())).all()

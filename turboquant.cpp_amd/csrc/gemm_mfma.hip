@@ -17,7 +17,8 @@
 //    v_mfma_f32_32x32x16_bf16 do not collide); while one buffer is multiplied the next tile is written into
 //    the other and the one after that is on its way from memory.
 //  * gemm_few_tiles_kernel, for up to some hundred rows of one matrix: smaller tiles through a ring of LDS buffers, the same sums.
-//  * gemm_phases_kernel (gemm_phases.hip), for experts with many rows: tiles of up to 256 x 256, the same sums.
+//  * gemm_phases_kernel (gemm_phases.hip), for experts with many rows and for many rows of one matrix where k is in whole tiles: tiles
+//    of up to 256 x 256, the same sums.
 //
 // Operand layouts (wave of 64 lanes): 16x16x32: A lane l = row l%16, k 8*(l/16)..+7; B lane l = column l%16,
 // same k; D lane l = column l%16, rows 4*(l/16)+v, v<4.  32x32x16: A lane l = row l%32, k 8*(l/32)..+7;
@@ -975,6 +976,80 @@ static bool gated_pair_in_tiles_of_64(int M, int N) {
   return lower <= 256 || (taller > 256 && lower <= 512);
 }
 
+// How long gemm_phases takes for a product of one matrix in tiles of 64 mi rows, k in runs, us: 8 in front of and behind a tile's steps
+// of 64, and a step's time, which grows with how many compute units are at work beside it (the clock falls with the power they draw):
+// the first figure where few are, the second where all are.  Fitted to 1,400 timings (80 to 13,197 rows, 64 to 151,936 columns, k 1,024 to
+// 20,480): 4 % above them on average, 9 % off in the root of the mean square, and the height it names loses 0.1 % to the best one.
+static double phases_time(int M, int N, int K, bool dual, int mi, int runs) {
+  static const double few[5] = {0, 0.50, 0.62, 0.84, 1.10}, all[5] = {0, 0.60, 0.86, 1.10, 1.48};
+  const int cols = dual ? 128 : 256, steps = (K / TBK + runs - 1) / runs;
+  const int64_t tiles = (int64_t)((M + 64 * mi - 1) / (64 * mi)) * ((N + cols - 1) / cols) * runs;
+  const double busy = (double)(tiles % 256) / 256;
+  return (double)(tiles / 256) * (8 + all[mi] * steps) + (busy > 0 ? 8 + steps * (few[mi] + (all[mi] - few[mi]) * busy) : 0);
+}
+static double phases_best(int M, int N, int K, bool dual, int runs, int* rows) {
+  double best = 0;
+  for (int mi = 1; mi <= 4 && (mi == 1 || M > 64 * (mi - 1)); ++mi) {
+    const double t = phases_time(M, N, K, dual, mi, runs);
+    if (mi == 1 || t < best) best = t, *rows = 64 * mi;
+  }
+  return best;
+}
+
+// Whether a product of one matrix, of more than 64 rows that follow one another, goes in the tiles of gemm_phases rather than those of
+// gemm_few_tiles or the tile kernel: k in whole tiles, and
+//  * more than 1,024 rows: always (us by the tile kernel and by gemm_phases: 1,280 rows by 2,048 x 2,048 31.8 and 25.3, 3,001 by 3,072 x
+//    2,048 84.6 and 44.5, 13,197 by 6,144 x 2,048 424 and 271; gated pairs of 2,048 rows by 5,632 x 2,048 186 and 88);
+//  * 513 to 1,024 where tiles of 64 x 128 do not find a compute unit each (264 of them, 700 by 3,072 x 2,048, 29.5 and 25.5; 176,
+//    700 by 2,048 x 5,632, 45.6 and 53.1) and a tile has some steps (741 by 6,464 x 128 11.1 and 13.1);
+//  * up to 512 where there are more than two of them to a unit (528, 512 by 8,448 x 2,048, 39.0 and 29.6; 512, 200 by 16,384 x 2,048,
+//    26.8 and 26.2; 384, 512 by 6,144 x 2,048, 25.2 and 26.6; 256, 128 by 16,384 x 2,048, 17.9 and 24.7);
+//  * a gated pair of up to 1,024 where tiles of 64 x 64 do not find a unit each (264, 160 by 5,632 x 2,048, 27.1 and 23.9; 220, 320 by
+//    2,816 x 1,024, 16.1 and 16.0; 160, 256 by 2,560 x 3,584, 32.5 and 34.7).
+// And columns in whole pieces of 16 bytes of the result: without, a lane's four or eight columns side by side go out one by one (10,405
+// by 314 x 320 15.3 and 20.2, 4,377 by 5,006 x 2,752 141 and 162, 727 by 5,583 x 448 15.8 and 22.8).
+static bool phases_suit(int M, int N, int K, bool dual) {
+  if (M <= 64 || K % TBK || K < 2 * TBK || N % 8) return false;
+  const int64_t rows = (M + 63) / 64, narrow = rows * ((N + 63) / 64), wide = rows * ((N + 127) / 128);
+  if (M > 1024) return true;
+  return dual ? narrow > 256 : wide > (M > 512 ? 256 : 512) && K >= 512;
+}
+// Its runs of k where partial sums are wanted apart: what a run more saves must be more than writing and reading its sums takes.
+static int phases_runs(int M, int N, int K) {
+  int best = 1, rows;
+  double least = phases_best(M, N, K, false, 1, &rows);
+  for (int s = 2; s <= 4; s *= 2) {
+    const int per = (K / TBK + s - 1) / s;
+    if (per < 4 || K / TBK - per * (s - 1) < 2) break;
+    const double t = phases_best(M, N, K, false, s, &rows) + (s - 1) * ((double)M * N * 8 / 5e6);
+    if (t < least) least = t, best = s;
+  }
+  return best;
+}
+
+// Whether a product of many rows that the vendor's library would take is the faster one here.  kind 0: plain; 1: its result passes an
+// activation alone; 2: a gated pair, both into the activation type. The library's kernels leave their sums in float for a pass of its
+// own to apply the activation, so that against them stand 14 us (11.5 of an activation alone), the multiply-adds at 1,150 TFLOP/s and
+// that pass at 5.5 TB/s (us by the library and here: gated 2,048 by 5,632 x 2,048 105 and 88, 1,999 by 11,008 x 4,096 408 and 288,
+// 1,280 by 768 x 1,024 18 and 16, 900 by 1,024 x 4,096 31 and 40; an activation alone 3,001 by 8,448 x 2,048 127 and 103, 768 by
+// 1,408 x 2,048 19 and 23, 1,315 by 256 x 832 11 and 13).  A plain product the library does at the same rate, but not where its
+// columns are no whole number of tiles (2,048 by 6,288 x 2,048 67 and 49, 1,733 by 7,184 x 2,048 60 and 50, 3,258 by 8,224 x 2,048
+// 111 and 99; by 8,448 101 and 102), nor where k is very long (8,192 by 3,584 x 20,480 1,505 and 829): there where the tiles here
+// reach 950 TFLOP/s (600 of a very long k).  With many rows and a long k its choice of kernel is uneven: of 130 products of 9,000 to
+// 28,000 rows by 1,024 to 6,144 x 3,584 and 5,632 where these tiles reach 1,100 TFLOP/s the times here are 0.95 of the library's on
+// average (13,197 by 3,584 x 3,584 366 and 252, 12,000 by 6,144 x 5,632 782 and 641, 16,384 by 3,584 x 3,584 343 and 350; worst
+// 1.07), at k 2,048 they are level.
+TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
+  const bool dual = kind == 2;
+  if (!phases_suit(M, N, K, dual)) return 0;
+  int rows;
+  const double t = phases_best(M, N, K, dual, 1, &rows), flops = 2.0 * M * N * K * (dual ? 2 : 1);
+  if (kind) return (dual ? t : 0.95 * t) <= (dual ? 14 : 11.5) + flops / 1.15e9 + (double)M * N * (dual ? 10 : 6) / 5.5e6;
+  const double rate = flops / (t * 1e6);
+  if (K >= 16384) return rate >= 600;
+  return (N % 256 != 0 && rate >= 950) || (M >= 9000 && K >= 3584 && rate >= 1100);
+}
+
 // Into how many runs of k a plain product of M rows may be split when its partial sums are wanted apart.  Many
 // rows: a product whose tiles do not fill the chip twice, and that has k enough, goes faster in 2 to 4 runs, each
 // at least 1024 long, and up to 1,024 rows as tile_runs says.  17 to 64 rows of a narrow matrix with a long k in the
@@ -1015,6 +1090,7 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
     while (s < 8 && waves * s < 4096 && K / (16 * s) >= 128) s *= 2;
     return s;
   }
+  if (phases_suit(M, N, K, false)) return phases_runs(M, N, K);
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + TBN - 1) / TBN);
   int s = 1;
   while (s < 4 && tiles * s < 512 && K / (s * 2) >= 1024) s *= 2;
@@ -1100,7 +1176,11 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
     rc = launch_stream<4>(g, dual, out_act, 1, st, splits);
   } else {
     if ((N + TBN - 1) / TBN > 65535) return TQ_ERR_UNSUPPORTED;
-    if (few_tiles_suit(g, dual))
+    if (!a_rows && phases_suit(M, N, K, dual)) {
+      int rows;
+      phases_best(M, N, K, dual, splits, &rows);
+      rc = launch_gemm_phases_plain(g, rows, dual, out_act, st);
+    } else if (few_tiles_suit(g, dual))
       rc = launch_few_tiles(g, dual, out_act, splits, st);
     else if (M <= 64 * 16 && !dual)
       rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);

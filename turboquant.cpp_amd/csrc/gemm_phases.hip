@@ -22,6 +22,8 @@
 // through LDS, then as it is: 13,197 tokens by 8 of 64 experts of 2,560 x 3,584 beside a shared expert of 20,480, gated pairs 7,551 ->
 // 6,334 (1,223 TFLOP/s), second products 3,496 -> 3,051 (the experts alone 4,760 -> 3,739 and 2,590 -> 1,943 before); 2,048 tokens by 4
 // of 60 experts of 1,408 x 2,048 beside one of 5,632 293 -> 260 and 165 -> 154 (the experts alone 219 -> 173 and 147 -> 103 before).
+// Products of one matrix (`launch_gemm_phases_plain`) take the same tiles, 64 to 256 rows high as the compute units fill best; gemm_mfma.hip
+// has the rules and what they replace (2,048 rows by 2,048 columns with a bias, k 2,048, 62 -> 27 us; 3,001 by 3,072 99 -> 43).
 #include "common.h"
 
 #include "gemm_mfma.h"
@@ -60,6 +62,7 @@ __device__ __forceinline__ void gate_many(float (&v)[N], int kind) {
   }
 }
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 struct No {
   static constexpr bool value = false;
 };
@@ -256,6 +259,7 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
         bias[b][j][v] = n < g.N ? bias_at(g, n) : 0.f;
       }
   const bool aligned = g.ldc % V == 0 && (uintptr_t)g.out % 16 == 0;
+  const bool even = g.N % 2 == 0 && g.ldc % 2 == 0 && (uintptr_t)g.out % 8 == 0;      // columns in pairs at least
 #pragma unroll 1
   for (int i = 0; i < 2 * MI; ++i) {      // (kept a loop; the sums stay in registers since each case names its own)
     f32x4 sums[2][2];
@@ -302,6 +306,10 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
 #pragma unroll
             for (int k = 0; k < 4; ++k) packed[k] = f32_to_bf16(v[2 * k]).bits | (unsigned)f32_to_bf16(v[2 * k + 1]).bits << 16;
             *reinterpret_cast<u32x4*>(o) = packed;
+          } else if (even) {
+#pragma unroll
+            for (int k = 0; k < V; k += 2)
+              if (col + k < g.N) *reinterpret_cast<unsigned*>(o + k) = f32_to_bf16(v[k]).bits | (unsigned)f32_to_bf16(v[k + 1]).bits << 16;
           } else {
 #pragma unroll
             for (int k = 0; k < V; ++k)
@@ -311,6 +319,10 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
           float* o = (float*)g.out + row + col;
           if (wide) {
             *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
+          } else if (even) {
+#pragma unroll
+            for (int k = 0; k < V; k += 2)
+              if (col + k < g.N) *reinterpret_cast<f32x2*>(o + k) = f32x2{v[k], v[k + 1]};
           } else {
 #pragma unroll
             for (int k = 0; k < V; ++k)
@@ -323,9 +335,9 @@ __device__ __forceinline__ void phases_tile(const MfmaGemmArgs& g, const PhaseTi
 
 // Tile `logical` of a product in the order in which a die goes through its run of them.  A matrix per expert (the first product): expert
 // by expert, so that an expert's matrices are read by one die, and within an expert column by column with its items side by side.
-// One matrix (the second): tiles of 256 rows in bands of 8, down a band's columns, a run of k behind the other.
+// One matrix (the second): tiles of `rows` rows in bands of 8, down a band's columns, a run of k behind the other.
 template <bool DUAL>
-__device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int gx, int gy, PhaseTile& p) {
+__device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int gx, int gy, int rows, PhaseTile& p) {
   const int lane = threadIdx.x % 64;
   int tile_n, group = 0;
   if (g.tile_group) {
@@ -366,8 +378,8 @@ __device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int 
     }
     const int band = logical / (8 * gy), in_band = logical % (8 * gy), bh = min(8, gx - band * 8);
     tile_n = in_band / bh;
-    p.m0 = (band * 8 + in_band % bh) * 256;
-    p.units = min((g.M - p.m0 + 63) / 64, 4);
+    p.m0 = (band * 8 + in_band % bh) * rows;
+    p.units = min((g.M - p.m0 + 63) / 64, rows / 64);
   }
   p.w = g.w + (size_t)group * g.group_stride;
   p.w2 = DUAL ? g.w2 + (size_t)group * g.group_stride : p.w;
@@ -375,9 +387,9 @@ __device__ __forceinline__ void phase_tile_of(MfmaGemmArgs& g, int logical, int 
   p.n1 = DUAL ? p.n0 : p.n0 + 128;
 }
 template <bool DUAL, bool OUT_ACT>
-__device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int gy, bf16_t* lds) {
+__device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int gy, int rows, bf16_t* lds) {
   PhaseTile p;
-  phase_tile_of<DUAL>(g, logical, gx, gy, p);
+  phase_tile_of<DUAL>(g, logical, gx, gy, rows, p);
   switch (__builtin_amdgcn_readfirstlane(p.units)) {
     case 4: phases_tile<4, DUAL, OUT_ACT>(g, p, lds); break;
     case 3: phases_tile<3, DUAL, OUT_ACT>(g, p, lds); break;
@@ -387,11 +399,12 @@ __device__ __forceinline__ void phases(MfmaGemmArgs& g, int logical, int gx, int
 }
 
 // A die (workgroups are dealt to the 8 of them in turn) gets a contiguous run of the tiles of the first product and one of the
-// second, if there is one (n2 tiles, gx2 x gy2 a run of k): `first2`: the second's before the first's, else spread among them.
+// second, if there is one (n2 tiles of `rows2` rows, gx2 x gy2 a run of k): `first2`: the second's before the first's, else spread
+// among them.  A first without an order of rows is not there at all: the second alone.
 template <bool DUAL, bool OUT_ACT>
-__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gy, MfmaGemmArgs g2, int gx2, int gy2, int n2, int first2) {
+__global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gy, MfmaGemmArgs g2, int gx2, int gy2, int n2, int rows2, int first2) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  int gx = min(g.n_tiles[1], g.M / 64);
+  int gx = g.tile_group ? min(g.n_tiles[1], g.M / 64) : 0;
   const int id = blockIdx.x, die = id % 8, i = id / 8;
   const int n1 = gx * gy;
   const int q1 = n1 / 8, rem1 = n1 % 8, mine1 = q1 + (die < rem1 ? 1 : 0);
@@ -412,7 +425,27 @@ __global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gy
     gx = gx2;
     gy = gy2;
   }
-  phases<DUAL, OUT_ACT>(g, logical, gx, gy, (bf16_t*)smem);
+  phases<DUAL, OUT_ACT>(g, logical, gx, gy, rows2, (bf16_t*)smem);
+}
+
+static int launch_phases(const MfmaGemmArgs& g, int gy, int64_t n1, const MfmaGemmArgs& g2, int gx2, int gy2, int64_t n2, int rows2, int first2,
+                         bool dual, bool out_act, hipStream_t st) {
+  const int64_t per_die = (n1 + 7) / 8 + (n2 + 7) / 8;
+  if (per_die * 8 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
+  const int shmem = 160 * 1024;      // MI = 2 and 4; 144 KB where MI is 1 or 3
+#define TQ_PHASES(D, O)                                                                                                       \
+  do {                                                                                                                        \
+    if (hipFuncSetAttribute((const void*)gemm_phases_kernel<D, O>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem) != hipSuccess) \
+      return TQ_ERR_UNSUPPORTED;                                                                                              \
+    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), dim3((unsigned)(per_die * 8)), dim3(512), shmem, st, g, gy, g2, gx2, gy2,  \
+                       (int)n2, rows2, first2);                                                                               \
+  } while (0)
+  if (dual && out_act) TQ_PHASES(true, true);
+  else if (dual) TQ_PHASES(true, false);
+  else if (out_act) TQ_PHASES(false, true);
+  else TQ_PHASES(false, false);
+#undef TQ_PHASES
+  return 0;
 }
 
 // g2 (null: none): a second product, of one matrix and of the same kind, whose tiles fill the chip beside the first's; its k may be
@@ -432,21 +465,16 @@ int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual,
     // beside 5,632 261 and 266.  No side where spreading wins was found: the line is no border between two, only where the gain is sure.
     first2 = g2->k_per >= 3 * g.K / 2;
   }
-  const int64_t per_die = ((int64_t)gx * gy + 7) / 8 + (n2 + 7) / 8;
-  if (per_die * 8 > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
-  const int shmem = 160 * 1024;      // MI = 2 and 4; 144 KB where MI is 1 or 3
-#define TQ_PHASES(D, O)                                                                                                       \
-  do {                                                                                                                        \
-    if (hipFuncSetAttribute((const void*)gemm_phases_kernel<D, O>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem) != hipSuccess) \
-      return TQ_ERR_UNSUPPORTED;                                                                                              \
-    hipLaunchKernelGGL((gemm_phases_kernel<D, O>), dim3((unsigned)(per_die * 8)), dim3(512), shmem, st, g, gy, g2 ? *g2 : g, gx2, gy2, n2, first2); \
-  } while (0)
-  if (dual && out_act) TQ_PHASES(true, true);
-  else if (dual) TQ_PHASES(true, false);
-  else if (out_act) TQ_PHASES(false, true);
-  else TQ_PHASES(false, false);
-#undef TQ_PHASES
-  return 0;
+  return launch_phases(g, gy, (int64_t)gx * gy, g2 ? *g2 : g, gx2, gy2, n2, 256, first2, dual, out_act, st);
+}
+
+// A product of one matrix, whose rows follow one another, in tiles of `rows` (a multiple of 64 up to 256) rows; k may be in runs.
+int launch_gemm_phases_plain(const MfmaGemmArgs& g, int rows, bool dual, bool out_act, hipStream_t st) {
+  if (g.tile_group || g.a_rows) return TQ_ERR_BAD_ARG;
+  const int cols = dual ? 128 : 256;
+  const int64_t gx = (g.M + rows - 1) / rows, gy = (g.N + cols - 1) / cols, n = gx * gy * ((g.K + g.k_per - 1) / g.k_per);
+  if (n > (1 << 28)) return TQ_ERR_UNSUPPORTED;
+  return launch_phases(g, 1, 0, g, (int)gx, (int)gy, n, rows, 0, dual, out_act, st);
 }
 
 // Into how many runs the second product's k goes beside a first of M1 rows (at most): so many that none of its tiles takes longer than

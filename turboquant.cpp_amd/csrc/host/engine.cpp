@@ -126,6 +126,9 @@ bool vendor_product(const Ctx& c, const Product& p) {
   if (!(bf16_path() && s.vendor_min_rows > 0 && p.M >= s.vendor_min_rows && (p.K < 16384 || p.M >= 8192) &&
         p.w.wtype == TQ_BF16 && !s.capturing && !s.decode && tq_vendor_available()))
     return false;
+#if defined(TQ_ACT_BF16)
+  if (!(p.w2 && !p.out_act) && tq_gemm_here_rather(p.M, p.N, p.K, p.w2 ? 2 : 0)) return false;
+#endif
   if (!p.w2) return tq_vendor_takes(p.M, p.N, p.K, p.lda, p.out_act) != 0;
   const int64_t chunk = s.vendor_gated_rows > 0 ? s.vendor_gated_rows : 4096;
   const int rows = (int)(p.M < chunk ? p.M : chunk), last = (int)(p.M % chunk);

@@ -175,6 +175,7 @@ _OPTIONAL = {
     "tq_gemm_mfma": [_c_ptr, _c_i64, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int,
                      _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "tq_gemm_mfma_splits": [_c_int, _c_int, _c_int],
+    "tq_gemm_here_rather": [_c_int] * 4,
     "tq_gemm_phases_pair_splits": [_c_int] * 6,
     "tq_gemm_mfma_pair_splits": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "tq_gemm_mfma_pair": [_c_ptr, _c_ptr, _c_int, _c_ptr],
@@ -777,7 +778,7 @@ def qkv_rope_write(a: torch.Tensor, qkv_weight: torch.Tensor, qkv_bias: torch.Te
              and (qkv_bias is None or qkv_bias.dtype in _WTYPE))
     if not fused:
         # the vendor library's product has no bias of its own that costs nothing: the rotation adds it as it reads
-        late = qkv_bias is not None and a.dim() == 2 and _vendor_product(act, a, qkv_weight, T, K)
+        late = qkv_bias is not None and a.dim() == 2 and _vendor_here(act, a, qkv_weight, T, qkv_weight.shape[0], K)
         qkv = gemm(a, qkv_weight, act, bias=None if late else qkv_bias)
         return rope_kv_write(qkv, positions, seq_of_token, block_table, inv_freq, pairing, rotary_dim, k_pages, v_pages,
                              layer_offset, page_size, page_stride, num_heads, num_kv_heads, head_dim, act, runs=runs,
@@ -953,11 +954,11 @@ def _gemm_problem(k: str, a, w, act, bias, w2, out_act, a_rows, tile_group, n_ti
 
 # Plain bfloat16 products of many rows may go through the vendor's matrix library (hipBLASLt behind torch.mm), as the
 # reference's engine hands its plain products to a BLAS where it has one
-# (/root/reference/src/engine/tq_ops.c:296-305): measured on gfx950 it is 25 to 35 % faster than the tile kernel here
-# from 512 rows on ([2048, 2048] x [6144, 2048]: 48 against 63 us; 13,199 rows: 282 against 401), slower or equal
-# below and where k is long and the rows are not many ([4096, 20480] x [3584, 20480]: 724 against 687 us).  A call
+# (/root/reference/src/engine/tq_ops.c:296-305): measured on gfx950 it is level with this library's best tiles where its own divide
+# the result evenly, and ahead of them from some thousand rows down ([2048, 2048] x [6144, 2048]: 47 against 53 us, [768, 2048] x
+# [2048, 2048] 14 against 21); where this library is the faster one (``tq_gemm_here_rather``, with both sides' times) a product stays.  A call
 # into the library costs the host twice what a launch here costs, and a step of 512 to 767 rows is as long on the
-# host as on the chip (24 layers of 512 tokens: 9.7 ms through the library, 7.9 without), so it starts at 768 rows.
+# host as on the chip, so it starts at 768 rows.
 # TQ_PLAIN_PRODUCTS=own keeps every product in this library's kernels.  Products over experts, gated pairs whose
 # matrices lie apart, products with a bias that nothing behind them can add, products of few rows, decode steps,
 # steps under graph capture and the 32-bit path never leave them.
@@ -987,6 +988,12 @@ def _vendor_product(act, a, w, M: int, K: int) -> bool:
     return (_VENDOR and M >= VENDOR_MIN_ROWS and (K < 16384 or M >= 8192) and dtype_name(act) == "bfloat16"
             and w.dtype == torch.bfloat16 and a.stride(1) == 1 and w.is_contiguous()
             and not torch.cuda.is_current_stream_capturing())
+
+
+def _vendor_here(act, a, w, M: int, N: int, K: int, kind: int = 0) -> bool:
+    """Whether a product goes to the vendor's library: it may, and this library's tiles are not the faster ones (``kind`` 0: plain, 1: an
+    activation alone, 2: a gated pair; csrc/gemm_mfma.hip has the rule and both sides' times)."""
+    return _vendor_product(act, a, w, M, K) and not library(act).tq_gemm_here_rather(M, N, K, kind)
 
 
 def _vendor_gemm(a, w, out_act: bool) -> torch.Tensor:
@@ -1093,7 +1100,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
                              gather=gather), None, activation, act)
     if act_alone:
         _need(w2 is None and not partial_sums and not grouped and a_rows is None, k, "an activation alone is for plain products")
-        if (dtype_name(act) == "bfloat16" and not (bias is None and _vendor_product(act, a, w, M, K))
+        if (dtype_name(act) == "bfloat16" and not (bias is None and _vendor_here(act, a, w, M, N, K, 1))
                 and _use_mfma(act, a, w, K) and (bias is None or bias.dtype in _WTYPE)):
             out = torch.empty((M, N), dtype=adt, device=a.device)
             _run("gemm_mfma", lib.tq_gemm_mfma(_ptr(a), a.stride(0), None, 1, _ptr(w), None, gstride, None, None, _ptr(bias),
@@ -1101,11 +1108,11 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
                                                tile_rows, 1, gate + 256, _stream()))
             return out
         return act_rows(gemm(a, w, act, bias=bias), None, activation, act)
-    if not grouped and a_rows is None and bias is None and _vendor_product(act, a, w, M, K):
-        if w2 is None:
+    if not grouped and a_rows is None and bias is None:
+        if w2 is None and _vendor_here(act, a, w, M, N, K):
             out = _vendor_gemm(a, w, out_act)
             return out[None] if partial_sums else out
-        if out_act and _behind(w, w2):
+        if w2 is not None and out_act and _behind(w, w2) and _vendor_here(act, a, w, M, N, K, 2):
             return _vendor_gated(a, w, N, K, gate, act)
     if _use_mfma(act, a, w, K) and (bias is None or bias.dtype in _WTYPE):
         splits = lib.tq_gemm_mfma_splits(M, N, K) if partial_sums else 1
