@@ -201,3 +201,48 @@ def test_runs_of_k_of_one_matrix(ops):
             x, y = a[:, z * per:(z + 1) * per].double(), w[:, z * per:(z + 1) * per].double()
             want = x @ y.T + (bias.double() if z == 0 else 0.0)
             assert ((got[z].double() - want).abs() <= (per + 4) * 2.0 ** -24 * (x.abs() @ y.abs().T + bias.double().abs())).all()
+
+
+# tiles: fewer than the chip's compute units, some for each of them, and crowded experts that leave one die with more than the others
+@pytest.mark.parametrize("counts,N", [([70] * 5, 300), ([130, 1, 64, 200] * 20, 1300), ([2900] + [65] * 30, 1300), ([300] * 9 + [0] * 40 + [60], 4100)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_tiles_dealt_from_a_queue(ops, counts, N, gated):
+    """An order's first two products take their tiles from its queues, a third one a tile to a workgroup, in a captured graph all of
+    them: the same results, alone and with another product beside, which the order's next use of its memory does not change."""
+    K = 320
+    st, _slot, te, nt = order(ops, counts)
+    live, T = st >= 0, sum(counts)
+    x, w = drawn((T, K), 1), drawn((len(counts), N, K), 2, 0.1)
+    form = dict(w2=drawn(w.shape, 3, 0.1), out_act=True) if gated else dict()
+    run = lambda nt, rows: ops.gemm(x, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=rows, **form)[live]
+    want = run(nt, 64)
+    assert nt.queues.left == [2, 1]
+    for left in ([2], [], []):
+        assert torch.equal(run(nt, 64 + ops.TILE_PAIRS), want) and nt.queues.left == left
+    assert torch.equal(run(nt.clone(), 64 + ops.TILE_PAIRS), want)      # numbers without queues
+    for _ in range(3):
+        nt = order(ops, counts)[3]
+        a, b = drawn((700, 128), 6), drawn((N, 128), 7, 0.1)
+        first = dict(a=x, w=w, a_rows=st, tile_group=te, n_tiles=nt, tile_rows=64 + ops.TILE_PAIRS, **form)
+        second = dict(a=a, w=b, **(dict(w2=drawn(b.shape, 8, 0.1), out_act=True) if gated else {}))
+        y1, y2 = ops.gemm_pair(first, dict(second), "bfloat16")
+        assert nt.queues.left == [2] and torch.equal(y1[live], want)
+        assert torch.equal(y2, ops.gemm(second.pop("a"), second.pop("w"), "bfloat16", **second))
+    nt = order(ops, counts)[3]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.gemm(x, w, "bfloat16", a_rows=st, tile_group=te, n_tiles=nt, tile_rows=64 + ops.TILE_PAIRS, **form)
+    assert nt.queues.left == [2, 1]
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(got[live], want)
+
+
+def test_what_names_no_queue_is_refused(ops):
+    st, _slot, te, nt = order(ops, [70])
+    h, w, out = drawn((st.numel(), 128), 1), drawn((1, 64, 128), 2), torch.empty((st.numel(), 64), device=DEV)
+    call = lambda rows: ops.library("bfloat16").tq_gemm_mfma(h.data_ptr(), 128, st.data_ptr(), 0, w.data_ptr(), None, 64 * 128, te.data_ptr(), nt.data_ptr(),
+                                                            None, 0, out.data_ptr(), 64, 0, st.numel(), 64, 128, rows, 1, 0, torch.cuda.current_stream().cuda_stream)
+    assert call(64 + ops.TILE_QUEUE) != 0 and call(64 + ops.TILE_PAIRS + 3 * ops.TILE_QUEUE) != 0

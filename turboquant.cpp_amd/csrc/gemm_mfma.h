@@ -75,6 +75,6 @@ __device__ __forceinline__ void load_to_lds16(const bf16_t* src, bf16_t* wave_ba
 }
 
 // gemm_phases.hip: products of many rows (K a multiple of TBK, 2 TBK and more) with a matrix per expert, by the row order's items; g2 (or
-// null): another of one matrix in the same launch, whose k may be in runs of k_per
-int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, bool dual, bool out_act, hipStream_t st);
+// null): another of one matrix in the same launch, whose k may be in runs of k_per; queue: eight zeros, for this launch alone, or null
+int launch_gemm_phases(const MfmaGemmArgs& g, const MfmaGemmArgs* g2, int* queue, bool dual, bool out_act, hipStream_t st);
 int launch_gemm_phases_plain(const MfmaGemmArgs& g, int rows, bool dual, bool out_act, hipStream_t st);

@@ -1101,10 +1101,20 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
   return s;
 }
 
+// The queue that tile_rows names, or null, and tile_rows without it; false: what cannot be.
+static bool take_queue(int& tile_rows, const int* n_tiles, int** queue) {
+  const int which = tile_rows / TQ_TILE_QUEUE;
+  *queue = nullptr;
+  if (tile_rows < TQ_TILE_QUEUE) return true;
+  tile_rows %= TQ_TILE_QUEUE;
+  *queue = const_cast<int*>(n_tiles) + 16 * which;
+  return which <= 2 && n_tiles && tile_rows == 64 + TQ_TILE_PAIRS;
+}
+
 // a: bfloat16 [.., K] with row stride lda (a multiple of 8, as K must be); w, w2: bfloat16.
 // tile_rows: with tile_group set, the padding unit of the row order (16, 32, 64, 128 or 256); else a hint that is
 // ignored.  64 + TQ_TILE_PAIRS: units of 64 taken two or four at a time, by the items that the row order lists behind its
-// row tiles (tile_group[M / 64 ..], n_tiles[1]).
+// row tiles (tile_group[M / 64 ..], n_tiles[1]); with TQ_TILE_QUEUE once or twice on top, dealt from the order's first or second queue.
 // splits > 1 (as tq_gemm_mfma_splits says, for a plain product into float): run z of k goes to out + z * M * ldc,
 // the bias to run 0; the sum over the runs is the caller's.
 // gate: the activation of the gated pair; without w2 and with TQ_GEMM_ACT_ALONE added, the activation that the plain
@@ -1124,6 +1134,8 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
   if (splits > 1 && (dual || out_act || tile_group || a_rows || splits != tq_gemm_mfma_splits(M, N, K))) return TQ_ERR_BAD_ARG;
   const int k_per = ((K + TBK - 1) / TBK + splits - 1) / splits * TBK;
   if (splits > 1 && (int64_t)(splits - 1) * k_per >= K) return TQ_ERR_BAD_ARG;
+  int* queue;
+  if (!take_queue(tile_rows, n_tiles, &queue)) return TQ_ERR_BAD_ARG;
   MfmaGemmArgs g{(const bf16_t*)a, lda, a_rows, a_gather, (const bf16_t*)w, (const bf16_t*)w2, group_stride,
                  tile_group, n_tiles, bias, bias_type, out, ldc, M, N, K, splits > 1 ? k_per : K, (int64_t)M * ldc, gate, 1,
                  alone ? gate + 1 : 0, tq_pair_limit_host};
@@ -1138,7 +1150,7 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
     } else if (tile_rows == 64 || tile_rows == 64 + TQ_TILE_PAIRS) {
       if ((N + TBN - 1) / TBN > 65535 || M % 64) return TQ_ERR_UNSUPPORTED;
       if (tile_rows != 64 && K % TBK == 0 && K >= 2 * TBK)
-        rc = launch_gemm_phases(g, nullptr, dual, out_act, st);
+        rc = launch_gemm_phases(g, nullptr, queue, dual, out_act, st);
       else
         rc = launch_tile<64, 2, 4>(g, dual, out_act, 1, st);
     } else if (tile_rows == 128) {     // experts with hundreds of rows each: the taller tile's rate for little padding
@@ -1222,7 +1234,7 @@ TQ_API int tq_gemm_phases_pair_splits(int M1, int N1, int K1, int M2, int N2, in
 // both not, both into the same type.  Either
 //  * few rows: both products that the streaming kernel takes 16 rows at a time (a matrix per expert with tile_rows 16, or
 //    one matrix with M <= 16).  The waves that split k are those of the first product (the larger one by convention);
-//  * or many, where tile_rows of the first is 64 + TQ_TILE_PAIRS: the first over experts by the row order's items, the second
+//  * or many, where tile_rows of the first is 64 + TQ_TILE_PAIRS (and a queue, as above): the first over experts by the row order's items, the second
 //    of one matrix whose rows follow one another, k of either a multiple of 64 and 128 and more (gemm_phases.hip).
 // splits2 > 1 (as tq_gemm_mfma_pair_splits says of few rows and tq_gemm_phases_pair_splits of many, for a plain second
 // product into float): run z of its k goes to out + z * M * ldc, the bias to run 0.
@@ -1231,7 +1243,10 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
   int row_tiles[2];
   bool dual[2], out_act[2];
   const int64_t* d[2] = {d1, d2};
-  const bool many = d1[17] == 64 + TQ_TILE_PAIRS;
+  int tile_rows1 = (int)d1[17];
+  int* queue;
+  if (!take_queue(tile_rows1, (const int*)d1[8], &queue)) return TQ_ERR_BAD_ARG;
+  const bool many = tile_rows1 == 64 + TQ_TILE_PAIRS;
   for (int i = 0; i < 2; ++i) {
     const int64_t* p = d[i];
     const int M = (int)p[14], N = (int)p[15], K = (int)p[16], tile_rows = (int)p[17];
@@ -1266,7 +1281,7 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
       g[1].k_per = (g[1].K / TBK + splits2 - 1) / splits2 * TBK;
       g[1].split_stride = (int64_t)g[1].M * g[1].ldc;
     }
-    if (const int rc = launch_gemm_phases(g[0], &g[1], dual[0], out_act[0], st)) return rc;
+    if (const int rc = launch_gemm_phases(g[0], &g[1], queue, dual[0], out_act[0], st)) return rc;
     TQ_LAUNCH_CHECK();
     return 0;
   }

@@ -218,7 +218,7 @@ void pair_desc(const Product& p, void* out, int tile_rows, int64_t* d) {
 // Whether a product over experts by items of several units and one of one matrix go out together (mirrors ops.gemm_pair).
 bool tiles_together(const Product& p1, const Product& p2) {
   auto suits = [](const Product& p) { return use_mfma(p.w, p.K) && p.K % 64 == 0 && p.K >= 128; };
-  return p1.tile_group && p1.tile_rows == 64 + TQ_TILE_PAIRS && !p2.tile_group && !p2.a_rows && p2.M >= 64 && suits(p1) && suits(p2);
+  return p1.tile_group && p1.tile_rows % TQ_TILE_QUEUE == 64 + TQ_TILE_PAIRS && !p2.tile_group && !p2.a_rows && p2.M >= 64 && suits(p1) && suits(p2);
 }
 
 // Two products that do not depend on each other; mirrors ops.gemm_pair (only the second may leave partial sums).
@@ -391,7 +391,7 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   int* sorted_token = (int*)c.arena.take((size_t)cap * 4);
   int* pair_slot = (int*)c.arena.take((size_t)n_pairs * 4);
   int* tile_expert = (int*)c.arena.take((size_t)(cap / unit) * 2 * 4);      // row tiles, then items
-  int* n_tiles = (int*)c.arena.take(2 * 4);
+  int* n_tiles = (int*)c.arena.take(48 * 4);      // two numbers and, from the 16th on, two queues
   auto route = [&]() -> int {
     RUN(c, "route",
         tq_route(normed32, f.router.ptr, gated ? f.shared_scale.ptr : nullptr, (int)f.router.wtype, E, k, (int)f.renormalize,
@@ -413,7 +413,8 @@ int moe_ffn(Ctx& c, const tq_moe_ffn_desc& f, const void* normed, const float* n
   *pending = Pending();
   pending->pair_slot = pair_slot, pending->weights = weights, pending->topk = k, pending->gate = gate;
   const bool beside = Is > 0 && tiles_together(eg, sg) && tiles_together(ed, sd);
-  if (rows != unit) {      // how many units an item holds (ops.expert_item_units)
+  if (rows != unit) {      // how many units an item holds (ops.expert_item_units), and a queue of tiles for either product
+    if (bf16_path()) order_unit += TQ_ORDER_QUEUES, eg.tile_rows += TQ_TILE_QUEUE, ed.tile_rows += 2 * TQ_TILE_QUEUE;
     const int64_t tiles = n_pairs * ((I + 127) / 128) / 256;
     if ((beside || tiles >= 256) && n_pairs >= (beside || tiles >= 450 ? 88 : 112) * (int64_t)E) order_unit += TQ_ITEMS_OF_FOUR;
   }

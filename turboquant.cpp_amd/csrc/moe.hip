@@ -574,11 +574,20 @@ __device__ __forceinline__ void rank_segment(const int* ids, int seg_beg, int se
   }
 }
 
+// A wave zeroes the queues behind n_tiles, if there are any, and takes what says so off the row tiles of an item.
+#define TQ_WITH_QUEUES 256
+__device__ __forceinline__ void clear_queues(int* __restrict__ n_tiles, int& per_item) {
+  if (!(per_item & TQ_WITH_QUEUES)) return;
+  per_item -= TQ_WITH_QUEUES;
+  if (threadIdx.x % TQ_WAVE < 32) n_tiles[16 + threadIdx.x % TQ_WAVE] = 0;
+}
+
 // Wave 0 of a workgroup turns the experts' padded sizes starts[e] into their first rows (an exclusive scan, each lane
 // a contiguous run of experts) and writes the row tiles' experts, the items and their numbers.
 __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int per_item, int cap,
                                             int* __restrict__ tile_expert, int* __restrict__ n_tiles) {
   const int lane = threadIdx.x % TQ_WAVE;
+  clear_queues(n_tiles, per_item);
   {
     const int chunk = (E + TQ_WAVE - 1) / TQ_WAVE;
     const int e0 = lane * chunk, e1 = min(E, e0 + chunk);
@@ -853,6 +862,7 @@ __global__ __launch_bounds__(64 * NW) void select_align_kernel(const float* __re
           }
         }
         for (int i = lane; i < cap; i += TQ_WAVE) sorted_token[i] = i < n * unit && i % unit == 0 ? 0 : -1;
+        clear_queues(n_tiles, per_item);
         if (lane == 0) n_tiles[0] = n_tiles[1] = n;
         return;
       }
@@ -873,11 +883,13 @@ __global__ __launch_bounds__(64 * NW) void select_align_kernel(const float* __re
   align_pairs<NW>(ids_l, T * topk, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, cnt, n_real);
 }
 
-// Row tiles that an item holds at most; takes TQ_ITEMS_OF_FOUR off `unit`.
+// Row tiles that an item holds at most, with TQ_WITH_QUEUES where there are queues to zero; takes TQ_ITEMS_OF_FOUR and TQ_ORDER_QUEUES
+// off `unit`.
 static int units_per_item(int& unit) {
-  if (unit < TQ_ITEMS_OF_FOUR) return 2;
-  unit -= TQ_ITEMS_OF_FOUR;
-  return 4;
+  int per_item = 2;
+  if (unit >= TQ_ITEMS_OF_FOUR) unit -= TQ_ITEMS_OF_FOUR, per_item = 4;
+  if (unit >= TQ_ORDER_QUEUES) unit -= TQ_ORDER_QUEUES, per_item += TQ_WITH_QUEUES;
+  return per_item;
 }
 
 // cap: rows that sorted_token holds, a multiple of unit and at least n_pairs + min(E, n_pairs) * (unit - 1);

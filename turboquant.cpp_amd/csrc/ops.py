@@ -843,6 +843,8 @@ EXPERT_16_UPTO, EXPERT_32_UPTO = 5, 10
 # time do better wherever the taller units did (see expert_tile_rows); tests lower them to run those kernels.
 EXPERT_128_FROM = EXPERT_256_FROM = 1 << 30
 TILE_PAIRS = 1024            # added to tile_rows 64: the units of an item, two or four of one expert, per workgroup (TQ_TILE_PAIRS)
+TILE_QUEUE = 2048            # added to that once or twice: the tiles are dealt from the order's first or second queue (TQ_TILE_QUEUE)
+ORDER_QUEUES = 1 << 29       # added to the row order's unit: two queues behind n_tiles, which the order zeroes (TQ_ORDER_QUEUES)
 ITEMS_OF_FOUR = 1 << 30      # added to the row order's unit: its items hold four row tiles instead of two (TQ_ITEMS_OF_FOUR)
 ITEMS_OF_FOUR_FROM = 112, 88 # rows per expert on average from which items may hold four units, by expert_item_units
 EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken several at a time
@@ -1094,7 +1096,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
             _run("gemm_mfma", lib.tq_gemm_mfma(_ptr(a), a.stride(0), _ptr(a_rows), int(gather), _ptr(w), None, gstride,
                                                _ptr(tile_group), _ptr(n_tiles), _ptr(bias),
                                                _WTYPE[bias.dtype] if bias is not None else 0, _ptr(out), N, 1, M, N, K,
-                                               tile_rows, 1, gate + 256, _stream()), "moe" if grouped else None)
+                                               _tile_queue(tile_rows, n_tiles), 1, gate + 256, _stream()), "moe" if grouped else None)
             return out
         return act_rows(gemm(a, w, act, bias=bias, a_rows=a_rows, tile_group=tile_group, n_tiles=n_tiles, tile_rows=tile_rows,
                              gather=gather), None, activation, act)
@@ -1121,7 +1123,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
         _run("gemm_mfma", lib.tq_gemm_mfma(_ptr(a), a.stride(0), _ptr(a_rows), int(gather), _ptr(w), _ptr(w2), gstride,
                                            _ptr(tile_group), _ptr(n_tiles), _ptr(bias),
                                            _WTYPE[bias.dtype] if bias is not None else 0, _ptr(out), N, int(out_act),
-                                           M, N, K, tile_rows, splits, gate, _stream()), "moe" if grouped else None)
+                                           M, N, K, _tile_queue(tile_rows, n_tiles), splits, gate, _stream()), "moe" if grouped else None)
         return out
     if _use_f32(act, a, w, K, gstride) and (w2 is None or w2.data_ptr() % 16 == 0):
         # a narrow matrix times few rows is cut into runs of k: they come back apart if the caller adds them up
@@ -1195,7 +1197,7 @@ def gemm_pair(first: dict, second: dict, act) -> tuple[torch.Tensor, torch.Tenso
         outs.append(out)
         vals = [_ptr(p["a"]), p["a"].stride(0), _ptr(p["a_rows"]), int(p["gather"]), _ptr(p["w"]), _ptr(p["w2"]), gstride,
                 _ptr(p["tile_group"]), _ptr(p["n_tiles"]), _ptr(p["bias"]),
-                _WTYPE[p["bias"].dtype] if p["bias"] is not None else 0, _ptr(out), N, int(p["out_act"]), M, N, K, tile_rows,
+                _WTYPE[p["bias"].dtype] if p["bias"] is not None else 0, _ptr(out), N, int(p["out_act"]), M, N, K, _tile_queue(tile_rows, p["n_tiles"]),
                 _gate_code(k, p["activation"]), struct.unpack("<I", struct.pack("<f", p["pair_limit"] or 0.0))[0]]
         descs.append((ctypes.c_int64 * 20)(*[0 if v is None else int(v) for v in vals]))
     _run(k, lib.tq_gemm_mfma_pair(descs[0], descs[1], splits, _stream()),
@@ -1400,8 +1402,36 @@ def _align_outputs(T: int, topk: int, num_experts: int, unit: int, dev):
     sorted_token = torch.empty((cap,), dtype=torch.int32, device=dev)
     pair_slot = torch.empty((T, topk), dtype=torch.int32, device=dev)
     tile_expert = torch.empty((2 * (cap // unit),), dtype=torch.int32, device=dev)      # row tiles, then items
-    n_tiles = torch.empty((2,), dtype=torch.int32, device=dev)
+    n_tiles = torch.empty((48 if unit == 64 else 2,), dtype=torch.int32, device=dev)
+    if unit == 64:
+        whole, n_tiles = n_tiles, n_tiles[:2]
+        n_tiles.queues = TileQueues(whole)
     return cap, sorted_token, pair_slot, tile_expert, n_tiles
+
+
+class TileQueues:
+    """What the products over experts of one row order take their tiles from in turn (csrc/gemm_phases.hip): two queues that the
+    order's kernels zero, behind the two numbers of ``n_tiles``, whose attribute ``queues`` this is.  A queue serves one
+    launch, so a product under graph capture, which may run any number of times, takes none."""
+
+    def __init__(self, whole: torch.Tensor):
+        self.whole = whole                      # int32 [48], the queues from the 16th on
+        self.left = [2, 1]
+
+    def take(self) -> int:
+        """What is added to a product's ``tile_rows``: TILE_QUEUE or twice that, 0 where no queue is left."""
+        if torch.cuda.is_current_stream_capturing():
+            return 0
+        try:
+            return self.left.pop() * TILE_QUEUE
+        except IndexError:
+            return 0
+
+
+def _tile_queue(tile_rows: int, n_tiles: torch.Tensor | None) -> int:
+    """``tile_rows`` as the matrix-core product is called with it, a queue of the order's with it if there is one."""
+    queues = getattr(n_tiles, "queues", None) if tile_rows == 64 + TILE_PAIRS else None
+    return tile_rows if queues is None else tile_rows + queues.take()
 
 
 def route(x32: torch.Tensor, router: torch.Tensor, shared_scale: torch.Tensor | None, top_k: int, renormalize: bool,
@@ -1470,9 +1500,10 @@ class RowUnit(int):
 
 
 def _order_unit(k: str, unit: int, item_units: int) -> int:
-    """The ``unit`` that the library is told, with how many row tiles an item holds at most (ITEMS_OF_FOUR)."""
+    """The ``unit`` that the library is told, with how many row tiles an item holds at most (ITEMS_OF_FOUR) and whether there are
+    queues to zero behind ``n_tiles`` (``_align_outputs``)."""
     _need(item_units in (2, 4), k, "an item holds up to 2 or 4 row tiles")
-    return unit + ITEMS_OF_FOUR if item_units == 4 else unit
+    return unit + (ITEMS_OF_FOUR if item_units == 4 else 0) + (ORDER_QUEUES if unit == 64 else 0)
 
 
 def moe_align(ids: torch.Tensor, num_experts: int, unit: int, act, item_units: int = 2):

@@ -17,6 +17,8 @@
 // added to a tile_rows of 64 of a product over experts: the units that the row order's items hold, two or four of one
 // expert, per workgroup (see tq_gemm_mfma)
 #define TQ_TILE_PAIRS 1024
+#define TQ_TILE_QUEUE 2048             /* added to that once or twice: its tiles are dealt from the order's first or second queue, one product each */
+#define TQ_ORDER_QUEUES (1 << 29)      /* added to the unit of the order of pairs by expert: n_tiles holds 48 ints, the last 32 of them two queues, which it zeroes */
 #define TQ_ITEMS_OF_FOUR (1 << 30)      /* added to the unit of the order of pairs by expert: its items hold four row tiles, not two */
 #define TQ_GEMM_ACT_ALONE 256      // added to tq_gemm_mfma's gate: the activation of a plain product's result
 
