@@ -246,3 +246,26 @@ def test_what_names_no_queue_is_refused(ops):
     call = lambda rows: ops.library("bfloat16").tq_gemm_mfma(h.data_ptr(), 128, st.data_ptr(), 0, w.data_ptr(), None, 64 * 128, te.data_ptr(), nt.data_ptr(),
                                                             None, 0, out.data_ptr(), 64, 0, st.numel(), 64, 128, rows, 1, 0, torch.cuda.current_stream().cuda_stream)
     assert call(64 + ops.TILE_QUEUE) != 0 and call(64 + ops.TILE_PAIRS + 3 * ops.TILE_QUEUE) != 0
+
+
+def test_the_gate_over_its_whole_range(ops):
+    """silu in the tiles' epilogue against the tile kernel's, to the last bit of the 16-bit result but where a rounding is near: factors
+    that make every product one value from -1e5 to 1e5, among them those where the exponential leaves the range, zeros, infinities and NaN."""
+    x = torch.cat([torch.linspace(-100, 100, 4097), torch.tensor([0.0, -0.0, 86.9, 87.1, -86.9, -87.1, -88.8, 1e5, -1e5, 1e-30, -1e-38, float("inf"), float("-inf"), float("nan")])])
+    M, K, N = 1280, 128, 264
+    a = torch.zeros(M, K)
+    a[:, 0] = 1.0
+    w = torch.zeros(N, K)
+    w[:, 0] = x[torch.arange(N) * 16 % 4097]
+    w[-14:, 0] = x[-14:]
+    w2 = torch.zeros(N, K)
+    w2[:, 0] = 1.0
+    a, w, w2 = (t.to(torch.bfloat16).to(DEV) for t in (a, w, w2))
+    every = torch.arange(M, dtype=torch.int32, device=DEV)
+    got = ops.gemm(a, w, "bfloat16", w2=w2, out_act=True)
+    want = ops.gemm(a, w, "bfloat16", w2=w2, out_act=True, a_rows=every)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+    z = w[:, 0].double().cpu()
+    exact = (z * torch.sigmoid(z)).expand(M, N)
+    finite = exact.isfinite() & (z.abs() < 87)
+    assert ((got.cpu().double() - exact).abs() <= exact.abs() * 2.0 ** -8 + 1e-40)[finite].all()

@@ -16,15 +16,17 @@
 // One workgroup fills a compute unit's LDS, so what stands between two tiles has nothing to hide behind: the end of a workgroup and the
 // start of the next (1.9 us on average, 5.8 for one in ten), the search for its tile (0.9), the first loads' way (3).  An order of rows has
 // queues for that (PhaseTiles): a workgroup stays, and a die that is through helps the others: 2,048 tokens by 4 of 60 experts of 1,408 x
-// 2,048 beside a shared one of 5,632 260 -> 244 us.  And with w as the products'
-// first operand a lane ends with columns side by side, and the outputs go from the registers into stores of 16 bytes a lane.
+// 2,048 beside a shared one of 5,632 260 -> 244 us.  With w as the products'
+// first operand a lane ends with columns side by side, and the outputs go from the registers into stores of 16 bytes a lane.  What is left
+// of an end is the gate's arithmetic, 31 instructions a value as expf, a division and a rounding by integers make it, 9.5 us a tile of 256 x
+// 128 beside 39 of its steps: 19 now (silu_within, f32_to_bf16), 244 -> 240 us there, 6,250 -> 6,053 at the size below.
 // What the matrix instructions cost is power: on random values the chip runs 32x32x16 products alone at 1,858 TFLOP/s and 16x16x32
 // products at 2,183 (1.7 GHz in this kernel either way, where 2.4 is the peak), so these are the small ones.  They add k in groups of
 // eight, one behind the other, as the large ones do: same bits.
 // Measured, us, with items of two units by 16 waves through a ring of three stages, then these tiles by 32x32x16 products and outputs
 // through LDS, then as it is: 13,197 tokens by 8 of 64 experts of 2,560 x 3,584 beside a shared expert of 20,480, gated pairs 7,551 ->
-// 6,334 (1,223 TFLOP/s), second products 3,496 -> 3,051 (the experts alone 4,760 -> 3,739 and 2,590 -> 1,943 before); 2,048 tokens by 4
-// of 60 experts of 1,408 x 2,048 beside one of 5,632 293 -> 260 and 165 -> 154 (the experts alone 219 -> 173 and 147 -> 103 before).
+// 6,053 (1,280 TFLOP/s), second products 3,496 -> 3,041 (the experts alone 4,760 -> 3,739 and 2,590 -> 1,943 before); 2,048 tokens by 4
+// of 60 experts of 1,408 x 2,048 beside one of 5,632 293 -> 240 and 165 -> 155 (the experts alone 219 -> 173 and 147 -> 103 before).
 // Products of one matrix (`launch_gemm_phases_plain`) take the same tiles, 64 to 256 rows high as the compute units fill best; gemm_mfma.hip
 // has the rules and what they replace (2,048 rows by 2,048 columns with a bias, k 2,048, 62 -> 27 us; 3,001 by 3,072 99 -> 43).
 #include "common.h"
@@ -49,9 +51,37 @@ __device__ __forceinline__ void loads_left() {      // at most N loads of this w
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// x / (1 + exp(-x)) of N values, none of them beyond 87 in size: the exponential as expf does it there, without its tests for the ends of
+// the range, and the quotient by a reciprocal that one step sharpens and the remainder, which is exact, corrects (within 0.5 of the last
+// place but for one in some millions; over all floats of that range 0.281 of the last place off 64 bits in the root of the mean square,
+// as with a division).  17 instructions instead of 25.
+template <int N>
+__device__ __forceinline__ void silu_within(float (&v)[N]) {
+#pragma clang fp contract(off)      // (p - n is to be of the rounded p, whose rest stands apart)
+  constexpr float LOG2E = 1.44269504088896341f, LOG2E_REST = 1.92596299112661746e-8f;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float x = v[j], p = -x * LOG2E, rest = fmaf(-x, LOG2E_REST, fmaf(-x, LOG2E, -p)), n = rintf(p);
+    const float d = 1.0f + ldexpf(__builtin_amdgcn_exp2f((p - n) + rest), (int)n);
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    const float q = x * r;
+    v[j] = fmaf(fmaf(-d, q, x), r, q);
+  }
+}
+
 // v[j] = f(v[j]), the switch once for all of them
 template <int N>
 __device__ __forceinline__ void gate_many(float (&v)[N], int kind) {
+  if (kind == TQ_GATE_silu) {
+    float far = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) far = fmaxf(far, fabsf(v[j]));
+    if (!__any(!(far < 87.f))) {
+      silu_within(v);
+      return;
+    }
+  }
   switch (kind) {
 #define TQ_GATE(name, expr)                          \
   case TQ_GATE_##name:                               \
@@ -314,12 +344,12 @@ __device__ __forceinline__ void phase_store(const PhaseOut& g, const f32x4 (&acc
           if (wide) {
             u32x4 packed;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) packed[k] = f32_to_bf16(v[2 * k]).bits | (unsigned)f32_to_bf16(v[2 * k + 1]).bits << 16;
+            for (int k = 0; k < 4; ++k) packed[k] = f32_to_bf16_pair(v[2 * k], v[2 * k + 1]);
             *reinterpret_cast<u32x4*>(o) = packed;
           } else if (even) {
 #pragma unroll
             for (int k = 0; k < V; k += 2)
-              if (col + k < g.N) *reinterpret_cast<unsigned*>(o + k) = f32_to_bf16(v[k]).bits | (unsigned)f32_to_bf16(v[k + 1]).bits << 16;
+              if (col + k < g.N) *reinterpret_cast<unsigned*>(o + k) = f32_to_bf16_pair(v[k], v[k + 1]);
           } else {
 #pragma unroll
             for (int k = 0; k < V; ++k)

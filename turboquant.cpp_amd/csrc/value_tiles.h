@@ -14,8 +14,8 @@ __device__ __forceinline__ f32x4 load4f(const bf16_t* p) {
 __device__ __forceinline__ void store4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ void store4(bf16_t* p, f32x4 v) {
   uint2 u;
-  u.x = (uint32_t)f32_to_bf16(v.x).bits | ((uint32_t)f32_to_bf16(v.y).bits << 16);
-  u.y = (uint32_t)f32_to_bf16(v.z).bits | ((uint32_t)f32_to_bf16(v.w).bits << 16);
+  u.x = f32_to_bf16_pair(v.x, v.y);
+  u.y = f32_to_bf16_pair(v.z, v.w);
   *reinterpret_cast<uint2*>(p) = u;
 }
 
