@@ -20,8 +20,8 @@
 // added to the unit of the order of pairs by expert: its items hold four row tiles instead of two (see moe.hip).  Above every unit:
 // a unit of rows may be any number whose rows fit the order.
 #define TQ_ITEMS_OF_FOUR (1 << 30)
-// The row order's n_tiles may hold more than its two numbers, 48 in all, of which the last 32, two runs of 16, are queues: zeroed with the
-// order where TQ_ORDER_QUEUES is added to its unit, each for one product (tile_rows with TQ_TILE_QUEUE added once or twice) behind it.
+// The row order's n_tiles may hold more than its two numbers, 48 in all, of which the last 32, two runs of 16, are queues: written with the
+// order (and the third, the experts that have rows) where TQ_ORDER_QUEUES is added to its unit, each for one product (tile_rows with TQ_TILE_QUEUE added once or twice) behind it.
 #define TQ_ORDER_QUEUES (1 << 29)
 #define TQ_TILE_QUEUE 2048
 #define TQ_GEMM_ACT_ALONE 256      // added to tq_gemm_mfma's gate: the activation of a plain product's result

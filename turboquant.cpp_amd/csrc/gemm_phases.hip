@@ -19,13 +19,13 @@
 // 2,048 beside a shared one of 5,632 260 -> 244 us.  With w as the products'
 // first operand a lane ends with columns side by side, and the outputs go from the registers into stores of 16 bytes a lane.  What is left
 // of an end is the gate's arithmetic, 31 instructions a value as expf, a division and a rounding by integers make it, 9.5 us a tile of 256 x
-// 128 beside 39 of its steps: 19 now (silu_within, f32_to_bf16), 244 -> 240 us there, 6,250 -> 6,053 at the size below.
+// 128 beside 39 of its steps: 19 now (silu_within, f32_to_bf16), 244 -> 240 us there.
 // What the matrix instructions cost is power: on random values the chip runs 32x32x16 products alone at 1,858 TFLOP/s and 16x16x32
 // products at 2,183 (1.7 GHz in this kernel either way, where 2.4 is the peak), so these are the small ones.  They add k in groups of
 // eight, one behind the other, as the large ones do: same bits.
 // Measured, us, with items of two units by 16 waves through a ring of three stages, then these tiles by 32x32x16 products and outputs
 // through LDS, then as it is: 13,197 tokens by 8 of 64 experts of 2,560 x 3,584 beside a shared expert of 20,480, gated pairs 7,551 ->
-// 6,053 (1,280 TFLOP/s), second products 3,496 -> 3,041 (the experts alone 4,760 -> 3,739 and 2,590 -> 1,943 before); 2,048 tokens by 4
+// 5,682 (1,363 TFLOP/s), second products 3,496 -> 3,041 (the experts alone 4,760 -> 3,739 and 2,590 -> 1,943 before); 2,048 tokens by 4
 // of 60 experts of 1,408 x 2,048 beside one of 5,632 293 -> 240 and 165 -> 155 (the experts alone 219 -> 173 and 147 -> 103 before).
 // Products of one matrix (`launch_gemm_phases_plain`) take the same tiles, 64 to 256 rows high as the compute units fill best; gemm_mfma.hip
 // has the rules and what they replace (2,048 rows by 2,048 columns with a bias, k 2,048, 62 -> 27 us; 3,001 by 3,072 99 -> 43).
@@ -553,6 +553,16 @@ __global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gy
   s.gx = g.tile_group ? min(g.n_tiles[1], g.M / 64) : 0;
   s.gy = gy, s.gx2 = gx2, s.gy2 = gy2, s.rows2 = rows2, s.first2 = first2, s.queue = queue;
   const int n1 = s.gx * gy;
+  if (queue) {
+    // Where the experts' matrices pass for many rows each, or for so few that nothing else counts, the second's tiles go first, all of
+    // them reading what their dies' L2 holds; between, where memory and the matrix instructions are about in balance (1,280 TFLOP/s
+    // against 5.5 TB/s: 230 rows), they are spread among those that wait for memory.  us spread and first, gated pairs of 60 experts of
+    // 1,408 x 2,048 beside one of 5,632: 60 rows each 191 and 179, 100 203 and 222, 137 241 and 253, 200 275 and 296, 260 361 and 369,
+    // 330 456 and 445, 1,650 1,848 and 1,795; 64 of 2,560 x 3,584 beside 20,480: 60 543 and 547, 137 713 and 751, 260 1,170 and 1,121,
+    // 1,650 6,190 and 5,688.
+    const int per_expert = s.n_units * 64 / max(g.n_tiles[2], 1);      // rows, padding among them
+    if (per_expert >= 270 || per_expert <= 100) s.first2 = 1;
+  }
   s.q1 = n1 / 8, s.rem1 = n1 % 8, s.q2 = n2 / 8, s.rem2 = n2 % 8;
   int die = blockIdx.x % 8, i = blockIdx.x / 8;
   if (queue) {

@@ -574,12 +574,14 @@ __device__ __forceinline__ void rank_segment(const int* ids, int seg_beg, int se
   }
 }
 
-// A wave zeroes the queues behind n_tiles, if there are any, and takes what says so off the row tiles of an item.
+// A wave zeroes the queues behind n_tiles (16..47; n_tiles[2] is the number of experts with rows then), if there are any, and takes what
+// says so off the row tiles of an item; false: there are none.
 #define TQ_WITH_QUEUES 256
-__device__ __forceinline__ void clear_queues(int* __restrict__ n_tiles, int& per_item) {
-  if (!(per_item & TQ_WITH_QUEUES)) return;
+__device__ __forceinline__ bool clear_queues(int* __restrict__ n_tiles, int& per_item) {
+  if (!(per_item & TQ_WITH_QUEUES)) return false;
   per_item -= TQ_WITH_QUEUES;
   if (threadIdx.x % TQ_WAVE < 32) n_tiles[16 + threadIdx.x % TQ_WAVE] = 0;
+  return true;
 }
 
 // Wave 0 of a workgroup turns the experts' padded sizes starts[e] into their first rows (an exclusive scan, each lane
@@ -587,13 +589,14 @@ __device__ __forceinline__ void clear_queues(int* __restrict__ n_tiles, int& per
 __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int per_item, int cap,
                                             int* __restrict__ tile_expert, int* __restrict__ n_tiles) {
   const int lane = threadIdx.x % TQ_WAVE;
-  clear_queues(n_tiles, per_item);
+  const bool queues = clear_queues(n_tiles, per_item);
   {
     const int chunk = (E + TQ_WAVE - 1) / TQ_WAVE;
     const int e0 = lane * chunk, e1 = min(E, e0 + chunk);
-    int sum = 0, isum = 0;
+    int sum = 0, isum = 0, live = 0;
     for (int e = e0; e < e1; ++e) {
       sum += starts[e];
+      live += starts[e] > 0;
       isum += (starts[e] / unit + per_item - 1) / per_item;
     }
     const int incl = wave_scan_add(sum), iincl = wave_scan_add(isum);
@@ -608,9 +611,11 @@ __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int pe
       }
       row += padded;
     }
+    const int used = queues ? wave_scan_add(live) : 0;
     if (lane == TQ_WAVE - 1) {
       n_tiles[0] = incl / unit;
       n_tiles[1] = iincl;
+      if (queues) n_tiles[2] = used;
     }
   }
 }
@@ -862,7 +867,7 @@ __global__ __launch_bounds__(64 * NW) void select_align_kernel(const float* __re
           }
         }
         for (int i = lane; i < cap; i += TQ_WAVE) sorted_token[i] = i < n * unit && i % unit == 0 ? 0 : -1;
-        clear_queues(n_tiles, per_item);
+        if (clear_queues(n_tiles, per_item) && lane == 0) n_tiles[2] = n;
         if (lane == 0) n_tiles[0] = n_tiles[1] = n;
         return;
       }
