@@ -71,20 +71,26 @@ __device__ __forceinline__ float group_sum(float v) {
 
 // One tile of 64 keys for 16 queries: scores from `kf` (reads the key operand of subtile kt, chunk u), softmax
 // update, and the product with the values from `vf` (value operand of d-tile dt, subtile kt).
-template <int ND, class KF, class VF>
+// SIDE: sums whose products take turns, so that none waits for the one before it (1: operands from memory, as few as may be in registers).
+template <int ND, int SIDE, class KF, class VF>
 __device__ __forceinline__ void attend_tile(const f32x4 (&qf)[ND], KF kf, VF vf, int key0, int pos_q, int lo_q, float scale,
                                             float cap, bool biased, float r1, float r2, int keep, bool sig, float pb,
                                             float& m_run, float& l_run, f32x4 (&acc)[ND]) {
   const int g = (threadIdx.x % 64) / 16;
   f32x4 s[4];
 #pragma unroll
-  for (int kt = 0; kt < 4; ++kt) {
-    s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < 4; k0 += SIDE) {
+#pragma unroll
+    for (int n = 0; n < SIDE; ++n) s[k0 + n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < ND; ++u) {
-      const f32x4 a = kf(kt, u);
+      f32x4 a[SIDE];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], qf[u][i], s[kt], 0, 0, 0);
+      for (int n = 0; n < SIDE; ++n) a[n] = kf(k0 + n, u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int n = 0; n < SIDE; ++n) s[k0 + n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][i], qf[u][i], s[k0 + n], 0, 0, 0);
     }
   }
   float m_tile = -INFINITY;
@@ -114,32 +120,46 @@ __device__ __forceinline__ void attend_tile(const f32x4 (&qf)[ND], KF kf, VF vf,
   const float alpha = m_run == -INFINITY ? 0.f : expf(m_run - m_new);
   l_run = l_run * alpha + l_tile;
   m_run = m_new;
+  constexpr int SV = SIDE < ND ? SIDE : ND;
 #pragma unroll
-  for (int dt = 0; dt < ND; ++dt) {
-    acc[dt] *= alpha;
+  for (int d0 = 0; d0 < ND; d0 += SV) {
+#pragma unroll
+    for (int n = 0; n < SV; ++n) acc[d0 + n] *= alpha;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      const f32x4 a = vf(dt, kt);
+      f32x4 a[SV];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], s[kt][i], acc[dt], 0, 0, 0);
+      for (int n = 0; n < SV; ++n) a[n] = vf(d0 + n, kt);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int n = 0; n < SV; ++n) acc[d0 + n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][i], s[kt][i], acc[d0 + n], 0, 0, 0);
     }
   }
 }
 
 // ------------------------------------------------------------------------------------------ runs of tokens
-template <int ND>
-__global__ __launch_bounds__(256) void attn_f32_prefill_kernel(AttnF32Args p, int blocks_per_seq) {
+// What bounds it: the float matrix instructions, so what counts
+// is that nothing waits in front of them.  FULL (heads that fill their last 16): a tile of keys and values is on its way in registers while
+// the one before is multiplied, and four sums take turns.  A die (workgroups are dealt to the 8 of them in turn) gets whole
+// heads of whole sequences, one after the other, the longest blocks first, so that a head's keys and values, 2 MB at 2,048 positions of
+// 128, are read from memory once.  16 sequences of 1 to 2,048 tokens (16,385 in all), 16 heads of 128, a layer: 2,230 us with tiles through LDS one by one, 1,260 so; one of 2,048 459 and 362.
+template <int ND, bool FULL>
+__global__ __launch_bounds__(256, 2) void attn_f32_prefill_kernel(AttnF32Args p, int blocks_per_seq, int pairs) {
   extern __shared__ __align__(16) float lds[];
   constexpr int HDP = 16 * ND, KLD = HDP + 4, VLD = AT + 4;
+  constexpr bool AHEAD = FULL && ND <= 8;      // (heads of 256: the registers are taken)
   float* Ks = lds;                    // [AT][KLD]
   float* Vt = lds + AT * KLD;         // [HDP][VLD]
-  const int seq = blockIdx.x / blocks_per_seq, blk = blockIdx.x % blocks_per_seq;
-  const int h = blockIdx.y, kvh = h / (p.nh / p.nkv);
+  const int pair = blockIdx.x / 8 / blocks_per_seq * 8 + blockIdx.x % 8, blk = blocks_per_seq - 1 - blockIdx.x / 8 % blocks_per_seq;
+  if (pair >= pairs) return;
+  const int seq = pair / p.nh, h = pair % p.nh, kvh = h / (p.nh / p.nkv);
   const int t0 = p.cu_seqlens[seq], n_new = p.cu_seqlens[seq + 1] - t0;
   if (blk * 64 >= n_new) return;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
   // head sizes that do not fill their last 16: the padding is multiplied by zeros of the queries, so it must hold numbers
-  for (int i = tid; i < AT * KLD + HDP * VLD; i += 256) lds[i] = 0.f;
+  if (!FULL)
+    for (int i = tid; i < AT * KLD + HDP * VLD; i += 256) lds[i] = 0.f;
   const int start = p.start[seq];
   const int* table = p.block_table + (size_t)p.slots[seq] * p.bt_stride;
   const int hd = p.hd;
@@ -177,27 +197,54 @@ __global__ __launch_bounds__(256) void attn_f32_prefill_kernel(AttnF32Args p, in
   const int wave_first = start + blk * 64 + wave * 16, wave_last = min(blk_last, wave_first + 15);
   const int wave_lo = reach_lo(wave_first, p.window, p.mod.chunk);
 
-  for (int tile = first_tile(blk_lo / AT, kept); tile * AT <= blk_last; tile = next_tile(tile, blk_lo / AT, kept)) {
+  f32x4 kr[AHEAD ? ND : 1], vr[AHEAD ? ND : 1];      // this thread's 16 bytes of the next tile's keys and values
+  auto fetch = [&](int tile) {
+    const int key0 = tile * AT, page = table[key0 / p.page_size];
+    if (page < 0) return page;
+    const float* kp = p.k_pool + (size_t)page * p.page_stride + ((size_t)kvh * p.page_size + key0 % p.page_size) * HDP;
+    const float* vp = p.v_pool + (size_t)page * p.page_stride + (size_t)kvh * p.page_size * HDP + key0 % p.page_size;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int idx = tid + 256 * i;
+      kr[AHEAD ? i : 0] = *reinterpret_cast<const f32x4*>(kp + 4 * idx);
+      vr[AHEAD ? i : 0] = *reinterpret_cast<const f32x4*>(vp + (size_t)(idx / (AT / 4)) * p.page_size + idx % (AT / 4) * 4);
+    }
+    return page;
+  };
+  int tile = first_tile(blk_lo / AT, kept), ahead = -1;
+  if (AHEAD && tile * AT <= blk_last) ahead = fetch(tile);
+  for (int next; tile * AT <= blk_last; tile = next) {
     const int key0 = tile * AT;
-    const int page = table[key0 / p.page_size];
+    const int page = AHEAD ? ahead : table[key0 / p.page_size];
+    next = next_tile(tile, blk_lo / AT, kept);
     __syncthreads();          // the tile before has been used by every wave
     if (page >= 0) {
-      const float* kp = p.k_pool + (size_t)page * p.page_stride + ((size_t)kvh * p.page_size + key0 % p.page_size) * hd;
-      const int per_row = hd / 4;
-      for (int idx = tid; idx < AT * per_row; idx += 256) {
-        const int row = idx / per_row, c = idx % per_row;
-        *reinterpret_cast<f32x4*>(&Ks[row * KLD + 4 * c]) = *reinterpret_cast<const f32x4*>(kp + (size_t)row * hd + 4 * c);
-      }
-      const float* vp = p.v_pool + (size_t)page * p.page_stride + (size_t)kvh * p.page_size * hd + key0 % p.page_size;
-      for (int idx = tid; idx < hd * (AT / 4); idx += 256) {
-        const int d = idx / (AT / 4), c = idx % (AT / 4);
-        *reinterpret_cast<f32x4*>(&Vt[d * VLD + 4 * c]) = *reinterpret_cast<const f32x4*>(vp + (size_t)d * p.page_size + 4 * c);
+      if constexpr (AHEAD) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+          const int idx = tid + 256 * i;
+          *reinterpret_cast<f32x4*>(&Ks[idx / (4 * ND) * KLD + idx % (4 * ND) * 4]) = kr[i];
+          *reinterpret_cast<f32x4*>(&Vt[idx / (AT / 4) * VLD + idx % (AT / 4) * 4]) = vr[i];
+        }
+      } else {
+        const float* kp = p.k_pool + (size_t)page * p.page_stride + ((size_t)kvh * p.page_size + key0 % p.page_size) * hd;
+        const int per_row = hd / 4;
+        for (int idx = tid; idx < AT * per_row; idx += 256) {
+          const int row = idx / per_row, c = idx % per_row;
+          *reinterpret_cast<f32x4*>(&Ks[row * KLD + 4 * c]) = *reinterpret_cast<const f32x4*>(kp + (size_t)row * hd + 4 * c);
+        }
+        const float* vp = p.v_pool + (size_t)page * p.page_stride + (size_t)kvh * p.page_size * hd + key0 % p.page_size;
+        for (int idx = tid; idx < hd * (AT / 4); idx += 256) {
+          const int d = idx / (AT / 4), c = idx % (AT / 4);
+          *reinterpret_cast<f32x4*>(&Vt[d * VLD + 4 * c]) = *reinterpret_cast<const f32x4*>(vp + (size_t)d * p.page_size + 4 * c);
+        }
       }
     }
     __syncthreads();
+    if (AHEAD && next * AT <= blk_last) ahead = fetch(next);
     if (page < 0) continue;             // a page that its group has given back: nothing of it is in anyone's reach
     if (key0 > wave_last || (key0 + AT <= wave_lo && key0 >= keep)) continue;
-    attend_tile<ND>(
+    attend_tile<ND, AHEAD ? 4 : 1>(
         qf, [&](int kt, int u) { return *reinterpret_cast<const f32x4*>(&Ks[(16 * kt + r) * KLD + 16 * u + 4 * g]); },
         [&](int dt, int kt) { return *reinterpret_cast<const f32x4*>(&Vt[(16 * dt + r) * VLD + 16 * kt + 4 * g]); },
         key0, pos_q, lo_q, p.scale, p.mod.cap, biased, r1, r2, keep, sig, pb, m_run, l_run, acc);
@@ -265,7 +312,7 @@ __global__ __launch_bounds__(64) void attn_f32_decode_kernel(AttnF32Args p, int 
     if (LINES) {
       const int r8 = r % 8, ch = 4 * (g + 4 * (r / 8));
       f32x4 k_next, v_next;
-      attend_tile<ND>(
+      attend_tile<ND, 1>(
           qf,
           [&](int kt, int u) {
             if (u % 2) return k_next;
@@ -289,7 +336,7 @@ __global__ __launch_bounds__(64) void attn_f32_decode_kernel(AttnF32Args p, int 
     } else {
       // (what lies beyond the head size is asked for at the tile's first address instead and replaced by zeros:
       // every lane loads, so that no load waits behind a branch)
-      attend_tile<ND>(
+      attend_tile<ND, 1>(
           qf,
           [&](int kt, int u) {
             const int d = 16 * u + 4 * g;
@@ -394,15 +441,16 @@ static int launch_attention_f32(const AttnF32Args& p, int B, int decode, int max
   }
   constexpr int HDP = 16 * ND;
   const size_t shmem = ((size_t)AT * (HDP + 4) + (size_t)HDP * (AT + 4)) * sizeof(float);
+  const auto kernel = p.hd == HDP ? attn_f32_prefill_kernel<ND, true> : attn_f32_prefill_kernel<ND, false>;
   if (shmem > 64 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_f32_prefill_kernel<ND>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;
   }
   const int blocks_per_seq = (max_new + 63) / 64;
   if (p.nh > 65535) return TQ_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(attn_f32_prefill_kernel<ND>, dim3((unsigned)B * blocks_per_seq, p.nh), dim3(256), shmem, st, p,
-                     blocks_per_seq);
+  const int64_t pairs = (int64_t)B * p.nh, workgroups = (pairs + 7) / 8 * 8 * blocks_per_seq;
+  if (workgroups > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)workgroups), dim3(256), shmem, st, p, blocks_per_seq, (int)pairs);
   return 0;
 }
 
