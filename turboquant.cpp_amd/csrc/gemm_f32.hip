@@ -15,7 +15,11 @@
 //    16,385 rows, ms, before and now: by 6,144 x 2,048 3.46 and 3.20 (129 TFLOP/s; the instructions alone give 153), by 2,048 x 5,632 3.48
 //    and 3.22, gated pair of twice 5,632 x 2,048 7.55 and 5.78; 60 experts of 1,408 x 2,048, four per token, 6.85 and
 //    6.12, their second product 3.80 and 3.22; 1,000 rows by twice 5,632 x 2,048 655 and 402 us.  Rings of two stages 1 to 3 % slower,
-//    of four level; four waves to a SIMD (128 registers) level.
+//    of four level; four waves to a SIMD (128 registers) level.  Then, with a wave's priority raised while it multiplies (a wave that
+//    asks for tiles or has just passed its barrier lets the one in the middle of its products go on), ms without and with: 3.29 and
+//    3.15, 3.21 and 3.11, 5.72 and 5.57; experts 6.09 and 6.05, 3.19 and 3.05; 1,000 rows 404 and 388 us.  All of a step's reads
+//    before its first product 2 to 4 % slower than a half at a time; waves whose rows all lie behind the last row without their products
+//    level to 1 % slower (the loop for each height takes registers that the reads ahead had).
 //    17 to 64 rows (a decode step of many sequences) are one row of tiles, at which multiply-adds and bytes of w
 //    are in balance; a narrow matrix is cut into runs of k so that the chip has enough workgroups.
 //  * gemm_f32_stream_kernel, for few rows (decoding; experts that few tokens chose): the work is reading w once.
@@ -205,7 +209,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (t + TSTAGES - 1 < steps) ask(t + TSTAGES - 1);
+    __builtin_amdgcn_s_setprio(1);
     multiply(ring + t % TSTAGES * STAGE);
+    __builtin_amdgcn_s_setprio(0);
   }
   if (left) {      // the last 4, 8 or 12 of k, through registers, zeros behind them
     __syncthreads();
