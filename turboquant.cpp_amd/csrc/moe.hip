@@ -9,6 +9,11 @@
 // a fixed share of the elements and the lanes' sums are added by a butterfly: one order for every token,
 // whatever else is in the batch.  Rows are dealt over a second grid dimension when
 // there are few tokens, so that decoding does not leave the chip to eight waves.
+// What bounds it: loads in a chain (a workgroup's activations, then its rows of wr), and for many tokens the multiply-adds and the sums
+// over the lanes.  So a workgroup asks for all its tokens' activations before it stores the first, and a wave's 32 sums change places on
+// the way (62 exchanges instead of 192 shuffles and additions).  us with the choice, before and now, 60 experts of 2,048 and a shared one,
+// bf16: one token 7.3 and 6.6, 97 8.8 and 7.8, 512 14.6 and 10.5, 1,733 27.7 and 17.6, 2,048 24.4 and 16.9, 11,000 93.7 and 66.1;
+// 256 experts, 2,048 tokens 76.2 and 53.3; 32-bit, 16,385 tokens 140 and 103.
 // router_select, one wave per token: top-k by logit, k rounds of a search in which >= lets the highest index
 // win among equal logits, so ids come out by descending logit (tq_moe.c:626-645).  Weights:
 //   renorm != 0: softmax over the selected logits (tq_moe.c:648-678), times wscale;
@@ -20,6 +25,7 @@
 #define TQ_ROUTE_SIGMOID 2
 #define TQ_ROUTE_PAIR_GROUPS 4
 #define RT 8   // most tokens per workgroup of router_logits
+#define TQ_ROUTER_MANY 240   // tokens from which on a workgroup of router_logits has eight waves and RT tokens
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void load4(const float* p, float* w) {
@@ -34,14 +40,41 @@ __device__ __forceinline__ void load4(const bf16_t* p, float* w) {
   w[3] = __uint_as_float(v.y & 0xffff0000u);
 }
 
+// The sums over the wave of N values (a power of two up to the wave's lanes): afterwards s[0] of lanes i * 64 / N and on is value i's.
+// Each value's is the sum that wave_sum gives, in its order, by fewer steps: at a step two values change places by halves, and one
+// addition makes the next sums of both.
+template <int N, int O>
+__device__ __forceinline__ void wave_sums(float* s) {
+  if constexpr (N > 1) {
+    const bool upper = (threadIdx.x & O) != 0;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const float a = s[i], b = s[i + N / 2];
+      if constexpr (O >= 16) {
+        typedef unsigned two __attribute__((ext_vector_type(2)));
+        const two t = __builtin_bit_cast(two, O == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                                                      : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false));
+        s[i] = __uint_as_float(t.x) + __uint_as_float(t.y);
+      } else {
+        const float own = upper ? b : a;
+        s[i] = with_lane_xor<O>(upper ? a : b, [own](float, float other) { return own + other; });
+      }
+    }
+    wave_sums<N / 2, O / 2>(s);
+  } else if constexpr (O > 0) {
+    s[0] = with_lane_xor<O>(s[0], LanesSum());
+    wave_sums<1, O / 2>(s);
+  }
+}
+
 // TG: tokens per workgroup (tokens beyond T are zeros in LDS and are not stored).  RW: rows of wr that a wave
 // takes at a time, so that one read of the activations from LDS serves RW rows.  Neither changes the order in
 // which a logit is summed: of every 512 elements lane l sums 4 l .. 4 l + 3 and 256 + 4 l .. 256 + 4 l + 3 (its
 // 16-byte reads from LDS then lie side by side with its neighbours'), block after block.  In LDS a token's row is
 // filled with zeros up to a multiple of 512, so the last block needs no predicate: there the weights are read
 // from the row's last elements instead, and multiplied by zeros.
-template <class W, int TG, int RW>
-__global__ __launch_bounds__(256) void router_logits_kernel(const float* __restrict__ x, const W* __restrict__ wr,
+template <class W, int TG, int RW, int TH>
+__global__ __launch_bounds__(TH, TH == 512 ? 4 : 1) void router_logits_kernel(const float* __restrict__ x, const W* __restrict__ wr,
                                                             const W* __restrict__ shared_w, int rows, int E,
                                                             float* __restrict__ logits, int T, int H,
                                                             const float* __restrict__ bias) {
@@ -55,12 +88,15 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float* __restr
     const int Hp4 = Hp / 4, H4 = H / 4;
     f32x4* dst = reinterpret_cast<f32x4*>(xs);
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    for (int j = threadIdx.x; j < Hp4; j += TH) {
+      f32x4 v[TG];
 #pragma unroll
-    for (int k = 0; k < TG; ++k)
-      for (int j = threadIdx.x; j < Hp4; j += blockDim.x)
-        dst[k * Hp4 + j] = k < nt && j < H4 ? reinterpret_cast<const f32x4*>(x + (size_t)(t0 + k) * H)[j] : zero;
+      for (int k = 0; k < TG; ++k) v[k] = k < nt && j < H4 ? reinterpret_cast<const f32x4*>(x + (size_t)(t0 + k) * H)[j] : zero;
+#pragma unroll
+      for (int k = 0; k < TG; ++k) dst[k * Hp4 + j] = v[k];
+    }
   } else {
-    for (int i = threadIdx.x; i < TG * Hp; i += blockDim.x) {
+    for (int i = threadIdx.x; i < TG * Hp; i += TH) {
       const int k = i / Hp, j = i % Hp;
       xs[i] = k < nt && j < H ? x[(size_t)(t0 + k) * H + j] : 0.f;
     }
@@ -68,20 +104,19 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float* __restr
   __syncthreads();
   // workgroups start at different rows, so that they do not all ask for the same row at once
   const int rot = (blockIdx.x * 5) % rows;
-  for (int idx = (blockIdx.y * 4 + wave) * RW; idx < rows; idx += gridDim.y * 4 * RW) {
+  for (int idx = (blockIdx.y * (TH / TQ_WAVE) + wave) * RW; idx < rows; idx += gridDim.y * (TH / TQ_WAVE) * RW) {
     const W* row[RW];
-    int e[RW];
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
       const int i = min(idx + r, rows - 1) + rot;
-      e[r] = i < rows ? i : i - rows;
-      row[r] = e[r] < E ? wr + (size_t)e[r] * H : shared_w;
+      const int e = i < rows ? i : i - rows;
+      row[r] = e < E ? wr + (size_t)e * H : shared_w;
     }
-    float s[RW][TG];
+    float s[RW * TG];
 #pragma unroll
     for (int r = 0; r < RW; ++r)
 #pragma unroll
-      for (int k = 0; k < TG; ++k) s[r][k] = 0.f;
+      for (int k = 0; k < TG; ++k) s[r * TG + k] = 0.f;
     if (vec) {
       const f32x4* xv = reinterpret_cast<const f32x4*>(xs);
       const int Hp4 = Hp / 4;
@@ -108,7 +143,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float* __restr
               const f32x4 c = xv[k * Hp4 + b / 4 + 64 + lane];
 #pragma unroll
               for (int r = 0; r < RW; ++r) {
-                float v = s[r][k];
+                float v = s[r * TG + k];
                 v = fmaf(a.x, w[u][r][0], v);
                 v = fmaf(a.y, w[u][r][1], v);
                 v = fmaf(a.z, w[u][r][2], v);
@@ -117,7 +152,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float* __restr
                 v = fmaf(c.y, w[u][r][5], v);
                 v = fmaf(c.z, w[u][r][6], v);
                 v = fmaf(c.w, w[u][r][7], v);
-                s[r][k] = v;
+                s[r * TG + k] = v;
               }
             }
           }
@@ -129,18 +164,17 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const float* __restr
         for (int r = 0; r < RW; ++r) {
           const float w = to_f32(row[r][j]);
 #pragma unroll
-          for (int k = 0; k < TG; ++k) s[r][k] = fmaf(xs[k * Hp + j], w, s[r][k]);
+          for (int k = 0; k < TG; ++k) s[r * TG + k] = fmaf(xs[k * Hp + j], w, s[r * TG + k]);
         }
       }
     }
-#pragma unroll
-    for (int r = 0; r < RW; ++r)
-#pragma unroll
-      for (int k = 0; k < TG; ++k) {
-        const float v = wave_sum(s[r][k]);
-        if (lane == 0 && k < nt && idx + r < rows)      // (a bias per expert, not for the shared expert's gate row)
-          logits[(size_t)(t0 + k) * rows + e[r]] = bias && e[r] < E ? v + bias[e[r]] : v;
-      }
+    wave_sums<RW * TG, TQ_WAVE / 2>(s);
+    constexpr int LANES = TQ_WAVE / (RW * TG);      // that hold one sum
+    const int r = lane / LANES / TG, k = lane / LANES % TG;
+    if (lane % LANES == 0 && k < nt && idx + r < rows) {      // (a bias per expert, not for the shared expert's gate row)
+      const int i = idx + r + rot, at = i < rows ? i : i - rows;
+      logits[(size_t)(t0 + k) * rows + at] = bias && at < E ? s[0] + bias[at] : s[0];
+    }
   }
 }
 
@@ -441,38 +475,44 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float* __restr
 
 static int launch_router_logits(const float* x, const void* wr, const void* shared_w, int wtype, int E,
                                 float* logits, int T, int H, hipStream_t st, const float* bias = nullptr) {
-  int tg = RT;
+  const int rows = E + (shared_w ? 1 : 0);
   const size_t hp = ((size_t)H + 511) / 512 * 512;      // a token's row in LDS
-  while (tg > 1 && (size_t)tg * hp * sizeof(float) > 32 * 1024) tg /= 2;   // small enough for several workgroups per CU
+  // Many tokens: 8 of them to a workgroup of eight waves, whatever LDS they take (a wave's read of 4 rows of wr serves 8 tokens).  The
+  // other form and this one, with the choice, us, 60 experts of 2,048 and a shared one: 160 tokens 8.4 and 8.6, 333 10.7 and 10.1,
+  // 512 12.9 and 10.5, 700 15.9 and 11.8; 256 experts: 64 16.5 and 16.5, 240 22.2 and 19.5, 512 27.3 and 24.2; rows of 3,584, 114 KB
+  // of LDS, 2,048 tokens 42.7 and 33.1.
+  const bool many = T >= TQ_ROUTER_MANY && hp * RT * sizeof(float) <= 160 * 1024;
+  int tg = RT;
+  while (!many && tg > 1 && (size_t)tg * hp * sizeof(float) > 32 * 1024) tg /= 2;   // small enough for several workgroups per CU
   const size_t shmem = (size_t)tg * hp * sizeof(float);
   if (shmem > 160 * 1024) return TQ_ERR_UNSUPPORTED;
-  const int rows = E + (shared_w ? 1 : 0);
-  const int groups = (T + tg - 1) / tg;
+  const int groups = (T + tg - 1) / tg, waves = many ? 8 : 4;
   // The rows are dealt over so many workgroups that the chip holds about 2048 of them: what a wave does is a
   // chain of loads, and only many waves hide it.  A wave takes 1, 2 or 4 rows at a time.
-  int row_groups = 2048 / groups;
-  row_groups = row_groups < 1 ? 1 : (row_groups > (rows + 3) / 4 ? (rows + 3) / 4 : row_groups);
-  const int rows_per_wave = (rows + row_groups * 4 - 1) / (row_groups * 4);
+  int row_groups = (many ? 512 : 2048) / groups;
+  row_groups = row_groups < 1 ? 1 : (row_groups > (rows + waves - 1) / waves ? (rows + waves - 1) / waves : row_groups);
+  const int rows_per_wave = (rows + row_groups * waves - 1) / (row_groups * waves);
   const int rw = rows_per_wave >= 4 ? 4 : (rows_per_wave >= 2 ? 2 : 1);
-#define TQ_ROUTER(TGV, RWV)                                                                                         \
+#define TQ_ROUTER(TGV, RWV, THV)                                                                                    \
   do {                                                                                                              \
     if (shmem > 48 * 1024)                                                                                          \
-      (void)hipFuncSetAttribute((const void*)router_logits_kernel<W, TGV, RWV>,                                           \
+      (void)hipFuncSetAttribute((const void*)router_logits_kernel<W, TGV, RWV, THV>,                                \
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);                                  \
-    hipLaunchKernelGGL((router_logits_kernel<W, TGV, RWV>), dim3(groups, row_groups), dim3(256), shmem, st, x,      \
+    hipLaunchKernelGGL((router_logits_kernel<W, TGV, RWV, THV>), dim3(groups, row_groups), dim3(THV), shmem, st, x, \
                        (const W*)wr, (const W*)shared_w, rows, E, logits, T, H, bias);                              \
   } while (0)
-#define TQ_ROUTER_RW(TGV)          \
-  do {                             \
-    if (rw == 4) TQ_ROUTER(TGV, 4); \
-    else if (rw == 2) TQ_ROUTER(TGV, 2); \
-    else TQ_ROUTER(TGV, 1);        \
+#define TQ_ROUTER_RW(TGV, THV)              \
+  do {                                      \
+    if (rw == 4) TQ_ROUTER(TGV, 4, THV);    \
+    else if (rw == 2) TQ_ROUTER(TGV, 2, THV); \
+    else TQ_ROUTER(TGV, 1, THV);            \
   } while (0)
   TQ_DISPATCH_W(wtype, {
-    if (tg == 8) TQ_ROUTER_RW(8);
-    else if (tg == 4) TQ_ROUTER_RW(4);
-    else if (tg == 2) TQ_ROUTER_RW(2);
-    else TQ_ROUTER_RW(1);
+    if (many) TQ_ROUTER_RW(8, 512);
+    else if (tg == 8) TQ_ROUTER_RW(8, 256);
+    else if (tg == 4) TQ_ROUTER_RW(4, 256);
+    else if (tg == 2) TQ_ROUTER_RW(2, 256);
+    else TQ_ROUTER_RW(1, 256);
   });
 #undef TQ_ROUTER_RW
 #undef TQ_ROUTER
