@@ -881,11 +881,10 @@ def expert_tile_rows(n_pairs: int, num_experts: int, act, a: torch.Tensor, w: to
 def expert_product_rows(unit: int, n_pairs: int, num_experts: int) -> int:
     """The ``tile_rows`` that a product over experts is called with when the row order has units of ``unit`` rows: from
     48 rows per expert on average, units of 64 up to two or four at a time by the order's items (``expert_item_units``,
-    csrc/gemm_phases.hip).  Measured on 60 experts of 1,408 x 2,048, four per token, evenly dealt, both products together
-    against items of two through a ring of LDS stages, which unit by unit trailed by 13 % and more: 253 us against 264 at 70 rows
-    per expert (items of two), 275 against 367 at 137 (of four), 480 against 541 at 273, 715 against 918 at 546; 64 experts
-    of 2,560 x 3,584 at 1,650 rows each 5.7 ms against 7.5.  Below 48 rows nearly every expert has one unit, and unit by
-    unit is level."""
+    csrc/gemm_phases.hip).  Both products together, us, unit by unit in the tile kernel and so: 60 experts of 1,408 x 2,048, four per
+    token, evenly dealt, 293 and 246 at 70 rows per expert, 379 and 325 at 137, 563 and 452 at 273, 958 and 722 at 546; 64 experts
+    of 2,560 x 3,584 678 and 663 at 48, 8,590 and 5,882 at 1,650.  Below 48 rows nearly every expert has one unit, and the
+    difference is small (244 and 237 at 48, 242 and 231 at 36, 244 and 227 at 24)."""
     if unit == 64 and n_pairs >= EXPERT_PAIRS_FROM * num_experts:
         return 64 + TILE_PAIRS
     return unit
