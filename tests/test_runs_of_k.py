@@ -1,0 +1,32 @@
+"""Into how many runs of k products of many rows go: what the library's rule says, without a GPU."""
+import ctypes
+
+import pytest
+
+from turboquant_cpp_amd.csrc import build
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return ctypes.CDLL(build.find_library("bfloat16") or build.build("bfloat16"))
+
+
+def tile_kernel_runs(M, N, K):
+    """Tiles of 128 x 128 that do not fill the chip twice, runs of 1,024 of k at least."""
+    runs = 1
+    while runs < 4 and -(-M // 128) * -(-N // 128) * runs < 512 and K // (2 * runs) >= 1024:
+        runs *= 2
+    return runs
+
+
+def test_many_rows_go_in_no_fewer_and_bounded_runs(lib):
+    """A run fewer is a longer sum of 32 bits, with a larger error; a run more is as much again for the next kernel to read.  Every run
+    has two steps of 64 and more."""
+    for M in (1025, 1500, 2048, 3001, 4096, 6000, 8192, 13197, 28000):
+        for N in (64, 128, 184, 1024, 2048, 3072, 3584, 4096, 5824, 6144, 8192, 20480):
+            for K in (128, 192, 512, 960, 2048, 2112, 3584, 4096, 5632, 8192, 11008, 19520, 20480):
+                runs, least = lib.tq_gemm_mfma_splits(M, N, K), tile_kernel_runs(M, N, K)
+                assert least <= runs <= 4, (M, N, K)
+                assert runs == least or runs * M * N * 4 <= 256 << 20, (M, N, K)
+                steps, per = K // 64, -(-(K // 64) // runs)
+                assert runs == 1 or steps - per * (runs - 1) >= 2, (M, N, K)

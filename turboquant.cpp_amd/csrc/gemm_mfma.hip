@@ -1014,11 +1014,13 @@ static bool phases_suit(int M, int N, int K, bool dual) {
   if (M > 1024) return true;
   return dual ? narrow > 256 : wide > (M > 512 ? 256 : 512) && K >= 512;
 }
-// Its runs of k where partial sums are wanted apart: what a run more saves must be more than writing and reading its sums takes.
-static int phases_runs(int M, int N, int K) {
-  int best = 1, rows;
-  double least = phases_best(M, N, K, false, 1, &rows);
-  for (int s = 2; s <= 4; s *= 2) {
+// Its runs of k where partial sums are wanted apart, `from` at least (the tile kernel's: fewer runs are longer sums, whose error against
+// 64 bits is the larger, 2.7e-7 of 2,048 products in one run and 1.9e-7 in two): what a run more saves must be more than writing and
+// reading its sums takes, and they stay within 256 MB, which the kernel behind reads.
+static int phases_runs(int M, int N, int K, int from) {
+  int best = from, rows;
+  double least = phases_best(M, N, K, false, from, &rows) + (from - 1) * ((double)M * N * 8 / 5e6);
+  for (int s = 2 * from; s <= 4 && (int64_t)s * M * N * 4 <= (256 << 20); s *= 2) {
     const int per = (K / TBK + s - 1) / s;
     if (per < 4 || K / TBK - per * (s - 1) < 2) break;
     const double t = phases_best(M, N, K, false, s, &rows) + (s - 1) * ((double)M * N * 8 / 5e6);
@@ -1052,7 +1054,8 @@ TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
 
 // Into how many runs of k a plain product of M rows may be split when its partial sums are wanted apart.  Many
 // rows: a product whose tiles do not fill the chip twice, and that has k enough, goes faster in 2 to 4 runs, each
-// at least 1024 long, and up to 1,024 rows as tile_runs says.  17 to 64 rows of a narrow matrix with a long k in the
+// at least 1024 long, and up to 1,024 rows as tile_runs says; in the tiles of gemm_phases in as many, or in more and shorter
+// ones (256 of k at least) where phases_runs expects them to be faster.  17 to 64 rows of a narrow matrix with a long k in the
 // streaming kernel (at most 8 waves over k): as many runs as bring about 4096 waves, each wave keeping 128 of k
 // (64 rows by 2,048 x 2,048: 13.4 us in two runs against 15.2 in one; by 2,048 x 5,632: 17.3 in four against 20.7
 // in two); from 33 rows on the tile kernel with its runs instead, where it may split k.  1 for up to 16 rows.
@@ -1090,10 +1093,10 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
     while (s < 8 && waves * s < 4096 && K / (16 * s) >= 128) s *= 2;
     return s;
   }
-  if (phases_suit(M, N, K, false)) return phases_runs(M, N, K);
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + TBN - 1) / TBN);
   int s = 1;
   while (s < 4 && tiles * s < 512 && K / (s * 2) >= 1024) s *= 2;
+  if (phases_suit(M, N, K, false)) return phases_runs(M, N, K, s);
   if (M <= 64 * 16) {      // tiles of 64 rows: more and shorter runs
     const int t = tile_runs(M, N, K);
     if (t > s) s = t;
