@@ -1,4 +1,4 @@
-"""Into how many runs of k products of many rows go: what the library's rule says, without a GPU."""
+"""Products of many rows: into how many runs of k they go and which leave for the vendor's library, as the rules say without a GPU."""
 import ctypes
 
 import pytest
@@ -30,3 +30,10 @@ def test_many_rows_go_in_no_fewer_and_bounded_runs(lib):
                 assert runs == least or runs * M * N * 4 <= 256 << 20, (M, N, K)
                 steps, per = K // 64, -(-(K // 64) // runs)
                 assert runs == 1 or steps - per * (runs - 1) >= 2, (M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(13197, 3584, 3584), (12000, 6144, 5632), (8192, 3584, 20480), (13197, 3584, 20480), (9000, 2048, 16384), (3258, 8224, 4096)])
+def test_plain_products_of_a_long_k_stay_with_the_library_that_adds_it_in_parts(lib, M, N, K):
+    """Its sums of 32 bits are the closer ones to 64 bits; an activation or a gate's result of 16 bits keeps nothing of that."""
+    assert not lib.tq_gemm_here_rather(M, N, K, 0)
+    assert lib.tq_gemm_here_rather(2048, 6288, 2048, 0) and lib.tq_gemm_here_rather(2048, 5632, 2048, 2)

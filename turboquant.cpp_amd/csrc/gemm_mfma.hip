@@ -1035,21 +1035,18 @@ static int phases_runs(int M, int N, int K, int from) {
 // that pass at 5.5 TB/s (us by the library and here: gated 2,048 by 5,632 x 2,048 105 and 88, 1,999 by 11,008 x 4,096 408 and 288,
 // 1,280 by 768 x 1,024 18 and 16, 900 by 1,024 x 4,096 31 and 40; an activation alone 3,001 by 8,448 x 2,048 127 and 103, 768 by
 // 1,408 x 2,048 19 and 23, 1,315 by 256 x 832 11 and 13).  A plain product the library does at the same rate, but not where its
-// columns are no whole number of tiles (2,048 by 6,288 x 2,048 67 and 49, 1,733 by 7,184 x 2,048 60 and 50, 3,258 by 8,224 x 2,048
-// 111 and 99; by 8,448 101 and 102), nor where k is very long (8,192 by 3,584 x 20,480 1,505 and 829): there where the tiles here
-// reach 950 TFLOP/s (600 of a very long k).  With many rows and a long k its choice of kernel is uneven: of 130 products of 9,000 to
-// 28,000 rows by 1,024 to 6,144 x 3,584 and 5,632 where these tiles reach 1,100 TFLOP/s the times here are 0.95 of the library's on
-// average (13,197 by 3,584 x 3,584 366 and 252, 12,000 by 6,144 x 5,632 782 and 641, 16,384 by 3,584 x 3,584 343 and 350; worst
-// 1.07), at k 2,048 they are level.
+// columns are no whole number of tiles (2,048 by 6,288 x 2,048 70 and 55, 1,733 by 7,184 x 2,048 62 and 54, 3,258 by 8,224 x 2,048
+// 120 and 109; by 8,448 101 and 102): there where the tiles here reach 950 TFLOP/s, and up to k 2,048.  Beyond, the library adds k in parts
+// for many a size: the slower kernel (13,197 by 3,584 x 3,584 367 us and 274 here, 8,192 by 3,584 x 20,480 1,305 and 860), but the
+// closer to 64 bits (3.45e-7 against 3.68e-7, 8.3e-7 against 9.2e-7; 17 of 66 sizes drawn from k 2,496 to 12,672, by 4 to 11 %), and a
+// result in float keeps what is gained.  Up to k 2,304 the error was the same in all of 24.  (A result of 16 bits is off by 1.7e-3.)
 TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
   const bool dual = kind == 2;
   if (!phases_suit(M, N, K, dual)) return 0;
   int rows;
   const double t = phases_best(M, N, K, dual, 1, &rows), flops = 2.0 * M * N * K * (dual ? 2 : 1);
   if (kind) return (dual ? t : 0.95 * t) <= (dual ? 14 : 11.5) + flops / 1.15e9 + (double)M * N * (dual ? 10 : 6) / 5.5e6;
-  const double rate = flops / (t * 1e6);
-  if (K >= 16384) return rate >= 600;
-  return (N % 256 != 0 && rate >= 950) || (M >= 9000 && K >= 3584 && rate >= 1100);
+  return K <= 2048 && N % 256 != 0 && flops / (t * 1e6) >= 950;
 }
 
 // Into how many runs of k a plain product of M rows may be split when its partial sums are wanted apart.  Many
