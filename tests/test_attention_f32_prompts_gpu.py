@@ -46,3 +46,17 @@ def test_prompts_against_64_bits(hd, lens, starts, nh, nkv, window):
                         hd ** -0.5, "float32", runs=runs)
     # scores are off by some roundings of sums of hd products, weights and their sums by as much: 1e-5 of values of about one
     assert (got.cpu().double() - torch.cat(want)).abs().max().item() < 1e-5
+
+
+def test_more_workgroups_than_a_dimension_of_the_grid_holds():
+    """The longest run is an upper bound: 17 million workgroups, most of them with nothing to do, whose threads are more than 32 bits count."""
+    from turboquant_cpp_amd.csrc import ops
+    page, hd, nh, lens = 64, 32, 3, [70, 5]
+    gen = torch.Generator().manual_seed(1)
+    kp, vp, q = (torch.randn(*s, generator=gen).to(DEV) for s in ((3, nh, page, hd), (3, nh, hd, page), (sum(lens), nh * hd)))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    table, pos, seq = i32([[2, 0], [1, 0]]), i32([p for n in lens for p in range(n)]), i32([i for i, n in enumerate(lens) for _ in range(n)])
+    def attend(longest):
+        runs = dict(cu_seqlens=i32([0, 70, 75]), slots=i32([0, 1]), start=i32([0, 0]), max_new=longest, max_end=70, decode=False)
+        return ops.attention(q, kp.flatten(), vp.flatten(), 0, pos, seq, table, page, nh * page * hd, nh, nh, hd, None, hd ** -0.5, "float32", runs=runs)
+    assert torch.equal(attend(64 * 2_900_000), attend(70))

@@ -27,6 +27,7 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define AT 64            // positions per tile
+#define F32_GRID_X (1 << 23)      // most workgroups of a prompt's launch in the grid's x, whose threads HIP counts in 32 bits; the others lie in y
 
 struct AttnF32Args {
   const float* q;          // [T][nh][hd]
@@ -151,7 +152,12 @@ __global__ __launch_bounds__(256, 2) void attn_f32_prefill_kernel(AttnF32Args p,
   constexpr bool AHEAD = FULL && ND <= 8;      // (heads of 256: the registers are taken)
   float* Ks = lds;                    // [AT][KLD]
   float* Vt = lds + AT * KLD;         // [HDP][VLD]
-  const int pair = blockIdx.x / 8 / blocks_per_seq * 8 + blockIdx.x % 8, blk = blocks_per_seq - 1 - blockIdx.x / 8 % blocks_per_seq;
+  int pair, blk;
+  auto find = [&](auto i) {
+    pair = (int)(i / 8 / blocks_per_seq * 8 + i % 8), blk = blocks_per_seq - 1 - (int)(i / 8 % blocks_per_seq);
+  };
+  if (gridDim.y == 1) find(blockIdx.x);
+  else find((uint64_t)blockIdx.y * gridDim.x + blockIdx.x);
   if (pair >= pairs) return;
   const int seq = pair / p.nh, h = pair % p.nh, kvh = h / (p.nh / p.nkv);
   const int t0 = p.cu_seqlens[seq], n_new = p.cu_seqlens[seq + 1] - t0;
@@ -448,9 +454,10 @@ static int launch_attention_f32(const AttnF32Args& p, int B, int decode, int max
   }
   const int blocks_per_seq = (max_new + 63) / 64;
   if (p.nh > 65535) return TQ_ERR_UNSUPPORTED;
-  const int64_t pairs = (int64_t)B * p.nh, workgroups = (pairs + 7) / 8 * 8 * blocks_per_seq;
-  if (workgroups > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)workgroups), dim3(256), shmem, st, p, blocks_per_seq, (int)pairs);
+  const int64_t pairs = (int64_t)B * p.nh, all = (pairs + 7) / 8 * 8 * blocks_per_seq;
+  const int64_t x = all < F32_GRID_X ? all : F32_GRID_X, y = (all + x - 1) / x;
+  if (pairs > 0x7ffffff0 || y > 65535) return TQ_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)x, (unsigned)y), dim3(256), shmem, st, p, blocks_per_seq, (int)pairs);
   return 0;
 }
 
