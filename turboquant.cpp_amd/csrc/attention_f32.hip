@@ -72,7 +72,7 @@ __device__ __forceinline__ float group_sum(float v) {
 
 // One tile of 64 keys for 16 queries: scores from `kf` (reads the key operand of subtile kt, chunk u), softmax
 // update, and the product with the values from `vf` (value operand of d-tile dt, subtile kt).
-// SIDE: sums whose products take turns, so that none waits for the one before it (1: operands from memory, as few as may be in registers).
+// SIDE: sums whose products take turns, so that none waits for the one before it (2: fewer registers; 1: operands from memory, as few as may be).
 template <int ND, int SIDE, class KF, class VF>
 __device__ __forceinline__ void attend_tile(const f32x4 (&qf)[ND], KF kf, VF vf, int key0, int pos_q, int lo_q, float scale,
                                             float cap, bool biased, float r1, float r2, int keep, bool sig, float pb,
@@ -140,26 +140,35 @@ __device__ __forceinline__ void attend_tile(const f32x4 (&qf)[ND], KF kf, VF vf,
 }
 
 // ------------------------------------------------------------------------------------------ runs of tokens
-// What bounds it: the float matrix instructions, so what counts
-// is that nothing waits in front of them.  FULL (heads that fill their last 16): a tile of keys and values is on its way in registers while
-// the one before is multiplied, and four sums take turns.  A die (workgroups are dealt to the 8 of them in turn) gets whole
-// heads of whole sequences, one after the other, the longest blocks first, so that a head's keys and values, 2 MB at 2,048 positions of
-// 128, are read from memory once.  16 sequences of 1 to 2,048 tokens (16,385 in all), 16 heads of 128, a layer: 2,230 us with tiles through LDS one by one, 1,260 so; one of 2,048 459 and 362.
+// What bounds it: the float matrix instructions, so what counts is that nothing waits in front of them.  FULL (heads that fill their
+// last 16): a tile of keys and values is on its way in registers while the one before is multiplied, and two or four sums take turns.
+// Workgroups follow each other sequence by sequence and within one the longest blocks first, a block's heads side by side: however many
+// heads there are, every die (workgroups are dealt to the 8 of them in turn) has its share of long and short blocks, and where the heads are
+// a multiple of 8 a head stays on one die, whose L2 holds its keys and values.  Whole heads to a die leave dies idle where heads are few or
+// reach little: us with blocks dealt in turn and tiles through LDS one by one, with whole heads to a die, and so: 12 heads of 64, 4,096
+// tokens that reach 256 positions 63, 88 and 55, that reach all 649, 499 and 410; 1 head of 128, 8,192 tokens 1,398, 1,425 and 913; 28
+// heads over 4 of keys and values, 2,048 tokens 824, 533 and 328; 16 of 128, 2,048 tokens 448, 349 and 285, 16 sequences of 1 to 2,048 (16,385) 2,243, 1,205
+// and 1,153.  (7 sequences of 400 tokens of 12 heads 69, 52 and 62: what is left there is a last sequence whose long blocks begin late.)
+// Heads of 64 take 128 registers, so that four workgroups share a compute unit: 16 heads, 4,096 tokens that reach 256 positions 77 and 66 us.
 template <int ND, bool FULL>
-__global__ __launch_bounds__(256, 2) void attn_f32_prefill_kernel(AttnF32Args p, int blocks_per_seq, int pairs) {
+__global__ __launch_bounds__(256, ND == 4 ? 4 : 2) void attn_f32_prefill_kernel(AttnF32Args p, int blocks_per_seq, int n_seqs) {
   extern __shared__ __align__(16) float lds[];
   constexpr int HDP = 16 * ND, KLD = HDP + 4, VLD = AT + 4;
   constexpr bool AHEAD = FULL && ND <= 8;      // (heads of 256: the registers are taken)
   float* Ks = lds;                    // [AT][KLD]
   float* Vt = lds + AT * KLD;         // [HDP][VLD]
-  int pair, blk;
+  int seq, h, blk;      // (a head's blocks of 64 tokens)
   auto find = [&](auto i) {
-    pair = (int)(i / 8 / blocks_per_seq * 8 + i % 8), blk = blocks_per_seq - 1 - (int)(i / 8 % blocks_per_seq);
+    const unsigned per_seq = (unsigned)p.nh * blocks_per_seq, in = i % per_seq;
+    seq = (int)(i / per_seq), h = in % p.nh, blk = blocks_per_seq - 1 - (int)(in / p.nh);
   };
-  if (gridDim.y == 1) find(blockIdx.x);
-  else find((uint64_t)blockIdx.y * gridDim.x + blockIdx.x);
-  if (pair >= pairs) return;
-  const int seq = pair / p.nh, h = pair % p.nh, kvh = h / (p.nh / p.nkv);
+  if (gridDim.y == 1) {
+    find(blockIdx.x);
+  } else {
+    find((uint64_t)blockIdx.y * gridDim.x + blockIdx.x);
+    if (seq >= n_seqs) return;
+  }
+  const int kvh = h / (p.nh / p.nkv);
   const int t0 = p.cu_seqlens[seq], n_new = p.cu_seqlens[seq + 1] - t0;
   if (blk * 64 >= n_new) return;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
@@ -250,7 +259,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_prefill_kernel(AttnF32Args p,
     if (AHEAD && next * AT <= blk_last) ahead = fetch(next);
     if (page < 0) continue;             // a page that its group has given back: nothing of it is in anyone's reach
     if (key0 > wave_last || (key0 + AT <= wave_lo && key0 >= keep)) continue;
-    attend_tile<ND, AHEAD ? 4 : 1>(
+    attend_tile<ND, AHEAD ? (ND == 4 ? 2 : 4) : 1>(
         qf, [&](int kt, int u) { return *reinterpret_cast<const f32x4*>(&Ks[(16 * kt + r) * KLD + 16 * u + 4 * g]); },
         [&](int dt, int kt) { return *reinterpret_cast<const f32x4*>(&Vt[(16 * dt + r) * VLD + 16 * kt + 4 * g]); },
         key0, pos_q, lo_q, p.scale, p.mod.cap, biased, r1, r2, keep, sig, pb, m_run, l_run, acc);
@@ -452,12 +461,11 @@ static int launch_attention_f32(const AttnF32Args& p, int B, int decode, int max
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;
   }
-  const int blocks_per_seq = (max_new + 63) / 64;
-  if (p.nh > 65535) return TQ_ERR_UNSUPPORTED;
-  const int64_t pairs = (int64_t)B * p.nh, all = (pairs + 7) / 8 * 8 * blocks_per_seq;
+  const int blocks_per_seq = (max_new - 1) / 64 + 1;
+  const int64_t per_seq = (int64_t)p.nh * blocks_per_seq, all = per_seq * B;
   const int64_t x = all < F32_GRID_X ? all : F32_GRID_X, y = (all + x - 1) / x;
-  if (pairs > 0x7ffffff0 || y > 65535) return TQ_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)x, (unsigned)y), dim3(256), shmem, st, p, blocks_per_seq, (int)pairs);
+  if (p.nh > 65535 || per_seq > 0x7fffffff || y > 65535) return TQ_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)x, (unsigned)y), dim3(256), shmem, st, p, blocks_per_seq, B);
   return 0;
 }
 
