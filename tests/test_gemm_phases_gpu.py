@@ -248,6 +248,17 @@ def test_what_names_no_queue_is_refused(ops):
     assert call(64 + ops.TILE_QUEUE) != 0 and call(64 + ops.TILE_PAIRS + 3 * ops.TILE_QUEUE) != 0
 
 
+@pytest.mark.parametrize("hint", [2048, 4096, 64 + 1024 + 2048, 1 << 30])
+def test_a_hint_of_any_size_is_ignored(ops, hint):
+    """Products of one matrix take no notice of the rows of a tile, alone and in pairs of few rows."""
+    for M in (5, 300, 1100):
+        a, w, w2, bias = drawn((M, 128), 1), drawn((256, 128), 2), drawn((128, 128), 3), drawn((256,), 4)
+        assert torch.equal(ops.gemm(a, w, "bfloat16", out_act=True, bias=bias, tile_rows=hint), ops.gemm(a, w, "bfloat16", out_act=True, bias=bias))
+        if M <= 16:
+            both = [ops.gemm_pair(dict(a=a, w=w, tile_rows=r), dict(a=a, w=w2, tile_rows=r), "bfloat16") for r in (16, hint)]
+            assert torch.equal(both[0][0], both[1][0]) and torch.equal(both[0][1], both[1][1])
+
+
 def test_the_gate_over_its_whole_range(ops):
     """silu in the tiles' epilogue against the tile kernel's, to the last bit of the 16-bit result but where a rounding is near: factors
     that make every product one value from -1e5 to 1e5, among them those where the exponential leaves the range, zeros, infinities and NaN."""

@@ -1101,11 +1101,11 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
   return s;
 }
 
-// The queue that tile_rows names, or null, and tile_rows without it; false: what cannot be.
-static bool take_queue(int& tile_rows, const int* n_tiles, int** queue) {
+// The queue that tile_rows names, or null, and tile_rows without it; false: what cannot be.  Without a tile_group it is a hint, whatever it says.
+static bool take_queue(int& tile_rows, const int* tile_group, const int* n_tiles, int** queue) {
   const int which = tile_rows / TQ_TILE_QUEUE;
   *queue = nullptr;
-  if (tile_rows < TQ_TILE_QUEUE) return true;
+  if (!tile_group || tile_rows < TQ_TILE_QUEUE) return true;
   tile_rows %= TQ_TILE_QUEUE;
   *queue = const_cast<int*>(n_tiles) + 16 * which;
   return which <= 2 && n_tiles && tile_rows == 64 + TQ_TILE_PAIRS;
@@ -1135,7 +1135,7 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
   const int k_per = ((K + TBK - 1) / TBK + splits - 1) / splits * TBK;
   if (splits > 1 && (int64_t)(splits - 1) * k_per >= K) return TQ_ERR_BAD_ARG;
   int* queue;
-  if (!take_queue(tile_rows, n_tiles, &queue)) return TQ_ERR_BAD_ARG;
+  if (!take_queue(tile_rows, tile_group, n_tiles, &queue)) return TQ_ERR_BAD_ARG;
   MfmaGemmArgs g{(const bf16_t*)a, lda, a_rows, a_gather, (const bf16_t*)w, (const bf16_t*)w2, group_stride,
                  tile_group, n_tiles, bias, bias_type, out, ldc, M, N, K, splits > 1 ? k_per : K, (int64_t)M * ldc, gate, 1,
                  alone ? gate + 1 : 0, tq_pair_limit_host};
@@ -1245,7 +1245,7 @@ TQ_API int tq_gemm_mfma_pair(const int64_t* d1, const int64_t* d2, int splits2, 
   const int64_t* d[2] = {d1, d2};
   int tile_rows1 = (int)d1[17];
   int* queue;
-  if (!take_queue(tile_rows1, (const int*)d1[8], &queue)) return TQ_ERR_BAD_ARG;
+  if (!take_queue(tile_rows1, (const int*)d1[7], (const int*)d1[8], &queue)) return TQ_ERR_BAD_ARG;
   const bool many = tile_rows1 == 64 + TQ_TILE_PAIRS;
   for (int i = 0; i < 2; ++i) {
     const int64_t* p = d[i];
