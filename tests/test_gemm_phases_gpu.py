@@ -79,6 +79,18 @@ def test_the_feed_forward_asks_for_items_of_four(ops, monkeypatch, form):
         assert T == 215 or max(of) > 2
 
 
+def test_a_unit_of_half_a_thousand_million_rows(ops):
+    """What says that there are queues is no number of rows: an order of 2 GB, one unit with one row."""
+    st, slot, te, nt = order(ops, [1], 1 << 29, 2)
+    assert nt.tolist() == [1, 1] and te.tolist() == [0, 0] and slot.tolist() == [[0]]
+    assert st.numel() == 1 << 29 and st[0] == 0 and (st[1:] == -1).all()
+    ids = torch.zeros((1, 1), dtype=torch.int32, device=DEV)
+    out = torch.zeros(64, dtype=torch.int32, device=DEV)
+    for bad in (0, -1, ops.ORDER_QUEUES, ops.ORDER_QUEUES + 63, ops.ORDER_QUEUES + ops.ITEMS_OF_FOUR + 65):
+        assert ops.library("bfloat16").tq_moe_align(ids.data_ptr(), 1, 1, 1, bad, 64, out.data_ptr(), out.data_ptr(), out.data_ptr(), out.data_ptr(),
+                                                    torch.cuda.current_stream().cuda_stream) == -1
+
+
 # k: 2, 3, 4, 5 and 9 steps of 64 (the rings hold 2 to 4 tiles); columns: less than a wave's 32, no multiple of 8, one more than a tile
 @pytest.mark.parametrize("K,N", [(128, 24), (192, 100), (256, 129), (320, 256), (576, 263)])
 @pytest.mark.parametrize("gated", [True, False])

@@ -21,8 +21,9 @@
 // a unit of rows may be any number whose rows fit the order.
 #define TQ_ITEMS_OF_FOUR (1 << 30)
 // The row order's n_tiles may hold more than its two numbers, 48 in all, of which the last 32, two runs of 16, are queues: written with the
-// order (and the third, the experts that have rows) where TQ_ORDER_QUEUES is added to its unit, each for one product (tile_rows with TQ_TILE_QUEUE added once or twice) behind it.
-#define TQ_ORDER_QUEUES (1 << 29)
+// order (and the third, the experts that have rows) where TQ_ORDER_QUEUES is added to its unit of 64, each for one product (tile_rows with TQ_TILE_QUEUE added once or twice) behind it.
+// The sign: no unit of rows has it, and with any other unit than 64 it stays a negative number, which is refused.
+#define TQ_ORDER_QUEUES (-0x7fffffff - 1)
 #define TQ_TILE_QUEUE 2048
 #define TQ_GEMM_ACT_ALONE 256      // added to tq_gemm_mfma's gate: the activation of a plain product's result
 

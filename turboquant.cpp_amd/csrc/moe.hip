@@ -932,8 +932,8 @@ __global__ __launch_bounds__(64 * NW) void select_align_kernel(const float* __re
 // off `unit`.
 static int units_per_item(int& unit) {
   int per_item = 2;
-  if (unit >= TQ_ITEMS_OF_FOUR) unit -= TQ_ITEMS_OF_FOUR, per_item = 4;
-  if (unit >= TQ_ORDER_QUEUES) unit -= TQ_ORDER_QUEUES, per_item += TQ_WITH_QUEUES;
+  if (unit == 64 + TQ_ORDER_QUEUES || unit == 64 + TQ_ITEMS_OF_FOUR + TQ_ORDER_QUEUES) unit -= TQ_ORDER_QUEUES, per_item += TQ_WITH_QUEUES;
+  if (unit >= TQ_ITEMS_OF_FOUR) unit -= TQ_ITEMS_OF_FOUR, per_item += 2;
   return per_item;
 }
 

@@ -844,7 +844,7 @@ EXPERT_16_UPTO, EXPERT_32_UPTO = 5, 10
 EXPERT_128_FROM = EXPERT_256_FROM = 1 << 30
 TILE_PAIRS = 1024            # added to tile_rows 64: the units of an item, two or four of one expert, per workgroup (TQ_TILE_PAIRS)
 TILE_QUEUE = 2048            # added to that once or twice: the tiles are dealt from the order's first or second queue (TQ_TILE_QUEUE)
-ORDER_QUEUES = 1 << 29       # added to the row order's unit: two queues behind n_tiles, which the order zeroes (TQ_ORDER_QUEUES)
+ORDER_QUEUES = -1 << 31      # added to the row order's unit of 64: two queues behind n_tiles, which the order zeroes (TQ_ORDER_QUEUES)
 ITEMS_OF_FOUR = 1 << 30      # added to the row order's unit: its items hold four row tiles instead of two (TQ_ITEMS_OF_FOUR)
 ITEMS_OF_FOUR_FROM = 112, 88 # rows per expert on average from which items may hold four units, by expert_item_units
 EXPERT_PAIRS_FROM = 48       # rows per expert on average from which units of 64 are taken several at a time

@@ -18,7 +18,7 @@
 // expert, per workgroup (see tq_gemm_mfma)
 #define TQ_TILE_PAIRS 1024
 #define TQ_TILE_QUEUE 2048             /* added to that once or twice: its tiles are dealt from the order's first or second queue, one product each */
-#define TQ_ORDER_QUEUES (1 << 29)      /* added to the unit of the order of pairs by expert: n_tiles holds 48 ints, the last 32 of them two queues, which it zeroes */
+#define TQ_ORDER_QUEUES (-0x7fffffff - 1)      /* added to a unit of 64 of the order of pairs by expert: n_tiles holds 48 ints, the last 32 of them two queues, which it zeroes */
 #define TQ_ITEMS_OF_FOUR (1 << 30)      /* added to the unit of the order of pairs by expert: its items hold four row tiles, not two */
 #define TQ_GEMM_ACT_ALONE 256      // added to tq_gemm_mfma's gate: the activation of a plain product's result
 
