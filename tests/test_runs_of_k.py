@@ -37,3 +37,23 @@ def test_plain_products_of_a_long_k_stay_with_the_library_that_adds_it_in_parts(
     """Its sums of 32 bits are the closer ones to 64 bits; an activation or a gate's result of 16 bits keeps nothing of that."""
     assert not lib.tq_gemm_here_rather(M, N, K, 0)
     assert lib.tq_gemm_here_rather(2048, 6288, 2048, 0) and lib.tq_gemm_here_rather(2048, 5632, 2048, 2)
+
+
+@pytest.mark.parametrize("N", [8, 16, 32])
+def test_few_columns_stay_in_the_tile_kernel(lib, N):
+    """Tiles of 256 columns are nearly empty there: only a long k in one run and one round of tiles makes up for it, and a gated pair."""
+    for M in (1025, 4096, 16384, 16385, 65536):
+        for K in (128, 512, 1024, 1984, 2048, 4096):
+            here = lib.tq_gemm_phases_rows(M, N, K, 0, 1)
+            assert (here > 0) == (K >= 2048 and M <= 16384), (M, K)
+            assert not lib.tq_gemm_phases_rows(M, N, K, 0, 2) and lib.tq_gemm_phases_rows(M, N, K, 1, 1)
+            assert lib.tq_gemm_mfma_splits(M, N, K) == tile_kernel_runs(M, N, K)
+            assert lib.tq_gemm_phases_rows(M, 40, K, 0, 1)
+
+
+def test_one_round_of_the_tile_kernel_stays_its_own(lib):
+    """Partial sums of up to 128 columns in the tile kernel's runs; more runs than its are for the other tiles."""
+    for M, N, K, here in ((16384, 64, 2048, 0), (14000, 128, 2048, 0), (8192, 40, 4096, 0), (16384, 136, 2048, 1), (12000, 64, 2048, 1), (20000, 64, 2048, 1)):
+        runs = lib.tq_gemm_mfma_splits(M, N, K)
+        assert runs > 1 and (lib.tq_gemm_phases_rows(M, N, K, 0, runs) > 0) == bool(here), (M, N, K)
+        assert runs == tile_kernel_runs(M, N, K) or lib.tq_gemm_phases_rows(M, N, K, 0, runs)

@@ -996,6 +996,14 @@ static double phases_best(int M, int N, int K, bool dual, int runs, int* rows) {
   return best;
 }
 
+// Runs of k in the tile kernel where partial sums are wanted apart (see tq_gemm_mfma_splits).
+static int tile_kernel_runs(int M, int N, int K) {
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + TBN - 1) / TBN);
+  int s = 1;
+  while (s < 4 && tiles * s < 512 && K / (s * 2) >= 1024) s *= 2;
+  return s;
+}
+
 // Whether a product of one matrix, of more than 64 rows that follow one another, goes in the tiles of gemm_phases rather than those of
 // gemm_few_tiles or the tile kernel: k in whole tiles, and
 //  * more than 1,024 rows: always (us by the tile kernel and by gemm_phases: 1,280 rows by 2,048 x 2,048 31.8 and 25.3, 3,001 by 3,072 x
@@ -1008,11 +1016,26 @@ static double phases_best(int M, int N, int K, bool dual, int runs, int* rows) {
 //    2,816 x 1,024, 16.1 and 16.0; 160, 256 by 2,560 x 3,584, 32.5 and 34.7).
 // And columns in whole pieces of 16 bytes of the result: without, a lane's four or eight columns side by side go out one by one (10,405
 // by 314 x 320 15.3 and 20.2, 4,377 by 5,006 x 2,752 141 and 162, 727 by 5,583 x 448 15.8 and 22.8).
-static bool phases_suit(int M, int N, int K, bool dual) {
+// Up to 32 columns are an eighth of these tiles, and a quarter of the tile kernel's: plain products of those only with k long enough,
+// rows that are one round of tiles of 64, and no partial sums apart (by 16 columns, us by the tile kernel and by gemm_phases: 4,096 x 512
+// 11.2 and 12.5, 4,096 x 2,048 20.1 and 18.4, 28,000 x 2,048 25.6 and 28.4; apart 16,384 x 2,048 15.8 and 23.1, 8,192 x 4,096 18.2 and
+// 21.3; a gated pair gains everywhere).  Partial sums of up to 128 columns, half of these tiles, stay where the tile kernel's runs are
+// just one round of its tiles (14,000 by 40 x 2,048 19.0 and 21.4, 16,384 by 64 x 2,048 21.6 and 25.8).  runs: of k, 1 where they are not apart.
+static bool phases_suit(int M, int N, int K, bool dual, int runs) {
   if (M <= 64 || K % TBK || K < 2 * TBK || N % 8) return false;
+  if (!dual && N <= 32 && (runs > 1 || K < 2048 || M > 64 * 256)) return false;
+  const int round = (M + 127) / 128 * runs;
+  if (runs > 1 && N <= 128 && runs == tile_kernel_runs(M, N, K) && round >= 200 && round <= 256) return false;
   const int64_t rows = (M + 63) / 64, narrow = rows * ((N + 63) / 64), wide = rows * ((N + 127) / 128);
   if (M > 1024) return true;
   return dual ? narrow > 256 : wide > (M > 512 ? 256 : 512) && K >= 512;
+}
+// The height of those tiles for a product of one matrix whose rows follow one another (dual: a gated pair), k in `splits` runs; 0: it goes in others.
+TQ_API int tq_gemm_phases_rows(int M, int N, int K, int dual, int splits) {
+  if (!phases_suit(M, N, K, dual != 0, splits)) return 0;
+  int rows;
+  phases_best(M, N, K, dual != 0, splits, &rows);
+  return rows;
 }
 // Its runs of k where partial sums are wanted apart, `from` at least (the tile kernel's: fewer runs are longer sums, whose error against
 // 64 bits is the larger, 2.7e-7 of 2,048 products in one run and 1.9e-7 in two): what a run more saves must be more than writing and
@@ -1042,7 +1065,7 @@ static int phases_runs(int M, int N, int K, int from) {
 // result in float keeps what is gained.  Up to k 2,304 the error was the same in all of 24.  (A result of 16 bits is off by 1.7e-3.)
 TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
   const bool dual = kind == 2;
-  if (!phases_suit(M, N, K, dual)) return 0;
+  if (!phases_suit(M, N, K, dual, 1)) return 0;
   int rows;
   const double t = phases_best(M, N, K, dual, 1, &rows), flops = 2.0 * M * N * K * (dual ? 2 : 1);
   if (kind) return (dual ? t : 0.95 * t) <= (dual ? 14 : 11.5) + flops / 1.15e9 + (double)M * N * (dual ? 10 : 6) / 5.5e6;
@@ -1090,10 +1113,8 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K) {
     while (s < 8 && waves * s < 4096 && K / (16 * s) >= 128) s *= 2;
     return s;
   }
-  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + TBN - 1) / TBN);
-  int s = 1;
-  while (s < 4 && tiles * s < 512 && K / (s * 2) >= 1024) s *= 2;
-  if (phases_suit(M, N, K, false)) return phases_runs(M, N, K, s);
+  int s = tile_kernel_runs(M, N, K);
+  if (phases_suit(M, N, K, false, s)) return phases_runs(M, N, K, s);
   if (M <= 64 * 16) {      // tiles of 64 rows: more and shorter runs
     const int t = tile_runs(M, N, K);
     if (t > s) s = t;
@@ -1188,11 +1209,9 @@ TQ_API int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gat
     rc = launch_stream<4>(g, dual, out_act, 1, st, splits);
   } else {
     if ((N + TBN - 1) / TBN > 65535) return TQ_ERR_UNSUPPORTED;
-    if (!a_rows && phases_suit(M, N, K, dual)) {
-      int rows;
-      phases_best(M, N, K, dual, splits, &rows);
+    if (const int rows = a_rows ? 0 : tq_gemm_phases_rows(M, N, K, dual, splits))
       rc = launch_gemm_phases_plain(g, rows, dual, out_act, st);
-    } else if (few_tiles_suit(g, dual))
+    else if (few_tiles_suit(g, dual))
       rc = launch_few_tiles(g, dual, out_act, splits, st);
     else if (M <= 64 * 16 && !dual)
       rc = launch_tile<64, 2, 4>(g, dual, out_act, splits, st);

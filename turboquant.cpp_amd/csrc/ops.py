@@ -176,6 +176,7 @@ _OPTIONAL = {
                      _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "tq_gemm_mfma_splits": [_c_int, _c_int, _c_int],
     "tq_gemm_here_rather": [_c_int] * 4,
+    "tq_gemm_phases_rows": [_c_int] * 5,
     "tq_gemm_phases_pair_splits": [_c_int] * 6,
     "tq_gemm_mfma_pair_splits": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "tq_gemm_mfma_pair": [_c_ptr, _c_ptr, _c_int, _c_ptr],

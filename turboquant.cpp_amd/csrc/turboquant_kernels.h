@@ -73,6 +73,7 @@ int tq_gemm_generic(const void* a, int64_t lda, const int* a_rows, int a_gather,
 // gemm_mfma.hip: bfloat16 products on the matrix cores (bfloat16 library)
 int tq_gemm_mfma_splits(int M, int N, int K);
 int tq_gemm_here_rather(int M, int N, int K, int kind);
+int tq_gemm_phases_rows(int M, int N, int K, int dual, int splits);
 int tq_gemm_mfma(const void* a, int64_t lda, const int* a_rows, int a_gather, const void* w, const void* w2,
         int64_t group_stride, const int* tile_group, const int* n_tiles, const void* bias, int bias_type,
         void* out, int64_t ldc, int out_is_act, int M, int N, int K, int tile_rows, int splits, int gate,
