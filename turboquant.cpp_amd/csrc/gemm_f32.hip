@@ -90,7 +90,8 @@ __device__ __forceinline__ void f32_to_lds16(const float* src, float* wave_base)
 
 // With `part` set the grid's z cuts k into runs of k_per_split and the sums of run z go to part[z] ([run][M][N], the
 // gated pair's second product behind all the first ones) as they are: gemm_f32_reduce_kernel finishes them.
-template <int MI, int NI, bool DUAL>
+// GO_FIRST: a wave in the middle of its products goes before those of the other workgroups on its SIMD.
+template <int MI, int NI, bool DUAL, bool GO_FIRST>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k_per_split, float* part) {
   constexpr int BM = 64 * MI, BN = 64 * NI, ROWS = BM + BN * (DUAL ? 2 : 1), STAGE = ROWS * TBK, L = ROWS / 64;
   __shared__ __align__(16) float ring[TSTAGES * STAGE];
@@ -209,9 +210,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(F32GemmArgs g, int k
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (t + TSTAGES - 1 < steps) ask(t + TSTAGES - 1);
-    __builtin_amdgcn_s_setprio(1);
+    if constexpr (GO_FIRST) __builtin_amdgcn_s_setprio(1);
     multiply(ring + t % TSTAGES * STAGE);
-    __builtin_amdgcn_s_setprio(0);
+    if constexpr (GO_FIRST) __builtin_amdgcn_s_setprio(0);
   }
   if (left) {      // the last 4, 8 or 12 of k, through registers, zeros behind them
     __syncthreads();
@@ -532,14 +533,27 @@ TQ_API int tq_gemm_f32(const void* a, int64_t lda, const int* a_rows, int a_gath
     const int columns = narrow ? 64 : 128;
     const dim3 grid((M + 64 * mi - 1) / (64 * mi), (N + columns - 1) / columns, runs);
     if (grid.y > 65535) return TQ_ERR_UNSUPPORTED;
+    // A wave's priority where workgroups share SIMDs, that is more than one to a compute unit, and not where one row of tiles waits for w.
+    // Three to a unit are a round of 768; up to three rounds whose last leaves more than a quarter of the chip empty go without, since those
+    // that go first leave the others of their unit behind, which then end alone (times with it over without, 17 to 4,096 rows by 2,048 to
+    // 32,000 columns, k 512 to 5,632: up to 256 workgroups 1.01 to 1.03, to 768 0.96 to 1.00; 1,000 to 1,024 1.00 to 1.14, 2,000 to 2,048 1.04 to
+    // 1.10; 1,376 and 1,536 0.96 to 0.98, 2,752 and more 0.97 to 1.00 (two of 30 1.02 and 1.06); one row of tiles of a gated pair up to 1.08).
+    const int64_t n = (int64_t)grid.x * grid.y;      // (of experts: at most)
+    const bool first = grid.x > 1 && n > 256 && (grouped || n <= 768 || n >= 3 * 768 || n % 768 == 0 || n % 768 >= 576);
+#define TQ_F32_TILE(...)                                                                                                     \
+  do {                                                                                                                       \
+    if (first) hipLaunchKernelGGL((gemm_f32_tile_kernel<__VA_ARGS__, true>), grid, dim3(256), 0, st, g, k_per_split, part);  \
+    else hipLaunchKernelGGL((gemm_f32_tile_kernel<__VA_ARGS__, false>), grid, dim3(256), 0, st, g, k_per_split, part);       \
+  } while (0)
     if (mi == 1) {
-      if (narrow) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
-      else if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, true>), grid, dim3(256), 0, st, g, k_per_split, part);
-      else hipLaunchKernelGGL((gemm_f32_tile_kernel<1, 2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
+      if (narrow) TQ_F32_TILE(1, 1, true);
+      else if (dual) TQ_F32_TILE(1, 2, true);
+      else TQ_F32_TILE(1, 2, false);
     } else {
-      if (dual) hipLaunchKernelGGL((gemm_f32_tile_kernel<2, 1, true>), grid, dim3(256), 0, st, g, k_per_split, part);
-      else hipLaunchKernelGGL((gemm_f32_tile_kernel<2, 2, false>), grid, dim3(256), 0, st, g, k_per_split, part);
+      if (dual) TQ_F32_TILE(2, 1, true);
+      else TQ_F32_TILE(2, 2, false);
     }
+#undef TQ_F32_TILE
   }
   if (runs > 1) {
     const unsigned blocks = (unsigned)(((int64_t)M * N + 255) / 256);
