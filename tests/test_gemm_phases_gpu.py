@@ -271,24 +271,45 @@ def test_a_hint_of_any_size_is_ignored(ops, hint):
             assert torch.equal(both[0][0], both[1][0]) and torch.equal(both[0][1], both[1][1])
 
 
-def test_the_gate_over_its_whole_range(ops):
-    """silu in the tiles' epilogue against the tile kernel's, to the last bit of the 16-bit result but where a rounding is near: factors
-    that make every product one value from -1e5 to 1e5, among them those where the exponential leaves the range, zeros, infinities and NaN."""
-    x = torch.cat([torch.linspace(-100, 100, 4097), torch.tensor([0.0, -0.0, 86.9, 87.1, -86.9, -87.1, -88.8, 1e5, -1e5, 1e-30, -1e-38, float("inf"), float("-inf"), float("nan")])])
-    M, K, N = 1280, 128, 264
-    a = torch.zeros(M, K)
-    a[:, 0] = 1.0
-    w = torch.zeros(N, K)
-    w[:, 0] = x[torch.arange(N) * 16 % 4097]
-    w[-14:, 0] = x[-14:]
-    w2 = torch.zeros(N, K)
-    w2[:, 0] = 1.0
+# Values of a wave of 32 columns beside each other: its form of the gate hangs on whether one of them is 87 or more in size.  To the ends of
+# the shorter form; where an exponential one rounding off gives the next float; zeros and the smallest normal floats; NaN; both forms'
+# values, and infinities, in one wave.
+ROUNDED = [-73.06429, -30.360157, -60.720314, -40.9672, -57.091183, -15.313667, -74.74527, -61.679783, -46.15222, -76.990776, -54.57411,
+           -7.829238, -29.549843, -19.86942, -79.04454, 79.04454]
+GATED = [[s * v for v in (86.99, 86.5, 86.0, 85.5, 84.0, 83.0, 80.0, 70.0) for s in (1, -1)] * 2,
+         ROUNDED * 2,
+         [0.0, -0.0, 1e-30, -1e-30, 2.0 ** -126, -(2.0 ** -126), 2.0 ** -110, -(2.0 ** -120)] * 4,
+         [float("nan")] * 32,
+         [0.0, -0.0, 86.5, -86.5, 87.0, -87.0, 88.0, -88.5, 1e5, -1e5, 1e-30, float("inf"), float("-inf"), float("nan"), 3.0, -3.0] * 2,
+         [(i - 15.5) * 0.05 for i in range(32)],
+         [(i - 15.5) * 3.0 for i in range(32)],
+         [(-1) ** i * 2.0 ** (-i) for i in range(32)]]
+
+
+@pytest.mark.parametrize("out_act", [True, False])
+def test_the_gate_over_its_whole_range(ops, out_act):
+    """silu in the tiles' epilogue is the tile kernel's, bit for bit: each value of GATED, and 127 smaller multiples of it, in waves of the
+    shorter form, of the longer one, and of values that would take either.  And it is the formula's."""
+    x = torch.tensor(GATED).flatten()
+    M, K, N = 1280, 128, x.numel()
+    a, w, w2 = torch.zeros(M, K), torch.zeros(N, K), torch.zeros(N, K)
+    a[:, :3] = (1.0 - torch.arange(M) % 128 / 256.0)[:, None]
+    rest = x
+    for k in range(3):      # a float is three of 16 bits
+        w[:, k] = rest.bfloat16().float()
+        rest = torch.where(x.isfinite(), rest - w[:, k], 0.0)
+    a[:, 3] = w2[:, 3] = 1.0
     a, w, w2 = (t.to(torch.bfloat16).to(DEV) for t in (a, w, w2))
-    every = torch.arange(M, dtype=torch.int32, device=DEV)
-    got = ops.gemm(a, w, "bfloat16", w2=w2, out_act=True)
-    want = ops.gemm(a, w, "bfloat16", w2=w2, out_act=True, a_rows=every)
+    assert ops.library("bfloat16").tq_gemm_phases_rows(M, N, K, 1, 1)
+    with ops.own_products(True):
+        got = ops.gemm(a, w, "bfloat16", w2=w2, out_act=out_act)
+        want = ops.gemm(a, w, "bfloat16", w2=w2, out_act=out_act, a_rows=torch.arange(M, dtype=torch.int32, device=DEV))
+        z = ops.gemm(a, w, "bfloat16")
+    finite = x.isfinite() & (x.abs() > 1e-29)
+    assert torch.equal(z[0].cpu()[finite], x[finite])
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
-    z = w[:, 0].double().cpu()
-    exact = (z * torch.sigmoid(z)).expand(M, N)
-    finite = exact.isfinite() & (z.abs() < 87)
-    assert ((got.cpu().double() - exact).abs() <= exact.abs() * 2.0 ** -8 + 1e-40)[finite].all()
+    z = z.double().cpu()
+    exact, inside = z * torch.sigmoid(z), z.abs() < 87
+    # a rounding to 16 bits; in 32 bits those of the exponential (one place of its own), the sum and the quotient
+    bound = exact.abs() * (2.0 ** -8 if out_act else 3 * 2.0 ** -23) + 2.0 ** -126
+    assert inside.sum() > 0.8 * inside.numel() and ((got.cpu().double() - exact).abs() <= bound)[inside].all()

@@ -51,14 +51,16 @@ __device__ __forceinline__ void loads_left() {      // at most N loads of this w
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
-// x / (1 + exp(-x)) of N values, none of them beyond 87 in size: the exponential as expf does it there, without its tests for the ends of
-// the range, and the quotient by a reciprocal that one step sharpens and the remainder, which is exact, corrects (within 0.5 of the last
-// place but for one in some millions; over all floats of that range 0.281 of the last place off 64 bits in the root of the mean square,
-// as with a division).  17 instructions instead of 25.
+// x / (1 + exp(-x)) of N values, none of them 87 or more in size, to the same bits as the general form (compared over all floats of that
+// range), so that it makes no difference which form the other values of a wave ask for.  What is left out is what only the ends of the
+// range need.  The exponential: reduction to a power of two (Cody and Waite), with log2(e) in two floats and the product's rounding error by
+// a fused multiply-add.  The second float is the one that expf has here, whose neighbour is as near: with that one 15 results were the next
+// float.  The quotient: a reciprocal that one Newton step sharpens, and one correction by the remainder, whose sign is changed so that -0
+// stays -0.  17 instructions instead of 25.
 template <int N>
 __device__ __forceinline__ void silu_within(float (&v)[N]) {
 #pragma clang fp contract(off)      // (p - n is to be of the rounded p, whose rest stands apart)
-  constexpr float LOG2E = 1.44269504088896341f, LOG2E_REST = 1.92596299112661746e-8f;
+  constexpr float LOG2E = 1.44269504088896341f, LOG2E_REST = 0x1.4ae0bep-26f;
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     const float x = v[j], p = -x * LOG2E, rest = fmaf(-x, LOG2E_REST, fmaf(-x, LOG2E, -p)), n = rintf(p);
@@ -66,7 +68,7 @@ __device__ __forceinline__ void silu_within(float (&v)[N]) {
     float r = __builtin_amdgcn_rcpf(d);
     r = fmaf(fmaf(-d, r, 1.0f), r, r);
     const float q = x * r;
-    v[j] = fmaf(fmaf(-d, q, x), r, q);
+    v[j] = fmaf(-fmaf(d, q, -x), r, q);
   }
 }
 
