@@ -172,32 +172,38 @@ def test_a_product_beside_the_experts(ops, T, K, N, K2, N2, gated):
             assert ((y2[z].double() - exact).abs() <= K2 * 2.0 ** -24 * (az.abs() @ bz.abs().T) + 2.0 ** -23 * exact.abs()).all()
 
 
-# rows, columns, k and the height of the tiles that suits: each height; the fewest rows of each rule (65 and 129, 513 to 1,024, 1,025);
-# a few columns past a tile, less than a wave's 32; two and three steps of k; a last tile of one row; and columns it leaves to the tile kernel
-@pytest.mark.parametrize("M,N,K", [(1025, 24, 128), (1100, 4200, 128), (700, 3104, 512), (65, 66048, 512), (1030, 4104, 192), (515, 16600, 512), (130, 33000, 576),
-                                   (2049, 6400, 192), (3001, 5000, 128), (2999, 8000, 320), (1025, 4100, 128)])
-def test_products_of_one_matrix(ops, M, N, K):
+# rows, columns, k and the height of the tiles that suits (0: it goes in others): each height; the fewest rows of each rule (65 and 129, 513 to
+# 1,024, 1,025); a few columns past a tile, less than a wave's 32; two and three steps of k; a last tile of one row; columns and a k left to the tile kernel
+@pytest.mark.parametrize("M,N,K,rows", [(1025, 24, 2048, 64), (1025, 40, 128, 64), (1100, 4200, 128, 128), (700, 3104, 512, 64), (65, 66048, 512, 128), (1030, 4104, 192, 128),
+                                        (515, 16600, 512, 192), (130, 33000, 576, 192), (2049, 6400, 192, 256), (3001, 5000, 128, 256), (2999, 8000, 320, 192),
+                                        (1025, 4100, 128, 0), (1025, 24, 128, 0)])
+def test_products_of_one_matrix(ops, M, N, K, rows):
     """Plain products in these tiles are the tile kernel's bits (which gathered rows keep to), with a bias, into either type, through an
     activation and in runs of k; and the formula's values."""
+    assert ops.library("bfloat16").tq_gemm_phases_rows(M, N, K, 0, 1) == rows
     a, w = drawn((M, K), 1), drawn((N, K), 2, 0.1)
     every = torch.arange(M, dtype=torch.int32, device=DEV)
     bias = torch.randn(N, generator=torch.Generator().manual_seed(4)).to(DEV)
     for form in (dict(), dict(bias=bias), dict(out_act=True, bias=bias.bfloat16()), dict(out_act=True, activation="gelu", act_alone=True, bias=bias)):
-        assert torch.equal(ops.gemm(a, w, "bfloat16", **form), ops.gemm(a, w, "bfloat16", a_rows=every, **form)), form
+        with ops.own_products(True):
+            assert torch.equal(ops.gemm(a, w, "bfloat16", **form), ops.gemm(a, w, "bfloat16", a_rows=every, **form)), form
     runs = ops.gemm(a, w, "bfloat16", bias=bias, partial_sums=True)
     x, y = a.double(), w.double()
     assert ((runs.double().sum(0) - (x @ y.T + bias.double())).abs() <= (K + 4) * 2.0 ** -24 * (x.abs() @ y.abs().T + bias.double().abs())).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 16500, 128), (1500, 2100, 192), (129, 20000, 128), (200, 16500, 192), (2049, 5000, 192), (1025, 8, 128)])
-def test_gated_pairs_of_one_matrix(ops, M, N, K):
+@pytest.mark.parametrize("M,N,K,rows", [(65, 16504, 128, 128), (1500, 2104, 192, 128), (129, 20000, 128, 192), (200, 16504, 192, 256), (2049, 5000, 192, 192),
+                                        (1025, 8, 128, 64), (1500, 2100, 192, 0)])
+def test_gated_pairs_of_one_matrix(ops, M, N, K, rows):
     """As above, of two matrices behind each other and apart, with and without a limit."""
+    assert ops.library("bfloat16").tq_gemm_phases_rows(M, N, K, 1, 1) == rows
     a, both = drawn((M, K), 1), drawn((2 * N, K), 2, 0.1)
     w, w2, every = both[:N], both[N:], torch.arange(M, dtype=torch.int32, device=DEV)
     for form in (dict(out_act=True), dict(), dict(out_act=True, pair_limit=0.6), dict(out_act=True, activation="gelu_tanh")):
-        want = ops.gemm(a, w, "bfloat16", w2=w2, a_rows=every, **form)
-        assert torch.equal(ops.gemm(a, w, "bfloat16", w2=w2.clone(), **form), want), form
-        assert torch.equal(ops.gemm(a, w, "bfloat16", w2=w2, **form), want) or M >= ops.VENDOR_MIN_ROWS, form
+        with ops.own_products(True):
+            want = ops.gemm(a, w, "bfloat16", w2=w2, a_rows=every, **form)
+            assert torch.equal(ops.gemm(a, w, "bfloat16", w2=w2.clone(), **form), want), form
+            assert torch.equal(ops.gemm(a, w, "bfloat16", w2=w2, **form), want), form
 
 
 def test_runs_of_k_of_one_matrix(ops):
@@ -269,6 +275,21 @@ def test_a_hint_of_any_size_is_ignored(ops, hint):
         if M <= 16:
             both = [ops.gemm_pair(dict(a=a, w=w, tile_rows=r), dict(a=a, w=w2, tile_rows=r), "bfloat16") for r in (16, hint)]
             assert torch.equal(both[0][0], both[1][0]) and torch.equal(both[0][1], both[1][1])
+
+
+# rows and columns of each kernel of plain products: streaming, tiles of few workgroups, the tile kernel, these tiles by 16 bytes and by pairs
+@pytest.mark.parametrize("M,N", [(3, 264), (40, 264), (300, 264), (1025, 261), (1100, 264)])
+def test_rounding_to_16_bits(ops, M, N):
+    """Results of 16 bits are the nearest, of two as near the even one: biases of 32 bits beside rows of zeros.  Among them both sides of
+    ties, the largest that stay finite, subnormal numbers of 16 bits, infinities and NaN."""
+    bits = [h << 16 | low for h in (0x3F80, 0x3F81, 0x0000, 0x0001, 0x007F, 0x0080, 0x7F7F, 0x7F7E, 0x4123) for low in (0, 1, 0x7FFF, 0x8000, 0x8001, 0xFFFF)]
+    bits += [b | 1 << 31 for b in bits] + [0x7F800000, 0xFF800000, 0x7F800001, 0x7FC00000, 0xFFFFFFFF]
+    bias = torch.tensor([bits[i % len(bits)] for i in range(N)], dtype=torch.int64).to(torch.int32).view(torch.float32)
+    a, w = torch.zeros(M, 128, dtype=torch.bfloat16, device=DEV), drawn((N, 128), 2)
+    with ops.own_products(True):
+        got = ops.gemm(a, w, "bfloat16", bias=bias.to(DEV), out_act=True).cpu()
+    want = bias.bfloat16().expand(M, N)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0))
 
 
 # Values of a wave of 32 columns beside each other: its form of the gate hangs on whether one of them is 87 or more in size.  To the ends of
