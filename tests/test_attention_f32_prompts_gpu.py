@@ -60,3 +60,19 @@ def test_more_workgroups_than_a_dimension_of_the_grid_holds():
         runs = dict(cu_seqlens=i32([0, 70, 75]), slots=i32([0, 1]), start=i32([0, 0]), max_new=longest, max_end=70, decode=False)
         return ops.attention(q, kp.flatten(), vp.flatten(), 0, pos, seq, table, page, nh * page * hd, nh, nh, hd, None, hd ** -0.5, "float32", runs=runs)
     assert torch.equal(attend(64 * 2_900_000), attend(70))
+
+
+def test_16_bit_prompts_refuse_more_workgroups_than_a_grid_holds():
+    """Their launch has one dimension: beyond what 32 bits count it would leave its output as it was, so it is an error."""
+    from turboquant_cpp_amd.csrc import ops
+    page, hd, nh, lens = 64, 32, 3, [70, 5]
+    gen = torch.Generator().manual_seed(1)
+    kp, vp, q = (torch.randn(*s, generator=gen).bfloat16().to(DEV) for s in ((3, nh, page, hd), (3, nh, hd, page), (sum(lens), nh * hd)))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    table, pos, seq = i32([[2, 0], [1, 0]]), i32([p for n in lens for p in range(n)]), i32([i for i, n in enumerate(lens) for _ in range(n)])
+    def attend(longest):
+        runs = dict(cu_seqlens=i32([0, 70, 75]), slots=i32([0, 1]), start=i32([0, 0]), max_new=longest, max_end=70, decode=False)
+        return ops.attention(q, kp.flatten(), vp.flatten(), 0, pos, seq, table, page, nh * page * hd, nh, nh, hd, None, hd ** -0.5, "bfloat16", runs=runs)
+    with pytest.raises(Exception):
+        attend(128 * 2_900_000)
+    assert torch.equal(attend(64 * 2_700_000 // nh), attend(70))

@@ -896,13 +896,14 @@ __global__ __launch_bounds__(128) void attn_join_diff_kernel(AttnArgs a, DiffArg
 }
 
 // ------------------------------------------------------------------------------------------ launch
+#define PREFILL_GRID 0xFFFFFF      // most workgroups of 256 of a launch: HIP counts the threads of a dimension in 32 bits, and what is beyond does not run
 template <int DT, int QG, bool EXACT, bool MOD, int VD = DT>
 static int launch_prefill_as(const AttnArgs& a, int B, int max_new, hipStream_t st) {
   const size_t shmem = (DT > ATTN_TWO_BUFFERS_UP_TO ? 1 : 2) * (EXACT ? (size_t)TILE * (a.hd + 16 * VD) : (size_t)TILE * (a.hd + KPAD) + (size_t)a.hd * VSTR) * sizeof(bf16_t);
   if (shmem > 48 * 1024)
     (void)hipFuncSetAttribute((const void*)attn_prefill_kernel<DT, QG, EXACT, MOD, VD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   const int n_blocks = (max_new + 64 * QG - 1) / (64 * QG);
-  if ((int64_t)n_blocks * a.nh * B > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
+  if ((int64_t)n_blocks * a.nh * B > PREFILL_GRID) return TQ_ERR_UNSUPPORTED;
   hipLaunchKernelGGL((attn_prefill_kernel<DT, QG, EXACT, MOD, VD>), dim3(n_blocks * a.nh * B), dim3(256), shmem, st, a, n_blocks, B, DiffArgs{});
   return 0;
 }
@@ -947,7 +948,7 @@ static int launch_diff_prefill(const AttnArgs& a, const DiffArgs& df, int B, int
   if (shmem > 48 * 1024)
     (void)hipFuncSetAttribute((const void*)attn_prefill_kernel<DT, 2, EXACT, false, DT, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   const int n_blocks = (max_new + 63) / 64;
-  if ((int64_t)n_blocks * a.nh * B > 0x7fffffff) return TQ_ERR_UNSUPPORTED;
+  if ((int64_t)n_blocks * a.nh * B > PREFILL_GRID) return TQ_ERR_UNSUPPORTED;
   hipLaunchKernelGGL((attn_prefill_kernel<DT, 2, EXACT, false, DT, true>), dim3(n_blocks * a.nh * B), dim3(256), shmem, st, a, n_blocks, B, df);
   return 0;
 }
