@@ -561,7 +561,8 @@ __global__ __launch_bounds__(512) void gemm_phases_kernel(MfmaGemmArgs g, int gy
     // against 5.5 TB/s: 230 rows), they are spread among those that wait for memory.  us spread and first, gated pairs of 60 experts of
     // 1,408 x 2,048 beside one of 5,632: 60 rows each 191 and 179, 100 203 and 222, 137 241 and 253, 200 275 and 296, 260 361 and 369,
     // 330 456 and 445, 1,650 1,848 and 1,795; 64 of 2,560 x 3,584 beside 20,480: 60 543 and 547, 137 713 and 751, 260 1,170 and 1,121,
-    // 1,650 6,190 and 5,688.
+    // 1,650 6,190 and 5,688.  (With padding 260 rows are 291 of the 60 and 290 of the 64: the upper line lies where the narrower experts lose
+    // 2 % and the wider gain 4, and between 200 and 260 nothing was timed.)
     const int per_expert = s.n_units * 64 / max(g.n_tiles[2], 1);      // rows, padding among them
     if (per_expert >= 270 || per_expert <= 100) s.first2 = 1;
   }
