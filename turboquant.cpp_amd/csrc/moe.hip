@@ -73,12 +73,10 @@ __device__ __forceinline__ void wave_sums(float* s) {
 // 16-byte reads from LDS then lie side by side with its neighbours'), block after block.  In LDS a token's row is
 // filled with zeros up to a multiple of 512, so the last block needs no predicate: there the weights are read
 // from the row's last elements instead, and multiplied by zeros.
+// xs: [TG][Hp] of LDS.  The workgroup takes the rows of its part out of `parts`; logit (token k of its, row e) goes to out[k * rows + e].
 template <class W, int TG, int RW, int TH>
-__global__ __launch_bounds__(TH, TH == 512 ? 4 : 1) void router_logits_kernel(const float* __restrict__ x, const W* __restrict__ wr,
-                                                            const W* __restrict__ shared_w, int rows, int E,
-                                                            float* __restrict__ logits, int T, int H,
-                                                            const float* __restrict__ bias) {
-  extern __shared__ __attribute__((aligned(16))) float xs[];      // [TG][Hp]
+__device__ __forceinline__ void token_logits(const float* __restrict__ x, const W* __restrict__ wr, const W* __restrict__ shared_w, int rows,
+                                             int E, float* out, int T, int H, const float* __restrict__ bias, float* xs, int part, int parts) {
   const int Hp = (H + 511) / 512 * 512;
   const int t0 = blockIdx.x * TG;
   const int nt = min(TG, T - t0);
@@ -104,7 +102,7 @@ __global__ __launch_bounds__(TH, TH == 512 ? 4 : 1) void router_logits_kernel(co
   __syncthreads();
   // workgroups start at different rows, so that they do not all ask for the same row at once
   const int rot = (blockIdx.x * 5) % rows;
-  for (int idx = (blockIdx.y * (TH / TQ_WAVE) + wave) * RW; idx < rows; idx += gridDim.y * (TH / TQ_WAVE) * RW) {
+  for (int idx = (part * (TH / TQ_WAVE) + wave) * RW; idx < rows; idx += parts * (TH / TQ_WAVE) * RW) {
     const W* row[RW];
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
@@ -173,9 +171,18 @@ __global__ __launch_bounds__(TH, TH == 512 ? 4 : 1) void router_logits_kernel(co
     const int r = lane / LANES / TG, k = lane / LANES % TG;
     if (lane % LANES == 0 && k < nt && idx + r < rows) {      // (a bias per expert, not for the shared expert's gate row)
       const int i = idx + r + rot, at = i < rows ? i : i - rows;
-      logits[(size_t)(t0 + k) * rows + at] = bias && at < E ? s[0] + bias[at] : s[0];
+      out[(size_t)k * rows + at] = bias && at < E ? s[0] + bias[at] : s[0];
     }
   }
+}
+
+template <class W, int TG, int RW, int TH>
+__global__ __launch_bounds__(TH, TH == 512 ? 4 : 1) void router_logits_kernel(const float* __restrict__ x, const W* __restrict__ wr,
+                                                            const W* __restrict__ shared_w, int rows, int E,
+                                                            float* __restrict__ logits, int T, int H,
+                                                            const float* __restrict__ bias) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];      // [TG][Hp]
+  token_logits<W, TG, RW, TH>(x, wr, shared_w, rows, E, logits + (size_t)blockIdx.x * TG * rows, T, H, bias, xs, blockIdx.y, gridDim.y);
 }
 
 // The group score of every lane's group where groups are runs of PER neighbouring lanes (a power of two): its largest value or, with
@@ -482,7 +489,9 @@ static int launch_router_logits(const float* x, const void* wr, const void* shar
   // 512 12.9 and 10.5, 700 15.9 and 11.8; 256 experts: 64 16.5 and 16.5, 240 22.2 and 19.5, 512 27.3 and 24.2; rows of 3,584, 114 KB
   // of LDS, 2,048 tokens 42.7 and 33.1.
   const bool many = T >= TQ_ROUTER_MANY && hp * RT * sizeof(float) <= 160 * 1024;
-  int tg = RT;
+  // Where two such workgroups do not share a unit and there are more than units: 4 of them (13,197 tokens of 3,584, with the choice and the order, 192 and 166 us).
+  const bool wide = many && T > 2048 && hp * RT * sizeof(float) > 80 * 1024;
+  int tg = wide ? 4 : RT;
   while (!many && tg > 1 && (size_t)tg * hp * sizeof(float) > 32 * 1024) tg /= 2;   // small enough for several workgroups per CU
   const size_t shmem = (size_t)tg * hp * sizeof(float);
   if (shmem > 160 * 1024) return TQ_ERR_UNSUPPORTED;
@@ -508,7 +517,8 @@ static int launch_router_logits(const float* x, const void* wr, const void* shar
     else TQ_ROUTER(TGV, 1, THV);            \
   } while (0)
   TQ_DISPATCH_W(wtype, {
-    if (many) TQ_ROUTER_RW(8, 512);
+    if (wide) TQ_ROUTER_RW(4, 512);
+    else if (many) TQ_ROUTER_RW(8, 512);
     else if (tg == 8) TQ_ROUTER_RW(8, 256);
     else if (tg == 4) TQ_ROUTER_RW(4, 256);
     else if (tg == 2) TQ_ROUTER_RW(2, 256);
@@ -625,11 +635,11 @@ __device__ __forceinline__ bool clear_queues(int* __restrict__ n_tiles, int& per
 }
 
 // Wave 0 of a workgroup turns the experts' padded sizes starts[e] into their first rows (an exclusive scan, each lane
-// a contiguous run of experts) and writes the row tiles' experts, the items and their numbers.
+// a contiguous run of experts) and (`write`) writes the row tiles' experts, the items and their numbers.
 __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int per_item, int cap,
-                                            int* __restrict__ tile_expert, int* __restrict__ n_tiles) {
+                                            int* __restrict__ tile_expert, int* __restrict__ n_tiles, bool write = true) {
   const int lane = threadIdx.x % TQ_WAVE;
-  const bool queues = clear_queues(n_tiles, per_item);
+  const bool queues = write && clear_queues(n_tiles, per_item);
   {
     const int chunk = (E + TQ_WAVE - 1) / TQ_WAVE;
     const int e0 = lane * chunk, e1 = min(E, e0 + chunk);
@@ -645,14 +655,14 @@ __device__ __forceinline__ void scan_starts(int* starts, int E, int unit, int pe
     for (int e = e0; e < e1; ++e) {
       const int padded = starts[e];
       starts[e] = row;
-      for (int j = 0; j < padded / unit; ++j) {
+      for (int j = 0; write && j < padded / unit; ++j) {
         tile_expert[row / unit + j] = e;
         if (j % per_item == 0) items[item++] = row / unit + j;
       }
       row += padded;
     }
     const int used = queues ? wave_scan_add(live) : 0;
-    if (lane == TQ_WAVE - 1) {
+    if (write && lane == TQ_WAVE - 1) {
       n_tiles[0] = incl / unit;
       n_tiles[1] = iincl;
       if (queues) n_tiles[2] = used;
@@ -726,6 +736,99 @@ __global__ __launch_bounds__(64 * AW) void moe_align_kernel(const int* __restric
                                                             int* __restrict__ n_tiles, int n_real) {
   extern __shared__ int cnt[];
   align_pairs<AW>(ids, n_pairs, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, cnt, n_real);
+}
+
+// The choice and the same order by many workgroups, for steps of more than a handful of tokens: two launches.
+//  * route_choose: a workgroup of eight waves has the logits of its TG tokens in LDS, a wave each chooses for them, and one wave ranks their
+//    pairs and leaves how many each expert has in table[workgroup][e];
+//  * route_place: every workgroup adds the table up for itself, all of it for the experts' first rows (the first workgroup writes the row tiles
+//    and items from them) and what stands before its own segments (a segment: the pairs of one workgroup of route_choose), and gives its pairs their rows.
+// The results are those of the one workgroup: pairs in order of expert and, within an expert, of pair.
+// What bounds them is waiting: a launch, the activations, the rows of wr twice, the choice; and a launch, the table, two barriers, a pair's
+// rank.  us by logits, choice and order apart (five launches; six from 8,192 pairs on) and by these, in a graph: 60 experts of 2,048 and a
+// shared one, four a token: 513 tokens 19.0 and 16.1, 1,024 20.6 and 17.4, 2,048 26.8 and 22.3, 3,001 38.3 and 29.5, 8,192 62.5 and 55.2; 32
+// of 1,024: 2,048 tokens 19.7 and 13.7; 64 of 3,584, eight a token: 1,500 48.3 and 31.6, 4,096 69.2 and 60.9; 256 experts, 2,048 tokens 78.2
+// and 63.3.
+template <class W, int TG>
+__global__ __launch_bounds__(512, 4) void route_choose_kernel(const float* __restrict__ x, const W* __restrict__ wr, const W* __restrict__ shared_w,
+                                                              int rows, int E, int T, int H, const float* __restrict__ bias, int topk, int renorm,
+                                                              int groups, int keep, const float* __restrict__ correction, int n_real,
+                                                              float wscale, int* __restrict__ ids, float* __restrict__ weights,
+                                                              float* __restrict__ shared_gate, int cap, int* __restrict__ sorted_token,
+                                                              int* __restrict__ pair_slot, int* __restrict__ table) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];      // [TG][Hp], then [TG][rows] logits, [TG][E] of the choice, [TG][topk] ids, [E] counts
+  const int Hp = (H + 511) / 512 * 512, t0 = blockIdx.x * TG, nt = min(TG, T - t0), wave = threadIdx.x / TQ_WAVE;
+  float* logits = xs + TG * Hp;
+  float* lg = logits + TG * rows;
+  int* ids_l = (int*)(lg + TG * E);
+  int* cnt = ids_l + TG * topk;
+  for (int i = blockIdx.x * 512 + threadIdx.x; i < cap; i += gridDim.x * 512) sorted_token[i] = -1;
+  for (int e = threadIdx.x; e < E; e += 512) cnt[e] = 0;
+  token_logits<W, TG, 4, 512>(x, wr, shared_w, rows, E, logits, T, H, bias, xs, 0, 1);
+  __syncthreads();
+  if (wave < nt)
+    select_token(logits + wave * rows, rows, E, topk, renorm, groups, keep, lg + wave * E, ids + (size_t)(t0 + wave) * topk, ids_l + wave * topk,
+                 weights + (size_t)(t0 + wave) * topk, shared_gate + t0 + wave, correction, n_real, wscale);
+  __syncthreads();
+  if (wave) return;
+  int my_e, my_rank;
+  rank_segment(ids_l, 0, nt * topk, E, cnt, pair_slot + (size_t)t0 * topk, false, my_e, my_rank);
+  __builtin_amdgcn_wave_barrier();
+  for (int e = threadIdx.x; e < E; e += TQ_WAVE) table[(size_t)blockIdx.x * E + e] = cnt[e];
+}
+
+// per: segments of a workgroup; seg: pairs of a segment.  LDS: [2][C][E] sums, [E] first rows, [per][E] a segment's first rows.
+#define RP 1024      // threads
+__global__ __launch_bounds__(RP) void route_place_kernel(const int* __restrict__ ids, int n_pairs, int E, int topk, int V, int per, int seg,
+                                                         const int* __restrict__ table, int unit, int per_item, int cap,
+                                                         int* __restrict__ sorted_token, int* __restrict__ pair_slot,
+                                                         int* __restrict__ tile_expert, int* __restrict__ n_tiles, int n_real) {
+  extern __shared__ int sm_p[];
+  const int C = max(RP / E, 1), v0 = blockIdx.x * per, v1 = min(v0 + per, V), n = v1 - v0;
+  int* all = sm_p;
+  int* before = all + C * E;
+  int* starts = before + C * E;
+  int* first = starts + E;
+  for (int idx = threadIdx.x; idx < n * E; idx += RP) first[idx] = table[(size_t)v0 * E + idx];
+  for (int idx = threadIdx.x; idx < C * E; idx += RP) {      // thread (c, e): segments c, c + C, ..
+    const int c = idx / E, e = idx % E;
+    int sum = 0, mine = 0;
+    for (int v = c; v < V; v += 8 * C) {
+      int t[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) t[u] = table[(size_t)min(v + u * C, V - 1) * E + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        sum += v + u * C < V ? t[u] : 0;
+        mine += v + u * C < v0 ? t[u] : 0;
+      }
+    }
+    all[idx] = sum;
+    before[idx] = mine;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += RP) {
+    int total = 0, mine = 0;
+    for (int c = 0; c < C; ++c) {
+      total += all[c * E + e];
+      mine += before[c * E + e];
+    }
+    starts[e] = e < n_real ? (total + unit - 1) / unit * unit : 0;
+    for (int s = 0; s < n; ++s) {
+      const int c = first[s * E + e];
+      first[s * E + e] = mine;
+      mine += c;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x / TQ_WAVE == 0) scan_starts(starts, E, unit, per_item, cap, tile_expert, n_tiles, blockIdx.x == 0);
+  __syncthreads();
+  const int beg = v0 * seg, end = min(v1 * seg, n_pairs);
+  for (int i = beg + threadIdx.x; i < end; i += RP) {
+    const int e = ids[i], r = starts[e] + first[(i - beg) / seg * E + e] + pair_slot[i];
+    pair_slot[i] = e < n_real ? r : -1;
+    if (e < n_real) sorted_token[r] = i / topk;
+  }
 }
 
 // The same order by several workgroups, for steps of many tokens (one workgroup's waves go through 32,768 pairs in
@@ -959,6 +1062,55 @@ TQ_API int tq_moe_align(const int* ids, int n_pairs, int E, int topk, int unit, 
   return moe_align_impl(ids, n_pairs, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, st, E);
 }
 
+// The choice and the order in two launches by many workgroups, or ROUTE_OTHERWISE: more activations or experts than the LDS holds, or so
+// many segments that every workgroup's way through the table costs more than the launches saved (256 experts, us apart and this way: 2,048
+// tokens, 65,536 counts, 78 and 63, 3,001 tokens, 96,256, 108 and 111, 8,192, 262,144, 191 and 224).
+// table: T * E ints.
+#define ROUTE_OTHERWISE (-1000)
+static int route_many(const float* x, const void* wr, const void* shared_w, const float* bias, int wtype, int E, int topk, int renorm,
+                      int groups, int keep, int* ids, float* weights, float* shared_gate, int* table, int unit, int per_item, int cap,
+                      int* sorted_token, int* pair_slot, int* tile_expert, int* n_tiles, int T, int H, hipStream_t st,
+                      const float* correction, int n_real, float wscale) {
+  if (topk < 1 || topk > 64 || topk > E || E > 8192) return TQ_ERR_UNSUPPORTED;
+  const int rows = E + (shared_w ? 1 : 0), n_pairs = T * topk;
+  if (unit < 1 || cap % unit != 0 || cap < n_pairs + (E < n_pairs ? E : n_pairs) * (unit - 1)) return TQ_ERR_BAD_ARG;
+  const size_t hp = ((size_t)H + 511) / 512 * 512;
+  auto lds = [&](int tg) { return (tg * (hp + rows + E + topk) + E) * 4; };
+  // So few tokens to a workgroup that there is one to a compute unit while they last, and where there are more, that two share one.
+  int tg = T <= 512 ? 2 : T <= 1024 ? 4 : 8;
+  while (tg > 1 && lds(tg) > (T > 2048 ? 80 : 160) * 1024) tg /= 2;
+  const int V = (T + tg - 1) / tg, fit = 12 * 1024 / E;      // segments whose first rows 48 KB hold
+  if (lds(tg) > 160 * 1024 || (int64_t)V * E > 65536) return ROUTE_OTHERWISE;
+  int per = (V + 63) / 64;
+  if (per < 16) per = 16;
+  if (per > fit) per = fit;
+  const int C = RP / E > 1 ? RP / E : 1;
+  const size_t lds_place = ((size_t)(2 * C + 1 + per) * E) * sizeof(int);
+  if (per < 1 || lds_place > 64 * 1024) return ROUTE_OTHERWISE;
+  const size_t shmem = lds(tg);
+#define TQ_CHOOSE(TGV)                                                                                                                    \
+  do {                                                                                                                                    \
+    if (shmem > 48 * 1024)                                                                                                                \
+      (void)hipFuncSetAttribute((const void*)route_choose_kernel<W, TGV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem); \
+    hipLaunchKernelGGL((route_choose_kernel<W, TGV>), dim3(V), dim3(512), shmem, st, x, (const W*)wr, (const W*)shared_w, rows, E, T, \
+                       H, bias, topk, renorm, groups, keep, correction, n_real, wscale, ids, weights, shared_gate, cap, sorted_token, \
+                       pair_slot, table);                                                                                                 \
+  } while (0)
+  TQ_DISPATCH_W(wtype, {
+    if (tg == 8) TQ_CHOOSE(8);
+    else if (tg == 4) TQ_CHOOSE(4);
+    else if (tg == 2) TQ_CHOOSE(2);
+    else TQ_CHOOSE(1);
+  });
+#undef TQ_CHOOSE
+  if (lds_place > 48 * 1024)
+    (void)hipFuncSetAttribute((const void*)route_place_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_place);
+  hipLaunchKernelGGL(route_place_kernel, dim3((V + per - 1) / per), dim3(RP), lds_place, st, ids, n_pairs, E, topk, V, per, tg * topk, table, unit,
+                     per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, n_real);
+  TQ_LAUNCH_CHECK();
+  return 0;
+}
+
 // tq_router_topk followed by tq_moe_align; up to 16 tokens take two kernels instead of three, and from 8,192 pairs on
 // several workgroups order the pairs (the same order).  logits: scratch of T * (E + 1) floats (T * E without a shared
 // gate vector); what it holds afterwards means nothing.
@@ -972,6 +1124,14 @@ static int route_impl(const float* x, const void* wr, const void* shared_w, cons
   if (!groups_ok(E, topk, groups, keep)) return TQ_ERR_BAD_ARG;
   const size_t shmem = ((size_t)(AW + 1) * E + (size_t)AW * topk + (size_t)AW * E) * 4;
   if (T > AW || shmem > 64 * 1024) {
+    // Fewer tokens: the rows of wr dealt over more workgroups than there are tokens gain more than a launch costs (us apart and in
+    // two launches: 60 experts, 200 tokens 12.8 and 14.7, 400 15.7 and 15.6, 512 16.1 and 15.7; 80, 400 16.5 and 17.7, 513 20.8 and 18.4;
+    // 256, 401 35.5 and 41.0, 700 44.6 and 45.2, 1,024 48.9 and 46.3).
+    if (T >= (E <= 128 ? 512 : 1024)) {
+      const int rc = route_many(x, wr, shared_w, bias, wtype, E, topk, renorm, groups, keep, ids, weights, shared_gate, (int*)logits, unit, per_item,
+                                cap, sorted_token, pair_slot, tile_expert, n_tiles, T, H, st, correction, n_real, wscale);
+      if (rc != ROUTE_OTHERWISE) return rc;
+    }
     const int rc = router_topk_impl(x, wr, shared_w, bias, wtype, E, topk, renorm, groups, keep, ids, weights,
                                     shared_gate, logits, T, H, st, correction, n_real, wscale);
     if (rc) return rc;
