@@ -1052,6 +1052,8 @@ static int phases_runs(int M, int N, int K, int from) {
   return best;
 }
 
+TQ_API int tq_gemm_mfma_splits(int M, int N, int K);
+
 // Whether a product of many rows that the vendor's library would take is the faster one here.  kind 0: plain; 1: its result passes an
 // activation alone; 2: a gated pair, both into the activation type. The library's kernels leave their sums in float for a pass of its
 // own to apply the activation, so that against them stand 14 us (11.5 of an activation alone), the multiply-adds at 1,150 TFLOP/s and
@@ -1063,8 +1065,17 @@ static int phases_runs(int M, int N, int K, int from) {
 // for many a size: the slower kernel (13,197 by 3,584 x 3,584 367 us and 274 here, 8,192 by 3,584 x 20,480 1,305 and 860), but the
 // closer to 64 bits (3.45e-7 against 3.68e-7, 8.3e-7 against 9.2e-7; 17 of 66 sizes drawn from k 2,496 to 12,672, by 4 to 11 %), and a
 // result in float keeps what is gained.  Up to k 2,304 the error was the same in all of 24.  (A result of 16 bits is off by 1.7e-3.)
+// kind 3: plain, and its partial sums are wanted apart.  Two and four runs of k are closer to 64 bits than the library is, and from k 8,192
+// on the faster ones too, with the sum and norm that read them (us by the library and here, error 1e-7: 3,258 rows by 2,048 x 8,448 118 and
+// 110, 5.8 and 4.0; 1,104 by 2,560 x 10,240 82 and 69, 6.4 and 3.1; 1,946 by 4,096 x 14,336 219 and 197, 7.6 and 5.3; of 70 sizes from 1,025
+// rows, 1,024 to 5,120 columns and k 8,192 on all, by 9 % in the median, but 8,192 columns of 8,192 lose 2 %; 800 by 2,048 x 8,448 51 and
+// 63).  Up to k 5,632 it is as often the other way round (2,048 columns, k 5,632: 0.95 to 1.08, k 3,072 0.88 to 0.95).
 TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
   const bool dual = kind == 2;
+  if (kind == 3) {
+    if (M > 1024 && N < 8192 && K >= 8192 && tq_gemm_mfma_splits(M, N, K) > 1 && phases_suit(M, N, K, false, 2)) return 1;
+    kind = 0;
+  }
   if (!phases_suit(M, N, K, dual, 1)) return 0;
   int rows;
   const double t = phases_best(M, N, K, dual, 1, &rows), flops = 2.0 * M * N * K * (dual ? 2 : 1);

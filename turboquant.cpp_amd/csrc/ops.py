@@ -994,7 +994,7 @@ def _vendor_product(act, a, w, M: int, K: int) -> bool:
 
 def _vendor_here(act, a, w, M: int, N: int, K: int, kind: int = 0) -> bool:
     """Whether a product goes to the vendor's library: it may, and this library's tiles are not the faster ones (``kind`` 0: plain, 1: an
-    activation alone, 2: a gated pair; csrc/gemm_mfma.hip has the rule and both sides' times)."""
+    activation alone, 2: a gated pair, 3: plain, its partial sums apart; csrc/gemm_mfma.hip has the rule and both sides' times)."""
     return _vendor_product(act, a, w, M, K) and not library(act).tq_gemm_here_rather(M, N, K, kind)
 
 
@@ -1111,7 +1111,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, act, bias: torch.Tensor | None = None
             return out
         return act_rows(gemm(a, w, act, bias=bias), None, activation, act)
     if not grouped and a_rows is None and bias is None:
-        if w2 is None and _vendor_here(act, a, w, M, N, K):
+        if w2 is None and _vendor_here(act, a, w, M, N, K, 3 if partial_sums else 0):
             out = _vendor_gemm(a, w, out_act)
             return out[None] if partial_sums else out
         if w2 is not None and out_act and _behind(w, w2) and _vendor_here(act, a, w, M, N, K, 2):
