@@ -336,16 +336,20 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
 // through LDS, one barrier a chunk; its share of o, to which waves 0, 1 and 2 add one of b's three tiles each once u is known,
 // goes along with the next chunk's u.  The next two chunks' operands are on their way meanwhile.  The blocks of a head lie H apart, so
 // that they run on one die (H a multiple of 8) and share what they read in its L2.
-// A chunk is a chain: 16 NB products with the state, the exchange, 8 NB products into the state, 1.8 us of which 0.64 are the products' (2,048 tokens
-// of 16 heads of 128 x 128: 118 us; with the token-by-token form both launches' work took 0.94 ms, 0.45 us a token).
-template <int NB>
-__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __restrict__ scratch,
+// A chunk is a chain: 8 NB products with the state, the exchange, in whose time 8 NB more are formed for o, and 8 NB into the state, 1.5 us of
+// which 0.64 are the products'.  2,048 tokens of 16 heads of 128 x 128, us: 97; 119 before with a wait for all loads on their way every two
+// chunks (see the loop; 116 without), the products for o in front of the exchange (109 behind it) and the key tiles' chains one behind the
+// other under conditions of their own.  Level: b's products between those into the state.  (Token by token both launches' work took 0.94 ms, 0.45
+// us a token.)
+// WHOLE: every wave has NB key tiles (D = 64 NB), so that nothing is under a condition and the tiles' chains of products go on side by side.
+template <int NB, bool WHOLE>
+__global__ __launch_bounds__(256, NB < 4 ? 2 : 1) void delta_chunk_scan_kernel(const float* __restrict__ scratch,
                                                                const int* __restrict__ cu_seqlens,
                                                                const int* __restrict__ slots, float* __restrict__ state,
                                                                int64_t state_stride, DeltaWindow window, DeltaDims dm,
                                                                float* __restrict__ o_raw) {
   __shared__ __align__(16) float ex[2][4][4][256];      // [buffer][wave][u, u, the chunk before's o, o][lane][4]
-  const int H = dm.H, D = dm.D, V = dm.V, ND = D / 16, VB = V / 16;
+  const int H = dm.H, D = WHOLE ? 64 * NB : dm.D, V = dm.V, ND = D / 16, VB = V / 16;
   const int h = blockIdx.x % H, vb = blockIdx.x / H, b = window.b0 + blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TQ_WAVE), lane = threadIdx.x % TQ_WAVE, r = lane % 16, g4 = lane / 16;
   int t0 = cu_seqlens[b], n = cu_seqlens[b + 1] - t0;
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
   for (int j = 0; j < NB; ++j) {
     const int db = wave + 4 * j;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s[j][i] = db < ND ? S[(size_t)(16 * db + 4 * g4 + i) * V] : 0.f;
+    for (int i = 0; i < 4; ++i) s[j][i] = WHOLE || db < ND ? S[(size_t)(16 * db + 4 * g4 + i) * V] : 0.f;
   }
   const dc_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   struct Operands {
@@ -378,7 +382,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
     auto tile = [&](int i) { return reinterpret_cast<const dc_f32x4*>(c + (size_t)i * 256)[lane]; };
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const int db = wave + 4 * j < ND ? wave + 4 * j : 0;
+      const int db = WHOLE || wave + 4 * j < ND ? wave + 4 * j : 0;
 #pragma unroll
       for (int tb = 0; tb < 2; ++tb) {
         to.w[tb][j] = tile(tb * ND + db);
@@ -415,7 +419,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
     }
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      if (wave + 4 * j < ND)
+      if (WHOLE || wave + 4 * j < ND)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -427,33 +431,39 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
       *reinterpret_cast<dc_f32x4*>(&to[wave][tb][lane * 4]) = pu[tb];
       *reinterpret_cast<dc_f32x4*>(&to[wave][2 + tb][lane * 4]) = po[tb];
     }
+    __syncthreads();
+    // the waves' shares in wave order, and U0; they come out of LDS while the products for o are formed
+    dc_f32x4 u[2], share[2][4];
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) share[tb][ww] = *reinterpret_cast<const dc_f32x4*>(&to[ww][tb][lane * 4]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      if (wave + 4 * j < ND)
+      if (WHOLE || wave + 4 * j < ND)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int tb = 0; tb < 2; ++tb) next[tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(in.q[tb][j][i], s[j][i], next[tb], 0, 0, 0);
     }
-    __syncthreads();
-    // the waves' shares in wave order, and U0
-    dc_f32x4 u[2];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb) {
-      u[tb] = *reinterpret_cast<const dc_f32x4*>(&to[0][tb][lane * 4]);
+      u[tb] = share[tb][0];
 #pragma unroll
-      for (int ww = 1; ww < 4; ++ww) u[tb] += *reinterpret_cast<const dc_f32x4*>(&to[ww][tb][lane * 4]);
+      for (int ww = 1; ww < 4; ++ww) u[tb] += share[tb][ww];
       u[tb] += in.u0[tb];
     }
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      s[j] *= in.g[j];
-      if (wave + 4 * j < ND)
+    for (int j = 0; j < NB; ++j) s[j] *= in.g[j];
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
+    for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in.k[j][tb][i], u[tb][i], s[j], 0, 0, 0);
-    }
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          if (WHOLE || wave + 4 * j < ND) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in.k[j][tb][i], u[tb][i], s[j], 0, 0, 0);
     if (!first) read_out(to, c - 1, false);
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb) po[tb] = next[tb];
@@ -487,17 +497,26 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
     }
     fetch(in, min(c + 2, chunks - 1));
   };
+  // Pairs behind the first chunk or the first two, so that the loop holds nothing but whole pairs: with a single chunk behind them the
+  // compiler made one body of both, and waited at its head for all loads on their way to move what they bring to other registers.
   Operands even, odd;
   fetch(even, 0);
-  fetch(odd, min(1, chunks - 1));
   one_chunk(0, even, true);
   int c = 1;
-#pragma unroll 1
-  for (; c + 1 < chunks; c += 2) {
-    one_chunk(c, odd, false);
-    one_chunk(c + 1, even, false);
+  if (chunks % 2 == 0) {
+    fetch(odd, 1);
+    one_chunk(1, odd, false);
+    c = 2;
   }
-  if (c < chunks) one_chunk(c, odd, false);
+  if (c < chunks) {
+    fetch(even, c);
+    fetch(odd, c + 1);
+#pragma unroll 1
+    for (; c < chunks; c += 2) {
+      one_chunk(c, even, false);
+      one_chunk(c + 1, odd, false);
+    }
+  }
   float (*to)[4][256] = ex[chunks & 1];
 #pragma unroll
   for (int tb = 0; tb < 2; ++tb) *reinterpret_cast<dc_f32x4*>(&to[wave][2 + tb][lane * 4]) = po[tb];
@@ -506,7 +525,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(const float* __re
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
     const int db = wave + 4 * j;
-    if (db < ND)
+    if (WHOLE || db < ND)
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[(size_t)(16 * db + 4 * g4 + i) * V] = s[j][i];
   }
@@ -570,8 +589,8 @@ TQ_API int tq_delta_chunks(const float* qn, const float* kn, const float* vc, co
 #undef TQ_PREP_CASE
 #undef TQ_PREP
     const dim3 grid((unsigned)(H * (V / 16)), w.B);
-#define TQ_SCAN(NB) \
-  hipLaunchKernelGGL(delta_chunk_scan_kernel<NB>, grid, dim3(256), 0, st, scratch, cu_seqlens, slots, state, state_stride, w, d, o_raw)
+#define TQ_SCAN(NB)                                                                                                                \
+  hipLaunchKernelGGL((nd == 4 * NB ? delta_chunk_scan_kernel<NB, true> : delta_chunk_scan_kernel<NB, false>), grid, dim3(256), 0, st, scratch, cu_seqlens, slots, state, state_stride, w, d, o_raw)
     if (nd <= 4) TQ_SCAN(1);
     else if (nd <= 8) TQ_SCAN(2);
     else TQ_SCAN(4);
