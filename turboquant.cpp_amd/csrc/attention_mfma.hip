@@ -161,7 +161,9 @@ __device__ __forceinline__ int v_swz(int d, int ch) { return d * TILE + ((ch ^ (
 // The part of a tile between its two products, for QG groups of 16 columns: s holds the tile's scores (rows of
 // block jt as tile_step says); afterwards m_run, l_run and o are brought to the new running maximum and pf holds the
 // probabilities 2^(s * scale2 - m) as the operand of the second product.
-template <int DT, int QG, bool MOD>
+// FLAT: nothing under a condition, for lds_tile_step, whose operands are on their way meanwhile (in the kernels that have no registers
+// left the conditions keep the compiler from more spills: heads of 96 with a distance bias 43 us with them and 91 without).
+template <int DT, int QG, bool MOD, bool FLAT = false>
 __device__ __forceinline__ void softmax_tile(f32x4 (&s)[QG][4], f32x4 (&o)[QG][DT], float (&m_run)[QG], float (&l_run)[QG],
                                              int pos0, const int (&p_q)[QG], const int (&lo_q)[QG], float scale2,
                                              bool masked, bf16x8 (&pf)[2][QG], const ColMod<QG, MOD>& cm) {
@@ -220,8 +222,10 @@ __device__ __forceinline__ void softmax_tile(f32x4 (&s)[QG][4], f32x4 (&o)[QG][D
     m_tile = group_max(m_tile) * scale2;
     const float m_new = fmaxf(m_run[g], m_tile);
     const bool any = m_new != -INFINITY;
-    const float alpha = any && m_run[g] != -INFINITY ? __builtin_amdgcn_exp2f(m_run[g] - m_new) : (any ? 0.f : 1.f);
     const float m_use = any ? m_new : 0.f;       // 2^(-inf - 0) = 0 for masked keys, also when all are masked
+    // (FLAT: 0 where no key was visible yet, whose sums are 0)
+    const float alpha = FLAT ? __builtin_amdgcn_exp2f(m_run[g] - m_use)
+                             : any && m_run[g] != -INFINITY ? __builtin_amdgcn_exp2f(m_run[g] - m_new) : (any ? 0.f : 1.f);
     float l_tile = 0.f;
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
@@ -343,6 +347,57 @@ __device__ __forceinline__ void tile_step(f32x4 (&o)[QG][VD], float (&m_run)[QG]
       }
     }
   }
+}
+
+// tile_step for a tile in LDS laid out by k_swz, v_swz (EXACT sizes): the same products in the same order.  The compiler asks for
+// two or three operands at a time and waits; here a tile's keys are all asked for before the first product and half of its values
+// before the softmax, which is worth 64 registers where a wave has one group of 16 columns or short heads (READS_AHEAD below): 3,001
+// tokens of 16 heads of 64 47 -> 43 us, of 128 with a distance bias 120 -> 105, with sigmoid weights 102 -> 88.
+template <int DT, int QG, bool MOD, int VD, bool DIFF>
+__device__ __forceinline__ void lds_tile_step(f32x4 (&o)[QG][VD], float (&m_run)[QG], float (&l_run)[QG],
+                                              const bf16x8 (&qf)[QG][(DT + 1) / 2], const bf16_t* kt, const bf16_t* vt, int pos0,
+                                              const int (&p_q)[QG], const int (&lo_q)[QG], float scale2, bool masked,
+                                              const ColMod<QG, MOD>& cm) {
+  constexpr int KS = DT / 2;
+  const int lane = threadIdx.x % 64, r = lane % 16, c = lane / 16;
+  f32x4 s[QG][4];
+  bf16x8 kf[4][KS];
+  auto load_k = [&](int jt) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kf[jt][ks] = ld16(kt + k_swz<DT>(32 * (jt / 2) + 8 * (r / 4) + 4 * (jt % 2) + r % 4, 4 * ks + c));
+  };
+  auto scores = [&](int jt) {
+#pragma unroll
+    for (int g = 0; g < QG; ++g) s[g][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int g = 0; g < QG; ++g)
+        if (!DIFF || (ks < KS / 2) == (g % 2 == 0))
+          s[g][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[jt][ks], qf[g][ks], s[g][jt], 0, 0, 0);
+  };
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) load_k(jt);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) scores(jt);
+  bf16x8 vf[2][VD];
+  auto load_v = [&](int pr) {
+#pragma unroll
+    for (int dt = 0; dt < VD; ++dt) vf[pr][dt] = ld16(vt + v_swz(16 * dt + r, 4 * pr + c));
+  };
+  load_v(0);
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8 pf[2][QG];
+  softmax_tile<VD, QG, MOD, true>(s, o, m_run, l_run, pos0, p_q, lo_q, scale2, masked, pf, cm);
+  load_v(1);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+    for (int dt = 0; dt < VD; ++dt)
+#pragma unroll
+      for (int g = 0; g < QG; ++g) o[g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pr][dt], pf[pr][g], o[g][dt], 0, 0, 0);
 }
 
 // Runs the wave's 16 columns over tiles [tile_beg, tile_end) straight from the cache pages.
@@ -479,9 +534,13 @@ __device__ __forceinline__ void load_query(bf16x8 (&qf)[(DT + 1) / 2], const bf1
 // VD < DT: the values' first 16 VD dimensions alone are summed and written (zeros behind them up to hd): an attention
 // whose keys are wider than its values, laid out at the keys' width.
 // DIFF: two maps a head, a token's two columns in two groups of one lane; they are made one where the output is normalised.
+// Waves to a SIMD: two, said as a maximum too, so that the compiler plans with the 256 registers that a wave has then anyway (heads
+// of 192 and values of 128, 3,001 tokens of 16 heads: 97 -> 76 us; heads of 256, 2,048 tokens of 8: 147 -> 80, whose
+// sums went to scratch memory; the numbers of a wave in scalar registers have a part in it).  Short heads gain by more waves; sizes known at run
+// time only stay without a maximum.
 template <int DT, int QG, bool EXACT, bool MOD, int VD = DT, bool DIFF = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF ? 8 : 16) ? 1 : 2))) void attn_prefill_kernel(AttnArgs a, int n_blocks, int B, DiffArgs df) {
-  constexpr bool ONEBUF = DT > ATTN_TWO_BUFFERS_UP_TO;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF ? 8 : 16) ? 1 : 2, DT > (DIFF ? 8 : 16) ? 1 : !EXACT ? 8 : DT > 4 ? 2 : 4))) void attn_prefill_kernel(AttnArgs a, int n_blocks, int B, DiffArgs df) {
+  constexpr bool ONEBUF = DT > ATTN_TWO_BUFFERS_UP_TO, READS_AHEAD = EXACT && DT * QG <= 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   static_assert(!DIFF || (QG % 2 == 0 && !MOD && VD == DT), "two maps a head: in pairs of groups, with plain scores");
   constexpr int QW = 16 * (DIFF ? QG / 2 : QG);
@@ -497,7 +556,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF 
   const int per_block = a.nh * B;
   const int blk = n_blocks - 1 - (int)blockIdx.x / per_block;
   const int h = (int)blockIdx.x % per_block % a.nh, seq = (int)blockIdx.x % per_block / a.nh;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, r = lane % 16, c = lane / 16;
+  const int tid = threadIdx.x, lane = tid % 64, r = lane % 16, c = lane / 16;
+  // (a number in a scalar register, except where hd is known at run time only: the compiler's code for heads between 256 and 512 gave NaN then)
+  const int wave = EXACT ? __builtin_amdgcn_readfirstlane(tid / 64) : tid / 64;
   const int t0 = a.cu_seqlens[seq], n = a.cu_seqlens[seq + 1] - t0;
   const int qb = blk * 4 * QW;
   if (qb >= n) return;
@@ -619,7 +680,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF 
     if ((tile >= wave_beg || tile < kept) && tile < wave_end) {
       const int pos0 = tile * TILE;
       const bool masked = pos0 + TILE - 1 > wave_first || pos0 < wave_lo_last;
-      tile_step<DT, QG, EXACT, EXACT, false, MOD, VD, DIFF>(o, m_run, l_run, qf, Ks + cur, kstr, Vs + cur, vstr, hd, pos0, p_q, lo_q,
+      if constexpr (READS_AHEAD) lds_tile_step<DT, QG, MOD, VD, DIFF>(o, m_run, l_run, qf, Ks + cur, Vs + cur, pos0, p_q, lo_q, a.scale * LOG2E, masked, cm);
+      else tile_step<DT, QG, EXACT, EXACT, false, MOD, VD, DIFF>(o, m_run, l_run, qf, Ks + cur, kstr, Vs + cur, vstr, hd, pos0, p_q, lo_q,
                                       a.scale * LOG2E, masked, cm);
     }
     __syncthreads();
