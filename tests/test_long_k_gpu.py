@@ -8,10 +8,10 @@ pytestmark = pytest.mark.gpu
 DEVICE = "cuda:0"
 
 
-# both sides of 1,024 rows, of k 8,192 and of 8,192 columns; remainders of rows and columns
+# both sides of 1,024 rows, of 1,024 and 8,192 columns and of k 8,192; remainders of rows and columns
 @pytest.mark.parametrize("rows,cols,k,here", [
-    (1024, 512, 8192, False), (1025, 512, 8192, True), (1025, 512, 8128, False), (1091, 1000, 8256, True), (2049, 768, 12288, True),
-    (1030, 8192, 8192, False),
+    (1024, 1024, 8192, False), (1025, 1024, 8192, True), (1025, 1016, 8192, False), (1025, 1024, 8128, False), (1091, 1032, 8256, True),
+    (2049, 1280, 12288, True), (1030, 8192, 8192, False),
 ])
 def test_partial_sums_of_a_long_k(rows, cols, k, here):
     gen = torch.Generator().manual_seed(rows + k)

@@ -1069,11 +1069,11 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K);
 // on the faster ones too, with the sum and norm that read them (us by the library and here, error 1e-7: 3,258 rows by 2,048 x 8,448 118 and
 // 110, 5.8 and 4.0; 1,104 by 2,560 x 10,240 82 and 69, 6.4 and 3.1; 1,946 by 4,096 x 14,336 219 and 197, 7.6 and 5.3; of 70 sizes from 1,025
 // rows, 1,024 to 5,120 columns and k 8,192 on all, by 9 % in the median, but 8,192 columns of 8,192 lose 2 %; 800 by 2,048 x 8,448 51 and
-// 63).  Up to k 5,632 it is as often the other way round (2,048 columns, k 5,632: 0.95 to 1.08, k 3,072 0.88 to 0.95).
+// 63; fewer than 1,024 columns were not timed and stay with the library).  Up to k 5,632 it is as often the other way round (2,048 columns, k 5,632: 0.95 to 1.08, k 3,072 0.88 to 0.95).
 TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
   const bool dual = kind == 2;
   if (kind == 3) {
-    if (M > 1024 && N < 8192 && K >= 8192 && tq_gemm_mfma_splits(M, N, K) > 1 && phases_suit(M, N, K, false, 2)) return 1;
+    if (M > 1024 && N >= 1024 && N < 8192 && K >= 8192 && tq_gemm_mfma_splits(M, N, K) > 1 && phases_suit(M, N, K, false, 2)) return 1;
     kind = 0;
   }
   if (!phases_suit(M, N, K, dual, 1)) return 0;
