@@ -535,11 +535,11 @@ __device__ __forceinline__ void load_query(bf16x8 (&qf)[(DT + 1) / 2], const bf1
 // whose keys are wider than its values, laid out at the keys' width.
 // DIFF: two maps a head, a token's two columns in two groups of one lane; they are made one where the output is normalised.
 // Waves to a SIMD: two, said as a maximum too, so that the compiler plans with the 256 registers that a wave has then anyway (heads
-// of 192 and values of 128, 3,001 tokens of 16 heads: 97 -> 76 us; heads of 256, 2,048 tokens of 8: 147 -> 80, whose
-// sums went to scratch memory; the numbers of a wave in scalar registers have a part in it).  Short heads gain by more waves; sizes known at run
-// time only stay without a maximum.
+// of 256, 2,048 tokens of 8: 147 -> 80 us, whose sums went to scratch memory; the numbers of a wave in scalar registers have a part in
+// it).  Short heads gain by more waves, and so do values narrower than keys behind a window (3,001 tokens of 16 heads of 192, values of
+// 128: 52 us behind 1,024 positions, 58 with the maximum, though 104 and 82 without a window); sizes known at run time stay without one.
 template <int DT, int QG, bool EXACT, bool MOD, int VD = DT, bool DIFF = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF ? 8 : 16) ? 1 : 2, DT > (DIFF ? 8 : 16) ? 1 : !EXACT ? 8 : DT > 4 ? 2 : 4))) void attn_prefill_kernel(AttnArgs a, int n_blocks, int B, DiffArgs df) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF ? 8 : 16) ? 1 : 2, DT > (DIFF ? 8 : 16) ? 1 : !EXACT || VD < DT ? 8 : DT > 4 ? 2 : 4))) void attn_prefill_kernel(AttnArgs a, int n_blocks, int B, DiffArgs df) {
   constexpr bool ONEBUF = DT > ATTN_TWO_BUFFERS_UP_TO, READS_AHEAD = EXACT && DT * QG <= 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   static_assert(!DIFF || (QG % 2 == 0 && !MOD && VD == DT), "two maps a head: in pairs of groups, with plain scores");
