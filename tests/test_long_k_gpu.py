@@ -24,3 +24,18 @@ def test_partial_sums_of_a_long_k(rows, cols, k, here):
     error = ((parts.double().sum(0) - exact).norm() / exact.norm()).item()
     # sums of 32 bits over k / 8 steps that round down: 6.2e-9 sqrt(k) as measured in one run of k, less in several
     assert error < 7e-9 * (k / parts.shape[0]) ** 0.5, error
+
+
+@pytest.mark.parametrize("first", [(4, 0), (0, 4)])
+def test_operands_between_16_bytes(first):
+    """Contiguous views that begin 8 bytes into memory: the tiles refuse them, the vendor's library does not."""
+    rows, cols, k = 1091, 1032, 8256
+    gen = torch.Generator().manual_seed(sum(first))
+
+    def at(rows, first, scale):
+        flat = (torch.randn(rows * k + 8, generator=gen) * scale).to(torch.bfloat16).to(DEVICE)
+        return flat[first:first + rows * k].view(rows, k)
+    a, w = at(rows, first[0], 1.0), at(cols, first[1], 0.02)
+    parts = ops.gemm(a, w, "bfloat16", partial_sums=True)
+    exact = a.double() @ w.double().t()
+    assert parts.shape[0] == 1 and ((parts[0].double() - exact).norm() / exact.norm()).item() < 7e-9 * k ** 0.5

@@ -57,3 +57,20 @@ def test_one_round_of_the_tile_kernel_stays_its_own(lib):
         runs = lib.tq_gemm_mfma_splits(M, N, K)
         assert runs > 1 and (lib.tq_gemm_phases_rows(M, N, K, 0, runs) > 0) == bool(here), (M, N, K)
         assert runs == tile_kernel_runs(M, N, K) or lib.tq_gemm_phases_rows(M, N, K, 0, runs)
+
+
+@pytest.mark.parametrize("kind,M,N,K", [(0, 2048, 6288, 2048), (1, 3001, 8448, 2048), (2, 2048, 5632, 2048), (3, 1091, 1032, 8256)])
+def test_operands_that_begin_between_16_bytes_leave_for_the_library(lib, monkeypatch, kind, M, N, K):
+    """The tiles refuse them, whatever their size says; the vendor's library takes any address."""
+    import torch
+
+    from turboquant_cpp_amd.csrc import ops
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops, "library", lambda act: lib)
+
+    def at(rows, first):
+        return torch.empty(rows * K + 8, dtype=torch.bfloat16)[first:first + rows * K].view(rows, K)
+    for a_first, w_first, leaves in ((0, 0, False), (8, 8, False), (4, 0, True), (0, 4, True), (1, 8, True)):
+        a, w = at(M, a_first), at(N, w_first)
+        assert a.is_contiguous() and w.is_contiguous()
+        assert ops._vendor_here("bfloat16", a, w, M, N, K, kind) is leaves, (a_first, w_first)

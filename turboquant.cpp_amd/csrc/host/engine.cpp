@@ -127,7 +127,9 @@ bool vendor_product(const Ctx& c, const Product& p) {
         p.w.wtype == TQ_BF16 && !s.capturing && !s.decode && tq_vendor_available()))
     return false;
 #if defined(TQ_ACT_BF16)
-  if (!(p.w2 && !p.out_act) && tq_gemm_here_rather(p.M, p.N, p.K, p.w2 ? 2 : p.partial ? 3 : 0)) return false;
+  // (the tiles here refuse matrices and rows that do not begin on 16 bytes; the library takes them)
+  const bool aligned = (uintptr_t)p.w.ptr % 16 == 0 && p.lda % 8 == 0;
+  if (aligned && !(p.w2 && !p.out_act) && tq_gemm_here_rather(p.M, p.N, p.K, p.w2 ? 2 : p.partial ? 3 : 0)) return false;
 #endif
   if (!p.w2) return tq_vendor_takes(p.M, p.N, p.K, p.lda, p.out_act) != 0;
   const int64_t chunk = s.vendor_gated_rows > 0 ? s.vendor_gated_rows : 4096;

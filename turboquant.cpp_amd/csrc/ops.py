@@ -994,8 +994,10 @@ def _vendor_product(act, a, w, M: int, K: int) -> bool:
 
 def _vendor_here(act, a, w, M: int, N: int, K: int, kind: int = 0) -> bool:
     """Whether a product goes to the vendor's library: it may, and this library's tiles are not the faster ones (``kind`` 0: plain, 1: an
-    activation alone, 2: a gated pair, 3: plain, its partial sums apart; csrc/gemm_mfma.hip has the rule and both sides' times)."""
-    return _vendor_product(act, a, w, M, K) and not library(act).tq_gemm_here_rather(M, N, K, kind)
+    activation alone, 2: a gated pair, 3: plain, its partial sums apart; csrc/gemm_mfma.hip has the rule and both sides' times).
+    The tiles read 16 bytes at a time and refuse operands that do not begin on as many; the library takes those."""
+    return _vendor_product(act, a, w, M, K) and not (a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.stride(0) % 8 == 0
+                                                     and library(act).tq_gemm_here_rather(M, N, K, kind))
 
 
 def _vendor_gemm(a, w, out_act: bool) -> torch.Tensor:
