@@ -74,3 +74,14 @@ def test_operands_that_begin_between_16_bytes_leave_for_the_library(lib, monkeyp
         a, w = at(M, a_first), at(N, w_first)
         assert a.is_contiguous() and w.is_contiguous()
         assert ops._vendor_here("bfloat16", a, w, M, N, K, kind) is leaves, (a_first, w_first)
+
+
+@pytest.mark.parametrize("M,N,K,here", [
+    (2048, 4096, 8192, True), (2049, 4096, 8192, False), (1280, 6144, 8192, True), (1281, 6144, 8192, False),      # 256 tiles in two runs, and more
+    (1091, 7168, 14336, False), (2713, 2944, 12928, False), (3258, 5120, 8192, False), (3258, 5120, 11008, True),      # 1.1e11, 1.0e11, 1.4e11, 1.8e11
+    (2209, 8128, 14528, True), (2209, 8192, 14528, False), (1024, 2048, 8448, False), (1025, 2048, 8448, True), (3258, 2048, 8128, False),
+    (3258, 1016, 8448, False), (3258, 2048, 8448, True)])
+def test_partial_sums_of_a_long_k_stay_in_one_round_of_tiles_or_where_they_are_many(lib, M, N, K, here):
+    """Beyond one tile to a compute unit the vendor's library is the faster one up to 1.4e11 multiply-adds."""
+    assert bool(lib.tq_gemm_here_rather(M, N, K, 3)) is here
+    assert not lib.tq_gemm_here_rather(M, N, K, 0)

@@ -1065,15 +1065,27 @@ TQ_API int tq_gemm_mfma_splits(int M, int N, int K);
 // for many a size: the slower kernel (13,197 by 3,584 x 3,584 367 us and 274 here, 8,192 by 3,584 x 20,480 1,305 and 860), but the
 // closer to 64 bits (3.45e-7 against 3.68e-7, 8.3e-7 against 9.2e-7; 17 of 66 sizes drawn from k 2,496 to 12,672, by 4 to 11 %), and a
 // result in float keeps what is gained.  Up to k 2,304 the error was the same in all of 24.  (A result of 16 bits is off by 1.7e-3.)
-// kind 3: plain, and its partial sums are wanted apart.  Two and four runs of k are closer to 64 bits than the library is, and from k 8,192
-// on the faster ones too, with the sum and norm that read them (us by the library and here, error 1e-7: 3,258 rows by 2,048 x 8,448 118 and
-// 110, 5.8 and 4.0; 1,104 by 2,560 x 10,240 82 and 69, 6.4 and 3.1; 1,946 by 4,096 x 14,336 219 and 197, 7.6 and 5.3; of 70 sizes from 1,025
-// rows, 1,024 to 5,120 columns and k 8,192 on all, by 9 % in the median, but 8,192 columns of 8,192 lose 2 %; 800 by 2,048 x 8,448 51 and
-// 63; fewer than 1,024 columns were not timed and stay with the library).  Up to k 5,632 it is as often the other way round (2,048 columns, k 5,632: 0.95 to 1.08, k 3,072 0.88 to 0.95).
+// kind 3: plain, and its partial sums are wanted apart.  Two and four runs of k are closer to 64 bits than the library is (2,048 columns,
+// k 8,448: 4.0e-7 and 5.8e-7; 1,024 columns in four 2.7e-7 and 5.7e-7).  Here they go from 1,025 rows, 1,024 to 8,191 columns and k 8,192 on where
+//  * their tiles are one round, one to a compute unit at most: 1.00 to 1.44 times as fast as the library, with the sum and norm that read them,
+//    in all of 84 such sizes (us by the library and here: 3,258 rows by 2,048 x 8,448 118 and 110; 2,421 by 2,080 x 9,472 106 and 104; 1,121 by
+//    5,744 x 12,032 171 and 146; 1,787 by 1,344 x 16,192 121 and 86), twice in 3 where the library takes a slower kernel (1,302 by 3,936 x
+//    14,912 308 and 141).  Of more rounds and fewer multiply-adds than the next line's, 33 of 37 lose (1,091 by 7,168 x 8,192 129 and 147, 2,713 by 2,944 x
+//    12,928 189 and 222, 5,644 by 1,296 x 8,960 137 and 169, 1,152 by 6,656 x 8,384 124 and 145);
+//  * or 1.4e11 multiply-adds: for three of four sizes the library takes kernels there that need half as long again and more (3,258 by 5,120 x
+//    11,008 577 and 368, 12,032 by 1,536 x 12,992 715 and 442; 1.23 to 1.78 in 40 of 54), else it is level (4,096 by 6,144 x 8,192 373 and 384,
+//    x 14,336 600 and 580, 8,636 by 1,904 x 14,208 448 and 448: 0.97 to 1.07).
+// (800 rows by 2,048 x 8,448 51 and 63; fewer than 1,024 columns were not timed.)  Up to k 5,632 it is as often the other way round (2,048
+// columns, k 5,632: 0.95 to 1.08, k 3,072 0.88 to 0.95).
 TQ_API int tq_gemm_here_rather(int M, int N, int K, int kind) {
   const bool dual = kind == 2;
   if (kind == 3) {
-    if (M > 1024 && N >= 1024 && N < 8192 && K >= 8192 && tq_gemm_mfma_splits(M, N, K) > 1 && phases_suit(M, N, K, false, 2)) return 1;
+    const int runs = M > 1024 && N >= 1024 && N < 8192 && K >= 8192 ? tq_gemm_mfma_splits(M, N, K) : 1;
+    if (runs > 1 && phases_suit(M, N, K, false, runs)) {
+      int rows;
+      phases_best(M, N, K, false, runs, &rows);
+      if ((int64_t)((M + rows - 1) / rows) * ((N + 255) / 256) * runs <= 256 || (int64_t)M * N * K >= 140000000000) return 1;
+    }
     kind = 0;
   }
   if (!phases_suit(M, N, K, dual, 1)) return 0;
