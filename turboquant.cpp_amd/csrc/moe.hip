@@ -489,8 +489,13 @@ static int launch_router_logits(const float* x, const void* wr, const void* shar
   // 512 12.9 and 10.5, 700 15.9 and 11.8; 256 experts: 64 16.5 and 16.5, 240 22.2 and 19.5, 512 27.3 and 24.2; rows of 3,584, 114 KB
   // of LDS, 2,048 tokens 42.7 and 33.1.
   const bool many = T >= TQ_ROUTER_MANY && hp * RT * sizeof(float) <= 160 * 1024;
-  // Where two such workgroups do not share a unit and there are more than units: 4 of them (13,197 tokens of 3,584, with the choice and the order, 192 and 166 us).
-  const bool wide = many && T > 2048 && hp * RT * sizeof(float) > 80 * 1024;
+  // Where two such workgroups do not share a unit (rows beyond 2,560), two of 4 tokens that do take as long for the same 8 tokens, 1.10 times as
+  // long with 256 experts and 0.85 with 16; but a last round of up to half the units then takes half a round, and a whole one with 8 (us with 8
+  // and with 4 tokens, the choice among them; rows of 3,584: 256 experts, 2,049 tokens 132 and 112, 3,072 136 and 121, 3,073 136 and 145, 4,096 142 and
+  // 156, 4,097 205 and 187, 8,192 273 and 296, 10,300 350 and 340, 13,197 458 and 469; 128 experts, 3,001 73 and 63, 4,096 78 and 81, 13,197 246 and
+  // 243; 64, 2,049 39 and 33, 4,096 47 and 47, 13,197 145 and 133; 16, 8,192 46 and 40; rows of 3,072, 4,096 and 5,120 alike).
+  const bool wide = many && T > 2048 && hp * RT * sizeof(float) > 80 * 1024 &&
+                    (E <= 64 || ((T - 1) % 2048 < 1024 && T <= (E <= 128 ? 16384 : 12288)));
   int tg = wide ? 4 : RT;
   while (!many && tg > 1 && (size_t)tg * hp * sizeof(float) > 32 * 1024) tg /= 2;   // small enough for several workgroups per CU
   const size_t shmem = (size_t)tg * hp * sizeof(float);
