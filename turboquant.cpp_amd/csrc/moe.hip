@@ -789,7 +789,7 @@ __global__ __launch_bounds__(RP) void route_place_kernel(const int* __restrict__
                                                          int* __restrict__ sorted_token, int* __restrict__ pair_slot,
                                                          int* __restrict__ tile_expert, int* __restrict__ n_tiles, int n_real) {
   extern __shared__ int sm_p[];
-  const int C = max(RP / E, 1), v0 = blockIdx.x * per, v1 = min(v0 + per, V), n = v1 - v0;
+  const int C = RP / E, v0 = blockIdx.x * per, v1 = min(v0 + per, V), n = v1 - v0;
   int* all = sm_p;
   int* before = all + C * E;
   int* starts = before + C * E;
@@ -1084,14 +1084,11 @@ static int route_many(const float* x, const void* wr, const void* shared_w, cons
   // So few tokens to a workgroup that there is one to a compute unit while they last, and where there are more, that two share one.
   int tg = T <= 512 ? 2 : T <= 1024 ? 4 : 8;
   while (tg > 1 && lds(tg) > (T > 2048 ? 80 : 160) * 1024) tg /= 2;
-  const int V = (T + tg - 1) / tg, fit = 12 * 1024 / E;      // segments whose first rows 48 KB hold
+  const int V = (T + tg - 1) / tg;
   if (lds(tg) > 160 * 1024 || (int64_t)V * E > 65536) return ROUTE_OTHERWISE;
-  int per = (V + 63) / 64;
-  if (per < 16) per = 16;
-  if (per > fit) per = fit;
-  const int C = RP / E > 1 ? RP / E : 1;
-  const size_t lds_place = ((size_t)(2 * C + 1 + per) * E) * sizeof(int);
-  if (per < 1 || lds_place > 64 * 1024) return ROUTE_OTHERWISE;
+  // (the callers' 512 tokens, 1,024 beyond 128 experts, leave at most 508 experts then, and route_place 42,672 bytes of LDS)
+  const int even = (V + 63) / 64, per = even < 16 ? 16 : even;
+  const size_t lds_place = ((size_t)(2 * (RP / E) + 1 + per) * E) * sizeof(int);
   const size_t shmem = lds(tg);
 #define TQ_CHOOSE(TGV)                                                                                                                    \
   do {                                                                                                                                    \
@@ -1108,8 +1105,6 @@ static int route_many(const float* x, const void* wr, const void* shared_w, cons
     else TQ_CHOOSE(1);
   });
 #undef TQ_CHOOSE
-  if (lds_place > 48 * 1024)
-    (void)hipFuncSetAttribute((const void*)route_place_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_place);
   hipLaunchKernelGGL(route_place_kernel, dim3((V + per - 1) / per), dim3(RP), lds_place, st, ids, n_pairs, E, topk, V, per, tg * topk, table, unit,
                      per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, n_real);
   TQ_LAUNCH_CHECK();
