@@ -789,9 +789,10 @@ def test_routing_in_one_call(ops, act, E, k, H, renorm, shared):
 @pytest.mark.parametrize("T,E,k,H,unit,skew", [(2048, 60, 4, 128, 64, False), (2500, 60, 4, 128, 64, True), (3000, 5, 3, 72, 16, False),
                                                 (1100, 130, 8, 64, 64, False), (40000, 64, 8, 64, 64, True)])
 def test_order_by_several_workgroups(ops, T, E, k, H, unit, skew):
-    """From 8,192 pairs on ``route`` orders the pairs with several workgroups (three launches, its table in the logits'
-    memory) where ``moe_align`` has one workgroup go through them: the same rows, tiles and items, also when most
-    tokens choose the same experts and when the last workgroup's waves have nothing left."""
+    """From 8,192 pairs on ``route`` orders the pairs with several workgroups (with the choice in two launches, or behind it in
+    three, its table in the logits' memory; test_route_in_two_launches_gpu.py names each) where ``moe_align`` has one
+    workgroup go through them: the same rows, tiles and items, also when most tokens choose the same experts and when the
+    last workgroup's waves have nothing left."""
     act = "bfloat16"
     x = rnd((T, H), torch.float32, 71)
     if skew:

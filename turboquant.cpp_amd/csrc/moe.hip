@@ -1067,29 +1067,68 @@ TQ_API int tq_moe_align(const int* ids, int n_pairs, int E, int topk, int unit, 
   return moe_align_impl(ids, n_pairs, E, topk, unit, per_item, cap, sorted_token, pair_slot, tile_expert, n_tiles, st, E);
 }
 
-// The choice and the order in two launches by many workgroups, or ROUTE_OTHERWISE: more activations or experts than the LDS holds, or so
-// many segments that every workgroup's way through the table costs more than the launches saved (256 experts, us apart and this way: 2,048
-// tokens, 65,536 counts, 78 and 63, 3,001 tokens, 96,256, 108 and 111, 8,192, 262,144, 191 and 224).
-// table: T * E ints.
-#define ROUTE_OTHERWISE (-1000)
-static int route_many(const float* x, const void* wr, const void* shared_w, const float* bias, int wtype, int E, int topk, int renorm,
-                      int groups, int keep, int* ids, float* weights, float* shared_gate, int* table, int unit, int per_item, int cap,
-                      int* sorted_token, int* pair_slot, int* tile_expert, int* n_tiles, int T, int H, hipStream_t st,
-                      const float* correction, int n_real, float wscale) {
-  if (topk < 1 || topk > 64 || topk > E || E > 8192) return TQ_ERR_UNSUPPORTED;
-  const int rows = E + (shared_w ? 1 : 0), n_pairs = T * topk;
-  if (unit < 1 || cap % unit != 0 || cap < n_pairs + (E < n_pairs ? E : n_pairs) * (unit - 1)) return TQ_ERR_BAD_ARG;
+// Whether the choice and the order go in two launches by many workgroups, and how: tg tokens to a workgroup of route_choose, V of those, per
+// of its segments to a workgroup of route_place.  What the launches saved and the order by many workgroups gain must be more than every
+// workgroup's own way through all rows of wr and the table of V counts per expert costs (us apart and this way; of 800 sizes drawn the way taken is
+// more than 4 % slower than the other form in 8, and 1.19 times as fast in the geometric mean):
+//  * rows of up to 5,120, of which router_logits has 8 tokens to a workgroup too:
+//    - 8 experts and more, fewer leaving most waves without rows (929 tokens, 5 of 4,096, one a token 13.0 and 16.6; 12,630, 3 of 2,560, two 55 and
+//      67), and up to 8 for every pair of a workgroup's, the table's way (1,145, 160 of 5,120, one 61 and 84; 1,210, 384 of 2,560, one 63 and 86; 512, 120
+//      of 3,584, four 24.5 and 27.8; 1,024, 128 of 1,024, one 16.4 and 19.1; but 1,500, 120 of 3,072, four 54 and 39), 6 with rows beyond 4,608 (512,
+//      96 of 5,120, four 28.5 and 29.3);
+//    - pairs whose order takes one workgroup some time (1,181, 8 of 3,072, two 15.0 and 16.5, 671, 17 of 1,000, one 10.6 and 11.5; 1,500, 8 of
+//      3,072, four 27.3 and 18.0, 906, 16 of 1,536, eight 21.9 and 14.1), or 16 experts of rows beyond 2,560, of which router_logits has a workgroup to
+//      a unit (868, 32 of 3,072, two 24.1 and 14.0);
+//    - not beyond 4,608 from 3,072 tokens on (5,120: 3,000 tokens of 16 experts 50 and 43, 4,096 52 and 53; of 8 44 and 49, of 32 64 and 74), 1,025 beyond
+//      128 experts (1,341 of 160, eight 81 and 95), nor between
+//      2,048 and 2,560 from 7,169 on (6,743 of 24, two 46 and 43; 13,980 of 16, four 70 and 77), which have half as many tokens to a workgroup here as
+//      there; nor with more than 192 experts just beyond 1,024 tokens, which leave half the units idle (1,115, 256 of 2,048, six 53 and 56; 1,220, 384
+//      of 3,072, six 95 and 100; 1,429, 359 of 2,560, six 89 and 79);
+//  * longer rows, of which router_logits has few tokens to a workgroup, from 10 experts on, 16 where there are fewer than 4 here (1,024, 249 of 6,144,
+//    four 196 and 86; 859, 10 of 8,192, six 35 and 23; 512, 33 of 10,240, one 34 and 26; but 1,280, 8 of 10,240, eight 40 and 46);
+//  * 512 tokens (1,024 beyond 128 experts): fewer leave compute units idle, over which the other form deals the rows of wr (60 experts, 200 tokens
+//    12.8 and 14.7, 400 15.7 and 15.6; 256, 401 35.5 and 41.0, 700 44.6 and 45.2, 1,024 48.9 and 46.3); a table of up to 65,536 counts (256 experts,
+//    2,048 tokens, 65,536 counts, 78 and 63, 3,001 tokens, 96,256, 108 and 111, 8,192, 262,144, 191 and 224).
+struct RouteMany {
+  int tg, V, per;
+  size_t lds;
+};
+static bool route_many_suits(int T, int E, int rows, int topk, int H, RouteMany* r) {
+  if (T < (E <= 128 ? 512 : 1024)) return false;
   const size_t hp = ((size_t)H + 511) / 512 * 512;
   auto lds = [&](int tg) { return (tg * (hp + rows + E + topk) + E) * 4; };
   // So few tokens to a workgroup that there is one to a compute unit while they last, and where there are more, that two share one.
   int tg = T <= 512 ? 2 : T <= 1024 ? 4 : 8;
   while (tg > 1 && lds(tg) > (T > 2048 ? 80 : 160) * 1024) tg /= 2;
   const int V = (T + tg - 1) / tg;
-  if (lds(tg) > 160 * 1024 || (int64_t)V * E > 65536) return ROUTE_OTHERWISE;
-  // (the callers' 512 tokens, 1,024 beyond 128 experts, leave at most 508 experts then, and route_place 42,672 bytes of LDS)
-  const int even = (V + 63) / 64, per = even < 16 ? 16 : even;
+  if (lds(tg) > 160 * 1024 || (int64_t)V * E > 65536) return false;
+  if (hp <= 5120) {
+    const bool tall = hp > 4608;
+    if (E < 8 || E > (tall ? 6 : 8) * tg * topk || (E > 192 && T > 1024 && T < 1408)) return false;
+    if ((int64_t)T * topk < (E < 10 ? 2560 : 2048) && (hp <= 2560 || E < 16)) return false;
+    if (tall ? T >= (E > 128 ? 1025 : 3072) : hp > 2048 && hp <= 2560 && T > 7168) return false;
+  } else if (E < (tg < 4 ? 16 : 10)) {
+    return false;
+  }
+  const int even = (V + 63) / 64;
+  *r = {tg, V, even < 16 ? 16 : even, lds(tg)};
+  return true;
+}
+TQ_API int tq_route_in_two(int T, int E, int shared, int topk, int H) {
+  RouteMany r;
+  return E > 0 && topk > 0 && H > 0 && route_many_suits(T, E, E + (shared ? 1 : 0), topk, H, &r);
+}
+// table: T * E ints.
+static int route_many(const RouteMany& r, const float* x, const void* wr, const void* shared_w, const float* bias, int wtype, int E, int topk,
+                      int renorm, int groups, int keep, int* ids, float* weights, float* shared_gate, int* table, int unit, int per_item, int cap,
+                      int* sorted_token, int* pair_slot, int* tile_expert, int* n_tiles, int T, int H, hipStream_t st,
+                      const float* correction, int n_real, float wscale) {
+  if (topk < 1 || topk > 64 || topk > E || E > 8192) return TQ_ERR_UNSUPPORTED;
+  const int rows = E + (shared_w ? 1 : 0), n_pairs = T * topk, tg = r.tg, V = r.V, per = r.per;
+  if (unit < 1 || cap % unit != 0 || cap < n_pairs + (E < n_pairs ? E : n_pairs) * (unit - 1)) return TQ_ERR_BAD_ARG;
+  const size_t shmem = r.lds;
+  // (V E <= 65,536 and T / V <= 8 leave at most 508 experts, and route_place 42,672 bytes of LDS)
   const size_t lds_place = ((size_t)(2 * (RP / E) + 1 + per) * E) * sizeof(int);
-  const size_t shmem = lds(tg);
 #define TQ_CHOOSE(TGV)                                                                                                                    \
   do {                                                                                                                                    \
     if (shmem > 48 * 1024)                                                                                                                \
@@ -1111,8 +1150,8 @@ static int route_many(const float* x, const void* wr, const void* shared_w, cons
   return 0;
 }
 
-// tq_router_topk followed by tq_moe_align; up to 16 tokens take two kernels instead of three, and from 8,192 pairs on
-// several workgroups order the pairs (the same order).  logits: scratch of T * (E + 1) floats (T * E without a shared
+// tq_router_topk followed by tq_moe_align, with the same results: up to 16 tokens in two launches, many as route_many_suits says in two others,
+// else in three, or five where several workgroups order the pairs (from 8,192 on).  logits: scratch of T * (E + 1) floats (T * E without a shared
 // gate vector); what it holds afterwards means nothing.
 // groups, keep: the choice within the best `keep` of `groups` groups of experts (1, 1: among all).
 static int route_impl(const float* x, const void* wr, const void* shared_w, const float* bias, int wtype, int E,
@@ -1124,14 +1163,10 @@ static int route_impl(const float* x, const void* wr, const void* shared_w, cons
   if (!groups_ok(E, topk, groups, keep)) return TQ_ERR_BAD_ARG;
   const size_t shmem = ((size_t)(AW + 1) * E + (size_t)AW * topk + (size_t)AW * E) * 4;
   if (T > AW || shmem > 64 * 1024) {
-    // Fewer tokens: the rows of wr dealt over more workgroups than there are tokens gain more than a launch costs (us apart and in
-    // two launches: 60 experts, 200 tokens 12.8 and 14.7, 400 15.7 and 15.6, 512 16.1 and 15.7; 80, 400 16.5 and 17.7, 513 20.8 and 18.4;
-    // 256, 401 35.5 and 41.0, 700 44.6 and 45.2, 1,024 48.9 and 46.3).
-    if (T >= (E <= 128 ? 512 : 1024)) {
-      const int rc = route_many(x, wr, shared_w, bias, wtype, E, topk, renorm, groups, keep, ids, weights, shared_gate, (int*)logits, unit, per_item,
-                                cap, sorted_token, pair_slot, tile_expert, n_tiles, T, H, st, correction, n_real, wscale);
-      if (rc != ROUTE_OTHERWISE) return rc;
-    }
+    RouteMany r;
+    if (route_many_suits(T, E, E + (shared_w ? 1 : 0), topk, H, &r))
+      return route_many(r, x, wr, shared_w, bias, wtype, E, topk, renorm, groups, keep, ids, weights, shared_gate, (int*)logits, unit, per_item, cap,
+                        sorted_token, pair_slot, tile_expert, n_tiles, T, H, st, correction, n_real, wscale);
     const int rc = router_topk_impl(x, wr, shared_w, bias, wtype, E, topk, renorm, groups, keep, ids, weights,
                                     shared_gate, logits, T, H, st, correction, n_real, wscale);
     if (rc) return rc;

@@ -189,6 +189,7 @@ int tq_router_topk(const float* x, const void* wr, const void* shared_w, int wty
         int* ids, float* weights, float* shared_gate, float* logits, int T, int H, hipStream_t st);
 int tq_moe_align(const int* ids, int n_pairs, int E, int topk, int unit, int cap, int* sorted_token,
         int* pair_slot, int* tile_expert, int* n_tiles, hipStream_t st);
+int tq_route_in_two(int T, int E, int shared, int topk, int H);
 int tq_route(const float* x, const void* wr, const void* shared_w, int wtype, int E, int topk, int renorm,
         int* ids, float* weights, float* shared_gate, float* logits, int unit, int cap, int* sorted_token,
         int* pair_slot, int* tile_expert, int* n_tiles, int T, int H, hipStream_t st);
