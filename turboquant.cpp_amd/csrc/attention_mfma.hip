@@ -144,7 +144,7 @@ __device__ __forceinline__ float group_sum(float v) {
 }
 
 
-// Where the workgroup's tiles lie in LDS when the head size is 64, 128 or 256 (rows of 8, 16 or 32 chunks of 16
+// Where the workgroup's tiles lie in LDS when the head size is 64, 128, 192, 256 or 512 (rows of 8 to 64 chunks of 16
 // bytes, no padding): chunk ch of key row `row` at chunk ch ^ g(row), where g numbers the 16 rows that one
 // operand read touches (rows r % 4 + 8 (r / 4) + const) 0..15, or 0..7 twice for rows of 8 chunks; chunk ch of value
 // row d (64 positions, 8 chunks) at chunk ch ^ (d & 7).  Measured: such reads run at about 210 bytes per clock
@@ -352,7 +352,8 @@ __device__ __forceinline__ void tile_step(f32x4 (&o)[QG][VD], float (&m_run)[QG]
 // tile_step for a tile in LDS laid out by k_swz, v_swz (EXACT sizes): the same products in the same order.  The compiler asks for
 // two or three operands at a time and waits; here a tile's keys are all asked for before the first product and half of its values
 // before the softmax, which is worth 64 registers where a wave has one group of 16 columns or short heads (READS_AHEAD below): 3,001
-// tokens of 16 heads of 64 47 -> 43 us, of 128 with a distance bias 120 -> 105, with sigmoid weights 102 -> 88.
+// tokens of 16 heads of 64 44.0 -> 41.5 us, with a distance bias 86 -> 83, of 128 64.5 -> 62.8, with a distance bias 109 -> 104, with sigmoid
+// weights 90 -> 87.
 template <int DT, int QG, bool MOD, int VD, bool DIFF>
 __device__ __forceinline__ void lds_tile_step(f32x4 (&o)[QG][VD], float (&m_run)[QG], float (&l_run)[QG],
                                               const bf16x8 (&qf)[QG][(DT + 1) / 2], const bf16_t* kt, const bf16_t* vt, int pos0,
@@ -520,7 +521,7 @@ __device__ __forceinline__ void load_query(bf16x8 (&qf)[(DT + 1) / 2], const bf1
 // QG groups of 16.  The cache already holds the step's keys and values.  Blocks are numbered from the end of the
 // sequences: a block attends to everything before it, so the longest ones start first and the short ones fill
 // the gaps that they leave.  The workgroup brings each tile of keys and values into one of two LDS buffers
-// (swizzled for head sizes 64, 128, 256; else key rows padded by KPAD and value rows VSTR long) while it works on
+// (swizzled for head sizes 64, 128, 192, 256 and 512; else key rows padded by KPAD and value rows VSTR long) while it works on
 // the other, and the tile after that is on its way from memory into registers meanwhile: one barrier per tile.
 #define KPAD 8
 #define VSTR 72
@@ -534,12 +535,14 @@ __device__ __forceinline__ void load_query(bf16x8 (&qf)[(DT + 1) / 2], const bf1
 // VD < DT: the values' first 16 VD dimensions alone are summed and written (zeros behind them up to hd): an attention
 // whose keys are wider than its values, laid out at the keys' width.
 // DIFF: two maps a head, a token's two columns in two groups of one lane; they are made one where the output is normalised.
-// Waves to a SIMD: two, said as a maximum too, so that the compiler plans with the 256 registers that a wave has then anyway (heads
-// of 256, 2,048 tokens of 8: 147 -> 80 us, whose sums went to scratch memory; the numbers of a wave in scalar registers have a part in
-// it).  Short heads gain by more waves, and so do values narrower than keys behind a window (3,001 tokens of 16 heads of 192, values of
-// 128: 52 us behind 1,024 positions, 58 with the maximum, though 104 and 82 without a window); sizes known at run time stay without one.
+// Waves to a SIMD: two (one for heads beyond 256), said as a maximum too, so that the compiler plans with the registers that a wave has then
+// anyway.  us without it, with it, with a wave's number in a scalar register alone, with both: heads of 256, 2,048 tokens of 8, whose sums went to
+// scratch memory, 137, 94, 80 and 79; a distance bias, 3,001 tokens of 16, heads of 64 93, 89, 94 and 86, of 128 120, 110, 114 and 109.  Heads of
+// 512, two prompts of 2,500 tokens of 16: 2,337 -> 2,059, 1,024 tokens 224 -> 202, with a distance bias 2,033 -> 1,859 (1,762 without the maximum).
+// Short heads gain by more waves, and so do values narrower than keys behind a short window (3,001 tokens of 16 heads of 192, values of 128: 52 us
+// behind 1,024 positions, 58 with the maximum, though 98 and 77 without a window); sizes known at run time stay without a maximum.
 template <int DT, int QG, bool EXACT, bool MOD, int VD = DT, bool DIFF = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF ? 8 : 16) ? 1 : 2, DT > (DIFF ? 8 : 16) ? 1 : !EXACT || VD < DT ? 8 : DT > 4 ? 2 : 4))) void attn_prefill_kernel(AttnArgs a, int n_blocks, int B, DiffArgs df) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF ? 8 : 16) ? 1 : 2, !EXACT || VD < DT ? 8 : DT > (DIFF ? 8 : 16) ? 1 : DT > 4 ? 2 : 4))) void attn_prefill_kernel(AttnArgs a, int n_blocks, int B, DiffArgs df) {
   constexpr bool ONEBUF = DT > ATTN_TWO_BUFFERS_UP_TO, READS_AHEAD = EXACT && DT * QG <= 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   static_assert(!DIFF || (QG % 2 == 0 && !MOD && VD == DT), "two maps a head: in pairs of groups, with plain scores");
@@ -557,7 +560,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DT > (DIFF 
   const int blk = n_blocks - 1 - (int)blockIdx.x / per_block;
   const int h = (int)blockIdx.x % per_block % a.nh, seq = (int)blockIdx.x % per_block / a.nh;
   const int tid = threadIdx.x, lane = tid % 64, r = lane % 16, c = lane / 16;
-  // (a number in a scalar register, except where hd is known at run time only: the compiler's code for heads between 256 and 512 gave NaN then)
+  // (In a scalar register, except where hd is known at run time only.  For heads between 256 and 512 that, together with the factor of softmax_tile
+  // without conditions, gave NaN: a query's 16 bytes lay half in accumulation registers and half in scratch memory then, and where the compiler
+  // brought them back into accumulation registers it left one of the four out.  Nothing built here has a value in both.)
   const int wave = EXACT ? __builtin_amdgcn_readfirstlane(tid / 64) : tid / 64;
   const int t0 = a.cu_seqlens[seq], n = a.cu_seqlens[seq + 1] - t0;
   const int qb = blk * 4 * QW;
