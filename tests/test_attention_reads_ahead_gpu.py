@@ -14,8 +14,9 @@ DEV = "cuda:0"
 PAGE = 64
 
 
-def paged(lens, old, nkv, hd, seed, gone=None):
-    """Caches of ``old[i] + lens[i]`` positions; pages before position ``gone[i]`` hold NaN.  Keys and values [n, nkv, hd] too."""
+def paged(lens, old, nkv, hd, seed, gone=None, width=None):
+    """Caches of ``old[i] + lens[i]`` positions; pages before position ``gone[i]`` hold NaN; values are zeros from ``width`` on.  Keys and values
+    [n, nkv, hd] too."""
     g = torch.Generator(DEV).manual_seed(seed)
     ends = [a + b for a, b in zip(lens, old)]
     pages = [-(-e // PAGE) for e in ends]
@@ -26,6 +27,7 @@ def paged(lens, old, nkv, hd, seed, gone=None):
     ks, vs, at = [], [], 0
     for i, (e, n) in enumerate(zip(ends, pages)):
         k, v = (torch.randn(n * PAGE, nkv, hd, generator=g, device=DEV).bfloat16() for _ in range(2))
+        v[..., width or hd:] = 0
         ids = order[at:at + n]
         at += n
         first = gone[i] // PAGE if gone else 0
@@ -67,12 +69,16 @@ def visible(n, old, window, keep, chunk):
     ([230], [700], {"window": 130, "keep": 5, "sigmoid": 1}), ([300], [0], {"sigmoid": 1, "gate": 1}), ([400], [0], {"bias": 1}),
     ([200], [100], {"chunk": 192, "bias": 1, "sink": 1}), ([385], [0], {"gate": 1})])
 def test_prompts_against_64_bits(hd, lens, old, mod):
-    nh, nkv = 4, 2
+    check_prompts(hd, lens, old, mod)
+
+
+def check_prompts(hd, lens, old, mod, nh=4):
+    nkv = 2
     window, keep, chunk = mod.get("window"), mod.get("keep", 0), mod.get("chunk")
     gone = None
     if (window or chunk) and not keep:
         gone = [max(o - window + 1, 0) if window else o // chunk * chunk for o in old]
-    kp, vp, table, ks, vs, q, runs, positions, seq = paged(lens, old, nkv, hd, sum(lens) + hd, gone)
+    kp, vp, table, ks, vs, q, runs, positions, seq = paged(lens, old, nkv, hd, sum(lens) + hd, gone, mod.get("values"))
     g = torch.Generator(DEV).manual_seed(1)
     tokens = sum(lens)
     q = torch.randn(tokens, nh, hd, generator=g, device=DEV).bfloat16()
@@ -90,6 +96,9 @@ def test_prompts_against_64_bits(hd, lens, old, mod):
         more["head_gate"] = f32(tokens, nh)
     if "window" in mod or "keep" in mod:
         more["keep_first"] = keep
+    if "values" in mod:
+        more["value_width"] = mod["values"]
+    width = mod.get("values", hd)
     scale = 1.7 * hd ** -0.5
     got = ops.attention(q.reshape(tokens, nh * hd), kp, vp, 0, positions, seq, table, PAGE, nkv * PAGE * hd, nh, nkv, hd, window, scale,
                         "bfloat16", runs=runs, chunk=chunk, **more).double().view(tokens, nh, hd)
@@ -97,7 +106,7 @@ def test_prompts_against_64_bits(hd, lens, old, mod):
     for i, (n, o) in enumerate(zip(lens, old)):
         see, dist = visible(n, o, window, keep, chunk)
         for h in range(nh):
-            s = scale * q[at:at + n, h].double() @ ks[i][:, h // 2].T
+            s = scale * q[at:at + n, h].double() @ ks[i][:, h // (nh // nkv)].T
             if "cap" in mod:
                 s = mod["cap"] * torch.tanh(s / mod["cap"])
             if "bias" in mod:
@@ -112,15 +121,20 @@ def test_prompts_against_64_bits(hd, lens, old, mod):
                 p = torch.softmax(s, 1)[:, :o + n]
             if "gate" in mod:
                 p = p * torch.sigmoid(more["head_gate"][at:at + n, h].double())[:, None]
-            v = vs[i][:, h // 2]
+            v = vs[i][:, h // (nh // nkv), :width]
             want, bound = p @ v, (2 ** -7 + 2 ** -12) * (p @ v.abs())
-            assert ((got[at:at + n, h] - want).abs() <= bound).all(), (i, h)
+            assert ((got[at:at + n, h, :width] - want).abs() <= bound).all(), (i, h)
+            assert not got[at:at + n, h, width:].any()
         at += n
 
 
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("lens,old", [([193], [0]), ([193, 64, 1], [0] * 3), ([700], [0]), ([200], [130])])
 def test_two_maps_a_head(hd, lens, old):
+    check_two_maps(hd, lens, old)
+
+
+def check_two_maps(hd, lens, old):
     nh, nkv, lam, eps, post = 4, 2, 0.4, 1e-5, 0.6
     kp, vp, table, ks, vs, q, runs, positions, seq = paged(lens, old, nkv, hd, 7 + sum(lens) + hd)
     g = torch.Generator(DEV).manual_seed(2)
