@@ -334,7 +334,7 @@ __global__ __launch_bounds__(512, 4) void delta_chunk_prep_kernel(const float* _
 // wave w keeps the rows of the state in key tiles w, w + 4, ... as accumulators, which are the operands of the products with the state as
 // they stand (the key channels of a product are taken in the order 0, 4, 8, 12, 1, 5, ...).  Each wave's share of u passes
 // through LDS, one barrier a chunk; its share of o, to which waves 0, 1 and 2 add one of b's three tiles each once u is known,
-// goes along with the next chunk's u.  The next two chunks' operands are on their way meanwhile.  The blocks of a head lie H apart, so
+// goes along with the next chunk's u.  In the loop the next two chunks' operands are on their way meanwhile.  The blocks of a head lie H apart, so
 // that they run on one die (H a multiple of 8) and share what they read in its L2.
 // A chunk is a chain: 8 NB products with the state, the exchange, in whose time 8 NB more are formed for o, and 8 NB into the state, 1.5 us of
 // which 0.64 are the products'.  2,048 tokens of 16 heads of 128 x 128, us: 97; 119 before with a wait for all loads on their way every two
@@ -499,6 +499,10 @@ __global__ __launch_bounds__(256, NB < 4 ? 2 : 1) void delta_chunk_scan_kernel(c
   };
   // Pairs behind the first chunk or the first two, so that the loop holds nothing but whole pairs: with a single chunk behind them the
   // compiler made one body of both, and waited at its head for all loads on their way to move what they bring to other registers.
+  // Those first chunks ask for their operands as they begin, and the loop asks again for what the last of them asked for.  Tried instead: the first
+  // two on their way together, and the loop beginning with what is on its way already; the body is longer then, and slower (both launches, us with
+  // one body, so tried and as it is: 64 tokens of 16 heads of 128 x 128 26.1, 25.6 and 25.0, 128 29.6, 28.6 and 28.2, 256 36.8, 34.8 and 34.1, 2,048
+  // 164, 147 and 144, 3,001 236, 210 and 206; 64 tokens of 8 of 256 x 128 38.3, 35.5 and 34.6).
   Operands even, odd;
   fetch(even, 0);
   one_chunk(0, even, true);
