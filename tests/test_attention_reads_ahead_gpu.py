@@ -164,3 +164,19 @@ def check_two_maps(hd, lens, old):
             bound = z * f * (slack + r.abs() * (slack * slack).mean(1, keepdim=True).sqrt() * f / post) + 2 ** -8 * want.abs()
             assert ((got[at:at + n, h] - want).abs() <= 1.1 * bound).all(), (i, h)
         at += n
+
+
+@pytest.mark.parametrize("hd", [64, 128, 96, 256])
+def test_scores_and_sinks_of_minus_infinity(hd):
+    """A sink of -inf counts nothing where a key has a finite score; where none has, the sums stay what they began as: 0 over 1."""
+    nh, nkv, n = 2, 2, 200
+    kp, vp, table, ks, vs, q, runs, positions, seq = paged([n], [0], nkv, hd, hd)
+    q = torch.rand(n, nh * hd, generator=torch.Generator(DEV).manual_seed(1), device=DEV).add(0.5).bfloat16()
+    kp[table[0].long(), 0, :, 3] = -torch.inf      # the first head's scores are -inf, the second's finite
+    sink = torch.full((nh,), -torch.inf, device=DEV)
+    got = ops.attention(q, kp, vp, 0, positions, seq, table, PAGE, nkv * PAGE * hd, nh, nkv, hd, None, hd ** -0.5, "bfloat16", runs=runs, sink=sink)
+    got = got.double().view(n, nh, hd)
+    assert not got[:, 0].any()
+    see, _ = visible(n, 0, None, 0, None)
+    p = torch.softmax((hd ** -0.5 * q.view(n, nh, hd)[:, 1].double() @ ks[0][:, 1].T).masked_fill(~see, -torch.inf), 1)
+    assert ((got[:, 1] - p @ vs[0][:, 1]).abs() <= (2 ** -7 + 2 ** -12) * (p @ vs[0][:, 1].abs())).all()

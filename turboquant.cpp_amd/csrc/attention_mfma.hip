@@ -223,8 +223,7 @@ __device__ __forceinline__ void softmax_tile(f32x4 (&s)[QG][4], f32x4 (&o)[QG][D
     const float m_new = fmaxf(m_run[g], m_tile);
     const bool any = m_new != -INFINITY;
     const float m_use = any ? m_new : 0.f;       // 2^(-inf - 0) = 0 for masked keys, also when all are masked
-    // (FLAT: 0 where no key was visible yet, whose sums are 0)
-    const float alpha = FLAT ? __builtin_amdgcn_exp2f(m_run[g] - m_use)
+    const float alpha = FLAT ? __builtin_amdgcn_exp2f(any ? m_run[g] - m_new : 0.f)
                              : any && m_run[g] != -INFINITY ? __builtin_amdgcn_exp2f(m_run[g] - m_new) : (any ? 0.f : 1.f);
     float l_tile = 0.f;
 #pragma unroll
