@@ -25,7 +25,8 @@
 // Tokens from which a run goes in chunks: a chunk costs the same whatever it holds, and the two launches 20 us before the first.
 // Chunks and token by token, us, 16 heads of 128 x 128: one sequence of 32 tokens 24 and 23, of 48 25 and 30, of 96 27 and 51, of
 // 1,024 90 and 475; 64 sequences of 32 tokens 195 and 212, of 48 295 and 288, of 64 302 and 364, of 256 970 and 1,291.  Heads of
-// 256 x 256, whose scan spills 196 bytes a lane: 38 and 42 for one of 48 tokens, 1,107 and 1,266 for 64 of them.  Narrow heads in a
+// 256 x 256, whose scan kept 196 bytes a lane in scratch memory then: 38 and 42 for one of 48 tokens, 1,107 and 1,266 for 64 of them (without
+// any, as now, both launches of 2,048 tokens of 8 heads of 256 x 128 take 222 us instead of 325).  Narrow heads in a
 // crowded step, where a chunk's pairs weigh more than the state, are the exception: 64 sequences of 64 tokens and 32 heads of 64 x 64
 // 225 and 215, 16 heads of 128 x 16 135 and 107, while one sequence of 256 tokens of these takes 27 and 127, 38 and 137.
 #define DC_FROM 48
